@@ -41,6 +41,7 @@
 #include <vector>
 
 #include "diso_hip.h"
+#include "diso_bits.h"
 #include "diso_scan_word.h"
 #include "diso_tables.h"
 
@@ -64,6 +65,7 @@ struct Geo {
     int off;         // stored sample (i,j,k) sits at conceptual (i+off, j+off, k+off)
     int nchunk;      // ceil(g2 / 64)
     int64_t nseg;    // g0 * g1 * nchunk
+    double rchunk, rg1;  // 1 / nchunk, 1 / g1 (seg_pos)
 };
 
 template <typename S>
@@ -147,111 +149,6 @@ __device__ __forceinline__ S interp_t(S d0, S d1, S iso) {
     return (d1 != d0) ? clamp01<S>((iso - d0) / (d1 - d0)) : S(0.5);  // src/cumc.cu:356
 }
 
-// The eight corner samples of the cell anchored at (x,y,z): c[dx][dy][dz].
-template <typename S>
-struct Corners {
-    S c[2][2][2];
-};
-
-template <typename S>
-__device__ __forceinline__ Corners<S> load_corners(const In<S> &in, int x, int y, int z) {
-    Corners<S> k;
-#pragma unroll
-    for (int dx = 0; dx < 2; ++dx)
-#pragma unroll
-        for (int dy = 0; dy < 2; ++dy)
-#pragma unroll
-            for (int dz = 0; dz < 2; ++dz) k.c[dx][dy][dz] = sample(in, x + dx, y + dy, z + dz);
-    return k;
-}
-
-// MC cube code, Bourke corner order (src/cumc.cu:107,455-472).
-template <typename S>
-__device__ __forceinline__ int mc_code(const Corners<S> &k, S iso) {
-    int code = 0;
-    code |= (k.c[0][0][0] >= iso) << 0;
-    code |= (k.c[1][0][0] >= iso) << 1;
-    code |= (k.c[1][1][0] >= iso) << 2;
-    code |= (k.c[0][1][0] >= iso) << 3;
-    code |= (k.c[0][0][1] >= iso) << 4;
-    code |= (k.c[1][0][1] >= iso) << 5;
-    code |= (k.c[1][1][1] >= iso) << 6;
-    code |= (k.c[0][1][1] >= iso) << 7;
-    return code;
-}
-
-// DMC cube code, Morton corner order (src/cudualmc.cu:95-104,796-813).
-template <typename S>
-__device__ __forceinline__ int dmc_code(const Corners<S> &k, S iso) {
-    int code = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) code |= (k.c[i & 1][(i >> 1) & 1][(i >> 2) & 1] >= iso) << i;
-    return code;
-}
-
-// getGoodCellCode (src/cudualmc.cu:815-839): an ambiguous case is inverted when its face
-// neighbour in the tabulated direction exists and is ambiguous too. `cases` is the DMC case table.
-template <typename S>
-__device__ __forceinline__ int dmc_good_code(const In<S> &in, const uint64_t *cases, int code, int x,
-                                             int y, int z) {
-    const int dir = DISO_DMC_DIR(cases[code]);
-    if (dir != 7) {
-        // neighbour along axis comp, +1 or -1; selected arithmetically (no indexed arrays, so the
-        // grid parameters can stay in registers)
-        const int comp = dir >> 1, step = (dir & 1) ? 1 : -1;
-        const int on0 = comp == 0, on1 = comp == 1, on2 = comp == 2;
-        const int nx = x + on0 * step, ny = y + on1 * step, nz = z + on2 * step;
-        const int c = on0 * nx + on1 * ny + on2 * nz;
-        const int lim = on0 * in.geo.g0 + on1 * in.geo.g1 + on2 * in.geo.g2;
-        if (c >= 0 && c < lim - 1) {
-            const int ncode = dmc_code(load_corners(in, nx, ny, nz), in.iso);
-            if (DISO_DMC_DIR(cases[ncode]) != 7) code ^= 0xff;
-        }
-    }
-    return code;
-}
-
-// dmc_good_code for a cell whose eight corners are all stored samples (`own` = index of corner
-// (0,0,0)): the face neighbour shares four corners with the cell, whose bits come from `code`
-// (Morton order: bit (dx | dy << 1 | dz << 2)); only its far face, the plane two steps past the
-// cell (step +1) or one step before it (step -1), is read, at the cell's index plus strides.
-template <typename S>
-__device__ __forceinline__ int dmc_good_code_stored(const In<S> &in, const uint64_t *cases, int code, int x, int y,
-                                                    int z, int64_t own) {
-    const int dir = DISO_DMC_DIR(cases[code]);
-    if (dir == 7) return code;
-    const Geo &g = in.geo;
-    const int comp = dir >> 1, plus = dir & 1;
-    const int c = comp == 0 ? x : (comp == 1 ? y : z);
-    const int lim = comp == 0 ? g.g0 : (comp == 1 ? g.g1 : g.g2);
-    const int nc = plus ? c + 1 : c - 1;  // the neighbour's anchor along comp
-    if (nc < 0 || nc >= lim - 1) return code;
-    const int64_t sz = 1, sy = g.n2, sx = (int64_t)g.n1 * g.n2;
-    // strides of comp and of the face's two other axes a < b
-    const int64_t sc = comp == 0 ? sx : (comp == 1 ? sy : sz);
-    const int64_t sa = comp == 0 ? sy : sx, sb = comp == 2 ? sy : sz;
-    const int a = comp == 0 ? 1 : 0, b = comp == 2 ? 1 : 2;
-    // far plane: conceptual c + 2 (step +1) or c - 1 (step -1); outside the stored grid it is pad
-    const int fc = plus ? c + 2 : c - 1;
-    const int nfc = comp == 0 ? g.n0 : (comp == 1 ? g.n1 : g.n2);
-    const bool stored = (unsigned)(fc - g.off) < (unsigned)nfc;
-    const int64_t f0 = own + (plus ? 2 * sc : -sc);
-    const int wc = 1 << comp;  // bit weight of comp in the corner index
-    constexpr int kLow[3] = {0x55, 0x33, 0x0f};  // corners with offset 0 along x, y, z
-    const int low = comp == 0 ? kLow[0] : (comp == 1 ? kLow[1] : kLow[2]);
-    // shared face: the neighbour's offset-0 corners are the cell's offset-1 ones (step +1), or its
-    // offset-1 corners the cell's offset-0 ones (step -1)
-    int ncode = plus ? ((code >> wc) & low) : ((code << wc) & ~low & 0xff);
-    const int fbit = plus ? wc : 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int ja = j & 1, jb = j >> 1;
-        const S v = stored ? in.sdf[f0 + ja * sa + jb * sb] : in.pad;
-        ncode |= (int)(v >= in.iso) << (fbit | (ja << a) | (jb << b));
-    }
-    return DISO_DMC_DIR(cases[ncode]) != 7 ? code ^ 0xff : code;
-}
-
 __device__ __forceinline__ int popc3(int m) { return (m & 1) + ((m >> 1) & 1) + ((m >> 2) & 1); }
 
 // ------------------------------------------------------------------------------------------
@@ -312,31 +209,66 @@ struct SegBase {
 // additions, not products.
 __device__ __forceinline__ int64_t xstride(const Geo &g) { return (int64_t)g.g1 * g.nchunk; }
 
-// Position classification word, written by the count pass for every lane of every segment
-// (segment-major: word s * 64 + lane), read by the later passes instead of re-deriving it from
-// the samples: bits 0-7 the code of the cell anchored at the position (MC: Bourke corner order;
-// DMC: Morton corner order after the face-neighbour rule), bits 8-10 the crossing mask of the
-// three edges the position owns (+x, +y, +z), bit 11 whether its own sample is >= iso, bits 12-14
-// the cell's face count (MC: triangles, 0..5; DMC: patches, 0..4). Bits 0-10 and 12-14 are 0
-// where no cell is anchored.
-__device__ __forceinline__ int info_code(uint32_t w) { return (int)(w & 0xffu); }
-__device__ __forceinline__ int info_mask(uint32_t w) { return (int)((w >> 8) & 7u); }
-__device__ __forceinline__ int info_inside(uint32_t w) { return (int)((w >> 11) & 1u); }
-__device__ __forceinline__ int info_count(uint32_t w) { return (int)((w >> 12) & 7u); }
+// Classification of a grid's positions, one bit per position of a segment in 64-bit planes (bit l =
+// lane l), written by the count pass after the segment bases and read by the later passes instead
+// of the samples:
+//   inside  the position's own sample is >= iso (pad samples included);
+//   X, Y, Z the edge owned along that axis crosses the surface;
+//   A       the cell anchored here is cut by the surface (active);
+//   m0, m1  DMC: the cell's patch count minus one, in binary (0 unless active);
+//   codes   per position, the code of the active cell anchored there (MC: Bourke corner order; DMC:
+//           Morton corner order after the face-neighbour rule). Written only in segments that hold
+//           an active cell, and only meaningful at active positions.
+// Where no cell is anchored, X, Y, Z and A are 0.
+//
+// The active cells, in the grid's linear order, are dealt to the emission's waves in units of 64:
+//   abase   active cells before the segment's first position, modulo 2^16;
+//   unit    unit u's first cell (number 64 u) lies in segment unit[u];
+//   nunits  the number of units (only where a grid can hold a cell: at least four segments).
+struct Plane2 {
+    uint64_t a, b;
+};
 
-__device__ __forceinline__ const uint16_t *info_of(const SegBase *seg, const Geo &g) {
-    return reinterpret_cast<const uint16_t *>(seg + g.nseg + 2);
+struct Planes {
+    Plane2 *xy, *za, *m;  // (X, Y), (Z, A), (m0, m1; DMC only), one entry per segment
+    uint8_t *codes;       // 64 per segment
+    uint64_t *inside;
+    uint32_t *unit;
+    uint32_t *nunits;
+    uint8_t *flags;       // DISO_TOTAL_* flags of the samples of a run of segments, at its first
+    uint16_t *abase;
+};
+constexpr int64_t kSegStateBytes = 128;  // per segment: 48 + 64 + 8 + 4 + 1 + 1 + 2
+
+// The planes behind the bases of `n` segments (seg[n], seg[n + 1] are the totals).
+__host__ __device__ inline Planes planes_at(void *after, int64_t n) {
+    uint8_t *b = static_cast<uint8_t *>(after);
+    Planes q;
+    q.xy = reinterpret_cast<Plane2 *>(b);
+    q.za = q.xy + n;
+    q.m = q.za + n;
+    q.codes = b + n * 48;
+    q.inside = reinterpret_cast<uint64_t *>(b + n * 112);
+    q.unit = reinterpret_cast<uint32_t *>(b + n * 120);
+    q.nunits = reinterpret_cast<uint32_t *>(b + n * 124);
+    q.flags = b + n * 125;
+    q.abase = reinterpret_cast<uint16_t *>(b + n * 126);
+    return q;
+}
+__host__ __device__ inline Planes planes_of(const SegBase *seg, int64_t nseg) {
+    return planes_at(const_cast<SegBase *>(seg + nseg + 2), nseg);
 }
 
 // A grid's segments as the emission and backward passes see them: its bases (seg[s], s from 0;
-// seg[nseg] is the base after its last segment), its classification words, and the base values
+// seg[nseg] is the base after its last segment), its classification planes, and the base values
 // of its first segment (v0, f0), which are subtracted to index its own outputs. A grid extracted
 // alone has v0 = f0 = 0; in a batch the scan runs over all grids' segments in order.
 struct SegCtx {
-    const SegBase *seg;
-    const uint16_t *info;
+    const SegBase *__restrict__ seg;
+    const Plane2 *__restrict__ xy, *__restrict__ za;
     int64_t v0, f0;
 };
+__device__ __forceinline__ SegCtx seg_ctx(const SegBase *seg, const Planes &q) { return SegCtx{seg, q.xy, q.za, 0, 0}; }
 
 // ------------------------------------------------------------------------------------------
 // Register windows and edge geometry shared by the emission and backward kernels
@@ -412,14 +344,17 @@ struct Win {
     __device__ __forceinline__ S operator()(int dx, int dy, int dz) const { return v[dx - X0][dy - Y0][dz - Z0]; }
 };
 
-// Segment of a wave: its row (px, py) and chunk, from the wave-uniform segment id.
+// A segment's row (px, py) and chunk. The quotients come from double reciprocals: (n + 1/2) / d is at
+// least 1 / (2 d) away from an integer, and for n < 2^32 the product is off by less than 2^-20 (and
+// by less than 2^-40 where d is large enough for that to matter), so its integer part is n / d.
+// Three instructions where an integer division takes about twenty.
 struct SegPos {
     int px, py, chunk;
 };
+__device__ __forceinline__ uint32_t div_rcp(uint32_t n, double r) { return (uint32_t)(((double)n + 0.5) * r); }
 __device__ __forceinline__ SegPos seg_pos(const Geo &g, int64_t s) {
-    const uint32_t su = (uint32_t)s, nc = (uint32_t)g.nchunk, g1 = (uint32_t)g.g1;
-    const uint32_t row = su / nc;
-    return SegPos{(int)(row / g1), (int)(row % g1), (int)(su % nc)};
+    const uint32_t su = (uint32_t)s, row = div_rcp(su, g.rchunk), px = div_rcp(row, g.rg1);
+    return SegPos{(int)px, (int)(row - px * (uint32_t)g.g1), (int)(su - row * (uint32_t)g.nchunk)};
 }
 
 // The position of segment lo + i, read from lane i of a lane-parallel seg_pos (i uniform).
@@ -578,14 +513,18 @@ __device__ __forceinline__ int find_group(const int64_t *__restrict__ rf, int m,
 }
 
 // ------------------------------------------------------------------------------------------
-// Pass 1: classify, count, scan (single pass)
+// Pass 1: classify, count, scan
 //
-// The grid of segments is split into G contiguous ranges, one per block (G ~ 4 blocks per CU).
-// A block counts its segments (writing each segment's counts into
-// `seg`), publishes its aggregate as one self-contained 64-bit word, reads the aggregates of all
-// its predecessors in parallel (a look-back over the whole window at once: no chain of inclusive
-// prefixes, so the wait is one memory latency rather than one per predecessor), and finally scans
-// its own segment counts into segment bases. Aggregate words are accessed with agent-scope
+// mask_kernel streams the samples once and keeps one bit per position: whether the sample is >=
+// iso. count_kernel then works on those bits, one lane per segment (diso_bits.h), and scans the
+// segment counts in the same launch.
+//
+// The scan (single pass). The segments are split into G contiguous ranges, one per block. A block
+// counts its segments (writing each segment's planes, and its counts into `seg`), publishes its
+// aggregate as one self-contained 64-bit word, reads the aggregates of all its predecessors in
+// parallel (a look-back over the whole window at once: no chain of inclusive prefixes, so the wait
+// is one memory latency rather than one per predecessor), and finally scans its own segment counts
+// into segment bases. Aggregate words are accessed with agent-scope
 // atomics only, so they are coherent across the XCDs' L2s without fences. Two word buffers
 // alternate between calls; each call clears the one the next call uses (up to the extent that
 // was written), and the last block advances the epoch once every block has published (and so has
@@ -600,66 +539,21 @@ __device__ __forceinline__ int find_group(const int64_t *__restrict__ rf, int m,
 struct CtlHeader {
     uint32_t epoch;     // calls completed on this block (diso_scan_word.h)
     uint32_t dirty[2];  // words written in each buffer since it was last cleared
-    uint32_t pad[13];
+    uint32_t nan;       // set by mask_kernel when it meets a NaN, cleared by the count's last block
+    uint32_t pad[12];
 };
 
 constexpr int kCountWaves = 8;
 constexpr int kCountBlock = kCountWaves * kWave;
-constexpr int64_t kMaxCountBlocks = 8192;
+constexpr int64_t kMaxCountBlocks = 4096;  // two words each
 constexpr int kCountBlocksPerCU = 4;
+constexpr int64_t kCountLds = 6144;  // segments of a block whose counts stay in LDS (24 KiB)
 
 __device__ __forceinline__ uint64_t ld_relaxed(const uint64_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void st_relaxed(uint64_t *p, uint64_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Per-position counts for pass 1: nv = crossing edges owned (MC vertices / DMC quads);
-// nf = MC triangles / DMC patches; fl = sample flags of the position's own sample; the position's
-// classification word.
-template <typename S>
-using CornerWin = Win<S, 0, 2, 0, 2, 0, 2>;
-
-template <typename S>
-__device__ __forceinline__ void count_position(const In<S> &in, int ALGO, const uint64_t *cases,
-                                               const CornerWin<S> &w, int *nv, int *nf, uint32_t *fl,
-                                               uint32_t *info) {
-    const int px = w.px, py = w.py, pz = w.pz;
-    const S v = w(0, 0, 0);
-    *fl = in_data(in, px, py, pz) ? ((v < in.iso ? DISO_TOTAL_HAS_BELOW : 0u) |
-                                     (v > in.iso ? DISO_TOTAL_HAS_ABOVE : 0u) | (v != v ? DISO_TOTAL_HAS_NAN : 0u))
-                                  : 0u;
-    *nv = 0;
-    *nf = 0;
-    *info = (uint32_t)(v >= in.iso) << 11;
-    if (!is_anchor(in, px, py, pz)) return;
-    const int m = own_mask(v, w(1, 0, 0), w(0, 1, 0), w(0, 0, 1), in.iso);
-    *nv = popc3(m);
-    int code;
-    if (ALGO == DISO_MC) {
-        Corners<S> k;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) k.c[i & 1][(i >> 1) & 1][(i >> 2) & 1] = w(i & 1, (i >> 1) & 1, (i >> 2) & 1);
-        code = mc_code(k, in.iso);
-        *nf = DISO_MC_NTRI(cases[code]);
-    } else {
-        code = 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) code |= (w(i & 1, (i >> 1) & 1, (i >> 2) & 1) >= in.iso) << i;
-        if (code != 0 && code != 255)
-            code = w.interior ? dmc_good_code_stored(in, cases, code, px, py, pz, data_index(in, px, py, pz))
-                              : dmc_good_code(in, cases, code, px, py, pz);
-        *nf = DISO_DMC_NPATCH(cases[code]);
-    }
-    *info |= (uint32_t)code | ((uint32_t)m << 8) | ((uint32_t)*nf << 12);
-}
-
-// Wave sums of two per-lane counts in [0, 7]: one DPP scan of both as 10-bit fields.
-__device__ __forceinline__ void wave_totals2(int a, int b, int *ta, int *tb) {
-    const uint32_t t = (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_dpp((uint32_t)a | (uint32_t)b << 10), kWave - 1);
-    *ta = (int)(t & 0x3ff);
-    *tb = (int)((t >> 10) & 0x3ff);
 }
 
 __device__ __forceinline__ int64_t wave_incl64(int64_t v) {
@@ -685,224 +579,232 @@ struct CountSrc {
     int64_t nseg;            // segments of the launch
 };
 
-// Counts segments [wlo, whi) (one wave, in order; its position advances without divisions) and
-// adds the wave's totals to (wv, wf, wfl). WRITE: also record each segment's counts (lane 0),
-// every lane's classification word and (BATCH) the grids' sample flags; without WRITE the range
-// is only summed (a block recounting a predecessor's range, see the look-back).
-// Whether count_range_tails applies to a grid: rows of at least two chunks whose last chunk holds
-// at most 32 positions (the z extent a few positions past a multiple of 64, as 256 + 2 pad
-// samples is).
-__device__ __forceinline__ bool short_tails(const Geo &g) {
-    return g.nchunk >= 2 && g.g2 - kWave * (g.nchunk - 1) <= kWave / 2;
-}
-
-// A count loop's position in one grid: the segment's row and chunk, and the offset of the stored
-// row (px - off, py - off) in samples, kept by additions as the loop advances segment by segment
-// (instead of 64-bit products per segment; meaningful only where the row is stored).
-// Whether a segment's corner window is all stored samples is kept the same way: rows (px..px+1,
-// py..py+1) stored, updated when the row changes, and the chunk within [clo, chi], the chunks
-// whose z extent z0 .. z0 + 64 is stored.
-struct CountPos {
-    SegPos sp;
-    int64_t rowoff;
-    bool rowin;
-    int clo, chi;
-    __device__ __forceinline__ bool interior() const { return rowin && sp.chunk >= clo && sp.chunk <= chi; }
-};
-__device__ __forceinline__ bool rows_stored(const Geo &g, int px, int py) {
-    return px - g.off >= 0 && px + 1 - g.off < g.n0 && py - g.off >= 0 && py + 1 - g.off < g.n1;
-}
-__device__ __forceinline__ CountPos count_pos(const Geo &g, int64_t s) {
-    const SegPos sp = seg_pos(g, s);
-    // chunk c is inside when 64 c - off >= 0 and 64 c + 64 - off < n2
-    const int clo = (g.off + kWave - 1) / kWave, hi = g.n2 + g.off - kWave - 1;
-    return CountPos{sp, ((int64_t)(sp.px - g.off) * g.n1 + (sp.py - g.off)) * g.n2, rows_stored(g, sp.px, sp.py), clo,
-                    hi >= 0 ? hi / kWave : -1};
-}
-__device__ __forceinline__ void count_advance(const Geo &g, CountPos &c) {
-    if (++c.sp.chunk == g.nchunk) {
-        c.sp.chunk = 0;
-        c.rowoff += g.n2;
-        if (++c.sp.py == g.g1) {
-            c.sp.py = 0;
-            ++c.sp.px;
-            c.rowoff += (int64_t)(g.n1 - g.g1) * g.n2;
-        }
-        c.rowin = rows_stored(g, c.sp.px, c.sp.py);
-    }
-}
-
-// The corner window of a wave's segment at `c` (pz = chunk * 64 + lane): a window of stored
-// samples from the row offset, else load_box's general path.
+// The grid that segment s of a batch belongs to.
 template <typename S>
-__device__ __forceinline__ void load_count_window(const In<S> &in, CornerWin<S> &w, const CountPos &c) {
-    if (!w.interior) {  // wave-uniform
-        w.template load_box<0, 2, 0, 2, 0, 2>(in);
-        return;
-    }
-    const Geo &g = in.geo;
-    const int64_t sy = g.n2, sx = (int64_t)g.n1 * g.n2;
-    const S *p = in.sdf + c.rowoff + (w.pz - g.off);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int k = 0; k < 2; ++k) w.v[i][j][k] = p[i * sx + j * sy + k];
-}
-
-// Counts the segments [wlo, whi) of one grid whose segment 0 is segment `first` of the launch
-// (a short_tails grid): its full segments one per wave iteration, then its last-chunk segments
-// ("tails") several per iteration, P lanes each (P = tail positions rounded up to a power of two),
-// so that a wave iteration is not spent on a few positions. A tail's remaining words (positions
-// past the grid) all hold the pad sample's inside bit. Same counts, words and flags as one segment
-// per iteration; returns the grid's sample flags of the range.
-template <typename S, bool WRITE>
-__device__ __forceinline__ uint32_t count_range_tails(const In<S> &in, int algo, int64_t first, SegBase *seg,
-                                                      uint16_t *info, const uint64_t *cases, int64_t wlo, int64_t whi,
-                                                      int lane, int64_t &wv, int64_t &wf) {
-    const Geo &g = in.geo;
-    const int nc = g.nchunk, last = nc - 1, tailr = g.g2 - kWave * last;
-    uint32_t gfl = 0;
-    CountPos cp = count_pos(g, wlo - first);
-    for (int64_t s = wlo; s < whi; ++s) {  // wave-uniform
-        const SegPos sp = cp.sp;
-        if (sp.chunk != last) {
-            int nv, nf;
-            uint32_t fl, iw;
-            CornerWin<S> w(sp.px, sp.py, sp.chunk * kWave + lane, cp.interior());
-            load_count_window(in, w, cp);
-            count_position<S>(in, algo, cases, w, &nv, &nf, &fl, &iw);
-            int tv, tf;
-            wave_totals2(nv, nf, &tv, &tf);
-            if constexpr (WRITE) {
-                info[s * kWave + lane] = (uint16_t)iw;
-                if (lane == 0) {
-                    seg[s].v = tv;
-                    seg[s].f = tf;
-                }
-            }
-            wv += tv;
-            wf += tf;
-            gfl |= fl;
-        }
-        count_advance(g, cp);
-    }
-    // tails of the range: segments t0, t0 + nc, ... below whi (t0 - first = last mod nc)
-    const int64_t t0 = wlo + ((last - (wlo - first) % nc) + nc) % nc;
-    const int64_t nt = t0 < whi ? (whi - 1 - t0) / nc + 1 : 0;
-    int P = 1;
-    while (P < tailr) P <<= 1;
-    const int per = kWave / P, t = lane / P, i = lane % P;
-    const uint16_t beyond = (uint16_t)((uint32_t)(in.pad >= in.iso) << 11);  // word of a position past the grid
-    for (int64_t b = 0; b < nt; b += per) {  // wave-uniform
-        const bool valid = b + t < nt && i < tailr;
-        const int64_t st = t0 + (b + t < nt ? b + t : 0) * nc;
-        const SegPos tp = seg_pos(g, st - first);  // per lane
-        int nv, nf;
-        uint32_t fl, iw;
-        CornerWin<S> w(in, tp.px, tp.py, last * kWave + i, last * kWave);
-        w.template load_box<0, 2, 0, 2, 0, 2>(in);
-        count_position<S>(in, algo, cases, w, &nv, &nf, &fl, &iw);
-        if (!valid) nv = nf = 0, fl = 0;
-        int sv = nv, sf = nf;  // per-tail sums over its P lanes
-        for (int o = 1; o < P; o <<= 1) {
-            sv += __shfl_xor(sv, o, kWave);
-            sf += __shfl_xor(sf, o, kWave);
-        }
-        if constexpr (WRITE) {
-            if (valid) info[st * kWave + i] = (uint16_t)iw;
-            if (valid && i == 0) {
-                seg[st].v = sv;
-                seg[st].f = sf;
-            }
-            const int ng = nt - b < per ? (int)(nt - b) : per, cw = kWave - tailr;
-            for (int k = lane; k < ng * cw; k += kWave)
-                info[(t0 + (b + k / cw) * nc) * kWave + tailr + k % cw] = beyond;
-        }
-        int tv, tf;
-        wave_totals2(nv, nf, &tv, &tf);
-        wv += tv;
-        wf += tf;
-        gfl |= fl;
-    }
-    return gfl;
-}
-
-template <typename S, int ALGO, bool BATCH, bool WRITE>
-__device__ __forceinline__ void count_range(const CountSrc<S> &src, const BatchGrid<S> *__restrict__ grids,
-                                            SegBase *seg, uint16_t *info, const uint64_t (*s_case)[256],
-                                            int64_t wlo, int64_t whi, int lane, int64_t &wv, int64_t &wf,
-                                            uint32_t &wfl) {
-    if constexpr (!BATCH) {
-        if (short_tails(src.in.geo)) {
-            wfl |= count_range_tails<S, WRITE>(src.in, ALGO, 0, seg, info, s_case[0], wlo, whi, lane, wv, wf);
-            return;
-        }
-    }
-    // BATCH: the range may span several grids; one pass of the outer loop per grid, with that
-    // grid's parameters held in scalar registers for the inner loop.
-    int gi = 0;
-    if constexpr (BATCH)
-        while (gi + 1 < src.ngrids && wlo >= grids[gi + 1].seg_first) ++gi;
-    for (int64_t s = wlo; s < whi;) {  // wave-uniform
-        In<S> in;
-        if constexpr (BATCH)
-            in = load_uniform(&grids[gi].in);
+__device__ __forceinline__ int batch_grid_of(const BatchGrid<S> *__restrict__ grids, int n, int64_t s) {
+    int lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (grids[mid].seg_first <= s)
+            lo = mid;
         else
-            in = src.in;
-        const int algo = BATCH ? grids[gi].algo : ALGO;
-        const int64_t first = BATCH ? grids[gi].seg_first : 0;
-        const int64_t end = (BATCH && gi + 1 < src.ngrids && grids[gi + 1].seg_first < whi) ? grids[gi + 1].seg_first
-                                                                                          : whi;
-        const uint64_t *cases = s_case[(BATCH && algo != DISO_MC) ? 1 : 0];
-        uint32_t gfl = 0;  // the grid's sample flags
-        if (BATCH && short_tails(in.geo)) {
-            gfl = count_range_tails<S, WRITE>(in, algo, first, seg, info, cases, s, end, lane, wv, wf);
+            hi = mid;
+    }
+    return lo;
+}
+
+__device__ __forceinline__ int64_t readlane64(int64_t v, int i) {
+    return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), i) << 32) |
+                     (uint32_t)__builtin_amdgcn_readlane((int)v, i));
+}
+
+// Inside planes and sample flags of the segments [lo, lo + n) (n <= kMaskTile) of one grid, whose
+// first segment is segment `first` of the launch. Stored samples are read in words of 64 from the
+// row's first (chunk c's word: samples 64 c .. 64 c + 63), kMaskLoads samples per lane in flight;
+// each compare's lane mask is the word's bits, kept in lane i + 1 for segment lo + i and in lane 0
+// for the chunk before the tile's first segment. With the virtual pad a segment's plane is its word
+// moved up by the pad sample, the bit below it from the previous chunk's word; so a last chunk that
+// holds only pad and the last sample needs no load of its own.
+constexpr int kMaskTile = 32;
+constexpr int kMaskLoads = 16;
+template <typename S>
+__device__ __forceinline__ void mask_tile(const In<S> &in, int64_t first, int64_t lo, int n, const Planes &out,
+                                          uint32_t *nan, int lane) {
+    const Geo &g = in.geo;
+    const int64_t sg = lo - first + lane - 1;  // segment of this lane's word
+    const SegPos sp = seg_pos(g, sg >= 0 ? sg : 0);
+    const int x = sp.px - g.off, y = sp.py - g.off, z0 = sp.chunk * kWave;
+    const bool row = (unsigned)x < (unsigned)g.n0 && (unsigned)y < (unsigned)g.n1;
+    const int64_t ro = row ? ((int64_t)x * g.n1 + y) * g.n2 + z0 : 0;
+    uint64_t todo = __ballot(row && z0 < g.n2 && sg >= 0 && lane <= n);
+    uint32_t ilo = 0, ihi = 0, elo = 0, ehi = 0;
+    while (todo) {  // wave-uniform
+        S v[kMaskLoads];
+        int at[kMaskLoads];
+#pragma unroll
+        for (int j = 0; j < kMaskLoads; ++j) {
+            // (past the last word to do: that word again)
+            at[j] = todo ? (int)__builtin_ctzll(todo) : at[j ? j - 1 : 0];
+            todo &= todo - 1;
+            const int left = g.n2 - 1 - __builtin_amdgcn_readlane(z0, at[j]);  // samples past the row: the last one
+            v[j] = in.sdf[readlane64(ro, at[j]) + (lane < left ? lane : left)];
+        }
+#pragma unroll
+        for (int j = 0; j < kMaskLoads; ++j) {
+            const uint64_t inside = __ballot(v[j] >= in.iso);
+            const uint64_t equal = __ballot(!(v[j] < in.iso || v[j] > in.iso));  // == iso, or NaN
+            const bool mine = lane == at[j];
+            ilo = mine ? (uint32_t)inside : ilo;
+            ihi = mine ? (uint32_t)(inside >> 32) : ihi;
+            elo = mine ? (uint32_t)equal : elo;
+            ehi = mine ? (uint32_t)(equal >> 32) : ehi;
+        }
+    }
+    const uint64_t have = row ? diso_bits::low_bits(g.n2 - z0) : 0ull;  // the word's stored samples
+    const uint64_t I = ((uint64_t)ihi << 32 | ilo) & have, E = (uint64_t)ehi << 32 | elo;
+    // flags of the tile's own words; a chunk beyond the stored samples has none
+    const uint64_t own = lane >= 1 && lane <= n ? have : 0ull;
+    uint32_t fl = ((~I & ~E & own) ? DISO_TOTAL_HAS_BELOW : 0u) | ((I & ~E & own) ? DISO_TOTAL_HAS_ABOVE : 0u) |
+                  ((~I & E & own) ? DISO_TOTAL_HAS_NAN : 0u);
+    fl = wave_or(fl);
+    if ((fl & DISO_TOTAL_HAS_NAN) && lane == 0) __hip_atomic_store(nan, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // the previous lane's top bit (its chunk precedes this one, unless this is the row's first)
+    const uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(I >> 32), 0x138, 0xf, 0xf, false) >> 31;
+    const uint64_t grid = diso_bits::low_bits(g.g2 - z0);
+    uint64_t plane = I, stored = have;
+    if (g.off) {  // uniform
+        plane = (I << 1) | (sp.chunk > 0 ? (uint64_t)before : 0ull);
+        stored = row ? diso_bits::low_bits(g.n2 + 1 - z0) & (sp.chunk > 0 ? ~0ull : ~1ull) : 0ull;
+    }
+    if (in.pad >= in.iso) plane |= grid & ~stored;
+    if (lane >= 1 && lane <= n) {
+        out.inside[lo + lane - 1] = plane;
+        out.flags[lo + lane - 1] = lane == 1 ? (uint8_t)fl : (uint8_t)0;
+    }
+}
+
+template <typename S, bool BATCH>
+__global__ __launch_bounds__(kBlock) void mask_kernel(CountSrc<S> src, const BatchGrid<S> *__restrict__ grids,
+                                                      Planes out, uint8_t *ctl) {
+    const int lane = threadIdx.x % kWave;
+    const int64_t lo = ((int64_t)blockIdx.x * kWavesPerBlock + wave_id()) * kMaskTile;
+    const int64_t hi = lo + kMaskTile < src.nseg ? lo + kMaskTile : src.nseg;
+    uint32_t *nan = &reinterpret_cast<CtlHeader *>(ctl)->nan;
+    if (lo >= hi) return;
+    if constexpr (!BATCH) {
+        mask_tile<S>(src.in, 0, lo, (int)(hi - lo), out, nan, lane);
+    } else {
+        int gi = batch_grid_of(grids, src.ngrids, lo);
+        for (int64_t s = lo; s < hi; ++gi) {  // the tile may span several grids
+            const In<S> in = load_uniform(&grids[gi].in);
+            const int64_t first = grids[gi].seg_first;
+            const int64_t end = first + in.geo.nseg < hi ? first + in.geo.nseg : hi;
+            mask_tile<S>(in, first, s, (int)(end - s), out, nan, lane);
             s = end;
         }
-        CountPos cp = count_pos(in.geo, s - first);
-        for (; s < end; ++s) {
-            int nv, nf;
-            uint32_t fl, iw;
-            const SegPos sp = cp.sp;
-            CornerWin<S> w(sp.px, sp.py, sp.chunk * kWave + lane, cp.interior());
-            load_count_window(in, w, cp);
-            count_position<S>(in, algo, cases, w, &nv, &nf, &fl, &iw);
-            count_advance(in.geo, cp);  // next segment of the grid
-            int tv, tf;
-            wave_totals2(nv, nf, &tv, &tf);
-            if constexpr (WRITE) {
-                info[s * kWave + lane] = (uint16_t)iw;
-                if (lane == 0) {
-                    seg[s].v = tv;
-                    seg[s].f = tf;
+    }
+}
+
+// An edge with a NaN end does not cross: takes such edges out of a segment's crossings (from the
+// samples; only called when the launch holds a NaN).
+template <typename S>
+__device__ __forceinline__ void drop_nan_edges(const In<S> &in, const SegPos &sp, uint64_t &X, uint64_t &Y, uint64_t &Z) {
+#pragma unroll 1
+    for (int l = 0; l < kWave; ++l) {
+        const int z = sp.chunk * kWave + l;
+        const S a = sample(in, sp.px, sp.py, z), x = sample(in, sp.px + 1, sp.py, z), y = sample(in, sp.px, sp.py + 1, z),
+                u = sample(in, sp.px, sp.py, z + 1);
+        X &= ~((uint64_t)(a != a || x != x) << l);
+        Y &= ~((uint64_t)(a != a || y != y) << l);
+        Z &= ~((uint64_t)(a != a || u != u) << l);
+    }
+}
+
+// Counts the segments [lo, hi) of one grid whose first segment is segment `first` of the launch, one
+// lane per segment, tiles of 64 segments dealt to the block's waves (the first to wave `turn`); adds
+// each lane's totals to (wv, wf) and its sample flags to fl. WRITE: also records each segment's
+// planes, codes and counts; without WRITE the range is only summed (a block recounting a
+// predecessor's range, see the look-back).
+template <typename S, bool DMC, bool WRITE>
+__device__ __forceinline__ void count_tiles(const In<S> &in, int64_t first, int64_t lo, int64_t hi, int wave, int lane,
+                                            bool has_nan, const Planes &P, SegBase *seg, int64_t &wv, int64_t &wf,
+                                            int64_t &wa, uint32_t &fl, uint32_t *s_cnt, int64_t block_lo) {
+    const Geo &g = in.geo;
+    const int64_t sx = xstride(g), sy = g.nchunk;
+    for (int64_t base = lo + (int64_t)wave * kWave; base < hi; base += kCountBlock) {  // wave-uniform
+        const int64_t s = base + lane;
+        const bool valid = s < hi;
+        const int64_t sv = valid ? s : hi - 1;
+        const SegPos sp = seg_pos(g, sv - first);
+        const diso_bits::Place pl{sp.px, sp.py, sp.chunk, g.g0, g.g1, g.g2, g.nchunk};
+        const uint64_t *ip = P.inside + sv;
+        uint64_t X = 0, Y = 0, Z = 0, A = 0, m0 = 0, m1 = 0;
+        int nf = 0;
+        diso_bits::classify<DMC>(
+            pl, valid, [&](int dx, int dy, int dc) { return ip[dx * sx + dy * sy + dc]; },
+            [&](uint32_t b) { return __any(b != 0) != 0; },
+            [&](int h, const diso_bits::Classified &c) {
+                X |= (uint64_t)c.X << (32 * h);
+                Y |= (uint64_t)c.Y << (32 * h);
+                Z |= (uint64_t)c.Z << (32 * h);
+                A |= (uint64_t)c.A << (32 * h);
+                m0 |= (uint64_t)c.m0 << (32 * h);
+                m1 |= (uint64_t)c.m1 << (32 * h);
+                nf += c.nf;
+                if constexpr (WRITE) {
+                    if (c.A) {
+                        uint32_t w[8];
+                        diso_bits::codes_of(c.code, w);
+                        uint4 *d = reinterpret_cast<uint4 *>(P.codes + s * kWave + 32 * h);
+                        d[0] = uint4{w[0], w[1], w[2], w[3]};
+                        d[1] = uint4{w[4], w[5], w[6], w[7]};
+                    }
                 }
+            });
+        if (has_nan) drop_nan_edges(in, sp, X, Y, Z);  // uniform
+        const int nv = diso_bits::popc64(X) + diso_bits::popc64(Y) + diso_bits::popc64(Z), na = diso_bits::popc64(A);
+        wv += nv;
+        wf += nf;
+        wa += na;
+        if (valid) fl |= P.flags[s];
+        if constexpr (WRITE) {
+            if (valid) {
+                // counts of at most 192, 320 and 64, for the segment bases
+                const uint32_t cnt = (uint32_t)nv | (uint32_t)nf << 8 | (uint32_t)na << 24;
+                if (s_cnt)
+                    s_cnt[s - block_lo] = cnt;
+                else
+                    seg[s].v = (int64_t)cnt;
+                P.xy[s] = Plane2{X, Y};
+                P.za[s] = Plane2{Z, A};
+                if (DMC) P.m[s] = Plane2{m0, m1};
             }
-            wv += tv;
-            wf += tf;
-            gfl |= fl;
         }
-        wfl |= gfl;
-        if constexpr (BATCH) {
+    }
+}
+
+// count_tiles over the segments [lo, hi) of the launch.
+template <typename S, int ALGO, bool BATCH, bool WRITE>
+__device__ __forceinline__ void count_range(const CountSrc<S> &src, const BatchGrid<S> *__restrict__ grids,
+                                            SegBase *seg, const Planes &P, bool has_nan, int64_t lo, int64_t hi,
+                                            int wave, int lane, int64_t &wv, int64_t &wf, int64_t &wa,
+                                            uint32_t &wfl, uint32_t *s_cnt, int64_t block_lo) {
+    if constexpr (!BATCH) {
+        count_tiles<S, ALGO == DISO_DMC, WRITE>(src.in, 0, lo, hi, wave, lane, has_nan, P, seg, wv, wf, wa, wfl,
+                                             s_cnt, block_lo);
+    } else {
+        // the range may span several grids: one pass per grid, its parameters in scalar registers
+        int gi = batch_grid_of(grids, src.ngrids, lo);
+        for (int64_t s = lo; s < hi; ++gi) {  // block-uniform
+            const In<S> in = load_uniform(&grids[gi].in);
+            const int64_t first = grids[gi].seg_first;
+            const int64_t end = first + in.geo.nseg < hi ? first + in.geo.nseg : hi;
+            uint32_t gfl = 0;
+            if (grids[gi].algo == DISO_MC)
+                count_tiles<S, false, WRITE>(in, first, s, end, wave, lane, has_nan, P, seg, wv, wf, wa, gfl, s_cnt, block_lo);
+            else
+                count_tiles<S, true, WRITE>(in, first, s, end, wave, lane, has_nan, P, seg, wv, wf, wa, gfl, s_cnt, block_lo);
+            wfl |= gfl;
             if constexpr (WRITE) {
                 gfl = wave_or(gfl);
                 if (lane == 0 && gfl) atomicOr(src.gflags + gi, gfl);
             }
-            ++gi;
+            s = end;
         }
     }
 }
 
 template <typename S, int ALGO, bool BATCH>
-__global__ __launch_bounds__(kCountBlock, (BATCH ? 3 : kCountBlocksPerCU) * kCountWaves / 4) void count_kernel(
-    CountSrc<S> src, const BatchGrid<S> *__restrict__ grids, SegBase *seg, uint16_t *info, uint8_t *ctl,
-    int64_t nblocks) {
-    __shared__ uint64_t s_case[BATCH ? 2 : 1][256];
-    __shared__ int64_t s_v[kCountWaves], s_f[kCountWaves];
+__global__ __launch_bounds__(kCountBlock, kCountWaves / 2) void count_kernel(CountSrc<S> src,
+                                                                           const BatchGrid<S> *__restrict__ grids,
+                                                                           SegBase *seg, Planes planes, uint8_t *ctl,
+                                                                           int64_t nblocks) {
+    __shared__ int64_t s_v[kCountWaves], s_f[kCountWaves], s_a[kCountWaves];
     __shared__ uint32_t s_fl[kCountWaves];
     __shared__ uint32_t s_epoch, s_dirty_other, s_next;
-    __shared__ uint64_t s_word;
+    __shared__ uint64_t s_word, s_word2;
+    __shared__ uint32_t s_cnt[kCountLds];
+    __shared__ uint64_t s_sum[2][kCountWaves];
 
     CtlHeader *hdr = reinterpret_cast<CtlHeader *>(ctl);
     uint64_t *words = reinterpret_cast<uint64_t *>(ctl + kCtlHeader);
@@ -911,92 +813,86 @@ __global__ __launch_bounds__(kCountBlock, (BATCH ? 3 : kCountBlocksPerCU) * kCou
     const int64_t b = blockIdx.x;
     const int64_t lo = b * nseg / nblocks, hi = (b + 1) * nseg / nblocks;
 
-    for (int i = tid; i < 256; i += kCountBlock) {
-        if (BATCH) {
-            s_case[0][i] = kMcCase[i];
-            s_case[BATCH ? 1 : 0][i] = kDmcCase[i];
-        } else {
-            s_case[0][i] = ALGO == DISO_MC ? kMcCase[i] : kDmcCase[i];
-        }
-    }
     if (tid == 0) {
         const uint32_t ep = __hip_atomic_load(&hdr->epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s_epoch = ep;
         s_dirty_other = __hip_atomic_load(&hdr->dirty[diso_scan::buffer_of(ep) ^ 1u], __ATOMIC_RELAXED,
                                           __HIP_MEMORY_SCOPE_AGENT);
     }
-    __syncthreads();
+    const bool has_nan = __builtin_amdgcn_readfirstlane(
+                             (int)__hip_atomic_load(&hdr->nan, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0;
+
+    // The block's sums of one set of per-lane counts, in every thread. Two barriers.
+    auto block_sums = [&](int64_t &v, int64_t &f, int64_t &a, uint32_t &fl) {
+        v = wave_sum64(v);
+        f = wave_sum64(f);
+        a = wave_sum64(a);
+        fl = wave_or(fl);
+        __syncthreads();  // s_v / s_f / s_a reuse
+        if (lane == 0) {
+            s_v[wave] = v;
+            s_f[wave] = f;
+            s_a[wave] = a;
+            s_fl[wave] = fl;
+        }
+        __syncthreads();
+        v = f = a = 0;
+        fl = 0;
+#pragma unroll
+        for (int w = 0; w < kCountWaves; ++w) {
+            v += s_v[w];
+            f += s_f[w];
+            a += s_a[w];
+            fl |= s_fl[w];
+        }
+    };
+
+    // 1. Count: the block's segments, one lane each; the counts of up to kCountLds segments stay in
+    // LDS (more: in `seg`) for phase 4.
+    const bool in_lds = hi - lo <= kCountLds;
+    int64_t av = 0, af = 0, aa = 0;
+    uint32_t afl = 0;
+    count_range<S, ALGO, BATCH, true>(src, grids, seg, planes, has_nan, lo, hi, wave, lane, av, af, aa, afl,
+                                          in_lds ? s_cnt : nullptr, lo);
+    block_sums(av, af, aa, afl);  // (its barriers also make the header reads visible)
     const uint32_t epoch = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_epoch);
     const uint32_t parity = diso_scan::buffer_of(epoch), tag = diso_scan::tag_of(epoch);
-    uint64_t *cur = words + (int64_t)parity * kMaxCountBlocks;
-
-    // 1. Count: wave w takes the w-th eighth of the block's segments, in order; lane 0 records
-    // each segment's counts, every lane its classification word.
-    int64_t wv = 0, wf = 0;
-    uint32_t wfl = 0;
-    count_range<S, ALGO, BATCH, true>(src, grids, seg, info, s_case, lo + (hi - lo) * wave / kCountWaves,
-                                      lo + (hi - lo) * (wave + 1) / kCountWaves, lane, wv, wf, wfl);
-    wfl = wave_or(wfl);
-    if (lane == 0) {
-        s_v[wave] = wv;
-        s_f[wave] = wf;
-        s_fl[wave] = wfl;
+    // block j's two words: words 2 j (vertices, faces, flags) and 2 j + 1 (active cells)
+    uint64_t *cur = words + (int64_t)parity * 2 * kMaxCountBlocks;
+    if (tid == 0) {
+        st_relaxed(cur + 2 * b, diso_scan::pack(av, af, afl, tag));
+        st_relaxed(cur + 2 * b + 1, diso_scan::pack_cells(aa, tag));
     }
-    __syncthreads();
-    int64_t av = 0, af = 0;
-    uint32_t afl = 0;
-#pragma unroll
-    for (int w = 0; w < kCountWaves; ++w) {
-        av += s_v[w];
-        af += s_f[w];
-        afl |= s_fl[w];
-    }
-    if (tid == 0) st_relaxed(cur + b, diso_scan::pack(av, af, afl, tag));
 
     // 2. Exclusive prefix of this block = sum of all predecessors' aggregates. A predecessor that
     // has not published within `recount_spins` reads is not waited for any longer: this block
     // counts that range itself (read-only; the same sums), so no block waits on one that may not
     // be running (several launches sharing the device fill the XCDs' slots). The last block alone
-    // waits for every predecessor's word: a block publishes after reading the epoch, so once all
+    // waits for every predecessor's words: a block publishes after reading the epoch, so once all
     // have published the last block may advance it; every other block ends in bounded time, so the
     // blocks it waits for are all dispatched.
     const bool last = b == nblocks - 1;
     const uint32_t spin_limit = last ? kSpinLimit / (uint32_t)(kMaxCountBlocks / kCountBlock) : src.recount_spins;
-    int64_t pv = 0, pf = 0;
-    uint32_t pfl = 0;
+    int64_t ev = 0, ef = 0, ea = 0;
+    uint32_t efl = 0;
     uint32_t miss = 0;  // bit k: predecessor tid + k * kCountBlock did not publish in time
     for (int64_t j = tid, k = 0; j < b; j += kCountBlock, ++k) {
-        uint64_t w;
+        uint64_t w, w2;
         uint32_t spins = 0;
         do {
-            w = ld_relaxed(cur + j);
-        } while (!diso_scan::published(w, tag) && ++spins < spin_limit);
-        if (!diso_scan::published(w, tag)) {
+            w = ld_relaxed(cur + 2 * j);
+            w2 = ld_relaxed(cur + 2 * j + 1);
+        } while (!(diso_scan::published(w, tag) && diso_scan::published(w2, tag)) && ++spins < spin_limit);
+        if (!(diso_scan::published(w, tag) && diso_scan::published(w2, tag))) {
             miss |= 1u << k;
         } else {
-            pv += diso_scan::count_v(w);
-            pf += diso_scan::count_f(w);
-            pfl |= diso_scan::flags_of(w);
+            ev += diso_scan::count_v(w);
+            ef += diso_scan::count_f(w);
+            ea += diso_scan::count_cells(w2);
+            efl |= diso_scan::flags_of(w);
         }
     }
-    pv = wave_sum64(pv);
-    pf = wave_sum64(pf);
-    pfl = wave_or(pfl);
-    __syncthreads();  // s_v / s_f reuse
-    if (lane == 0) {
-        s_v[wave] = pv;
-        s_f[wave] = pf;
-        s_fl[wave] = pfl;
-    }
-    __syncthreads();
-    int64_t ev = 0, ef = 0;
-    uint32_t efl = 0;
-#pragma unroll
-    for (int w = 0; w < kCountWaves; ++w) {
-        ev += s_v[w];
-        ef += s_f[w];
-        efl |= s_fl[w];
-    }
+    block_sums(ev, ef, ea, efl);
     // the missing predecessors, lowest first, one at a time by the whole block
     for (;;) {
         if (tid == 0) s_next = 0xffffffffu;
@@ -1008,36 +904,29 @@ __global__ __launch_bounds__(kCountBlock, (BATCH ? 3 : kCountBlocksPerCU) * kCou
         if (last) efl |= DISO_TOTAL_SCAN_TIMEOUT;  // never expected: the epoch may advance early
         if (tid == (int)(j % kCountBlock)) {  // one read for the whole block: every wave takes the same branch
             miss &= ~(1u << (j / kCountBlock));
-            s_word = ld_relaxed(cur + j);
+            s_word = ld_relaxed(cur + 2 * (int64_t)j);
+            s_word2 = ld_relaxed(cur + 2 * (int64_t)j + 1);
         }
         __syncthreads();
-        const uint64_t w = s_word;
-        int64_t rv = 0, rf = 0;
+        const uint64_t w = s_word, w2 = s_word2;
+        int64_t rv = 0, rf = 0, ra = 0;
         uint32_t rfl = 0;
-        if (__builtin_amdgcn_readfirstlane((int)diso_scan::published(w, tag))) {  // published meanwhile
-            rv = diso_scan::count_v(w);
-            rf = diso_scan::count_f(w);
-            rfl = diso_scan::flags_of(w);
-            if (wave != 0) rv = rf = 0, rfl = 0;  // count it once
+        if (__builtin_amdgcn_readfirstlane((int)(diso_scan::published(w, tag) && diso_scan::published(w2, tag)))) {
+            if (tid == 0) {  // published meanwhile; counted once
+                rv = diso_scan::count_v(w);
+                rf = diso_scan::count_f(w);
+                ra = diso_scan::count_cells(w2);
+                rfl = diso_scan::flags_of(w);
+            }
         } else {
-            const int64_t jl = (int64_t)j * nseg / nblocks, jh = ((int64_t)j + 1) * nseg / nblocks;
-            count_range<S, ALGO, BATCH, false>(src, grids, seg, info, s_case, jl + (jh - jl) * wave / kCountWaves,
-                                               jl + (jh - jl) * (wave + 1) / kCountWaves, lane, rv, rf, rfl);
-            rfl = wave_or(rfl);
+            count_range<S, ALGO, BATCH, false>(src, grids, seg, planes, has_nan, (int64_t)j * nseg / nblocks,
+                                               ((int64_t)j + 1) * nseg / nblocks, wave, lane, rv, rf, ra, rfl, nullptr, 0);
         }
-        __syncthreads();  // s_v / s_f reuse
-        if (lane == 0) {  // rv, rf are wave-uniform sums
-            s_v[wave] = rv;
-            s_f[wave] = rf;
-            s_fl[wave] = rfl;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int w2 = 0; w2 < kCountWaves; ++w2) {
-            ev += s_v[w2];
-            ef += s_f[w2];
-            efl |= s_fl[w2];
-        }
+        block_sums(rv, rf, ra, rfl);
+        ev += rv;
+        ef += rf;
+        ea += ra;
+        efl |= rfl;
     }
     if (last && tid == 0) {
         SegBase *tot = seg + nseg;
@@ -1045,8 +934,10 @@ __global__ __launch_bounds__(kCountBlock, (BATCH ? 3 : kCountBlocksPerCU) * kCou
         tot[0].f = ef + af;
         tot[1].v = (int64_t)(efl | afl);
         tot[1].f = ALGO;
-        __hip_atomic_store(&hdr->dirty[parity], (uint32_t)nblocks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (nseg >= 4) *planes.nunits = (uint32_t)((ea + aa + kWave - 1) / kWave);
+        __hip_atomic_store(&hdr->dirty[parity], (uint32_t)(2 * nblocks), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(&hdr->dirty[parity ^ 1u], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&hdr->nan, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(&hdr->epoch, epoch + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 
@@ -1055,44 +946,47 @@ __global__ __launch_bounds__(kCountBlock, (BATCH ? 3 : kCountBlocksPerCU) * kCou
         const int64_t n = (int64_t)__builtin_amdgcn_readfirstlane((int)s_dirty_other);
         const int64_t per = (n + nblocks - 1) / nblocks;
         const int64_t c0 = b * per, c1 = c0 + per < n ? c0 + per : n;
-        uint64_t *other = words + (int64_t)(parity ^ 1u) * kMaxCountBlocks;
+        uint64_t *other = words + (int64_t)(parity ^ 1u) * 2 * kMaxCountBlocks;
         for (int64_t i = c0 + tid; i < c1; i += kCountBlock) st_relaxed(other + i, 0ull);
     }
 
-    // 4. Segment bases: block-wide exclusive scan of this block's segment counts.
-    __syncthreads();  // s_v / s_f reuse; phase-1 counts complete
+    // 4. Segment bases: exclusive scan of the block's segment counts, 512 segments at a time. A wave's
+    // sums fit 16-bit fields (64 segments: at most 12,288 vertices, 20,480 faces, 4,096 cells).
+    __syncthreads();  // s_v / s_f / s_a reuse; phase-1 counts complete
     for (int64_t base = lo; base < hi; base += kCountBlock) {
         const int64_t s = base + tid;
-        int64_t cv = 0, cf = 0;
-        if (s < hi) {
-            cv = (int64_t)__hip_atomic_load(reinterpret_cast<uint64_t *>(&seg[s].v), __ATOMIC_RELAXED,
-                                            __HIP_MEMORY_SCOPE_AGENT);
-            cf = (int64_t)__hip_atomic_load(reinterpret_cast<uint64_t *>(&seg[s].f), __ATOMIC_RELAXED,
-                                            __HIP_MEMORY_SCOPE_AGENT);
-        }
-        const int64_t iv = wave_incl64(cv), jf = wave_incl64(cf);
-        if (lane == kWave - 1) {
-            s_v[wave] = iv;
-            s_f[wave] = jf;
-        }
+        uint32_t c = 0;
+        if (s < hi)
+            c = in_lds ? s_cnt[s - lo]
+                       : (uint32_t)__hip_atomic_load(reinterpret_cast<uint64_t *>(&seg[s].v), __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t cvf = (c & 0xff) | ((c >> 8) & 0xffff) << 16, ca = c >> 24;
+        const uint32_t ivf = wave_incl_dpp(cvf), ia = wave_incl_dpp(ca);
+        const int par = (int)((base - lo) / kCountBlock) & 1;  // two sets of sums: one barrier a round
+        if (lane == kWave - 1) s_sum[par][wave] = (uint64_t)ivf | (uint64_t)ia << 32;
         __syncthreads();
-        int64_t ov = ev, of = ef, tv = 0, tf = 0;
+        int64_t ov = ev, of = ef, oa = ea;
 #pragma unroll
         for (int w = 0; w < kCountWaves; ++w) {
+            const uint64_t t = s_sum[par][w];
+            const int64_t tv = (int64_t)(t & 0xffff), tf = (int64_t)((t >> 16) & 0xffff), ta = (int64_t)(t >> 32);
             if (w < wave) {
-                ov += s_v[w];
-                of += s_f[w];
+                ov += tv;
+                of += tf;
+                oa += ta;
             }
-            tv += s_v[w];
-            tf += s_f[w];
+            ev += tv;
+            ef += tf;
+            ea += ta;
         }
         if (s < hi) {
-            seg[s].v = ov + iv - cv;
-            seg[s].f = of + jf - cf;
+            seg[s].v = ov + (int64_t)((ivf & 0xffff) - (cvf & 0xffff));
+            seg[s].f = of + (int64_t)((ivf >> 16) - (cvf >> 16));
+            const int64_t a0 = oa + (int64_t)(ia - ca);
+            planes.abase[s] = (uint16_t)a0;
+            const int64_t u = (a0 + kWave - 1) / kWave;  // the unit, if any, that starts in this segment
+            if (u * kWave < a0 + (int64_t)ca) planes.unit[u] = (uint32_t)s;
         }
-        ev += tv;
-        ef += tf;
-        __syncthreads();
     }
 }
 
@@ -1112,41 +1006,10 @@ __global__ __launch_bounds__(kCountBlock, (BATCH ? 3 : kCountBlocksPerCU) * kCou
 // (diso_set_param).
 constexpr int kMaxRun = kWave;
 
-// Bit i: segment lo + i has faces (MC triangles / DMC patches), i.e. seg[s + 1].f != seg[s].f
-// (the entry after the last segment is the totals entry).
-__device__ __forceinline__ uint64_t run_active(const SegBase *__restrict__ seg, int64_t lo, int64_t hi, int lane) {
-    const int64_t s = lo + lane;
-    return __ballot(s < hi && seg[s + 1].f != seg[s].f);
-}
-
-// The segments of a run with work (bits of `act`, segment lo + bit), taken by the block's waves
-// from a shared counter as each becomes free (their costs differ, so a fixed round-robin deal
-// leaves waves idle while the block, and its LDS, stays resident). A wave loads its next
-// segment (load(bit)) before it processes the current one (work(loaded)). *s_take must be zero
-// and visible to every wave of the block on entry.
-template <typename Load, typename Work>
-__device__ __forceinline__ void run_segments(uint64_t act, uint32_t *s_take, int lane, Load load, Work work) {
-    const int nact = __popcll(act);
-    auto grab = [&]() {
-        uint32_t k = 0;
-        if (lane == 0) k = atomicAdd(s_take, 1u);  // LDS
-        return __builtin_amdgcn_readfirstlane((int)k);
-    };
-    auto kth = [&](int k) {  // bit of the k-th active segment
-        const bool hit = ((act >> lane) & 1) && lanes_below(act) == k;
-        return (int)__builtin_ctzll(__ballot(hit));
-    };
-    int k = grab();
-    if (k >= nact) return;  // wave-uniform
-    auto nxt = load(kth(k));
-    for (;;) {
-        const auto cur = nxt;
-        k = grab();
-        const bool more = k < nact;  // wave-uniform
-        if (more) nxt = load(kth(k));
-        work(cur);
-        if (!more) break;
-    }
+// Per-lane bit of a wave-uniform plane, and the lanes' count of set bits below them.
+__device__ __forceinline__ int bit_of(uint64_t plane) { return __builtin_amdgcn_inverse_ballot_w64(plane) ? 1 : 0; }
+__device__ __forceinline__ int mask_of(uint64_t X, uint64_t Y, uint64_t Z) {
+    return bit_of(X) | (bit_of(Y) << 1) | (bit_of(Z) << 2);
 }
 
 struct OutCfg {
@@ -1225,165 +1088,241 @@ __device__ __forceinline__ void store_vertex(S *__restrict__ verts, int64_t i, i
     }
 }
 
-// The vertex ids of a cell's 12 edges, relative to its segment's first MC vertex. A corner on
-// table edge e lies on an edge owned by the cell at (cell + edge offset); its id is that owner's
-// first vertex plus the rank of the edge's axis among the owner's crossing axes (what
-// create_cell_mc_tris_kernel finds by linear search, src/cumc.cu:586-608). Owners are the cell,
-// its +x, +y, +x+y neighbours (rows R00, R10, R01, R11 of the chunk; rNN = first vertex, nNN =
-// count, mNN = crossing mask) and their +z neighbours, whose first vertex is the current one's
-// first vertex plus its count (cNNn = x-crossing flag of the +z neighbour).
-__device__ __forceinline__ void edge_ids(int32_t *c, int32_t r00, int32_t r10, int32_t r01, int32_t r11, int m00,
-                                         int m10, int m01, int m11, int c00n, int c10n) {
-    const int n00 = popc3(m00), n10 = popc3(m10), n01 = popc3(m01), n11 = popc3(m11);
-    c[0] = r00;
-    c[1] = r10 + n10 - 1;
-    c[2] = r00 + n00;
-    c[3] = r00 + n00 - 1;
-    c[4] = r01;
-    c[5] = r11 + n11 - 1;
-    c[6] = r01 + n01;
-    c[7] = r01 + n01 - 1;
-    c[8] = r00 + (m00 & 1);
-    c[9] = r10 + (m10 & 1);
-    c[10] = r10 + n10 + c10n;
-    c[11] = r00 + n00 + c00n;
+// Active cells in units of 64, one lane per cell, whatever segments they lie in (so that lanes are
+// full on sparse surfaces too). A unit's cells are found from the segments between its first one and
+// the next unit's first one: lane i loads segment U0 + i and each segment with cells writes them to
+// `list` at its place. Where more than 64 segments lie in between (a sparse stretch), each lane
+// searches its cell's segment instead. Returns the number of cells; lane k < n gets cell k's segment
+// (of the launch) and position in it, the other lanes a copy of one of them.
+struct UnitGrid {
+    const SegBase *__restrict__ seg;  // launch-level arrays
+    Planes P;
+    int64_t first, last;  // the grid's first and last segment
+    int64_t v0, f0;       // bases of its first segment
+};
+
+// Position of the r-th set bit of m (r < popcount).
+__device__ __forceinline__ int select64(uint64_t m, int r) {
+    uint32_t w = (uint32_t)m;
+    int p = 0, c = __popc(w);
+    if (r >= c) r -= c, w = (uint32_t)(m >> 32), p = 32;
+#pragma unroll
+    for (int h = 16; h; h >>= 1) {
+        c = __popc(w & ((1u << h) - 1));
+        const bool up = r >= c;
+        r -= up ? c : 0;
+        p += up ? h : 0;
+        w = up ? w >> h : w;
+    }
+    return p;
 }
 
-// MC emission. Vertex item = (lane, axis) of an owned crossing edge, in the reference's order
-// (cell, then axis x < y < z; src/cumc.cu:370-410); triangle item = (lane, triangle of its cell),
-// whose three corners' table edges come from the cell's case word.
-// Cell codes and crossing masks come from the count pass's classification words.
+__device__ __forceinline__ int unit_cells(const UnitGrid &G, uint32_t u, uint32_t nunits, uint16_t *list, int lane,
+                                          uint32_t *s_out, int *l_out) {
+    const int64_t a = G.P.unit[u], b = u + 1 < nunits ? (int64_t)G.P.unit[u + 1] : G.last;
+    const int64_t U0 = a > G.first ? a : G.first, U1 = b < G.last ? b : G.last;
+    const uint16_t c0 = (uint16_t)(u * (uint32_t)kWave);  // number of the unit's first cell
+    if (U1 - U0 < kWave) {  // wave-uniform
+        const bool in = lane <= (int)(U1 - U0);
+        const uint64_t A = in ? G.P.za[U0 + lane].b : 0ull;
+        const int st = in ? (int)(int16_t)(uint16_t)(G.P.abase[U0 + lane] - c0) : 0;
+        const int s0 = __builtin_amdgcn_readfirstlane(st);
+        const int k0 = s0 > 0 ? s0 : 0;  // cells of the unit that belong to the grid before (a batch)
+        int n = 0;
+        for (uint64_t act = __ballot(A != 0); act; act &= act - 1) {
+            const int j = (int)__builtin_ctzll(act);
+            const uint64_t m = (uint64_t)readlane64((int64_t)A, j);
+            const int at = __builtin_amdgcn_readlane(st, j) - k0;
+            if (at >= kWave - k0) break;
+            const int k = at + lanes_below(m);
+            if (__builtin_amdgcn_inverse_ballot_w64(m) && k >= 0 && k < kWave - k0) list[k] = (uint16_t)(j << 6 | lane);
+            n = at + (int)__popcll(m);
+        }
+        n = n < kWave - k0 ? n : kWave - k0;
+        wave_lds_sync();
+        const int w = n > 0 ? list[lane < n ? lane : n - 1] : 0;
+        *s_out = (uint32_t)(U0 + (w >> 6));
+        *l_out = w & 63;
+        wave_lds_sync();
+        return n;
+    }
+    const int s0 = (int)(int16_t)(uint16_t)(G.P.abase[U0] - c0), k0 = s0 > 0 ? s0 : 0;
+    const int c = k0 + lane;  // this lane's cell of the unit
+    int64_t lo = U0, hi = U1;
+    while (lo < hi) {  // the last segment whose cells start at or before c
+        const int64_t mid = (lo + hi + 1) >> 1;
+        if ((int)(int16_t)(uint16_t)(G.P.abase[mid] - c0) <= c)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    const uint64_t A = G.P.za[lo].b;
+    const int r = c - (int)(int16_t)(uint16_t)(G.P.abase[lo] - c0);
+    const uint64_t ok = __ballot(c < kWave && r < (int)__popcll(A));
+    const int n = (int)__popcll(ok);  // the valid lanes are the first ones
+    const int l = (ok >> lane) & 1 ? select64(A, r) : 0;
+    const int from = lane < n ? lane : 0;
+    *s_out = (uint32_t)__shfl((int)(uint32_t)lo, from, kWave);
+    *l_out = __shfl(l, from, kWave);
+    return n;
+}
+
+// The units of a launch as a wave goes through them: XCD x takes the x-th eighth, its waves in turn,
+// so that at any time an XCD's waves work on neighbouring cells (whose rows share its L2). Calls
+// f(unit) for each of this wave's units. The grid has a multiple of eight blocks.
+template <typename F>
+__device__ __forceinline__ void for_units(uint32_t lo, uint32_t hi, int64_t block, int64_t nblocks, int wave, F f) {
+    const uint32_t n = hi - lo, xcd = (uint32_t)(block % 8), per = (uint32_t)(nblocks / 8) * kWavesPerBlock;
+    const uint32_t u0 = lo + (uint32_t)((uint64_t)n * xcd / 8), u1 = lo + (uint32_t)((uint64_t)n * (xcd + 1) / 8);
+    for (uint32_t u = u0 + (uint32_t)(block / 8) * kWavesPerBlock + (uint32_t)wave; u < u1; u += per) f(u);
+}
+
+__device__ __forceinline__ int bit_at(uint64_t w, int l) {
+    return (int)((((l & 32) ? (uint32_t)(w >> 32) : (uint32_t)w) >> (l & 31)) & 1u);
+}
+
+// MC emission, one unit of 64 active cells at a time: its vertices are the crossing edges its cells
+// own (all owners of crossing edges are active), its triangles those of its cells; both are
+// contiguous rows, in the reference's order (src/cumc.cu:370-410,564-649). Vertex item = (cell,
+// axis); triangle item = (cell, triangle), whose corners' table edges come from the case word.
 struct McEmitLds {
-    int32_t cand[kWave][12];  // vertex id of each table edge, relative to the segment's first vertex
-    uint64_t cw[kWave];       // case word of each lane's cell
-    uint16_t tri[kWave * 5 + 1];  // triangle items: lane << 3 | triangle of the lane's cell
-    uint8_t vert[kWave * 3 + 1];  // vertex items: lane * 4 + axis
+    int32_t cand[kWave][12];  // vertex id of each table edge, relative to the unit's first vertex
+    int32_t cx[kWave], cy[kWave], cz[kWave];
+    uint64_t cw[kWave];           // the cells' case words
+    uint16_t tri[kWave * 5 + 1];  // triangle items: cell << 3 | triangle
+    uint8_t vert[kWave * 3 + 1];  // vertex items: cell * 4 + axis
     // (the last entry of each list takes the writes of the lanes with nothing to list there)
 };
 
-// What an MC segment reads from memory before any work (loaded one segment ahead): the
-// classification words of rows 00, 10, 01, 11 at z and of rows 00, 10 at z + 1, and the bases.
-struct McSegIn {
-    int64_t s;
-    SegPos sp;
-    uint32_t w00, w10, w01, w11, n00, n10;
-    int64_t vabs, fabs;
-    int32_t d10, d01, d11;  // first vertices of rows +x, +y, +x+y relative to the segment's
+// Vertices of a row before position l (b = bits below l), and the row's counts at l.
+struct RowEdges {
+    uint64_t X, Y, Z;
+    __device__ __forceinline__ int below(uint64_t b) const {
+        return (int)__popcll(X & b) + (int)__popcll(Y & b) + (int)__popcll(Z & b);
+    }
 };
 
-template <typename S>
-__device__ __forceinline__ McSegIn mc_load(const In<S> &in, const SegCtx &sc, int64_t s, SegPos sp, int lane) {
-    const Geo &g = in.geo;
-    const SegBase *__restrict__ seg = sc.seg;
-    const uint16_t *info = sc.info;
-    McSegIn d;
-    d.s = s;
-    d.sp = sp;
-    // This row has cells, so rows +x, +y, +x+y exist; +z words are read within the row only.
-    const int pz = sp.chunk * kWave + lane;
-    const int64_t s10 = s + xstride(g), s01 = s + g.nchunk, s11 = s10 + g.nchunk;
-    d.vabs = seg[s].v;
-    d.fabs = seg[s].f;
-    d.d10 = (int32_t)(seg[s10].v - d.vabs);
-    d.d01 = (int32_t)(seg[s01].v - d.vabs);
-    d.d11 = (int32_t)(seg[s11].v - d.vabs);
-    d.w00 = info[s * kWave + lane];
-    d.w10 = info[s10 * kWave + lane];
-    d.w01 = info[s01 * kWave + lane];
-    d.w11 = info[s11 * kWave + lane];
-    const bool zn = pz + 1 < g.g2;
-    d.n00 = zn ? info[s * kWave + lane + 1] : 0u;
-    d.n10 = zn ? info[s10 * kWave + lane + 1] : 0u;
-    return d;
-}
-
-// One segment that has triangles.
 template <typename S, bool DEF>
-__device__ __forceinline__ void emit_mc_segment(const In<S> &in, const SegCtx &sc, const McSegIn &d,
-                                                S *__restrict__ verts, void *__restrict__ faces, const OutCfg &out,
-                                                const Norm<S> &nm, const uint64_t *s_case, McEmitLds &L,
-                                                int lane) {
-    wave_lds_sync();  // the previous segment's LDS reads are done
-    const int64_t tbase = d.fabs - sc.f0;
-    const int px = d.sp.px, py = d.sp.py;
-    const int z0 = d.sp.chunk * kWave;
-    const int64_t vabs = d.vabs, vbase = vabs - sc.v0;
-    const uint32_t w00 = d.w00;
-    const int m00 = info_mask(w00), m10 = info_mask(d.w10), m01 = info_mask(d.w01), m11 = info_mask(d.w11);
-    const int c00n = info_mask(d.n00) & 1, c10n = info_mask(d.n10) & 1;
-    const uint64_t cw = s_case[info_code(w00)];  // Bourke corner order (src/cumc.cu:107)
-    const int ntri = DISO_MC_NTRI(cw);
+__device__ __forceinline__ void emit_mc_unit(const In<S> &in, const UnitGrid &G, uint32_t u, uint32_t nunits,
+                                             S *__restrict__ verts, void *__restrict__ faces, const OutCfg &out,
+                                             const Norm<S> &nm, const uint64_t *s_case, McEmitLds &L, int lane) {
+    wave_lds_sync();  // the previous unit's LDS reads are done
+    uint32_t s;
+    int l;
+    const int n = unit_cells(G, u, nunits, L.tri, lane, &s, &l);
+    if (n == 0) return;  // wave-uniform
+    const Geo &g = in.geo;
+    const SegPos sp = seg_pos(g, (int64_t)s - G.first);
+    const bool on = lane < n;
+    const uint64_t b = (1ull << l) - 1;
 
-    // exclusive prefixes over the lanes of the rows' vertex counts and of the triangle counts, in
-    // two packed scans of 10-bit fields (wave totals <= 320)
-    const uint32_t cA = (uint32_t)popc3(m00) | (uint32_t)popc3(m10) << 10 | (uint32_t)popc3(m01) << 20;
-    const uint32_t cB = (uint32_t)ntri | (uint32_t)popc3(m11) << 10;
-    const uint32_t iA = wave_incl_dpp(cA), iB = wave_incl_dpp(cB);
-    const uint32_t eA = iA - cA, eB = iB - cB;
-    const uint32_t tA = (uint32_t)__builtin_amdgcn_readlane((int)iA, kWave - 1),
-                   tB = (uint32_t)__builtin_amdgcn_readlane((int)iB, kWave - 1);
-    const int p00 = (int)(eA & 0x3ff), tv = (int)(tA & 0x3ff);
-    const int pt = (int)(eB & 0x3ff), tt = (int)(tB & 0x3ff);
-    const int32_t r10 = d.d10 + (int32_t)((eA >> 10) & 0x3ff);
-    const int32_t r01 = d.d01 + (int32_t)((eA >> 20) & 0x3ff);
-    const int32_t r11 = d.d11 + (int32_t)((eB >> 10) & 0x3ff);
-
-    // list writes without per-lane branches: what is not listed goes to the spare last entry
-    {
-        int r = p00;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const int on = (m00 >> a) & 1;
-            L.vert[on ? r : 3 * kWave] = (uint8_t)(lane * 4 + a);
-            r += on;
-        }
+    // the cell's row and rows +x, +y, +x+y (an active cell has them): edges owned there
+    const int64_t s10 = (int64_t)s + xstride(g), s01 = (int64_t)s + g.nchunk, s11 = s10 + g.nchunk;
+    const uint32_t code = G.P.codes[(int64_t)s * kWave + l];
+    const Plane2 *__restrict__ XY = G.P.xy, *__restrict__ ZA = G.P.za;
+    const RowEdges e00{XY[s].a, XY[s].b, ZA[s].a}, e10{XY[s10].a, XY[s10].b, ZA[s10].a}, e01{XY[s01].a, XY[s01].b, ZA[s01].a},
+        e11{XY[s11].a, XY[s11].b, ZA[s11].a};
+    const int64_t v10 = G.seg[s10].v, v01 = G.seg[s01].v, v11 = G.seg[s11].v;
+    // x edges at z + 1 in rows 00 and 10
+    int xn00 = l < kWave - 1 ? bit_at(e00.X, l + 1) : 0, xn10 = l < kWave - 1 ? bit_at(e10.X, l + 1) : 0;
+    if (l == kWave - 1 && sp.chunk + 1 < g.nchunk) {
+        xn00 = (int)(XY[s + 1].a & 1);
+        xn10 = (int)(XY[s10 + 1].a & 1);
     }
-    edge_ids(L.cand[lane], p00, r10, r01, r11, m00, m10, m01, m11, c00n, c10n);
-    L.cw[lane] = cw;
+
+    // first vertex and triangle of the unit: those of its first cell
+    const uint64_t b0 = (uint64_t)readlane64((int64_t)b, 0);
+    const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
+    const Plane2 q0 = load_uniform(&XY[s0]), w0 = load_uniform(&ZA[s0]);
+    const int64_t vabs = G.seg[s0].v + RowEdges{q0.a, q0.b, w0.a}.below(b0), vbase = vabs - G.v0;
+    const bool before = __builtin_amdgcn_inverse_ballot_w64(w0.b & b0);  // its segment's cells before it
+    const uint32_t bt = before ? (uint32_t)DISO_MC_NTRI(s_case[G.P.codes[(int64_t)s0 * kWave + lane]]) : 0u;
+    const int64_t tbase = G.seg[s0].f - G.f0 + __builtin_amdgcn_readlane((int)wave_incl_dpp(bt), kWave - 1);
+
+    const uint64_t cw = s_case[code];
+    const int ntri = on ? DISO_MC_NTRI(cw) : 0;
+    const int x00 = bit_at(e00.X, l), y00 = bit_at(e00.Y, l), z00 = bit_at(e00.Z, l);
+    const int n00 = x00 + y00 + z00;
+    const int x10 = bit_at(e10.X, l), n10 = x10 + bit_at(e10.Y, l) + bit_at(e10.Z, l);
+    const int n01 = bit_at(e01.X, l) + bit_at(e01.Y, l) + bit_at(e01.Z, l);
+    const int n11 = bit_at(e11.X, l) + bit_at(e11.Y, l) + bit_at(e11.Z, l);
+    // exclusive prefixes of the vertices (<= 192) and triangles (<= 320) in one scan
+    const uint32_t c = on ? (uint32_t)n00 | (uint32_t)ntri << 16 : 0u;
+    const uint32_t ic = wave_incl_dpp(c), ec = ic - c, tc = (uint32_t)__builtin_amdgcn_readlane((int)ic, kWave - 1);
+    const int pv = (int)(ec & 0xffff), pt = (int)(ec >> 16), tv = (int)(tc & 0xffff), tt = (int)(tc >> 16);
+    const int32_t r10 = (int32_t)(v10 - vabs) + e10.below(b), r01 = (int32_t)(v01 - vabs) + e01.below(b),
+                  r11 = (int32_t)(v11 - vabs) + e11.below(b);
+
+    if (on) {
+        // A corner on table edge e lies on an edge owned by the cell at (cell + edge offset); its id is
+        // that owner's first vertex plus the rank of the edge's axis among the owner's crossing axes
+        // (what create_cell_mc_tris_kernel finds by linear search, src/cumc.cu:586-608). Owners are the
+        // cell, its +x, +y, +x+y neighbours and their +z neighbours, whose first vertex is the current
+        // one's first vertex plus its count.
+        int32_t *d = L.cand[lane];
+        d[0] = pv;
+        d[1] = r10 + n10 - 1;
+        d[2] = pv + n00;
+        d[3] = pv + n00 - 1;
+        d[4] = r01;
+        d[5] = r11 + n11 - 1;
+        d[6] = r01 + n01;
+        d[7] = r01 + n01 - 1;
+        d[8] = pv + x00;
+        d[9] = r10 + x10;
+        d[10] = r10 + n10 + xn10;
+        d[11] = pv + n00 + xn00;
+        L.cx[lane] = sp.px;
+        L.cy[lane] = sp.py;
+        L.cz[lane] = sp.chunk * kWave + l;
+        L.cw[lane] = cw;
+    }
+    // list writes without per-lane branches: what is not listed goes to the spare last entry
+    L.vert[on && x00 ? pv : 3 * kWave] = (uint8_t)(lane * 4);
+    L.vert[on && y00 ? pv + x00 : 3 * kWave] = (uint8_t)(lane * 4 + 1);
+    L.vert[on && z00 ? pv + x00 + y00 : 3 * kWave] = (uint8_t)(lane * 4 + 2);
 #pragma unroll
     for (int t = 0; t < 5; ++t) L.tri[t < ntri ? pt + t : 5 * kWave] = (uint16_t)((lane << 3) | t);
     wave_lds_sync();
 
     for (int k = lane; k < tv; k += kWave) {
         const int it = L.vert[k], src = it >> 2, a = it & 3;
-        const V3<S> p = edge_vertex<S, DEF>(in, px, py, z0 + src, a);
+        const V3<S> p = edge_vertex<S, DEF>(in, L.cx[src], L.cy[src], L.cz[src], a);
         store_vertex(verts, vbase + k, out.vcap, epilogue(p, out.flags, nm));
     }
-    // triangle k of the segment per lane: its cell's case word once, the three corners' table
-    // edges and vertex ids (independent LDS reads), then the three indices as one row
+    // triangle k of the unit per lane: its cell's case word once, the three corners' table edges and
+    // vertex ids (independent LDS reads), then the three indices as one row
     for (int k = lane; k < tt; k += kWave) {
         const int64_t f = tbase + k;
         if (f >= out.fcap) continue;
         const int it = L.tri[k], src = it >> 3, t = it & 7;
-        const uint64_t cw = L.cw[src];
+        const uint64_t w = L.cw[src];
         const int32_t *cand = L.cand[src];
-        store_tri(faces, f, vbase + cand[DISO_MC_EDGE(cw, 3 * t)], vbase + cand[DISO_MC_EDGE(cw, 3 * t + 1)],
-                  vbase + cand[DISO_MC_EDGE(cw, 3 * t + 2)], out.flags);
+        store_tri(faces, f, vbase + cand[DISO_MC_EDGE(w, 3 * t)], vbase + cand[DISO_MC_EDGE(w, 3 * t + 1)],
+                  vbase + cand[DISO_MC_EDGE(w, 3 * t + 2)], out.flags);
     }
 }
 
+__device__ __forceinline__ void load_mc_cases(uint64_t *s_case) {
+    for (int i = threadIdx.x; i < 256; i += kBlock) s_case[i] = kMcCase[i];
+}
+
 template <typename S, bool DEF>
-__global__ __launch_bounds__(kBlock, 7) void emit_mc_kernel(In<S> in, const SegBase *__restrict__ seg,
-                                                         S *__restrict__ verts, void *__restrict__ faces,
-                                                         OutCfg out, Norm<S> nm, int run, int64_t nblocks) {
+__global__ __launch_bounds__(kBlock, 6) void emit_mc_kernel(In<S> in, const SegBase *__restrict__ seg, Planes planes,
+                                                         S *__restrict__ verts, void *__restrict__ faces, OutCfg out,
+                                                         Norm<S> nm) {
     __shared__ uint64_t s_case[256];
     __shared__ McEmitLds s_lds[kWavesPerBlock];
-    __shared__ uint32_t s_take;
-    const int tid = threadIdx.x, wave = wave_id(), lane = tid % kWave;
-    for (int i = tid; i < 256; i += kBlock) s_case[i] = kMcCase[i];
-    if (tid == 0) s_take = 0;
-    __syncthreads();
-    const Geo &g = in.geo;
-    const SegCtx sc{seg, info_of(seg, g), 0, 0};
-    const SegBase *tot = seg + g.nseg;
+    const int wave = wave_id(), lane = threadIdx.x % kWave;
+    const SegBase *tot = seg + in.geo.nseg;
     if (tot[0].v > out.vcap || tot[0].f > out.fcap) return;
-    const int64_t lo = xcd_block(blockIdx.x, nblocks) * run, hi = lo + run < g.nseg ? lo + run : g.nseg;
-    // segments of the run with triangles (hence owned crossings)
-    const uint64_t act = run_active(seg, lo, hi, lane);
-    const SegPos lp = seg_pos(g, lo + lane);
-    run_segments(
-        act, &s_take, lane, [&](int i) { return mc_load<S>(in, sc, lo + i, pos_of_lane(lp, i), lane); },
-        [&](const McSegIn &d) { emit_mc_segment<S, DEF>(in, sc, d, verts, faces, out, nm, s_case, s_lds[wave], lane); });
+    load_mc_cases(s_case);
+    __syncthreads();
+    const uint32_t nunits = *planes.nunits;
+    const UnitGrid G{seg, planes, 0, in.geo.nseg - 1, 0, 0};
+    for_units(0, nunits, blockIdx.x, gridDim.x, wave, [&](uint32_t u) {
+        emit_mc_unit<S, DEF>(in, G, u, nunits, verts, faces, out, nm, s_case, s_lds[wave], lane);
+    });
 }
 
 // DMC emission. Patch-vertex item = (lane, patch): the mean of the MC vertices on the patch's
@@ -1422,41 +1361,61 @@ __device__ constexpr bool tables_agree() {
 }
 static_assert(tables_agree(), "edge / quad tables");
 
-// Edge kinds of a segment's cells, by owner row (dx, dy) and axis: 0: row 00 x, 1: row 00 y,
-// 2: row 00 z, 3: row 10 y, 4: row 10 z, 5: row 01 x, 6: row 01 z, 7: row 11 z (the owner of an
-// edge is the position it starts from; row dxy is (px + dx, py + dy)). The x and y edges of the
-// last cell's top face start at z0 + 64 (the "halo", kinds 8..11 for 0, 1, 3, 5 there).
-// Cell edge e (table numbering) as (kind | top << 3) in 5 bits: top = the edge starts at z + 1.
-__device__ constexpr int edge_kind(int e) {
-    return eax(e) == 0 ? (eoy(e) ? 5 : 0) : eax(e) == 1 ? (eox(e) ? 3 : 1) : (eox(e) + 2 * eoy(e) == 0 ? 2 : eox(e) + 2 * eoy(e) == 1 ? 4 : eox(e) + 2 * eoy(e) == 2 ? 6 : 7);
-}
-__device__ constexpr uint64_t edge_kind_table() {
-    uint64_t t = 0;
-    for (int e = 0; e < 12; ++e) t |= (uint64_t)(edge_kind(e) | (eoz(e) << 3)) << (5 * e);
-    return t;
-}
-// A cell's top edges (dz = 1) are all of kinds 0, 1, 3 or 5.
-__device__ constexpr bool top_kinds_ok() {
-    for (int e = 0; e < 12; ++e)
-        if (eoz(e) && !((1 << edge_kind(e)) & 0x2b)) return false;
+// Edges of a dual cell that start at its own z (the other four, on its top face, are the next
+// position's): kinds 0..7 in ascending edge number, with the edge's offsets and axis as bit masks
+// over the kinds. Top edges 2, 6, 10, 11 are kinds 0, 3, 7, 6 of the next position.
+__device__ constexpr int kind_edge(int k) { return k + (k >= 2) + (k >= 5); }  // 0 1 3 4 5 7 8 9
+constexpr int kTopEdges[4] = {2, 6, 10, 11}, kTopKinds[4] = {0, 3, 7, 6};
+constexpr int kKindX = 0x92, kKindY = 0x38, kKindAxisZ = 0x36, kKindAxisY = 0xC0;
+__device__ constexpr bool kinds_ok() {
+    for (int k = 0; k < 8; ++k) {
+        const int e = kind_edge(k);
+        if (eoz(e) || eox(e) != ((kKindX >> k) & 1) || eoy(e) != ((kKindY >> k) & 1) ||
+            eax(e) != ((kKindAxisZ >> k) & 1 ? 2 : (kKindAxisY >> k) & 1))
+            return false;
+    }
+    for (int t = 0; t < 4; ++t) {
+        const int e = kTopEdges[t], d = kind_edge(kTopKinds[t]);
+        if (!eoz(e) || eox(e) != eox(d) || eoy(e) != eoy(d) || eax(e) != eax(d)) return false;
+    }
     return true;
 }
-static_assert(top_kinds_ok(), "top edges outside the halo slot entries");
-constexpr int kEdgeSlots = 255;  // MC vertices kept per segment; beyond, patches recompute theirs
+static_assert(kinds_ok(), "edge kinds");
+// The kinds that cross in a cell of code c (Morton corner order); a cell of the inverted code has
+// the same. And the top edges that cross, as kinds of the next position.
+__host__ __device__ constexpr uint32_t own_kinds(uint32_t c) {
+    const uint32_t x = c ^ (c >> 1), y = c ^ (c >> 2), z = c ^ (c >> 4);
+    return (x & 1) | (z & 2) | (z & 1) << 2 | (x & 4) << 1 | (z & 8) << 1 | (z & 4) << 3 | (y & 3) << 6;
+}
+__host__ __device__ constexpr uint32_t top_kinds(uint32_t c) {
+    const uint32_t x = c ^ (c >> 1), y = c ^ (c >> 2);
+    return ((x >> 4) & 1) | ((x >> 6) & 1) << 3 | ((y >> 4) & 3) << 6;
+}
+
+// MC vertices kept per unit; a unit with more recomputes them per patch. White noise averages 256
+// per unit (8 kinds, half of them crossing, 64 cells) and stays below 320.
+constexpr int kEdgeSlots = 320;
 
 template <typename S>
 struct DmcEmitLds {
-    uint8_t code[8][kWave];    // codes of the cells (-i,-j,-k) around the lane, ci = 4i + 2j + k
-    int16_t pre[8][kWave];     // their first DMC vertex, relative to the first of row (-i,-j)
-    int32_t rowb[4];           // first DMC vertex of row (-i,-j), relative to the segment's first
-    uint8_t patch[kWave * 4 + 1];  // patch items: lane * 4 + patch
-    uint16_t quad[kWave * 3 + 1];  // quad items: lane * 8 + axis * 2 + leaving
+    // entry k + 1: cell k's first edge slot (bits 0-9), whether its sample is inside (bit 10), the
+    // kinds that cross (bits 16-23), its code (bits 24-31); entry 0: the code of the cell below cell
+    // 0; entry n + 1: the slots and kinds of the position above the last cell
+    uint32_t cw[kWave + 2];
+    int32_t cx[kWave + 1], cy[kWave + 1], cz[kWave + 1];  // the cells' positions (and that one's)
+    uint16_t pp[kWave];            // patches of the unit before the cell's
+    uint8_t patch[kWave * 4 + 1];  // patch items: cell * 4 + patch
+    uint8_t quad[kWave * 3 + 1];   // quad items: cell * 4 + axis
     // (the last entry of each list takes the writes of the lanes with nothing to list there)
-    // slot of the lane's edge of each kind (0xff: does not cross); entry kWave of kinds 0, 1, 3
-    // and 5 holds the halo position z0 + 64's (the only kinds a cell's top edges have)
-    uint8_t slot[8][kWave + 1];
-    uint16_t eitem[kEdgeSlots + 1];  // edge items: lane << 4 | kind; the last takes non-crossing edges' writes
-    S ev[3][kEdgeSlots + 1];         // their MC vertices; the last entry holds zeros
+    uint16_t eitem[kEdgeSlots + 1];  // edge items, from slot 1: cell * 8 + kind (entry 0: spare)
+    union {
+        struct {  // neighbour rows -x, -y, -x-y, until the quads are written
+            int32_t nf[3][kWave];  // first patch of the row's cell at z, relative to the unit's first
+            uint32_t nc[kWave];    // codes: row -x at z and z - 1, row -y at z and z - 1
+            uint8_t nd[kWave];     // code: row -x-y at z
+        };
+        S ev[3][kEdgeSlots + 1];  // then the MC vertices by slot; entry 0 holds zeros
+    };
 };
 
 // Edge masks of the patches of every DMC case, 16 bits per patch (patch k in bits 16k..16k+11),
@@ -1479,20 +1438,6 @@ constexpr PatchEdgeTable make_patch_edges() {
 }
 __constant__ PatchEdgeTable kDmcPatchEdges = make_patch_edges();
 
-// Quad stencil of each edge type as one word: cell index ci of corner j in bits 3j..3j+2, edge id
-// in bits 12+4j..15+4j.
-struct StencilTable {
-    uint32_t w[6];
-};
-constexpr StencilTable make_stencil() {
-    StencilTable t{};
-    for (int ty = 0; ty < 6; ++ty)
-        for (int j = 0; j < 4; ++j)
-            t.w[ty] |= ((uint32_t)stencil_ci(ty, j) << (3 * j)) | ((uint32_t)stencil_eid(ty, j) << (12 + 4 * j));
-    return t;
-}
-__constant__ StencilTable kStencil = make_stencil();
-
 // 1/n for the possible patch sizes (n = 1..7), correctly rounded at compile time.
 template <typename S>
 struct RcpTable {
@@ -1513,245 +1458,243 @@ __device__ __forceinline__ float rcp_small<float>(int n) { return kRcpF.r[n]; }
 template <>
 __device__ __forceinline__ double rcp_small<double>(int n) { return kRcpD.r[n]; }
 
-// What a DMC segment reads from memory before any work: its classification words (own row,
-// rows -x, -y, -x-y at z and z - 1, rows +x, +y, +x+y at z, and the halo position z0 + 64) and the
-// bases. Loaded one segment ahead, so the loads of the next segment overlap this one's work.
-struct DmcSegIn {
-    int64_t s;
-    SegPos sp;
-    uint32_t w0, w10, w01, w11, h00, h10, h01;
-    uint32_t cur[4], prev[4];  // codes of cells (-i,-j,0) and (-i,-j,-1), index 2i + j
-    int64_t vabs, pabs;
-    int32_t rowd[4];  // first DMC vertex of row (-i, -j), relative to the segment's
-};
-
-template <typename S>
-__device__ __forceinline__ DmcSegIn dmc_load(const In<S> &in, const SegCtx &sc, int64_t s, SegPos sp, int lane) {
-    const Geo &g = in.geo;
-    const SegBase *__restrict__ seg = sc.seg;
-    const uint16_t *info = sc.info;
-    DmcSegIn d;
-    d.s = s;
-    d.sp = sp;
-    const int px = sp.px, py = sp.py, chunk = sp.chunk, pz = chunk * kWave + lane;
-    d.vabs = seg[s].v;
-    d.pabs = seg[s].f;
-    const int64_t s10 = s + xstride(g), s01 = s + g.nchunk, s11 = s10 + g.nchunk;
-    d.w0 = info[s * kWave + lane];
-    d.w10 = info[s10 * kWave + lane];
-    d.w01 = info[s01 * kWave + lane];
-    d.w11 = info[s11 * kWave + lane];
-    d.h00 = d.h10 = d.h01 = 0;
-    if (lane == kWave - 1 && pz + 1 < g.g2) {  // position z0 + 64, in the row's next segment
-        d.h00 = info[s * kWave + lane + 1];
-        d.h10 = info[s10 * kWave + lane + 1];
-        d.h01 = info[s01 * kWave + lane + 1];
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const bool row = px - i >= 0 && py - j >= 0;  // wave-uniform
-            const int64_t r = row ? s - i * xstride(g) - j * g.nchunk : s;
-            d.rowd[2 * i + j] = row ? (int32_t)(seg[r].f - d.pabs) : 0;
-            d.cur[2 * i + j] = (i || j) ? (row ? info[r * kWave + lane] : 0u) : d.w0;
-            d.prev[2 * i + j] = (row && !(i && j) && pz >= 1) ? info[r * kWave + lane - 1] : 0u;
-        }
-    return d;
+// Patches before position l of a segment (b = bits below l).
+__device__ __forceinline__ int patches_below(uint64_t A, Plane2 m, uint64_t b) {
+    return (int)__popcll(A & b) + (int)__popcll(m.a & b) + 2 * (int)__popcll(m.b & b);
+}
+// MC vertex of an edge as a patch sums it: zero where the edge does not cross (on NaN samples only,
+// for an edge whose ends' inside bits differ).
+template <typename S, bool DEF>
+__device__ __forceinline__ V3<S> patch_edge_vertex(const In<S> &in, int x, int y, int z, int axis) {
+    const EdgeEnds<S, DEF> e = edge_ends<S, DEF>(in, x, y, z, axis);
+    const V3<S> p = lerp_vertex<S, DEF>(x, y, z, axis, e.d0, e.d1, e.f0, e.f1, in.iso);
+    const bool nan = e.d0 != e.d0 || e.d1 != e.d1;
+    return V3<S>{nan ? S(0) : p.x, nan ? S(0) : p.y, nan ? S(0) : p.z};
 }
 
-// One segment that has patches (hence cells, so rows +x, +y exist).
+// One unit of 64 active cells: its patch vertices and the quads of the edges its cells own. Both are
+// contiguous rows of the output, in the cells' order.
 template <typename S, bool DEF>
-__device__ __forceinline__ void emit_dmc_segment(const In<S> &in, const SegCtx &sc, const DmcSegIn &d,
-                                                 S *__restrict__ verts, void *__restrict__ faces,
-                                                 uint8_t *__restrict__ vinfo, const OutCfg &out, const Norm<S> &nm,
-                                                 DmcEmitLds<S> &L, int lane) {
-    wave_lds_sync();  // the previous segment's LDS reads are done
-    const int64_t pabs = d.pabs, pbase = pabs - sc.f0;
-    const int px = d.sp.px, py = d.sp.py;
-    const int z0 = d.sp.chunk * kWave;
-    const int64_t qbase = d.vabs - sc.v0;
-    const uint32_t w0 = d.w0;
-    // Crossing masks of the rows the cells' edges start from: 10, 01, 11 (this z) and the halo.
-    const int m00 = info_mask(w0), m10 = info_mask(d.w10), m01 = info_mask(d.w01), m11 = info_mask(d.w11);
-    const int h00 = info_mask(d.h00), h10 = info_mask(d.h10), h01 = info_mask(d.h01);
-    // Exclusive prefixes over the lanes, in two packed scans of 10-bit fields (wave totals <= 448):
-    // the patch counts of rows (0,0) (the segment's own; also the first vertices of row (0,0)'s
-    // cells below), (0,-1), (-1,0) and (-1,-1) at this z, and the owned crossing edges (quads).
-    const int np = info_count(w0);
-    const uint32_t cA = (uint32_t)np | (uint32_t)info_count(d.cur[1]) << 10 | (uint32_t)info_count(d.cur[2]) << 20;
-    const uint32_t cB = (uint32_t)info_count(d.cur[3]) | (uint32_t)popc3(m00) << 10;
-    const uint32_t iA = wave_incl_dpp(cA), iB = wave_incl_dpp(cB);
-    const uint32_t eA = iA - cA, eB = iB - cB;
-    const uint32_t tA = (uint32_t)__builtin_amdgcn_readlane((int)iA, kWave - 1),
-                   tB = (uint32_t)__builtin_amdgcn_readlane((int)iB, kWave - 1);
-    const int pp = (int)(eA & 0x3ff), tp = (int)(tA & 0x3ff);
-    const int pq = (int)((eB >> 10) & 0x3ff), tq = (int)((tB >> 10) & 0x3ff);
-    const int rowpre[4] = {pp, (int)((eA >> 10) & 0x3ff), (int)((eA >> 20) & 0x3ff), (int)(eB & 0x3ff)};
-    // Codes and first vertices of the cells (-i, -j, 0) and (-i, -j, -1).
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t cur = d.cur[2 * i + j], prev = d.prev[2 * i + j];
-            const int b = rowpre[2 * i + j];
-            if (lane == 0) L.rowb[2 * i + j] = d.rowd[2 * i + j];
-            L.code[4 * i + 2 * j][lane] = (uint8_t)info_code(cur);
-            L.pre[4 * i + 2 * j][lane] = (int16_t)b;
-            L.code[4 * i + 2 * j + 1][lane] = (uint8_t)info_code(prev);
-            L.pre[4 * i + 2 * j + 1][lane] = (int16_t)(b - info_count(prev));
-        }
-    // list writes without per-lane branches: what is not listed goes to the spare last entry
+__device__ __forceinline__ void emit_dmc_unit(const In<S> &in, const UnitGrid &G, uint32_t u, uint32_t nunits,
+                                              S *__restrict__ verts, void *__restrict__ faces,
+                                              uint8_t *__restrict__ vinfo, const OutCfg &out, const Norm<S> &nm,
+                                              const uint64_t *s_case, DmcEmitLds<S> &L, int lane) {
+    wave_lds_sync();  // the previous unit's LDS reads are done
+    uint32_t s;
+    int l;
+    const int n = unit_cells(G, u, nunits, L.eitem, lane, &s, &l);
+    if (n == 0) return;  // wave-uniform
+    const Geo &g = in.geo;
+    const SegPos sp = seg_pos(g, (int64_t)s - G.first);
+    const int px = sp.px, py = sp.py, z = sp.chunk * kWave + l;
+    const bool on = lane < n;
+
+    // Loads: the cell's own planes and code; of rows -x, -y, -x-y the patch planes, the base and the
+    // codes at z and z - 1 (a cell that shares a crossing edge with an active one is active, so the
+    // codes that are used have been written).
+    const Plane2 qxy = G.P.xy[s], qza = G.P.za[s];
+    const bool rx = px > 0, ry = py > 0, rz = z > 0;
+    const int64_t sx = rx ? xstride(g) : 0, sy = ry ? g.nchunk : 0;
+    const int64_t s10 = (int64_t)s - sx, s01 = (int64_t)s - sy, s11 = rx && ry ? (int64_t)s - sx - sy : (int64_t)s;
+    const int below1 = rz ? 1 : 0;
+    const uint8_t *cd = G.P.codes + l;
+    uint32_t code = cd[(int64_t)s * kWave];
+    uint32_t cx0 = cd[s10 * kWave], cx1 = (cd - below1)[s10 * kWave];
+    uint32_t cy0 = cd[s01 * kWave], cy1 = (cd - below1)[s01 * kWave];
+    uint32_t cxy = cd[s11 * kWave];
+    uint32_t cz1 = (cd - below1)[(int64_t)s * kWave];
+    const uint64_t inside = G.P.inside[s];
+    const uint64_t ax = G.P.za[s10].b, ay = G.P.za[s01].b, aw = G.P.za[s11].b;
+    const Plane2 mx = G.P.m[s10], my = G.P.m[s01], mw = G.P.m[s11];
+    const int64_t fx = G.seg[s10].f, fy = G.seg[s01].f, fw = G.seg[s11].f, fs = G.seg[s].f;
+    const uint64_t b = (1ull << l) - 1;
+
+    // first patch and first quad of the unit: those of its first cell
+    const uint64_t b0 = (uint64_t)readlane64((int64_t)b, 0);
+    const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)s);
+    const Plane2 q0 = load_uniform(&G.P.xy[s0]), w0 = load_uniform(&G.P.za[s0]), m0 = load_uniform(&G.P.m[s0]);
+    const int64_t pbase = G.seg[s0].f - G.f0 + patches_below(w0.b, m0, b0);
+    const int64_t qbase = G.seg[s0].v - G.v0 + RowEdges{q0.a, q0.b, w0.a}.below(b0);
+    const int64_t pabs = pbase + G.f0;
+
+    // crossing kinds of the edges at the cell's own z; where the owner's row anchors no cells, or
+    // (top edges) the next position, an edge counts as not crossing
+    const bool gx = px + 1 < g.g0 - 1, gy = py + 1 < g.g1 - 1, gz = z + 1 < g.g2 - 1;
+    const uint32_t keep = (gx ? 0xffu : 0x7du) & (gy ? 0xffu : 0xd7u) & (gx && gy ? 0xffu : 0xefu);
+    const uint64_t cwd = s_case[code];
+    const uint32_t kb = on ? (uint32_t)(cwd >> 56) & keep : 0u;
+    const int np = on ? DISO_DMC_NPATCH(cwd) : 0;
+    const int ex = on ? bit_at(qxy.a, l) : 0, ey = on ? bit_at(qxy.b, l) : 0, ez = on ? bit_at(qza.a, l) : 0;
+    // exclusive prefixes of the edge slots (<= 512), patches (<= 256) and quads (<= 192): one scan
+    const uint32_t c = (uint32_t)__popc(kb) | (uint32_t)np << 10 | (uint32_t)(ex + ey + ez) << 20;
+    const uint32_t ic = wave_incl_dpp(c), ec = ic - c;
+    const uint32_t tc = (uint32_t)__builtin_amdgcn_readlane((int)ic, kWave - 1);
+    const int pe = (int)(ec & 0x3ff), pp = (int)((ec >> 10) & 0x3ff), pq = (int)(ec >> 20);
+    const int te = (int)(tc & 0x3ff), tp = (int)((tc >> 10) & 0x3ff), tq = (int)(tc >> 20);
+    // the position above the last cell: its crossing kinds are that cell's top edges
+    const uint32_t lcode = (uint32_t)__builtin_amdgcn_readlane((int)code, n - 1);
+    const uint32_t lkeep = (uint32_t)__builtin_amdgcn_readlane((int)(gz ? keep : 0u), n - 1);
+    const uint32_t hk = top_kinds(lcode) & lkeep;
+    const int nslot = te + __popc(hk);
+    const bool slots = nslot <= kEdgeSlots;  // wave-uniform
+
+    if (on) {
+        // bit 11: the top edges are the next cell's (they cross only where its position has a cell)
+        L.cw[lane + 1] = (uint32_t)(pe + 1) | (uint32_t)bit_at(inside, l) << 10 | (gz ? 1u << 11 : 0u) | kb << 16 | code << 24;
+        L.cx[lane] = px;
+        L.cy[lane] = py;
+        L.cz[lane] = z;
+        L.pp[lane] = (uint16_t)pp;
+    }
+    if (lane == n - 1) {
+        L.cx[n] = px;
+        L.cy[n] = py;
+        L.cz[n] = z + 1;
+        L.cw[n + 1] = (uint32_t)(te + 1) | hk << 16;
+    }
+    if (lane == 0) L.cw[0] = (rz ? cz1 : 0u) << 24;
+    // list writes without per-lane branches: what is not listed goes to the spare entry
 #pragma unroll
     for (int k = 0; k < 4; ++k) L.patch[k < np ? pp + k : 4 * kWave] = (uint8_t)(lane * 4 + k);
-    {
-        // an owned crossing edge leaves the inside when the position's sample is >= iso
-        // (type a + 3, src/cudualmc.cu:782-788)
-        const int leaving = info_inside(w0);
-        int q = pq;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const int on = (m00 >> a) & 1;
-            L.quad[on ? q : 3 * kWave] = (uint16_t)(lane * 8 + a * 2 + leaving);
-            q += on;
-        }
-    }
-    // Edge slots: kinds 0..7 at every lane, then the halo kinds 8..11 (lane 63 only).
-    const int kbits = (m00 & 7) | (((m10 >> 1) & 3) << 3) | ((m01 & 1) << 5) | (((m01 >> 2) & 1) << 6) |
-                      (((m11 >> 2) & 1) << 7);
-    const int hbits = (h00 & 3) | (((h10 >> 1) & 1) << 2) | ((h01 & 1) << 3);
-    // Slots are numbered kind by kind, lanes in order within a kind: the lane's exclusive prefix
-    // per kind from two DPP scans of the kind bits spread into 8-bit fields (x * 0x204081 moves bit
-    // i of a 4-bit x to bit 8i), the kinds' wave totals from the scans' last lane; the halo kinds
-    // (lane 63 only) follow all of them.
-    const uint32_t c0 = ((uint32_t)(kbits & 15) * 0x204081u) & 0x01010101u;
-    const uint32_t c1 = ((uint32_t)(kbits >> 4) * 0x204081u) & 0x01010101u;
-    const uint32_t i0 = wave_incl_dpp(c0), i1 = wave_incl_dpp(c1);
-    const uint32_t e0 = i0 - c0, e1 = i1 - c1;
-    const uint32_t t0 = (uint32_t)__builtin_amdgcn_readlane((int)i0, kWave - 1),
-                   t1 = (uint32_t)__builtin_amdgcn_readlane((int)i1, kWave - 1);
-    const int hb = __builtin_amdgcn_readlane(hbits, kWave - 1);
-    int nslot = 0, myslot[12];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        const int sh = 8 * (k & 3);
-        const int ex = (int)(((k < 4 ? e0 : e1) >> sh) & 0xff);
-        myslot[k] = ((kbits >> k) & 1) ? nslot + ex : -1;
-        L.slot[k][lane] = (uint8_t)myslot[k];
-        nslot += (int)(((k < 4 ? t0 : t1) >> sh) & 0xff);
-    }
-#pragma unroll
-    for (int h = 0; h < 4; ++h) {
-        // hb is wave-uniform, so every lane writes the same halo entry (kinds 0, 1, 3, 5)
-        const int hs = ((hb >> h) & 1) ? nslot + __popc(hb & ((1 << h) - 1)) : -1;
-        myslot[8 + h] = ((hbits >> h) & 1) ? hs : -1;
-        L.slot[h < 2 ? h : 2 * h - 1][kWave] = (uint8_t)hs;
-    }
-    nslot += __popc(hb);
-    const bool slots = nslot <= kEdgeSlots;  // wave-uniform
+    L.quad[ex ? pq : 3 * kWave] = (uint8_t)(lane * 4);
+    L.quad[ey ? pq + ex : 3 * kWave] = (uint8_t)(lane * 4 + 1);
+    L.quad[ez ? pq + ex + ey : 3 * kWave] = (uint8_t)(lane * 4 + 2);
     if (slots) {
-        // slots are < kEdgeSlots here, so the edges that do not cross (-1 & 0xff) all write the
-        // spare last item, and no lane needs its own branch
+        int r = pe + 1;
 #pragma unroll
-        for (int k = 0; k < 12; ++k) L.eitem[myslot[k] & 0xff] = (uint16_t)((lane << 4) | k);
+        for (int k = 0; k < 8; ++k) {
+            const int x = (int)((kb >> k) & 1);
+            L.eitem[x ? r : 0] = (uint16_t)(lane * 8 + k);
+            r += x;
+        }
+        if (lane < 8 && ((hk >> lane) & 1)) L.eitem[te + 1 + __popc(hk & ((1u << lane) - 1))] = (uint16_t)(n * 8 + lane);
     }
+    // neighbour rows (where there is none, the quad corner is one before the segment's first patch)
+    const int32_t own0 = (int32_t)(fs - pabs);
+    L.nf[0][lane] = rx ? (int32_t)(fx - pabs) + patches_below(ax, mx, b) : own0;
+    L.nf[1][lane] = ry ? (int32_t)(fy - pabs) + patches_below(ay, my, b) : own0;
+    L.nf[2][lane] = rx && ry ? (int32_t)(fw - pabs) + patches_below(aw, mw, b) : own0;
+    L.nc[lane] = (rx ? cx0 | (rz ? cx1 << 8 : 0u) : 0u) | (ry ? cy0 << 16 | (rz ? cy1 << 24 : 0u) : 0u);
+    L.nd[lane] = (uint8_t)(rx && ry ? cxy : 0u);
     wave_lds_sync();
 
+    // quads: corner 0 is the own cell's vertex; corners B, C, D those of the other three cells around
+    // the edge (X: -y, -y below, below; Y: below, -x below, -x; Z: -x, -x-y, -y), in that order or,
+    // where the edge leaves the inside, in reverse. A cell below a row's cell at z has its patches
+    // right before that cell's.
+    const bool vec = ((uintptr_t)faces & 15) == 0;  // a quad's four indices in 16-byte stores
+    for (int k = lane; k < tq; k += kWave) {
+        const int64_t qi = qbase + k;
+        if (qi >= out.fcap) continue;
+        const int it = L.quad[k], src = it >> 2, axis = it & 3;
+        const uint32_t w = L.cw[src + 1], wb = L.cw[src] >> 24, nc = L.nc[src], nd = L.nd[src];
+        const int32_t f0 = L.pp[src], fx0 = L.nf[0][src], fy0 = L.nf[1][src], fw0 = L.nf[2][src];
+        const bool isx = axis == 0, isy = axis == 1;
+        const uint32_t czb = L.cz[src] > 0 ? wb : 0u;
+        const uint64_t wa = s_case[w >> 24];
+        const uint64_t wB = s_case[isx ? (nc >> 16) & 0xff : (isy ? czb : nc & 0xff)];
+        const uint64_t wC = s_case[isx ? nc >> 24 : (isy ? (nc >> 8) & 0xff : nd)];
+        const uint64_t wD = s_case[isx ? czb : (isy ? nc & 0xff : (nc >> 16) & 0xff)];
+        const int pa = (int)(wa >> (isx ? 0 : (isy ? 24 : 9))) & 7;         // edges 0, 8, 3
+        const int pB = (int)(wB >> (isx ? 12 : (isy ? 33 : 3))) & 7;        // edges 4, 11, 1
+        const int pC = (int)(wC >> (isx ? 18 : (isy ? 30 : 15))) & 7;       // edges 6, 10, 5
+        const int pD = (int)(wD >> (isx ? 6 : (isy ? 27 : 21))) & 7;        // edges 2, 9, 7
+        const int32_t va = f0 + (pa == 7 ? -1 : pa);
+        const int32_t vB = (isx ? fy0 : (isy ? f0 - DISO_DMC_NPATCH(wB) : fx0)) + (pB == 7 ? -1 : pB);
+        const int32_t vC = (isx ? fy0 - DISO_DMC_NPATCH(wC) : (isy ? fx0 - DISO_DMC_NPATCH(wC) : fw0)) + (pC == 7 ? -1 : pC);
+        const int32_t vD = (isx ? f0 - DISO_DMC_NPATCH(wD) : (isy ? fx0 : fy0)) + (pD == 7 ? -1 : pD);
+        const bool leaving = (w >> 10) & 1;
+        const int32_t rel[4] = {va, leaving ? vD : vB, vC, leaving ? vB : vD};
+        store_quad(faces, qi, pbase, rel, out.flags, vec);
+    }
+    wave_lds_sync();  // the neighbour rows' entries give way to the vertices
+
     if (slots) {
+        if (lane < 3) L.ev[lane][0] = S(0);
         // MC vertex of every crossing edge of the cells, once
         for (int i = lane; i < nslot; i += kWave) {
-            const int it = L.eitem[i], l = it >> 4, k0 = it & 15;
-            const int k = k0 < 8 ? k0 : (k0 == 8 ? 0 : (k0 == 9 ? 1 : (k0 == 10 ? 3 : 5)));
-            // kinds 3, 4, 7 start at dx = 1; 5, 6, 7 at dy = 1; 2, 4, 6, 7 run along z, 1 and 3 along y
-            const int dx = (0x98 >> k) & 1, dy = (0xE0 >> k) & 1, a = (0xD4 >> k) & 1 ? 2 : (0x0A >> k) & 1;
-            const V3<S> p = edge_vertex<S, DEF>(in, px + dx, py + dy, z0 + (k0 < 8 ? l : kWave), a);
-            L.ev[0][i] = p.x;
-            L.ev[1][i] = p.y;
-            L.ev[2][i] = p.z;
+            const int it = L.eitem[i + 1], src = it >> 3, k = it & 7;
+            const int dx = (kKindX >> k) & 1, dy = (kKindY >> k) & 1, a = (kKindAxisZ >> k) & 1 ? 2 : (kKindAxisY >> k) & 1;
+            const V3<S> p = patch_edge_vertex<S, DEF>(in, L.cx[src] + dx, L.cy[src] + dy, L.cz[src], a);
+            L.ev[0][i + 1] = p.x;
+            L.ev[1][i + 1] = p.y;
+            L.ev[2][i + 1] = p.z;
         }
         wave_lds_sync();
     }
 
-    constexpr uint64_t kKinds = edge_kind_table();
     for (int k = lane; k < tp; k += kWave) {
         const int it = L.patch[k], src = it >> 2, pk = it & 3;
-        unsigned em = (unsigned)(kDmcPatchEdges.m[L.code[0][src]] >> (16 * pk)) & 0xfffu;
+        const uint32_t w0 = L.cw[src + 1];
+        unsigned em = (unsigned)(kDmcPatchEdges.m[w0 >> 24] >> (16 * pk)) & 0xfffu;
         const int num = __popc(em);
-        S sx = S(0), sy = S(0), sz = S(0);
+        S sx2 = S(0), sy2 = S(0), sz2 = S(0);
         if (slots) {
-            // the slots of all twelve edges first (independent reads), then all twelve vertices
-            // added in ascending edge order, edges outside the patch (and, on NaN samples only,
-            // patch edges that do not cross) reading the zero entry: the running sum starts at
-            // +0 and so is never -0, and adding +0 leaves it unchanged
+            // the slots of all twelve edges first, then all twelve vertices added in ascending edge
+            // order, edges outside the patch (or not counted as crossing) reading the zero entry: the
+            // running sum starts at +0 and so is never -0, and adding +0 leaves it unchanged
+            const uint32_t w1 = L.cw[src + 2];
+            const uint32_t k0 = (w0 >> 16) & 0xff, k1 = (w0 >> 11) & 1 ? (w1 >> 16) & 0xff : 0u;
+            int r0 = (int)(w0 & 0x3ff);
+            const int r1 = (int)(w1 & 0x3ff);
             int sl[12];
 #pragma unroll
-            for (int e = 0; e < 12; ++e) {
-                const int v = (int)(kKinds >> (5 * e)) & 31, kd = v & 7, top = v >> 3;
-                // a top edge belongs to the next position (lane src + 1, or the halo entry after lane 63)
-                const int sv = L.slot[kd][src + top];
-                sl[e] = ((em >> e) & 1) ? sv : kEdgeSlots;
+            for (int k2 = 0; k2 < 8; ++k2) {
+                const int e = kind_edge(k2), x = (int)(k0 >> k2) & 1;
+                sl[e] = (x & (int)(em >> e)) ? r0 : 0;
+                r0 += x;
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int e = kTopEdges[t], kd = kTopKinds[t];
+                sl[e] = ((k1 >> kd) & (em >> e) & 1) ? r1 + __popc(k1 & ((1u << kd) - 1)) : 0;
             }
 #pragma unroll
             for (int e = 0; e < 12; ++e) {
-                sx += L.ev[0][sl[e]];
-                sy += L.ev[1][sl[e]];
-                sz += L.ev[2][sl[e]];
+                sx2 += L.ev[0][sl[e]];
+                sy2 += L.ev[1][sl[e]];
+                sz2 += L.ev[2][sl[e]];
             }
         } else {
-            const int z = z0 + src;
+            const int x0 = L.cx[src], y0 = L.cy[src], z0 = L.cz[src];
+            const bool okx = x0 + 1 < g.g0 - 1, oky = y0 + 1 < g.g1 - 1, okz = z0 + 1 < g.g2 - 1;
             while (em) {  // ascending edge order
                 const int e = __ffs(em) - 1;
                 em &= em - 1;
-                const V3<S> p = edge_vertex<S, DEF>(in, px + eox(e), py + eoy(e), z + eoz(e), eax(e));
-                sx += p.x;
-                sy += p.y;
-                sz += p.z;
+                if ((eox(e) && !okx) || (eoy(e) && !oky) || (eoz(e) && !okz)) continue;
+                const V3<S> p = patch_edge_vertex<S, DEF>(in, x0 + eox(e), y0 + eoy(e), z0 + eoz(e), eax(e));
+                sx2 += p.x;
+                sy2 += p.y;
+                sz2 += p.z;
             }
         }
         const S r = rcp_small<S>(num);
-        store_vertex(verts, pbase + k, out.vcap, epilogue(V3<S>{sx * r, sy * r, sz * r}, out.flags, nm));
+        store_vertex(verts, pbase + k, out.vcap, epilogue(V3<S>{sx2 * r, sy2 * r, sz2 * r}, out.flags, nm));
         if (pbase + k < out.vcap) put(vinfo + pbase + k, (uint8_t)(num | (pk << 3)));
-    }
-    const bool vec = ((uintptr_t)faces & 15) == 0;  // a quad's four indices in 16-byte stores
-    for (int k = lane; k < tq; k += kWave) {
-        const int it = L.quad[k], src = it >> 3, ty = ((it >> 1) & 3) + 3 * (it & 1);
-        const int64_t q = qbase + k;
-        if (q >= out.fcap) continue;
-        const uint32_t stw = kStencil.w[ty];
-        int32_t rel[4];  // corner ids relative to the segment's first DMC vertex
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int ci = (stw >> (3 * j)) & 7, eid = (stw >> (12 + 4 * j)) & 15;
-            const int p = DISO_DMC_PATCH_OF(kDmcCase[L.code[ci][src]], eid);
-            // dmcEdgeOffset is -1 for a non-crossing edge (never the case on a padded grid)
-            rel[j] = L.rowb[ci >> 1] + L.pre[ci][src] + (p == 7 ? -1 : p);
-        }
-        store_quad(faces, q, pbase, rel, out.flags, vec);
     }
 }
 
+// The DMC case words with each code's own_kinds in the free top byte, in LDS.
+__device__ __forceinline__ void load_dmc_cases(uint64_t *s_case) {
+    for (int i = threadIdx.x; i < 256; i += kBlock) s_case[i] = kDmcCase[i] | (uint64_t)own_kinds((uint32_t)i) << 56;
+}
+
 template <typename S, bool DEF>
-__global__ __launch_bounds__(kBlock, 6) void emit_dmc_kernel(In<S> in, const SegBase *__restrict__ seg,
+__global__ __launch_bounds__(kBlock, 5) void emit_dmc_kernel(In<S> in, const SegBase *__restrict__ seg, Planes planes,
                                                           S *__restrict__ verts, void *__restrict__ faces,
-                                                          uint8_t *__restrict__ vinfo, OutCfg out, Norm<S> nm,
-                                                          int run, int64_t nblocks) {
+                                                          uint8_t *__restrict__ vinfo, OutCfg out, Norm<S> nm) {
+    __shared__ uint64_t s_case[256];
     __shared__ DmcEmitLds<S> s_lds[kWavesPerBlock];
-    __shared__ uint32_t s_take;
-    const int tid = threadIdx.x, wave = wave_id(), lane = tid % kWave;
-    if (tid == 0) s_take = 0;
-    if (lane < 3) s_lds[wave].ev[lane][kEdgeSlots] = S(0);  // the zero entry of the patch sums
-    __syncthreads();
-    const Geo &g = in.geo;
-    const SegCtx sc{seg, info_of(seg, g), 0, 0};
-    const SegBase *tot = seg + g.nseg;
+    const int wave = wave_id(), lane = threadIdx.x % kWave;
+    const SegBase *tot = seg + in.geo.nseg;
     if (tot[0].v > out.fcap || tot[0].f > out.vcap) return;
-    const int64_t lo = xcd_block(blockIdx.x, nblocks) * run, hi = lo + run < g.nseg ? lo + run : g.nseg;
-    // segments of the run with patches (hence owned crossings)
-    const uint64_t act = run_active(seg, lo, hi, lane);
-    const SegPos lp = seg_pos(g, lo + lane);
-    run_segments(
-        act, &s_take, lane, [&](int i) { return dmc_load<S>(in, sc, lo + i, pos_of_lane(lp, i), lane); },
-        [&](const DmcSegIn &d) { emit_dmc_segment<S, DEF>(in, sc, d, verts, faces, vinfo, out, nm, s_lds[wave], lane); });
+    load_dmc_cases(s_case);
+    __syncthreads();
+    const uint32_t nunits = *planes.nunits;
+    const UnitGrid G{seg, planes, 0, in.geo.nseg - 1, 0, 0};
+    for_units(0, nunits, blockIdx.x, gridDim.x, wave, [&](uint32_t u) {
+        emit_dmc_unit<S, DEF>(in, G, u, nunits, verts, faces, vinfo, out, nm, s_case, s_lds[wave], lane);
+    });
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1900,7 +1843,8 @@ struct BwdSegIn {
     SegPos sp;
     int64_t v;
     int32_t dm0, d0m;  // first vertices of rows -x, -y relative to the segment's
-    uint32_t w00, wm0, w0m, wzm;
+    RowEdges e00, em0, e0m;  // crossing planes of the segment and of rows -x, -y
+    uint64_t zp;             // and the z plane of the previous chunk
 };
 
 template <bool RECOMP>
@@ -1914,13 +1858,14 @@ __device__ __forceinline__ BwdSegIn bwd_load(const Geo &g, const SegCtx &sc, int
     d.v = seg[s].v;
     d.dm0 = sm0 >= 0 ? (int32_t)(seg[sm0].v - d.v) : 0;
     d.d0m = s0m >= 0 ? (int32_t)(seg[s0m].v - d.v) : 0;
-    d.w00 = d.wm0 = d.w0m = d.wzm = 0;
+    d.e00 = d.em0 = d.e0m = RowEdges{0, 0, 0};
+    d.zp = 0;
     if constexpr (!RECOMP) {
-        const uint16_t *info = sc.info;
-        d.w00 = info[s * kWave + lane];
-        if (sm0 >= 0) d.wm0 = info[sm0 * kWave + lane];
-        if (s0m >= 0) d.w0m = info[s0m * kWave + lane];
-        if (sp.chunk * kWave + lane > 0) d.wzm = info[s * kWave + lane - 1];
+        const Plane2 *__restrict__ xy = sc.xy, *__restrict__ za = sc.za;
+        d.e00 = RowEdges{xy[s].a, xy[s].b, za[s].a};
+        if (sm0 >= 0) d.em0 = RowEdges{xy[sm0].a, xy[sm0].b, za[sm0].a};
+        if (s0m >= 0) d.e0m = RowEdges{xy[s0m].a, xy[s0m].b, za[s0m].a};
+        if (sp.chunk > 0) d.zp = za[s - 1].a;
     }
     return d;
 }
@@ -1953,10 +1898,10 @@ __device__ __forceinline__ void bwd_segment(const In<S> &in, const SegCtx &sc, c
         m0m = is_anchor(in, px, py - 1, pz) ? own_mask(w(0, -1, 0), w(1, -1, 0), c, w(0, -1, 1), iso) : 0;
         mzm = is_anchor(in, px, py, pz - 1) ? crosses(w(0, 0, -1), c, iso) << 2 : 0;
     } else {
-        m00 = info_mask(sg.w00);
-        mm0 = info_mask(sg.wm0);
-        m0m = info_mask(sg.w0m);
-        mzm = info_mask(sg.wzm);
+        m00 = mask_of(sg.e00.X, sg.e00.Y, sg.e00.Z);
+        mm0 = mask_of(sg.em0.X, sg.em0.Y, sg.em0.Z);
+        m0m = mask_of(sg.e0m.X, sg.e0m.Y, sg.e0m.Z);
+        mzm = bit_of(diso_bits::down1(sg.e00.Z, sg.zp)) << 2;
     }
     // slots 0-2: edges the vertex owns; 3-5: the x edge of -x, the y edge of -y, the z edge of -z
     const int inc_m = (mm0 & 1) | (m0m & 2) | (mzm & 4);
@@ -2055,7 +2000,7 @@ __global__ __launch_bounds__(kBlock) void bwd_mc_kernel(In<S> in, const SegBase 
     __shared__ BwdLds<S> s_lds[kWavesPerBlock];
     const int tid = threadIdx.x, wave = wave_id(), lane = tid % kWave;
     const Geo &g = in.geo;
-    const SegCtx sc{seg, info_of(seg, g), 0, 0};
+    const SegCtx sc = seg_ctx(seg, planes_of(seg, g.nseg));
     const int64_t lo = xcd_block(blockIdx.x, nblocks) * run, hi = lo + run < g.nseg ? lo + run : g.nseg;
     const int64_t t = lo + lane;
     const SegPos lp = seg_pos(g, t);
@@ -2137,14 +2082,15 @@ __global__ __launch_bounds__(kBlock) void dmc_edge_grad_kernel(const void *__res
 
 
 template <typename S>
-__device__ __forceinline__ SegCtx batch_ctx(const BatchGrid<S> &G, const SegBase *seg, const uint16_t *info) {
-    return SegCtx{seg + G.seg_first, info + G.seg_first * kWave, seg[G.seg_first].v, seg[G.seg_first].f};
+__device__ __forceinline__ SegCtx batch_ctx(const BatchGrid<S> &G, const SegBase *seg, const Planes &q) {
+    const int64_t f = G.seg_first;
+    return SegCtx{seg + f, q.xy + f, q.za + f, seg[f].v, seg[f].f};
 }
 
 template <typename S>
 __global__ void batch_totals_kernel(const BatchGrid<S> *__restrict__ grids, int n, int64_t nseg,
-                                    const SegBase *__restrict__ seg, uint32_t *__restrict__ gflags,
-                                    diso_totals_t *__restrict__ out) {
+                                    const SegBase *__restrict__ seg, Planes planes, uint32_t *__restrict__ gflags,
+                                    uint32_t *__restrict__ range, diso_totals_t *__restrict__ out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const SegBase a = seg[grids[i].seg_first], e = seg[i + 1 < n ? grids[i + 1].seg_first : nseg];
@@ -2155,65 +2101,78 @@ __global__ void batch_totals_kernel(const BatchGrid<S> *__restrict__ grids, int 
     out[i].flags = (int64_t)(gflags[i] | ((uint32_t)seg[nseg + 1].v & DISO_TOTAL_SCAN_TIMEOUT));
     out[i].n_crossing = cross;
     gflags[i] = 0u;  // ready for the next batch
+    // the grid's units: from the one that holds its first cell (the last to start before the grid's
+    // segments, which may end before them too) to the last that starts in them
+    const uint32_t nu = nseg >= 4 ? *planes.nunits : 0u;
+    auto lower = [&](int64_t s) {  // units that start before segment s
+        uint32_t lo = 0, hi = nu;
+        while (lo < hi) {
+            const uint32_t mid = lo + (hi - lo) / 2;
+            if ((int64_t)planes.unit[mid] < s)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        return lo;
+    };
+    const uint32_t u0 = lower(grids[i].seg_first), u1 = lower(i + 1 < n ? grids[i + 1].seg_first : nseg);
+    range[2 * i] = u0 > 0 ? u0 - 1 : 0u;
+    range[2 * i + 1] = u1;
+}
+
+// Batched emission: a grid's blocks go through its units in turn. Units are of the whole batch, so a
+// grid's first and last may hold cells of its neighbours too (unit_cells leaves them out).
+template <typename S, typename F>
+__device__ __forceinline__ void batch_units(const BatchGrid<S> *__restrict__ grids, const int32_t *__restrict__ gl,
+                                            const int64_t *__restrict__ rf, int m, const SegBase *__restrict__ seg,
+                                            const Planes &planes, const uint32_t *__restrict__ range, int64_t nblocks,
+                                            int wave, F f) {
+    const int64_t b = xcd_block(blockIdx.x, nblocks);
+    const int j = find_group(rf, m, b);
+    const int gi = gl[j];
+    const BatchGrid<S> &B = grids[gi];
+    if (B.nv > B.vcap || B.nf > B.fcap) return;
+    const In<S> in = B.in;
+    const int64_t first = B.seg_first;
+    const UnitGrid G{seg, planes, first, first + in.geo.nseg - 1, seg[first].v, seg[first].f};
+    const OutCfg out{B.flags, B.vcap, B.fcap};
+    const uint32_t nunits = *planes.nunits, hi = range[2 * gi + 1], step = (uint32_t)(rf[j + 1] - rf[j]) * kWavesPerBlock;
+    for (uint32_t u = range[2 * gi] + (uint32_t)(b - rf[j]) * kWavesPerBlock + (uint32_t)wave; u < hi; u += step)
+        f(in, G, B, out, u, nunits);
 }
 
 template <typename S, bool DEF>
-__global__ __launch_bounds__(kBlock, 7) void emit_mc_batch_kernel(const BatchGrid<S> *__restrict__ grids,
+__global__ __launch_bounds__(kBlock, 6) void emit_mc_batch_kernel(const BatchGrid<S> *__restrict__ grids,
                                                                const int32_t *__restrict__ gl,
                                                                const int64_t *__restrict__ rf, int m,
-                                                               const SegBase *__restrict__ seg,
-                                                               const uint16_t *__restrict__ info, int64_t nblocks) {
+                                                               const SegBase *__restrict__ seg, Planes planes,
+                                                               const uint32_t *__restrict__ range, int64_t nblocks) {
     __shared__ uint64_t s_case[256];
     __shared__ McEmitLds s_lds[kWavesPerBlock];
-    __shared__ uint32_t s_take;
-    const int tid = threadIdx.x, wave = wave_id(), lane = tid % kWave;
-    for (int i = tid; i < 256; i += kBlock) s_case[i] = kMcCase[i];
-    if (tid == 0) s_take = 0;
+    const int wave = wave_id(), lane = threadIdx.x % kWave;
+    load_mc_cases(s_case);
     __syncthreads();
-    const int64_t b = xcd_block(blockIdx.x, nblocks);
-    const int j = find_group(rf, m, b);
-    const BatchGrid<S> &G = grids[gl[j]];
-    if (G.nv > G.vcap || G.nf > G.fcap) return;
-    const In<S> in = G.in;
-    const SegCtx sc = batch_ctx(G, seg, info);
-    const OutCfg out{G.flags, G.vcap, G.fcap};
-    const int64_t lo = (b - rf[j]) * G.run, hi = lo + G.run < in.geo.nseg ? lo + G.run : in.geo.nseg;
-    const uint64_t act = run_active(sc.seg, lo, hi, lane);
-    const SegPos lp = seg_pos(in.geo, lo + lane);
-    run_segments(
-        act, &s_take, lane, [&](int i) { return mc_load<S>(in, sc, lo + i, pos_of_lane(lp, i), lane); },
-        [&](const McSegIn &d) {
-            emit_mc_segment<S, DEF>(in, sc, d, G.verts, G.faces, out, G.nm, s_case, s_lds[wave], lane);
-        });
+    batch_units(grids, gl, rf, m, seg, planes, range, nblocks, wave,
+                [&](const In<S> &in, const UnitGrid &G, const BatchGrid<S> &B, const OutCfg &out, uint32_t u, uint32_t nunits) {
+                    emit_mc_unit<S, DEF>(in, G, u, nunits, B.verts, B.faces, out, B.nm, s_case, s_lds[wave], lane);
+                });
 }
 
 template <typename S, bool DEF>
-__global__ __launch_bounds__(kBlock, 6) void emit_dmc_batch_kernel(const BatchGrid<S> *__restrict__ grids,
+__global__ __launch_bounds__(kBlock, 5) void emit_dmc_batch_kernel(const BatchGrid<S> *__restrict__ grids,
                                                                 const int32_t *__restrict__ gl,
                                                                 const int64_t *__restrict__ rf, int m,
-                                                                const SegBase *__restrict__ seg,
-                                                                const uint16_t *__restrict__ info, int64_t nblocks) {
+                                                                const SegBase *__restrict__ seg, Planes planes,
+                                                                const uint32_t *__restrict__ range, int64_t nblocks) {
+    __shared__ uint64_t s_case[256];
     __shared__ DmcEmitLds<S> s_lds[kWavesPerBlock];
-    __shared__ uint32_t s_take;
-    const int tid = threadIdx.x, wave = wave_id(), lane = tid % kWave;
-    if (tid == 0) s_take = 0;
-    if (lane < 3) s_lds[wave].ev[lane][kEdgeSlots] = S(0);  // the zero entry of the patch sums
+    const int wave = wave_id(), lane = threadIdx.x % kWave;
+    load_dmc_cases(s_case);
     __syncthreads();
-    const int64_t b = xcd_block(blockIdx.x, nblocks);
-    const int j = find_group(rf, m, b);
-    const BatchGrid<S> &G = grids[gl[j]];
-    if (G.nv > G.vcap || G.nf > G.fcap) return;
-    const In<S> in = G.in;
-    const SegCtx sc = batch_ctx(G, seg, info);
-    const OutCfg out{G.flags, G.vcap, G.fcap};
-    const int64_t lo = (b - rf[j]) * G.run, hi = lo + G.run < in.geo.nseg ? lo + G.run : in.geo.nseg;
-    const uint64_t act = run_active(sc.seg, lo, hi, lane);
-    const SegPos lp = seg_pos(in.geo, lo + lane);
-    run_segments(
-        act, &s_take, lane, [&](int i) { return dmc_load<S>(in, sc, lo + i, pos_of_lane(lp, i), lane); },
-        [&](const DmcSegIn &d) {
-            emit_dmc_segment<S, DEF>(in, sc, d, (S *)G.verts, G.faces, G.vinfo, out, G.nm, s_lds[wave], lane);
-        });
+    batch_units(grids, gl, rf, m, seg, planes, range, nblocks, wave,
+                [&](const In<S> &in, const UnitGrid &G, const BatchGrid<S> &B, const OutCfg &out, uint32_t u, uint32_t nunits) {
+                    emit_dmc_unit<S, DEF>(in, G, u, nunits, (S *)B.verts, B.faces, B.vinfo, out, B.nm, s_case, s_lds[wave], lane);
+                });
 }
 
 // Per-edge upstream gradients of every DMC grid of the batch: blocks of kBlock quads of one grid.
@@ -2239,7 +2198,7 @@ __global__ __launch_bounds__(kBlock) void bwd_batch_kernel(const BatchGrid<S> *_
                                                            const int32_t *__restrict__ gl,
                                                            const int64_t *__restrict__ rf, int m,
                                                            const SegBase *__restrict__ seg,
-                                                           const uint16_t *__restrict__ info,
+                                                           Planes planes,
                                                            const S *__restrict__ ge, int64_t nblocks) {
     __shared__ BwdLds<S> s_lds[kWavesPerBlock];
     const int tid = threadIdx.x, wave = wave_id(), lane = tid % kWave;
@@ -2248,7 +2207,7 @@ __global__ __launch_bounds__(kBlock) void bwd_batch_kernel(const BatchGrid<S> *_
     const BatchGrid<S> &G = grids[gl[j]];
     const In<S> in = G.in;
     const Geo &g = in.geo;
-    const SegCtx sc = batch_ctx(G, seg, info);
+    const SegCtx sc = batch_ctx(G, seg, planes);
     // DMC grids gather the per-edge gradients (already divided by the normalisation)
     const AdjIn<S> adj = G.algo == DISO_DMC ? AdjIn<S>{ge + 3 * G.q_first, G.nf, G.flags & ~DISO_FLAG_NORMALIZE, G.nm}
                                             : AdjIn<S>{G.adj, G.nv, G.flags, G.nm};
@@ -2498,14 +2457,16 @@ bool make_geo(int64_t X, int64_t Y, int64_t Z, int flags, Geo *g) {
     g->off = pad / 2;
     g->nchunk = (g->g2 + kWave - 1) / kWave;
     g->nseg = (int64_t)g->g0 * g->g1 * g->nchunk;
+    g->rchunk = 1.0 / g->nchunk;
+    g->rg1 = 1.0 / g->g1;
     // Per-block aggregates must fit the 29/30-bit fields of the scan words; segment ids 32 bits.
     return (int64_t)g->g0 * g->g1 * g->g2 < (1ll << 36) && g->nseg < (1ll << 32);
 }
 
-// Segment bases (+ two totals entries), then one 16-bit classification word per lane.
+// Segment bases (+ two totals entries), then the classification planes.
 int64_t bases_bytes_for(const Geo &g) { return (g.nseg + 2) * (int64_t)sizeof(SegBase); }
-int64_t seg_bytes_for(const Geo &g) { return bases_bytes_for(g) + g.nseg * kWave * 2; }
-int64_t ctl_bytes_for(const Geo &) { return kCtlHeader + 2 * kMaxCountBlocks * (int64_t)sizeof(uint64_t); }
+int64_t seg_bytes_for(const Geo &g) { return bases_bytes_for(g) + g.nseg * kSegStateBytes; }
+int64_t ctl_bytes_for(const Geo &) { return kCtlHeader + 4 * kMaxCountBlocks * (int64_t)sizeof(uint64_t); }
 
 // Number of count blocks: about kCountBlocksPerCU per CU of the current device, so that every
 // block is resident at once, and never more than the segments or the word buffer allow.
@@ -2539,10 +2500,16 @@ int64_t count_blocks(int64_t nseg, int resident_per_cu) {
     const int per_cu = want < resident_per_cu ? want : resident_per_cu;
     int64_t nb = (int64_t)cu_count() * per_cu;
     const int64_t min_nb = (nseg + (1ll << 20) - 1) >> 20;  // <= 2^20 segments per block keeps the
+    const int64_t full = (nseg + kCountBlock - 1) / kCountBlock;
+    if (nb > full) nb = full;   // a lane per segment: no more blocks than full waves
     if (nb < min_nb) nb = min_nb;                          // aggregate fields from overflowing
     if (nb > kMaxCountBlocks) nb = kMaxCountBlocks;
     if (nb > nseg) nb = nseg;
     return nb < 1 ? 1 : nb;
+}
+
+int64_t mask_blocks(int64_t nseg) {
+    return (nseg + kMaskTile * kWavesPerBlock - 1) / (kMaskTile * kWavesPerBlock);
 }
 
 template <typename S>
@@ -2565,15 +2532,19 @@ int launch_count(int algo, const void *sdf, double iso, const Geo &g, void *seg,
     src.recount_spins = (uint32_t)g_params.recount_spins;
     (void)ctl_bytes;
     SegBase *sb = (SegBase *)seg;
-    uint16_t *info = reinterpret_cast<uint16_t *>(sb + g.nseg + 2);
+    const Planes P = planes_of(sb, g.nseg);
+    hipLaunchKernelGGL((mask_kernel<S, false>), dim3((unsigned)mask_blocks(g.nseg)), dim3(kBlock), 0, st, src,
+                       (const BatchGrid<S> *)nullptr, P, (uint8_t *)ctl);
+    int rc = check_hip(hipGetLastError(), "mask kernel launch");
+    if (rc) return rc;
     if (algo == DISO_MC) {
         const int64_t nb = count_blocks(g.nseg, count_resident_per_cu<count_kernel<S, DISO_MC, false>>());
         hipLaunchKernelGGL((count_kernel<S, DISO_MC, false>), dim3((unsigned)nb), dim3(kCountBlock), 0, st, src,
-                           (const BatchGrid<S> *)nullptr, sb, info, (uint8_t *)ctl, nb);
+                           (const BatchGrid<S> *)nullptr, sb, P, (uint8_t *)ctl, nb);
     } else {
         const int64_t nb = count_blocks(g.nseg, count_resident_per_cu<count_kernel<S, DISO_DMC, false>>());
         hipLaunchKernelGGL((count_kernel<S, DISO_DMC, false>), dim3((unsigned)nb), dim3(kCountBlock), 0, st, src,
-                           (const BatchGrid<S> *)nullptr, sb, info, (uint8_t *)ctl, nb);
+                           (const BatchGrid<S> *)nullptr, sb, P, (uint8_t *)ctl, nb);
     }
     return check_hip(hipGetLastError(), "count kernel launch");
 }
@@ -2591,30 +2562,39 @@ Norm<S> norm_of(const Geo &g) {
     return nm;
 }
 
+// Blocks of a unit emission whose cells number at most `cells` (a cell has at least one triangle /
+// patch, so a face / vertex capacity bounds them): a wave per unit, at most kUnitBlocksPerCU blocks
+// per CU (then each wave goes through several units), a multiple of the eight XCDs.
+constexpr int kUnitBlocksPerCU = 10;
+int64_t unit_blocks(int64_t cells) {
+    int64_t nb = cells / (kWave * kWavesPerBlock) + 1;
+    const int64_t most = (int64_t)cu_count() * kUnitBlocksPerCU;
+    if (nb > most) nb = most;
+    return (nb + 7) / 8 * 8;
+}
+
 template <typename S>
 int launch_emit(int algo, const void *sdf, const void *deform, double iso, int flags, const Geo &g,
                 const void *seg, void *verts, int64_t vcap, void *faces, int64_t fcap, void *vinfo, hipStream_t st) {
     In<S> in = make_in<S>(sdf, deform, iso, g);
     const Norm<S> nm = norm_of<S>(g);
-    const int64_t nb = row_blocks(g);
     const SegBase *sb = (const SegBase *)seg;
     const OutCfg out{flags, vcap, fcap};
-    const dim3 grid((unsigned)nb), block(kBlock);
-    const int run = run_for(g.nseg);
+    if (g.nseg < 4) return DISO_OK;  // no cell
+    const Planes P = planes_of(sb, g.nseg);
+    const dim3 block(kBlock), grid((unsigned)unit_blocks(algo == DISO_MC ? fcap : vcap));
     if (algo == DISO_MC) {
         if (deform)
-            hipLaunchKernelGGL((emit_mc_kernel<S, true>), grid, block, 0, st, in, sb, (S *)verts, faces, out, nm,
-                               run, nb);
+            hipLaunchKernelGGL((emit_mc_kernel<S, true>), grid, block, 0, st, in, sb, P, (S *)verts, faces, out, nm);
         else
-            hipLaunchKernelGGL((emit_mc_kernel<S, false>), grid, block, 0, st, in, sb, (S *)verts, faces, out, nm,
-                               run, nb);
+            hipLaunchKernelGGL((emit_mc_kernel<S, false>), grid, block, 0, st, in, sb, P, (S *)verts, faces, out, nm);
     } else {
         if (deform)
-            hipLaunchKernelGGL((emit_dmc_kernel<S, true>), grid, block, 0, st, in, sb, (S *)verts, faces,
-                               (uint8_t *)vinfo, out, nm, run, nb);
+            hipLaunchKernelGGL((emit_dmc_kernel<S, true>), grid, block, 0, st, in, sb, P, (S *)verts, faces,
+                               (uint8_t *)vinfo, out, nm);
         else
-            hipLaunchKernelGGL((emit_dmc_kernel<S, false>), grid, block, 0, st, in, sb, (S *)verts, faces,
-                               (uint8_t *)vinfo, out, nm, run, nb);
+            hipLaunchKernelGGL((emit_dmc_kernel<S, false>), grid, block, 0, st, in, sb, P, (S *)verts, faces,
+                               (uint8_t *)vinfo, out, nm);
     }
     return check_hip(hipGetLastError(), "emit kernel launch");
 }
@@ -2740,7 +2720,7 @@ struct BatchLayout {
     int64_t nseg = 0;
     std::vector<Geo> geo;
     std::vector<int64_t> seg_first;
-    int64_t off_desc = 0, off_groups = 0, off_totals = 0, off_seg = 0, off_info = 0, total = 0;
+    int64_t off_desc = 0, off_groups = 0, off_totals = 0, off_seg = 0, off_planes = 0, off_range = 0, total = 0;
 };
 
 int64_t group_bytes(int n) { return align256((int64_t)n * 4) + align256((int64_t)(n + 1) * 8); }
@@ -2761,9 +2741,10 @@ bool batch_layout(const diso_grid_t *grids, int n, BatchLayout *L) {
     L->off_desc = 0;
     L->off_groups = align256((int64_t)n * (int64_t)sizeof(BatchGrid<double>));
     L->off_totals = L->off_groups + kBatchGroups * group_bytes(n);
-    L->off_seg = L->off_totals + align256((int64_t)n * (int64_t)sizeof(diso_totals_t));
-    L->off_info = L->off_seg + (nseg + 2) * (int64_t)sizeof(SegBase);
-    L->total = L->off_info + nseg * kWave * 2;
+    L->off_range = L->off_totals + align256((int64_t)n * (int64_t)sizeof(diso_totals_t));
+    L->off_seg = L->off_range + align256((int64_t)n * 8);
+    L->off_planes = L->off_seg + (nseg + 2) * (int64_t)sizeof(SegBase);
+    L->total = L->off_planes + nseg * kSegStateBytes;
     return true;
 }
 
@@ -2887,7 +2868,8 @@ template <typename S>
 struct BatchPtrs {
     BatchGrid<S> *desc;
     SegBase *seg;
-    uint16_t *info;
+    Planes planes;
+    uint32_t *range;  // first and end unit of each grid
     diso_totals_t *totals;
     const int32_t *gl(const BatchLayout &L, int k, uint8_t *ws) const {
         return (const int32_t *)(ws + L.off_groups + k * group_bytes(L.n));
@@ -2900,7 +2882,8 @@ struct BatchPtrs {
 template <typename S>
 BatchPtrs<S> batch_ptrs(void *ws, const BatchLayout &L) {
     uint8_t *b = (uint8_t *)ws;
-    return BatchPtrs<S>{(BatchGrid<S> *)(b + L.off_desc), (SegBase *)(b + L.off_seg), (uint16_t *)(b + L.off_info),
+    return BatchPtrs<S>{(BatchGrid<S> *)(b + L.off_desc), (SegBase *)(b + L.off_seg),
+                        planes_at(b + L.off_planes, L.nseg), (uint32_t *)(b + L.off_range),
                         (diso_totals_t *)(b + L.off_totals)};
 }
 
@@ -2915,13 +2898,16 @@ int batch_count(diso_grid_t *grids, const BatchLayout &L, void *ws, void *ctl, h
     src.ngrids = L.n;
     src.nseg = L.nseg;
     src.recount_spins = (uint32_t)g_params.recount_spins;
+    hipLaunchKernelGGL((mask_kernel<S, true>), dim3((unsigned)mask_blocks(L.nseg)), dim3(kBlock), 0, st, src,
+                       (const BatchGrid<S> *)P.desc, P.planes, (uint8_t *)ctl);
+    if ((rc = check_hip(hipGetLastError(), "batch mask kernel launch"))) return rc;
     const int64_t nb = count_blocks(L.nseg, count_resident_per_cu<count_kernel<S, DISO_MC, true>>());
     hipLaunchKernelGGL((count_kernel<S, DISO_MC, true>), dim3((unsigned)nb), dim3(kCountBlock), 0, st, src,
-                       (const BatchGrid<S> *)P.desc, P.seg, P.info, (uint8_t *)ctl, nb);
+                       (const BatchGrid<S> *)P.desc, P.seg, P.planes, (uint8_t *)ctl, nb);
     rc = check_hip(hipGetLastError(), "batch count kernel launch");
     if (rc) return rc;
     hipLaunchKernelGGL((batch_totals_kernel<S>), dim3((unsigned)((L.n + 255) / 256)), dim3(256), 0, st, P.desc, L.n,
-                       L.nseg, P.seg, src.gflags, P.totals);
+                       L.nseg, P.seg, P.planes, src.gflags, P.range, P.totals);
     rc = check_hip(hipGetLastError(), "batch totals kernel launch");
     if (rc) return rc;
     Staging &stg = staging();
@@ -2951,7 +2937,8 @@ int batch_emit(const diso_grid_t *grids, const BatchLayout &L, void *ws, hipStre
             return fail(DISO_E_CAPACITY, "grid %d: output buffers too small", i);
         if (!G.verts || !G.faces || (G.algo == DISO_DMC && !G.vinfo))
             return fail(DISO_E_INVALID, "grid %d: null output buffer", i);
-        gr[2 * (G.algo == DISO_DMC) + (G.deform != nullptr)].add(i, runs_of(L.geo[i], run_for(L.geo[i].nseg)));
+        gr[2 * (G.algo == DISO_DMC) + (G.deform != nullptr)].add(
+            i, (G.algo == DISO_DMC ? G.totals.n_verts : G.totals.n_faces / 2) / (kWave * kWavesPerBlock) + 1);
     }
     int rc = upload_batch<S>(ws, L, batch_desc<S>(grids, L), gr, 4, st);
     if (rc) return rc;
@@ -2965,10 +2952,10 @@ int batch_emit(const diso_grid_t *grids, const BatchLayout &L, void *ws, hipStre
         const int64_t *rf = P.rf(L, k, w);
         const int m = gr[k].m();
         switch (k) {
-            case 0: hipLaunchKernelGGL((emit_mc_batch_kernel<S, false>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.info, nb); break;
-            case 1: hipLaunchKernelGGL((emit_mc_batch_kernel<S, true>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.info, nb); break;
-            case 2: hipLaunchKernelGGL((emit_dmc_batch_kernel<S, false>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.info, nb); break;
-            default: hipLaunchKernelGGL((emit_dmc_batch_kernel<S, true>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.info, nb); break;
+            case 0: hipLaunchKernelGGL((emit_mc_batch_kernel<S, false>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, P.range, nb); break;
+            case 1: hipLaunchKernelGGL((emit_mc_batch_kernel<S, true>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, P.range, nb); break;
+            case 2: hipLaunchKernelGGL((emit_dmc_batch_kernel<S, false>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, P.range, nb); break;
+            default: hipLaunchKernelGGL((emit_dmc_batch_kernel<S, true>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, P.range, nb); break;
         }
         rc = check_hip(hipGetLastError(), "batch emit kernel launch");
         if (rc) return rc;
@@ -3016,10 +3003,10 @@ int batch_backward(const diso_grid_t *grids, const BatchLayout &L, void *ws, voi
         const int64_t *rf = P.rf(L, k, w);
         const int m = gr[k].m();
         switch (k) {
-            case 0: hipLaunchKernelGGL((bwd_batch_kernel<S, false, false>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.info, ge, nb); break;
-            case 1: hipLaunchKernelGGL((bwd_batch_kernel<S, false, true>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.info, ge, nb); break;
-            case 2: hipLaunchKernelGGL((bwd_batch_kernel<S, true, false>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.info, ge, nb); break;
-            default: hipLaunchKernelGGL((bwd_batch_kernel<S, true, true>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.info, ge, nb); break;
+            case 0: hipLaunchKernelGGL((bwd_batch_kernel<S, false, false>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
+            case 1: hipLaunchKernelGGL((bwd_batch_kernel<S, false, true>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
+            case 2: hipLaunchKernelGGL((bwd_batch_kernel<S, true, false>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
+            default: hipLaunchKernelGGL((bwd_batch_kernel<S, true, true>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
         }
         rc = check_hip(hipGetLastError(), "batch backward kernel launch");
         if (rc) return rc;
@@ -3037,7 +3024,7 @@ int batch_backward(const diso_grid_t *grids, const BatchLayout &L, void *ws, voi
 // from call to call (epoch-tagged words, each call clears the buffer the next one uses), so no
 // per-call clearing is needed. Every call on a device shares the one array: calls that overlap
 // in time on one device race.
-constexpr int64_t kNoallocCtlBytes = kCtlHeader + 2 * kMaxCountBlocks * (int64_t)sizeof(uint64_t);
+constexpr int64_t kNoallocCtlBytes = kCtlHeader + 4 * kMaxCountBlocks * (int64_t)sizeof(uint64_t);
 static_assert(kNoallocCtlBytes % 8 == 0, "control block is cleared in 8-byte words");
 static __device__ __align__(256) uint8_t scratch[kNoallocCtlBytes];
 

@@ -12,7 +12,8 @@
 // that block's range).
 //
 // Word layout: [63:62] tag (0 = empty), [61:59] sample flags, [58:29] face / patch count,
-// [28:0] vertex / quad count.
+// [28:0] vertex / quad count. A block publishes a second word beside it: [63:62] the same tag,
+// [61:0] its active cells; both must be published.
 //
 // Plain C++ (host and device), so the protocol is testable on the CPU.
 #pragma once
@@ -36,6 +37,8 @@ DISO_HD constexpr uint32_t tag_of(uint32_t epoch) { return 1u + epoch % 3u; }
 DISO_HD constexpr uint64_t pack(int64_t v, int64_t f, uint32_t flags, uint32_t tag) {
     return ((uint64_t)tag << 62) | ((uint64_t)(flags & 7u) << 59) | ((uint64_t)f << kCountBits) | (uint64_t)v;
 }
+DISO_HD constexpr uint64_t pack_cells(int64_t cells, uint32_t tag) { return ((uint64_t)tag << 62) | (uint64_t)cells; }
+DISO_HD constexpr int64_t count_cells(uint64_t w) { return (int64_t)(w & ((1ull << 62) - 1)); }
 DISO_HD constexpr bool published(uint64_t w, uint32_t tag) { return (uint32_t)(w >> 62) == tag; }
 DISO_HD constexpr int64_t count_v(uint64_t w) { return (int64_t)(w & ((1ull << kCountBits) - 1)); }
 DISO_HD constexpr int64_t count_f(uint64_t w) { return (int64_t)((w >> kCountBits) & ((1ull << kFaceBits) - 1)); }
