@@ -44,7 +44,7 @@ PARAM_RECOUNT_SPINS = 2
 PARAM_BUCKETS = 5  # size buckets of the run length and count blocks per CU (~32^3 .. ~512^3 grids)
 
 EXPORTS = [
-    "diso_seg_bytes", "diso_ctl_bytes", "diso_scratch_bytes", "diso_count", "diso_emit", "diso_backward",
+    "diso_seg_bytes", "diso_ctl_bytes", "diso_scratch_bytes", "diso_count", "diso_emit", "diso_extract", "diso_backward",
     "diso_read_totals", "diso_last_error", "diso_version", "diso_split_scratch_bytes", "diso_split",
     "diso_batch_seg_bytes", "diso_batch_ctl_bytes", "diso_batch_count", "diso_batch_emit", "diso_batch_scratch_bytes",
     "diso_batch_backward", "diso_set_param", "diso_get_param", "diso_totals_offset", "diso_count_noalloc",
@@ -99,6 +99,9 @@ def lib():
         L.diso_scratch_bytes.argtypes = [i32, i32, i64]
         L.diso_emit.restype = i32
         L.diso_emit.argtypes = [i32, i32, vp, vp, i64, i64, i64, dbl, i32, vp, i64, vp, i64, vp, i64, vp, vp]
+        L.diso_extract.restype = i32
+        L.diso_extract.argtypes = [i32, i32, vp, vp, i64, i64, i64, dbl, i32, vp, i64, vp, i64, vp, i64, vp, i64, vp,
+                                   ctypes.POINTER(Totals), vp]
         L.diso_backward.restype = i32
         L.diso_backward.argtypes = [i32, i32, vp, vp, i64, i64, i64, dbl, i32, vp, i64, vp, i64, vp, vp,
                                     i64, vp, vp, vp, i64, vp]

@@ -32,6 +32,7 @@
 // backward uses one hardware reciprocal per edge (gradients are compared within a tolerance).
 #include <hip/hip_runtime.h>
 
+#include <sched.h>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -543,6 +544,12 @@ struct CtlHeader {
     uint32_t pad[12];
 };
 
+// Where a waiting host reads a count's totals: in host memory that the device writes, `seq` last.
+struct HostTotals {
+    int64_t v, f, flags;
+    uint64_t seq;
+};
+
 constexpr int kCountWaves = 8;
 constexpr int kCountBlock = kCountWaves * kWave;
 constexpr int64_t kMaxCountBlocks = 4096;  // two words each
@@ -798,7 +805,8 @@ template <typename S, int ALGO, bool BATCH>
 __global__ __launch_bounds__(kCountBlock, kCountWaves / 2) void count_kernel(CountSrc<S> src,
                                                                            const BatchGrid<S> *__restrict__ grids,
                                                                            SegBase *seg, Planes planes, uint8_t *ctl,
-                                                                           int64_t nblocks) {
+                                                                           int64_t nblocks, HostTotals *host,
+                                                                           uint64_t seq) {
     __shared__ int64_t s_v[kCountWaves], s_f[kCountWaves], s_a[kCountWaves];
     __shared__ uint32_t s_fl[kCountWaves];
     __shared__ uint32_t s_epoch, s_dirty_other, s_next;
@@ -934,6 +942,13 @@ __global__ __launch_bounds__(kCountBlock, kCountWaves / 2) void count_kernel(Cou
         tot[0].f = ef + af;
         tot[1].v = (int64_t)(efl | afl);
         tot[1].f = ALGO;
+        if (host) {  // a host thread waits for `seq` (diso_extract)
+            auto put_host = [](auto *p, auto v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+            put_host(&host->v, ev + av);
+            put_host(&host->f, ef + af);
+            put_host(&host->flags, (int64_t)(efl | afl));
+            __hip_atomic_store(&host->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
         if (nseg >= 4) *planes.nunits = (uint32_t)((ea + aa + kWave - 1) / kWave);
         __hip_atomic_store(&hdr->dirty[parity], (uint32_t)(2 * nblocks), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(&hdr->dirty[parity ^ 1u], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2525,7 +2540,7 @@ In<S> make_in(const void *sdf, const void *deform, double iso, const Geo &g) {
 
 template <typename S>
 int launch_count(int algo, const void *sdf, double iso, const Geo &g, void *seg, void *ctl,
-                 int64_t ctl_bytes, hipStream_t st) {
+                 int64_t ctl_bytes, hipStream_t st, HostTotals *host = nullptr, uint64_t seq = 0) {
     CountSrc<S> src{};
     src.in = make_in<S>(sdf, nullptr, iso, g);
     src.nseg = g.nseg;
@@ -2540,11 +2555,11 @@ int launch_count(int algo, const void *sdf, double iso, const Geo &g, void *seg,
     if (algo == DISO_MC) {
         const int64_t nb = count_blocks(g.nseg, count_resident_per_cu<count_kernel<S, DISO_MC, false>>());
         hipLaunchKernelGGL((count_kernel<S, DISO_MC, false>), dim3((unsigned)nb), dim3(kCountBlock), 0, st, src,
-                           (const BatchGrid<S> *)nullptr, sb, P, (uint8_t *)ctl, nb);
+                           (const BatchGrid<S> *)nullptr, sb, P, (uint8_t *)ctl, nb, host, seq);
     } else {
         const int64_t nb = count_blocks(g.nseg, count_resident_per_cu<count_kernel<S, DISO_DMC, false>>());
         hipLaunchKernelGGL((count_kernel<S, DISO_DMC, false>), dim3((unsigned)nb), dim3(kCountBlock), 0, st, src,
-                           (const BatchGrid<S> *)nullptr, sb, P, (uint8_t *)ctl, nb);
+                           (const BatchGrid<S> *)nullptr, sb, P, (uint8_t *)ctl, nb, host, seq);
     }
     return check_hip(hipGetLastError(), "count kernel launch");
 }
@@ -2705,6 +2720,40 @@ int read_totals(const Geo &g, const void *seg, diso_totals_t *t, hipStream_t st,
     t->flags = tot[1].v;
     t->n_crossing = tot[0].v;
     return DISO_OK;
+}
+
+// This thread's landing place for totals written by the count kernel, kept for the life of the
+// process, and the number of its next call (a kernel of an abandoned call writes an old number).
+struct Landing {
+    HostTotals *host = nullptr;
+    uint64_t seq = 0;
+};
+Landing &landing() {
+    thread_local Landing l;
+    if (!l.host) {
+        void *q = nullptr;
+        if (hipHostMalloc(&q, sizeof(HostTotals), hipHostMallocCoherent | hipHostMallocMapped) == hipSuccess) {
+            l.host = (HostTotals *)q;
+            l.host->seq = 0;
+        }
+    }
+    return l;
+}
+
+// Waits until the count has written number `seq`. The stream's state is looked at only now and then
+// (it tells of a failed launch, or of work ahead in the stream that makes the wait long).
+int wait_totals(const HostTotals *h, uint64_t seq, hipStream_t st) {
+    for (uint32_t spins = 1;; ++spins) {
+        if (__atomic_load_n(&h->seq, __ATOMIC_ACQUIRE) == seq) return DISO_OK;
+        if (spins % 4096 == 0) {
+            const hipError_t e = hipStreamQuery(st);
+            if (e != hipSuccess && e != hipErrorNotReady) return check_hip(e, "count pass");
+            if (e == hipSuccess && __atomic_load_n(&h->seq, __ATOMIC_ACQUIRE) != seq)
+                return fail(DISO_E_HIP, "count pass ended without totals");
+            if (spins > (1u << 16)) sched_yield();
+        }
+        __builtin_ia32_pause();
+    }
 }
 
 // ---- batches
@@ -2903,7 +2952,8 @@ int batch_count(diso_grid_t *grids, const BatchLayout &L, void *ws, void *ctl, h
     if ((rc = check_hip(hipGetLastError(), "batch mask kernel launch"))) return rc;
     const int64_t nb = count_blocks(L.nseg, count_resident_per_cu<count_kernel<S, DISO_MC, true>>());
     hipLaunchKernelGGL((count_kernel<S, DISO_MC, true>), dim3((unsigned)nb), dim3(kCountBlock), 0, st, src,
-                       (const BatchGrid<S> *)P.desc, P.seg, P.planes, (uint8_t *)ctl, nb);
+                       (const BatchGrid<S> *)P.desc, P.seg, P.planes, (uint8_t *)ctl, nb, (HostTotals *)nullptr,
+                       (uint64_t)0);
     rc = check_hip(hipGetLastError(), "batch count kernel launch");
     if (rc) return rc;
     hipLaunchKernelGGL((batch_totals_kernel<S>), dim3((unsigned)((L.n + 255) / 256)), dim3(256), 0, st, P.desc, L.n,
@@ -3179,6 +3229,41 @@ int diso_emit(int algo, int dtype, const void *sdf, const void *deform, int64_t 
                                                   face_capacity, vinfo, st)
                              : launch_emit<double>(algo, sdf, deform, iso, flags, g, seg, verts, vert_capacity, faces,
                                                    face_capacity, vinfo, st);
+}
+
+int diso_extract(int algo, int dtype, const void *sdf, const void *deform, int64_t X, int64_t Y, int64_t Z, double iso,
+                 int flags, void *seg, int64_t seg_bytes, void *ctl, int64_t ctl_bytes, void *verts,
+                 int64_t vert_capacity, void *faces, int64_t face_capacity, void *vinfo, diso_totals_t *totals_host,
+                 void *stream) {
+    g_err[0] = 0;
+    Geo g;
+    int rc = check_common(algo, dtype, X, Y, Z, flags, &g);
+    if (rc) return rc;
+    if (!sdf || !seg || !ctl || !totals_host) return fail(DISO_E_INVALID, "null pointer argument");
+    if (seg_bytes < seg_bytes_for(g)) return fail(DISO_E_CAPACITY, "seg workspace too small");
+    if (ctl_bytes < ctl_bytes_for(g)) return fail(DISO_E_CAPACITY, "ctl workspace too small");
+    if (vert_capacity < 0 || face_capacity < 0) return fail(DISO_E_INVALID, "negative capacity");
+    if ((vert_capacity && !verts) || (face_capacity && !faces)) return fail(DISO_E_INVALID, "null output buffer");
+    if (algo == DISO_DMC && vert_capacity && !vinfo) return fail(DISO_E_INVALID, "DMC needs a vinfo buffer");
+    hipStream_t st = (hipStream_t)stream;
+    Landing &land = landing();
+    if (!land.host) return fail(DISO_E_HIP, "pinned allocation failed");
+    const uint64_t seq = ++land.seq;
+    const bool f32 = dtype == DISO_F32;
+    rc = f32 ? launch_count<float>(algo, sdf, iso, g, seg, ctl, ctl_bytes, st, land.host, seq)
+             : launch_count<double>(algo, sdf, iso, g, seg, ctl, ctl_bytes, st, land.host, seq);
+    if (rc) return rc;
+    rc = f32 ? launch_emit<float>(algo, sdf, deform, iso, flags, g, seg, verts, vert_capacity, faces, face_capacity, vinfo, st)
+             : launch_emit<double>(algo, sdf, deform, iso, flags, g, seg, verts, vert_capacity, faces, face_capacity, vinfo, st);
+    const int rw = wait_totals(land.host, seq, st);
+    if (rc || rw) return rc ? rc : rw;
+    const HostTotals h = *land.host;
+    totals_host->n_verts = algo == DISO_DMC ? h.f : h.v;
+    totals_host->n_faces = algo == DISO_DMC ? h.v : h.f;
+    totals_host->flags = h.flags;
+    totals_host->n_crossing = h.v;
+    if (h.flags & DISO_TOTAL_SCAN_TIMEOUT) return fail(DISO_E_TIMEOUT, "single-pass scan did not complete");
+    return DISO_OK;
 }
 
 int diso_backward(int algo, int dtype, const void *sdf, const void *deform, int64_t X, int64_t Y, int64_t Z,

@@ -73,33 +73,6 @@ def _stream(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
-_hiprt = None
-
-
-def _hip():
-    """The HIP runtime torch runs on (same soname, so the already loaded one), for the few
-    stream and event calls of the totals read-back."""
-    global _hiprt
-    if _hiprt is None:
-        h = ctypes.CDLL("libamdhip64.so.7")
-        vp, i32 = ctypes.c_void_p, ctypes.c_int
-        h.hipEventCreateWithFlags.argtypes = [ctypes.POINTER(vp), ctypes.c_uint]
-        h.hipEventRecord.argtypes = [vp, vp]
-        h.hipStreamWaitEvent.argtypes = [vp, vp, ctypes.c_uint]
-        h.hipMemcpyAsync.argtypes = [vp, vp, ctypes.c_size_t, i32, vp]
-        h.hipStreamSynchronize.argtypes = [vp]
-        for f in (h.hipEventCreateWithFlags, h.hipEventRecord, h.hipStreamWaitEvent, h.hipMemcpyAsync,
-                  h.hipStreamSynchronize):
-            f.restype = i32
-        _hiprt = h
-    return _hiprt
-
-
-def _hip_check(rc, what):
-    if rc != 0:
-        raise RuntimeError(f"diso_amd: {what} failed (hipError {rc})")
-
-
 class Extractor:
     def __init__(self, algo, dtype):
         if dtype not in _DTYPES:
@@ -109,7 +82,7 @@ class Extractor:
         self.code = _DTYPES[dtype]
         self._ctl = {}
         self._guess = {}  # (device, dims, flags) -> (vertices, faces) of the last call
-        self._side = {}  # device -> (side stream handle, pinned totals, event, side stream)
+        self._need = {}  # (dims, flags) -> workspace bytes (_sizes)
         _lib.lib()  # fail loudly now if the HIP library is not there
 
     def check_grid(self, grid, name="grid"):
@@ -120,10 +93,24 @@ class Extractor:
         if grid.dtype != self.dtype:
             raise RuntimeError(f"{name} type must match the {'mc' if self.algo == _lib.MC else 'dmc'} class")
 
+    def _sizes(self, dims, flags):
+        """Workspace bytes of a grid: the segment workspace, what of it a backward with these flags
+        keeps, and the control block (asked once per dims and flags)."""
+        key = (dims, flags)
+        got = self._need.get(key)
+        if got is None:
+            L = _lib.lib()
+            got = (L.diso_seg_bytes(*dims, flags & ~_lib.FLAG_RECOMPUTE), L.diso_seg_bytes(*dims, flags),
+                   L.diso_ctl_bytes(*dims, flags))
+            if min(got) < 0:
+                _lib.check(min(got), "workspace sizing")
+            if len(self._need) >= 256:
+                self._need.clear()
+            self._need[key] = got
+        return got
+
     def ctl_for(self, device, dims, flags):
-        need = _lib.lib().diso_ctl_bytes(*dims, flags)
-        if need < 0:
-            _lib.check(need, "workspace sizing")
+        need = self._sizes(dims, flags)[2]
         key = device.index
         ctl = self._ctl.get(key)
         if ctl is None or ctl.numel() < need:
@@ -136,9 +123,7 @@ class Extractor:
     def count(self, grid, iso, flags):
         dims = tuple(int(d) for d in grid.shape)
         L = _lib.lib()
-        nseg = L.diso_seg_bytes(*dims, flags & ~_lib.FLAG_RECOMPUTE)  # the full workspace
-        if nseg < 0:
-            _lib.check(nseg, "workspace sizing")
+        nseg = self._sizes(dims, flags)[0]
         seg = torch.empty(nseg, dtype=torch.uint8, device=grid.device)
         ctl = self.ctl_for(grid.device, dims, flags)
         tot = _lib.Totals()
@@ -149,13 +134,13 @@ class Extractor:
 
     def count_speculative(self, grid, deform, iso, flags):
         """The counting pass, and, when an earlier call on a grid of these dims gives a size
-        estimate, the emission queued right behind it into buffers of that size plus a margin:
-        the host then waits only for the counts (copied on a side stream as soon as the counting
-        kernel is done), so its work until the next launch overlaps the emission instead of
-        leaving the device idle. If the counts fit, `counted.spec` holds the emitted buffers
-        (emit() returns views of them); otherwise emit() runs the emission again at the exact
-        size (the queued one writes nothing when the counts exceed its capacities)."""
-        dims = tuple(int(d) for d in grid.shape)
+        estimate, the emission queued right behind it into buffers of that size plus a margin
+        (diso_extract): the host then waits only for the counts, which the counting kernel writes
+        to host memory, so its work until the next launch overlaps the emission instead of leaving
+        the device idle. If the counts fit, `counted.spec` holds the emitted buffers (emit() returns
+        views of them); otherwise emit() runs the emission again at the exact size (the queued one
+        writes nothing when the counts exceed its capacities)."""
+        dims = tuple(grid.shape)
         dev = grid.device
         key = (dev.index, dims, flags)
         guess = self._guess.get(key)
@@ -163,59 +148,26 @@ class Extractor:
             counted = self.count(grid, iso, flags)
             self._remember(key, counted.n_verts, counted.n_faces)
             return counted
-        L = _lib.lib()
-        nseg = L.diso_seg_bytes(*dims, flags & ~_lib.FLAG_RECOMPUTE)
-        off = L.diso_totals_offset(*dims, flags)
-        if nseg < 0 or off < 0:
-            _lib.check(min(nseg, off), "workspace sizing")
+        nseg = self._sizes(dims, flags)[0]
         seg = torch.empty(nseg, dtype=torch.uint8, device=dev)
         ctl = self.ctl_for(dev, dims, flags)
-        main = _stream(dev)
-        rc = L.diso_count(self.algo, self.code, _ptr(grid), *dims, float(iso), flags, _ptr(seg), nseg, _ptr(ctl),
-                          ctl.numel(), None, main)
-        _lib.check(rc, "count pass")
-        # the side stream copies the totals as soon as the count kernel is done
-        side, host, ev = self._side_for(dev)
-        hip = _hip()
-        _hip_check(hip.hipEventRecord(ev, main), "event record")
-        _hip_check(hip.hipStreamWaitEvent(side, ev, 0), "stream wait")
-        _hip_check(hip.hipMemcpyAsync(ctypes.c_void_p(host.data_ptr()), ctypes.c_void_p(seg.data_ptr() + off), 32,
-                                      2, side), "totals copy")  # 2: device to host
         dmc = self.algo == _lib.DMC
         vcap, fcap = guess[0] + guess[0] // 4 + 1024, guess[1] + guess[1] // 4 + 1024
-        idx = torch.int64 if flags & _lib.FLAG_INDEX64 else torch.int32
         verts = torch.empty((vcap, 3), dtype=self.dtype, device=dev)
-        faces = torch.empty((fcap, 4 if dmc else 3), dtype=idx, device=dev)
-        vinfo = torch.empty(vcap if dmc else 0, dtype=torch.uint8, device=dev)
-        rc = L.diso_emit(self.algo, self.code, _ptr(grid), _ptr(deform), *dims, float(iso), flags, _ptr(seg), nseg,
-                         _ptr(verts), vcap, _ptr(faces), fcap, _ptr(vinfo), main)
-        _lib.check(rc, "emit pass")
-        _hip_check(hip.hipStreamSynchronize(side), "totals wait")
-        crossing, other, tflags, _ = host.tolist()
+        faces = torch.empty((fcap, 4 if dmc else 3), dtype=torch.int64 if flags & _lib.FLAG_INDEX64 else torch.int32,
+                            device=dev)
+        vinfo = torch.empty(vcap, dtype=torch.uint8, device=dev) if dmc else None
         tot = _lib.Totals()
-        tot.n_verts, tot.n_faces = (other, crossing) if dmc else (crossing, other)
-        tot.flags, tot.n_crossing = tflags, crossing
-        if tflags & _lib.TOTAL_SCAN_TIMEOUT:
-            raise RuntimeError("diso_amd: count pass failed: single-pass scan did not complete")
-        counted = Counted(seg, tot, dims, float(iso), flags)
+        rc = _lib.lib().diso_extract(self.algo, self.code, grid.data_ptr(), 0 if deform is None else deform.data_ptr(),
+                                     *dims, iso, flags, seg.data_ptr(), nseg, ctl.data_ptr(), ctl.numel(),
+                                     verts.data_ptr(), vcap, faces.data_ptr(), fcap,
+                                     vinfo.data_ptr() if dmc else 0, tot, _stream(dev))
+        _lib.check(rc, "extraction")
+        counted = Counted(seg, tot, dims, iso, flags)
         if tot.n_verts <= vcap and tot.n_faces <= fcap:
             counted.spec = (verts, faces, vinfo)
         self._remember(key, tot.n_verts, tot.n_faces)
         return counted
-
-    def _side_for(self, dev):
-        """Per device: a side stream (default priority), a pinned 32-byte landing buffer and an
-        event without timing, created once."""
-        got = self._side.get(dev.index)
-        if got is None:
-            side = torch.cuda.Stream(device=dev)
-            host = torch.empty(4, dtype=torch.int64, pin_memory=True)
-            ev = ctypes.c_void_p()
-            with torch.cuda.device(dev):
-                _hip_check(_hip().hipEventCreateWithFlags(ctypes.byref(ev), 2), "event create")  # 2: no timing
-            got = (ctypes.c_void_p(side.cuda_stream), host, ev, side)
-            self._side[dev.index] = got
-        return got[:3]
 
     def _remember(self, key, n_verts, n_faces):
         if len(self._guess) >= 64 and key not in self._guess:
@@ -238,11 +190,11 @@ class Extractor:
             v, f, vi = counted.spec
             counted.spec = None
             verts, faces = _prefix(v, counted.n_verts), _prefix(f, counted.n_faces)
-            vinfo = _prefix(vi, counted.n_verts) if dmc else vi
+            vinfo = vi
         else:
             verts = torch.empty((counted.n_verts, 3), dtype=self.dtype, device=grid.device)
             faces = torch.empty((counted.n_faces, k), dtype=idx, device=grid.device)
-            vinfo = torch.empty(counted.n_verts if dmc else 0, dtype=torch.uint8, device=grid.device)
+            vinfo = torch.empty(counted.n_verts, dtype=torch.uint8, device=grid.device) if dmc else None
             rc = L.diso_emit(self.algo, self.code, _ptr(grid), _ptr(deform), *counted.dims, counted.iso, flags,
                              _ptr(counted.seg), counted.seg.numel(), _ptr(verts), counted.n_verts, _ptr(faces),
                              counted.n_faces, _ptr(vinfo), _stream(grid.device))
@@ -252,8 +204,7 @@ class Extractor:
         if flags & _lib.FLAG_RECOMPUTE:
             # The backward will re-derive the classification from the samples: keep only the
             # segment bases and release the classification words.
-            nb = L.diso_seg_bytes(*counted.dims, flags)
-            counted.seg = counted.seg[:nb].clone()
+            counted.seg = counted.seg[:self._sizes(counted.dims, flags)[1]].clone()
         return verts, faces
 
     def backward(self, grid, deform, counted, flags, adj_verts, adj_grid, adj_deform):

@@ -139,6 +139,17 @@ int diso_emit(int algo, int dtype, const void *sdf, const void *deform, int64_t 
               int64_t Z, double iso, int flags, const void *seg, int64_t seg_bytes, void *verts,
               int64_t vert_capacity, void *faces, int64_t face_capacity, void *vinfo, void *stream);
 
+/* Passes 1 and 2 in one call, for a caller that has output buffers whose capacities probably
+ * suffice (an estimate from an earlier grid): enqueues diso_count and diso_emit and returns as soon
+ * as the totals are known, which the counting pass writes to host memory itself, while the emission
+ * may still run. If the totals exceed the capacities nothing has been written: call diso_emit with
+ * larger buffers. The reference reads its counts back with three blocking copies (src/cumc.cu:651-723).
+ * Waits for the host, so it cannot be captured in a graph. */
+int diso_extract(int algo, int dtype, const void *sdf, const void *deform, int64_t X, int64_t Y,
+                 int64_t Z, double iso, int flags, void *seg, int64_t seg_bytes, void *ctl,
+                 int64_t ctl_bytes, void *verts, int64_t vert_capacity, void *faces,
+                 int64_t face_capacity, void *vinfo, diso_totals_t *totals_host, void *stream);
+
 /* Backward: gradients of sum(adj_verts * verts) with respect to sdf [X,Y,Z] and deform
  * [X,Y,Z,3] (adj_deform may be NULL). One thread per grid vertex gathers from its at most six
  * incident crossing edges, so there are no atomics and results are deterministic. Replaces
