@@ -127,17 +127,6 @@ __device__ __forceinline__ V3<S> deform_at(const In<S> &in, int x, int y, int z)
     return r;
 }
 
-// A cell is anchored at (x,y,z) when its +1 corner lies inside the grid (src/cumc.cu:278).
-template <typename S>
-__device__ __forceinline__ bool is_anchor(const In<S> &in, int x, int y, int z) {
-    return x >= 0 && y >= 0 && z >= 0 && x < in.geo.g0 - 1 && y < in.geo.g1 - 1 && z < in.geo.g2 - 1;
-}
-
-template <typename S>
-__device__ __forceinline__ bool crosses(S d0, S d1, S iso) {
-    return (d0 < iso && d1 >= iso) || (d1 < iso && d0 >= iso);  // src/cumc.cu:334-339
-}
-
 // clamp(x, a, b) = min(max(a, x), b) as in src/cumc.cu:80-91.
 template <typename S>
 __device__ __forceinline__ S clamp01(S v) {
@@ -149,8 +138,6 @@ template <typename S>
 __device__ __forceinline__ S interp_t(S d0, S d1, S iso) {
     return (d1 != d0) ? clamp01<S>((iso - d0) / (d1 - d0)) : S(0.5);  // src/cumc.cu:356
 }
-
-__device__ __forceinline__ int popc3(int m) { return (m & 1) + ((m >> 1) & 1) + ((m >> 2) & 1); }
 
 // ------------------------------------------------------------------------------------------
 // Wave primitives
@@ -198,6 +185,19 @@ __device__ __forceinline__ int64_t xcd_block(int64_t bid, int64_t nb) {
     int64_t q = nb / 8, r = nb % 8;
     int64_t xcd = bid % 8, k = bid / 8;
     return xcd * q + (xcd < r ? xcd : r) + k;
+}
+
+// The same in kStripes turns: an XCD takes one of every eight stripes of consecutive blocks, so that
+// work that is uneven over the grid (a surface's faces) is spread over the XCDs while neighbouring
+// rows still mostly share one. The grid is padded to `stripe_blocks` blocks; returns a block >= nb for
+// the padding. The 256^3 noisy gather, in one turn (an eighth of the grid per XCD: the planes of a
+// box's face fall to one) 176 us, in 2, 4, 8, 16, 32 turns 170, 141, 135, 131, 132 us.
+constexpr int64_t kStripes = 16;
+__host__ __device__ __forceinline__ int64_t stripe_len(int64_t nb) { return (nb + 8 * kStripes - 1) / (8 * kStripes); }
+__host__ __device__ __forceinline__ int64_t stripe_blocks(int64_t nb) { return stripe_len(nb) * 8 * kStripes; }
+__device__ __forceinline__ int64_t xcd_stripe(int64_t bid, int64_t nb) {
+    const int64_t c = stripe_len(nb), k = bid / 8, turn = k / c;
+    return (turn * 8 + bid % 8) * c + (k - turn * c);
 }
 
 struct SegBase {
@@ -272,78 +272,7 @@ struct SegCtx {
 __device__ __forceinline__ SegCtx seg_ctx(const SegBase *seg, const Planes &q) { return SegCtx{seg, q.xy, q.za, 0, 0}; }
 
 // ------------------------------------------------------------------------------------------
-// Register windows and edge geometry shared by the emission and backward kernels
-
-// Samples of a lane's neighbourhood held in registers: v[i][j][k] is the sample at
-// (px + X0 + i, py + Y0 + j, pz + Z0 + k). Only ever indexed with compile-time constants. Boxes
-// of it are loaded on demand (load_box), so a kernel can test cheaply for work before loading
-// the rest. When the whole window of the whole wave lies inside the stored grid (`interior`,
-// wave-uniform: px, py and the chunk are), samples are read through a row pointer without
-// per-sample range checks.
-template <typename S, int X0, int NX, int Y0, int NY, int Z0, int NZ>
-struct Win {
-    S v[NX][NY][NZ];
-    int px, py, pz;
-    bool interior;
-    // a window whose interior test the caller has made (a count loop keeps it by row)
-    __device__ __forceinline__ Win(int px_, int py_, int pz_, bool interior_)
-        : px(px_), py(py_), pz(pz_), interior(interior_) {}
-    __device__ __forceinline__ Win(const In<S> &in, int px_, int py_, int pz_, int z0) : px(px_), py(py_), pz(pz_) {
-        const Geo &g = in.geo;
-        interior = px + X0 - g.off >= 0 && px + X0 + NX - 1 - g.off < g.n0 && py + Y0 - g.off >= 0 &&
-                   py + Y0 + NY - 1 - g.off < g.n1 && z0 + Z0 - g.off >= 0 &&
-                   z0 + kWave - 1 + Z0 + NZ - 1 - g.off < g.n2;
-    }
-    template <int BX0, int BNX, int BY0, int BNY, int BZ0, int BNZ>
-    __device__ __forceinline__ void load_box(const In<S> &in) {
-        static_assert(BX0 >= X0 && BX0 + BNX <= X0 + NX && BY0 >= Y0 && BY0 + BNY <= Y0 + NY && BZ0 >= Z0 &&
-                          BZ0 + BNZ <= Z0 + NZ,
-                      "box outside the window");
-        const Geo &g = in.geo;
-        const int64_t sy = g.n2, sx = (int64_t)g.n1 * g.n2;
-        if (interior) {
-            const S *p = in.sdf + ((int64_t)(px + BX0 - g.off) * g.n1 + (py + BY0 - g.off)) * g.n2 + (pz + BZ0 - g.off);
-#pragma unroll
-            for (int i = 0; i < BNX; ++i)
-#pragma unroll
-                for (int j = 0; j < BNY; ++j)
-#pragma unroll
-                    for (int k = 0; k < BNZ; ++k) v[BX0 - X0 + i][BY0 - Y0 + j][BZ0 - Z0 + k] = p[i * sx + j * sy + k];
-        } else if (NX * NY > 4) {  // wide windows: per sample (fewer live scalar registers)
-#pragma unroll
-            for (int i = 0; i < BNX; ++i)
-#pragma unroll
-                for (int j = 0; j < BNY; ++j)
-#pragma unroll
-                    for (int k = 0; k < BNZ; ++k)
-                        v[BX0 - X0 + i][BY0 - Y0 + j][BZ0 - Z0 + k] = sample(in, px + BX0 + i, py + BY0 + j, pz + BZ0 + k);
-        } else {
-            // rows outside the stored grid read as the pad value (a wave-uniform test); inside a
-            // row, lanes whose z is outside load at a valid address and select the pad value
-            const int x0 = px + BX0 - g.off, y0 = py + BY0 - g.off;
-            const int64_t r0 = ((int64_t)x0 * g.n1 + y0) * g.n2;  // offset of row (x0, y0), maybe outside
-#pragma unroll
-            for (int i = 0; i < BNX; ++i)
-#pragma unroll
-                for (int j = 0; j < BNY; ++j) {
-                    if ((unsigned)(x0 + i) < (unsigned)g.n0 && (unsigned)(y0 + j) < (unsigned)g.n1) {
-                        const S *p = in.sdf + (r0 + i * sx + j * sy);
-#pragma unroll
-                        for (int k = 0; k < BNZ; ++k) {
-                            const int z = pz + BZ0 + k - g.off;
-                            const bool inz = (unsigned)z < (unsigned)g.n2;
-                            const S a = p[inz ? z : 0];
-                            v[BX0 - X0 + i][BY0 - Y0 + j][BZ0 - Z0 + k] = inz ? a : in.pad;
-                        }
-                    } else {
-#pragma unroll
-                        for (int k = 0; k < BNZ; ++k) v[BX0 - X0 + i][BY0 - Y0 + j][BZ0 - Z0 + k] = in.pad;
-                    }
-                }
-        }
-    }
-    __device__ __forceinline__ S operator()(int dx, int dy, int dz) const { return v[dx - X0][dy - Y0][dz - Z0]; }
-};
+// Edge geometry shared by the emission and backward kernels
 
 // A segment's row (px, py) and chunk. The quotients come from double reciprocals: (n + 1/2) / d is at
 // least 1 / (2 d) away from an integer, and for n < 2^32 the product is off by less than 2^-20 (and
@@ -386,12 +315,6 @@ __device__ constexpr int eox(int e) { return (0x622 >> e) & 1; }
 __device__ constexpr int eoy(int e) { return (0x0F0 >> e) & 1; }
 __device__ constexpr int eoz(int e) { return (0xC44 >> e) & 1; }
 __device__ constexpr int eax(int e) { return e >= 8 ? 1 : ((e & 1) ? 2 : 0); }
-
-// Crossing mask of the three edges a cell owns, from its sample and its +x, +y, +z neighbours.
-template <typename S>
-__device__ __forceinline__ int own_mask(S d0, S dx, S dy, S dz, S iso) {
-    return crosses(d0, dx, iso) | (crosses(d0, dy, iso) << 1) | (crosses(d0, dz, iso) << 2);
-}
 
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -497,7 +420,7 @@ struct BatchGrid {
     const S *adj;  // upstream vertex gradients [nv, 3]
     S *adj_sdf, *adj_deform;
     int64_t q_first;  // DMC: first row of its per-edge gradients in the batch scratch
-    int run;          // segments per emission / backward block: the run length of the grid's size bucket
+    int tile;           // segments per gathering wave (bwd_tile_of the grid's size bucket)
 };
 
 // j such that rf[j] <= b < rf[j + 1] (rf ascending, rf[0] = 0, rf[m] = total).
@@ -1020,12 +943,6 @@ __global__ __launch_bounds__(kCountBlock, kCountWaves / 2) void count_kernel(Cou
 // rest cost one lane-parallel load of the run's bases. The run length is a launch parameter
 // (diso_set_param).
 constexpr int kMaxRun = kWave;
-
-// Per-lane bit of a wave-uniform plane, and the lanes' count of set bits below them.
-__device__ __forceinline__ int bit_of(uint64_t plane) { return __builtin_amdgcn_inverse_ballot_w64(plane) ? 1 : 0; }
-__device__ __forceinline__ int mask_of(uint64_t X, uint64_t Y, uint64_t Z) {
-    return bit_of(X) | (bit_of(Y) << 1) | (bit_of(Z) << 2);
-}
 
 struct OutCfg {
     int flags;
@@ -1715,13 +1632,13 @@ __global__ __launch_bounds__(kBlock, 5) void emit_dmc_kernel(In<S> in, const Seg
 // ------------------------------------------------------------------------------------------
 // Backward (gather, deterministic)
 //
-// MC: one lane per grid vertex; its incident crossing edges (at most six: the three it owns and
-// the ones owned by its -x, -y, -z neighbours) become items of a dense per-wave list. Each item
-// computes the adjoint of its edge vertex (adjComputeMcVert, src/cumc.cu:412-453) for the lane's
-// endpoint; the owning lane adds its items up in a fixed order (slot 0..5), so results are
-// deterministic and no atomics are used. Item slots: 0/1/2 = edge along x/y/z owned by the
-// vertex (vertex is its start), 3/4/5 = edge along x/y/z owned by the -x/-y/-z neighbour
-// (vertex is its end).
+// MC: one lane per touched grid vertex (one with an incident crossing edge), compacted over a wave's
+// run of segments; its incident crossing edges (at most six: the three it owns and the ones owned by
+// its -x, -y, -z neighbours) become items of a dense per-wave list. Each item computes the adjoint of
+// its edge vertex (adjComputeMcVert, src/cumc.cu:412-453) for the lane's endpoint; the owning lane
+// adds its items up in a fixed order (slot 0..5), so results are deterministic and no atomics are
+// used. Item slots: 0/1/2 = edge along x/y/z owned by the vertex (vertex is its start), 3/4/5 = edge
+// along x/y/z owned by the -x/-y/-z neighbour (vertex is its end).
 //
 // DMC: dmc_edge_grad_kernel first turns the DMC vertex gradients into one upstream gradient per
 // crossing edge (MC vertex order = quad order): the sum over the quad's four corners of (gradient
@@ -1758,81 +1675,84 @@ struct Grad {
     S g, dx, dy, dz;
 };
 
-// d t / d d0 and d t / d d1 factors of t = (iso - d0) / (d1 - d0), and t itself.
+// 1 / dd of an edge, and the quotient a / dd. fp32: gradients are compared within a tolerance, so the
+// hardware reciprocal (within an ulp) stands for the division.
 template <typename S>
-__device__ __forceinline__ void interp_adjoint(S d0, S d1, S iso, S *t, S *k0, S *k1) {
-    *t = interp_t(d0, d1, iso);
-    const S dd = (d1 - d0) * (d1 - d0);
-    *k0 = (iso - d1) / dd;
-    *k1 = (d0 - iso) / dd;
-}
-// fp32: gradients are compared within a tolerance, so one hardware reciprocal replaces the three
-// correctly rounded divisions (a few ulp).
+struct EdgeQuot {
+    S dd;
+    __device__ __forceinline__ explicit EdgeQuot(S d) : dd(d) {}
+    __device__ __forceinline__ S of(S a) const { return a / dd; }
+};
 template <>
-__device__ __forceinline__ void interp_adjoint<float>(float d0, float d1, float iso, float *t, float *k0, float *k1) {
-    const float r = __builtin_amdgcn_rcpf(d1 - d0);
-    *t = d1 != d0 ? clamp01<float>((iso - d0) * r) : 0.5f;
-    const float r2 = r * r;
-    *k0 = (iso - d1) * r2;
-    *k1 = (d0 - iso) * r2;
-}
+struct EdgeQuot<float> {
+    float r;
+    __device__ __forceinline__ explicit EdgeQuot(float d) : r(__builtin_amdgcn_rcpf(d)) {}
+    __device__ __forceinline__ float of(float a) const { return a * r; }
+};
 
-// Adjoint of one edge vertex (v0 -> v0 + e_axis, upstream gradient gv) at endpoint `end`
-// (0 = v0, 1 = v1), with the endpoints' samples d0, d1 and deforms f0, f1 (src/cumc.cu:412-453).
+// Adjoint of one edge vertex (upstream gradient gv) at one of the edge's ends: at integer position c
+// with sample d and deform f; the other end (dO, fO) is one step along `axis` away, in direction dir
+// (1 or -1). With t = (iso - d0) / (d1 - d0) and the vertex p0 + (p1 - p0) t
+// (src/cumc.cu:343-368,412-453) the end's weight is w = (dO - iso) / (dO - d) at either end, and the
+// sample's gradient -w / (dO - d) * (pO - p) . gv.
 template <typename S, bool DEF>
-__device__ __forceinline__ Grad<S> edge_adjoint(int x, int y, int z, int axis, int end, S d0, S d1, V3<S> f0,
-                                                V3<S> f1, S iso, V3<S> gv) {
-    S t, k0, k1;
-    interp_adjoint(d0, d1, iso, &t, &k0, &k1);
-    S p0x = S(x), p0y = S(y), p0z = S(z);
-    S p1x = S(x + (axis == 0)), p1y = S(y + (axis == 1)), p1z = S(z + (axis == 2));
+__device__ __forceinline__ Grad<S> edge_adjoint(V3<S> c, int axis, S dir, S d, S dO, V3<S> f, V3<S> fO, S iso, V3<S> gv) {
+    const EdgeQuot<S> q(dO - d);
+    const S w = q.of(dO - iso);
+    S dot;
     if (DEF) {
-        p0x += f0.x;
-        p0y += f0.y;
-        p0z += f0.z;
-        p1x += f1.x;
-        p1y += f1.y;
-        p1z += f1.z;
-    }
-    const S adj_t = (p1x - p0x) * gv.x + (p1y - p0y) * gv.y + (p1z - p0z) * gv.z;
-    const S wgt = end ? t : S(1) - t;
-    Grad<S> r;
-    r.g = (end ? k1 : k0) * adj_t;
-    r.dx = wgt * gv.x;
-    r.dy = wgt * gv.y;
-    r.dz = wgt * gv.z;
-    return r;
-}
-
-template <typename S>
-__device__ __forceinline__ void store_grad(const In<S> &in, S *__restrict__ adj_sdf, S *__restrict__ adj_deform, int x,
-                                           int y, int z, Grad<S> acc, int flags) {
-    if (!in_data(in, x, y, z)) return;
-    const int64_t i = data_index(in, x, y, z);
-    if (flags & DISO_FLAG_ACCUMULATE) {
-        adj_sdf[i] += acc.g;
-        if (adj_deform) {
-            adj_deform[3 * i + 0] += acc.dx;
-            adj_deform[3 * i + 1] += acc.dy;
-            adj_deform[3 * i + 2] += acc.dz;
-        }
+        const S sx = ((c.x + (axis == 0 ? dir : S(0))) + fO.x) - (c.x + f.x);
+        const S sy = ((c.y + (axis == 1 ? dir : S(0))) + fO.y) - (c.y + f.y);
+        const S sz = ((c.z + (axis == 2 ? dir : S(0))) + fO.z) - (c.z + f.z);
+        dot = sx * gv.x + sy * gv.y + sz * gv.z;
     } else {
-        put(adj_sdf + i, acc.g);
-        if (adj_deform) {
-            put(adj_deform + 3 * i + 0, acc.dx);
-            put(adj_deform + 3 * i + 1, acc.dy);
-            put(adj_deform + 3 * i + 2, acc.dz);
-        }
+        dot = dir * (axis == 0 ? gv.x : (axis == 1 ? gv.y : gv.z));
     }
+    const S wc = clamp01<S>(w);
+    return Grad<S>{-(q.of(w) * dot), wc * gv.x, wc * gv.y, wc * gv.z};
 }
 
-// Per-wave LDS of the gather: the vertex id of each incident edge relative to the segment's first
-// vertex; the item list (lane * 8 + slot) and one round of item results.
+// Zeros p[a..b), by one wave: 16-byte stores between the aligned ends.
+template <typename S>
+__device__ __forceinline__ void fill_zero(S *__restrict__ p, int64_t a, int64_t b, int lane) {
+    typedef S vec __attribute__((ext_vector_type(16 / sizeof(S))));
+    constexpr int N = 16 / (int)sizeof(S);
+    const int64_t mis = (int64_t)(((uintptr_t)p / sizeof(S)) % N);  // elements past a 16-byte boundary
+    int64_t a1 = (a + mis + N - 1) / N * N - mis, b1 = (b + mis) / N * N - mis;
+    if (a1 >= b1) a1 = b1 = b;
+    if (a + lane < a1) put(p + a + lane, S(0));  // fewer than N elements, or (no aligned part) the whole
+    for (int64_t i = a + kWave + lane; i < a1; i += kWave) put(p + i, S(0));
+    for (int64_t i = a1 + (int64_t)lane * N; i < b1; i += kWave * N) put(reinterpret_cast<vec *>(p + i), vec(S(0)));
+    if (b1 + lane < b) put(p + b1 + lane, S(0));
+}
+
+// The gather's blocks are single waves, so that none waits for another's share. Per kBwdGroup
+// segments there is one that zeroes the gradients of the segments without a touched vertex (the
+// vector-memory counter is in order and covers stores: a gathering wave that issued these stores
+// would wait for them), and kBwdParts for each tile of at most kBwdTile segments, which gather 64
+// touched vertices at a time in turn (a tile of a surface that runs along z holds up to 512). On
+// 256^3 noisy / 203x256x181 smooth: tiles of 8 in one part 131 / 64 us, in two 127 / 60, in four 148 /
+// 64; tiles of 4 in one part 129 / 60, of 16 149 / 83; groups of 64, 32, 16 segments 127 / 60,
+// 128 / 55, 132 / 57. (A recomputing wave does not share a tile: each would recompute the planes.)
+constexpr int kBwdTile = 8;
+constexpr int kBwdGroup = 32;
+template <bool RECOMP>
+constexpr int kBwdParts = RECOMP ? 1 : 2;
+
+// LDS of a gathering wave.
 template <typename S>
 struct BwdLds {
-    int32_t id[6][kWave];
-    uint16_t item[kWave * 6];
-    Grad<S> res[2 * kWave];
+    uint64_t pl[kBwdTile][10];   // crossing planes: X, Y, Z of the segment, of rows -x, -y; Z of the previous chunk
+    int64_t at[kBwdTile];        // index of the sample at the segment's position 0 (as if it were stored)
+    int32_t base[kBwdTile][3];   // first vertex of the segment, of rows -x, -y, relative to the tile's first
+    int32_t px[kBwdTile], py[kBwdTile], z0[kBwdTile];  // its row, and its first z
+    uint32_t rows[kBwdTile];     // which neighbour rows are stored: +x, +y, -x, -y in bits 0, 1, 3, 4
+    int64_t idx[kWave];          // the chunk's vertices: sample index, integer position
+    S pos[3][kWave];
+    int32_t id[3][kWave];        // and first vertex ids: own edges, the x edge of -x, the y edge of -y
+    uint16_t list[kWave];        // the vertices: segment << 6 | position
+    uint16_t item[kWave * 6];    // vertex | slot << 6 | other end stored << 9 | id offset + 1 << 10
+    Grad<S> res[2 * kWave];      // one round of item results
 };
 
 // Whether segment t (-1: none) owns a crossing edge.
@@ -1849,187 +1769,340 @@ __device__ __forceinline__ bool seg_touched(const SegBase *__restrict__ seg, con
            (sp.chunk > 0 && seg_owns_crossing(seg, s - 1));
 }
 
-// What a gather segment reads before any work: the vertex bases of the segment and of rows -x, -y
-// (the segment's own base where the row does not exist) and, unless the masks are recomputed from
-// the samples, the classification words of the vertex and of its -x, -y, -z neighbours. Loaded one
-// segment ahead, so these loads overlap the previous segment's work.
-struct BwdSegIn {
-    int64_t s;
-    SegPos sp;
-    int64_t v;
-    int32_t dm0, d0m;  // first vertices of rows -x, -y relative to the segment's
-    RowEdges e00, em0, e0m;  // crossing planes of the segment and of rows -x, -y
-    uint64_t zp;             // and the z plane of the previous chunk
-};
-
-template <bool RECOMP>
-__device__ __forceinline__ BwdSegIn bwd_load(const Geo &g, const SegCtx &sc, int64_t s, SegPos sp, int lane) {
-    const SegBase *__restrict__ seg = sc.seg;
-    BwdSegIn d;
-    d.s = s;
-    d.sp = sp;
-    const int64_t sm0 = sp.px > 0 ? s - xstride(g) : -1;
-    const int64_t s0m = sp.py > 0 ? s - g.nchunk : -1;
-    d.v = seg[s].v;
-    d.dm0 = sm0 >= 0 ? (int32_t)(seg[sm0].v - d.v) : 0;
-    d.d0m = s0m >= 0 ? (int32_t)(seg[s0m].v - d.v) : 0;
-    d.e00 = d.em0 = d.e0m = RowEdges{0, 0, 0};
-    d.zp = 0;
-    if constexpr (!RECOMP) {
-        const Plane2 *__restrict__ xy = sc.xy, *__restrict__ za = sc.za;
-        d.e00 = RowEdges{xy[s].a, xy[s].b, za[s].a};
-        if (sm0 >= 0) d.em0 = RowEdges{xy[sm0].a, xy[sm0].b, za[sm0].a};
-        if (s0m >= 0) d.e0m = RowEdges{xy[s0m].a, xy[s0m].b, za[s0m].a};
-        if (sp.chunk > 0) d.zp = za[s - 1].a;
-    }
-    return d;
+__device__ __forceinline__ float from_lane(float v, int lane4) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(lane4, __float_as_int(v)));
+}
+__device__ __forceinline__ double from_lane(double v, int lane4) {
+    return __hiloint2double(__builtin_amdgcn_ds_bpermute(lane4, __double2hiint(v)),
+                            __builtin_amdgcn_ds_bpermute(lane4, __double2loint(v)));
 }
 
-// Gather of one touched segment.
-template <typename S, bool DEF, bool RECOMP>
-__device__ __forceinline__ void bwd_segment(const In<S> &in, const SegCtx &sc, const BwdSegIn &sg,
-                                            const AdjIn<S> &adj, S *__restrict__ adj_sdf,
-                                            S *__restrict__ adj_deform, BwdLds<S> &L, int lane) {
-    wave_lds_sync();  // the previous segment's LDS reads are done
-    const int px = sg.sp.px, py = sg.sp.py, chunk = sg.sp.chunk;
-    const int z0 = chunk * kWave, pz = z0 + lane;
-    const S iso = in.iso;
-    Grad<S> acc = {S(0), S(0), S(0), S(0)};
-    const int64_t vabs = sg.v, vbase = vabs - sc.v0;
-    // Crossing masks of the edges owned by the vertex and by its -x, -y, -z neighbours: from the
-    // classification words, or (RECOMP) from the samples of the vertex's neighbourhood.
-    int m00, mm0, m0m, mzm;
-    if constexpr (RECOMP) {
-        Win<S, -1, 3, -1, 3, -1, 3> w(in, px, py, pz, z0);
-        w.template load_box<0, 1, 0, 1, -1, 3>(in);
-        w.template load_box<-1, 1, 0, 1, 0, 2>(in);
-        w.template load_box<-1, 1, 1, 1, 0, 1>(in);
-        w.template load_box<1, 1, -1, 2, 0, 1>(in);
-        w.template load_box<0, 1, -1, 1, 0, 2>(in);
-        w.template load_box<0, 1, 1, 1, 0, 1>(in);
-        const S c = w(0, 0, 0);
-        m00 = is_anchor(in, px, py, pz) ? own_mask(c, w(1, 0, 0), w(0, 1, 0), w(0, 0, 1), iso) : 0;
-        mm0 = is_anchor(in, px - 1, py, pz) ? own_mask(w(-1, 0, 0), c, w(-1, 1, 0), w(-1, 0, 1), iso) : 0;
-        m0m = is_anchor(in, px, py - 1, pz) ? own_mask(w(0, -1, 0), w(1, -1, 0), c, w(0, -1, 1), iso) : 0;
-        mzm = is_anchor(in, px, py, pz - 1) ? crosses(w(0, 0, -1), c, iso) << 2 : 0;
-    } else {
-        m00 = mask_of(sg.e00.X, sg.e00.Y, sg.e00.Z);
-        mm0 = mask_of(sg.em0.X, sg.em0.Y, sg.em0.Z);
-        m0m = mask_of(sg.e0m.X, sg.e0m.Y, sg.e0m.Z);
-        mzm = bit_of(diso_bits::down1(sg.e00.Z, sg.zp)) << 2;
-    }
-    // slots 0-2: edges the vertex owns; 3-5: the x edge of -x, the y edge of -y, the z edge of -z
-    const int inc_m = (mm0 & 1) | (m0m & 2) | (mzm & 4);
-    const int mask = in_data(in, px, py, pz) ? (m00 | (inc_m << 3)) : 0;
-    // exclusive prefixes over the lanes of the rows' vertex counts (10-bit fields, totals <= 192)
-    // and of the items, in two DPP scans
-    const uint32_t cA = (uint32_t)popc3(m00) | (uint32_t)popc3(mm0) << 10 | (uint32_t)popc3(m0m) << 20;
-    const uint32_t cB = (uint32_t)__popc(mask);
-    const uint32_t iA = wave_incl_dpp(cA), iB = wave_incl_dpp(cB);
-    const uint32_t eA = iA - cA;
-    const int32_t r00 = (int32_t)(eA & 0x3ff);
-    const int32_t rm0 = sg.dm0 + (int32_t)((eA >> 10) & 0x3ff);
-    const int32_t r0m = sg.d0m + (int32_t)((eA >> 20) & 0x3ff);
-    const int first = (int)(iB - cB), total = __builtin_amdgcn_readlane((int)iB, kWave - 1);
+// Index of the first stored sample at or after a segment's first position: the samples of segments
+// [a, b) are the contiguous range [sample_start(a), sample_start(b)).
+__device__ __forceinline__ int64_t sample_start(const Geo &g, const SegPos &sp) {
+    const int64_t plane = (int64_t)g.n1 * g.n2;
+    const int x = sp.px - g.off, y = sp.py - g.off, z = sp.chunk * kWave - g.off;
+    if (x < 0) return 0;
+    if (x >= g.n0) return g.n0 * plane;
+    if (y < 0) return x * plane;
+    if (y >= g.n1) return (x + 1) * plane;
+    return x * plane + (int64_t)y * g.n2 + (z < 0 ? 0 : (z < g.n2 ? z : g.n2));
+}
 
-    L.id[0][lane] = r00;
-    L.id[1][lane] = r00 + (m00 & 1);
-    L.id[2][lane] = r00 + (m00 & 1) + ((m00 >> 1) & 1);
-    L.id[3][lane] = rm0;
-    L.id[4][lane] = r0m + (m0m & 1);
-    L.id[5][lane] = r00 - 1;
+// Inside and below bits of a segment's row of samples (wave-uniform row).
+struct SideBits {
+    uint64_t in, below;
+};
+template <typename S>
+__device__ __forceinline__ SideBits row_bits(const In<S> &in, int px, int py, int z0, int lane) {
+    const S v = sample(in, px, py, z0 + lane);
+    return SideBits{__ballot(v >= in.iso), __ballot(v < in.iso)};
+}
+__device__ __forceinline__ uint64_t cross_bits(SideBits a, SideBits b) { return (a.below & b.in) | (b.below & a.in); }
+__device__ __forceinline__ SideBits side_up(SideBits a, SideBits next, int bit) {
+    return SideBits{diso_bits::up1(a.in, next.in >> bit), diso_bits::up1(a.below, next.below >> bit)};
+}
+
+// The crossing planes of BwdLds::pl from the samples (the recomputing backward): returns them in
+// scalar registers, the same in every lane.
+struct BwdPlanes {
+    uint64_t w[10];
+};
+template <typename S>
+__device__ __forceinline__ BwdPlanes recompute_planes(const In<S> &in, const SegPos &sp, int lane) {
+    const Geo &g = in.geo;
+    const int px = sp.px, py = sp.py, z0 = sp.chunk * kWave;
+    const SideBits c = row_bits(in, px, py, z0, lane), xp = row_bits(in, px + 1, py, z0, lane),
+                   yp = row_bits(in, px, py + 1, z0, lane), xm = row_bits(in, px - 1, py, z0, lane),
+                   ym = row_bits(in, px, py - 1, z0, lane), xmyp = row_bits(in, px - 1, py + 1, z0, lane),
+                   xpym = row_bits(in, px + 1, py - 1, z0, lane);
+    // lanes 0-2: position z0 + 64 of rows (0,0), (-1,0), (0,-1); lane 3: position z0 - 1 of row (0,0)
+    const S e = sample(in, px - (lane == 1), py - (lane == 2), lane == 3 ? z0 - 1 : z0 + kWave);
+    const SideBits eb{__ballot(e >= in.iso), __ballot(e < in.iso)};
+    const uint64_t am = diso_bits::low_bits(g.g2 - 1 - z0);  // positions that anchor a cell
+    const bool ax = px < g.g0 - 1, ay = py < g.g1 - 1;
+    const uint64_t m00 = ax && ay ? am : 0ull, mx = px > 0 && ay ? am : 0ull, my = py > 0 && ax ? am : 0ull;
+    BwdPlanes r;
+    r.w[0] = cross_bits(c, xp) & m00;
+    r.w[1] = cross_bits(c, yp) & m00;
+    r.w[2] = cross_bits(c, side_up(c, eb, 0)) & m00;
+    r.w[3] = cross_bits(xm, c) & mx;
+    r.w[4] = cross_bits(xm, xmyp) & mx;
+    r.w[5] = cross_bits(xm, side_up(xm, eb, 1)) & mx;
+    r.w[6] = cross_bits(ym, xpym) & my;
+    r.w[7] = cross_bits(ym, c) & my;
+    r.w[8] = cross_bits(ym, side_up(ym, eb, 2)) & my;
+    const SideBits prev{eb.in >> 3, eb.below >> 3};
+    // the edge from z0 - 1 (in a previous chunk's top position)
+    r.w[9] = sp.chunk > 0 && ax && ay && (cross_bits(prev, c) & 1) && z0 - 1 < g.g2 - 1 ? 1ull << 63 : 0ull;
+    return r;
+}
+
+// Gather of up to 64 touched vertices (the first nv of L.list): lane k's gradients.
+template <typename S, bool DEF>
+__device__ __forceinline__ Grad<S> bwd_chunk(const In<S> &in, const AdjIn<S> &adj, int64_t vbase, int nv, BwdLds<S> &L,
+                                             int lane) {
+    const Geo &g = in.geo;
+    const int w = L.list[lane < nv ? lane : 0], j = w >> 6, l = w & 63;
+    const uint64_t *pl = L.pl[j];
+    const RowEdges e00{pl[0], pl[1], pl[2]}, em0{pl[3], pl[4], pl[5]}, e0m{pl[6], pl[7], pl[8]};
+    const uint64_t b = (1ull << l) - 1;
+    const int x = bit_at(e00.X, l), y = bit_at(e00.Y, l), z = bit_at(e00.Z, l);
+    const int xm = bit_at(em0.X, l), ym = bit_at(e0m.Y, l), zm = bit_at(diso_bits::down1(e00.Z, pl[9]), l);
+    const int mask = lane < nv ? x | y << 1 | z << 2 | xm << 3 | ym << 4 | zm << 5 : 0;
+    const int64_t idx = L.at[j] + l;
+    const int zs = L.z0[j] + l - g.off;
+    L.idx[lane] = idx;
+    if (DEF) {
+        L.pos[0][lane] = S(L.px[j]);
+        L.pos[1][lane] = S(L.py[j]);
+        L.pos[2][lane] = S(L.z0[j] + l);
+    }
+    L.id[0][lane] = L.base[j][0] + e00.below(b);
+    L.id[1][lane] = L.base[j][1] + em0.below(b);
+    L.id[2][lane] = L.base[j][2] + e0m.below(b) + bit_at(e0m.X, l);
+    // the other end is a stored sample (else it is the pad)
+    const uint32_t ok = L.rows[j] | (zs + 1 < g.n2 ? 4u : 0u) | (zs > 0 ? 32u : 0u);
+    const uint32_t cB = (uint32_t)__popc(mask), iB = wave_incl_dpp(cB);
+    const int first = (int)(iB - cB), last = (int)iB, total = __builtin_amdgcn_readlane((int)iB, kWave - 1);
     {
-        // (branch-free writes to a spare entry measured 2 us slower here)
+        const int off[6] = {1, 1 + x, 1 + x + y, 1, 1, 0};  // id offset + 1
         int r = first;
 #pragma unroll
         for (int sl = 0; sl < 6; ++sl)
-            if ((mask >> sl) & 1) L.item[r++] = (uint16_t)(lane * 8 + sl);
+            if ((mask >> sl) & 1) L.item[r++] = (uint16_t)(lane | sl << 6 | (int)((ok >> sl) & 1) << 9 | off[sl] << 10);
     }
     wave_lds_sync();
 
-    const int last = first + __popc(mask);
-    // Adjoint of item k (an edge and the endpoint that is this segment's vertex).
+    const int64_t sy = g.n2, sx = (int64_t)g.n1 * g.n2;
+    // Adjoint of item k (an edge and its end that is the vertex).
     auto item = [&](int k) {
-        const int it = L.item[k], src = it >> 3, slot = it & 7;
-        const int axis = slot % 3, end = slot >= 3;
-        // the edge runs from (x, y, z) along `axis`; the vertex is its start (slots 0-2) or its end
-        const int x = px - (slot == 3), y = py - (slot == 4), z = z0 + src - (slot == 5);
-        const EdgeEnds<S, DEF> e = edge_ends<S, DEF>(in, x, y, z, axis);
-        return edge_adjoint<S, DEF>(x, y, z, axis, end, e.d0, e.d1, e.f0, e.f1, iso,
-                                    load_adj(adj, vbase + L.id[slot][src]));
+        const int it = L.item[k], src = it & 63, slot = (it >> 6) & 7, end = slot >= 3, axis = end ? slot - 3 : slot;
+        const bool st = (it >> 9) & 1;
+        const int64_t i0 = L.idx[src], step = axis == 0 ? sx : (axis == 1 ? sy : 1);
+        const int64_t i1 = st ? (end ? i0 - step : i0 + step) : i0;
+        const int id = L.id[slot == 3 ? 1 : (slot == 4 ? 2 : 0)][src] + (it >> 10) - 1;
+        const S d = in.sdf[i0], dO = in.sdf[i1];
+        V3<S> c = {S(0), S(0), S(0)}, f = c, fO = c;
+        if (DEF) {
+            c = V3<S>{L.pos[0][src], L.pos[1][src], L.pos[2][src]};
+            const S *p0 = in.deform + 3 * i0, *p1 = in.deform + 3 * i1;
+            f = V3<S>{p0[0], p0[1], p0[2]};
+            const S u0 = p1[0], u1 = p1[1], u2 = p1[2];
+            fO = V3<S>{st ? u0 : S(0), st ? u1 : S(0), st ? u2 : S(0)};
+        }
+        const V3<S> gv = load_adj(adj, vbase + id);
+        return edge_adjoint<S, DEF>(c, axis, end ? S(-1) : S(1), d, st ? dO : in.pad, f, fO, in.iso, gv);
     };
+    Grad<S> acc = {S(0), S(0), S(0), S(0)};
     // Rounds of up to 128 items: with more than 64 left, each lane takes two (the second clamped
     // to the last item, its result unused), so both gathers are in flight together.
-    for (int b = 0; b < total; b += 2 * kWave) {
-        if (b + kWave < total) {  // wave-uniform
-            const int k1 = b + kWave + lane < total ? b + kWave + lane : total - 1;
-            const Grad<S> r0 = item(b + lane), r1 = item(k1);
+    for (int r = 0; r < total; r += 2 * kWave) {
+        if (r + kWave < total) {  // wave-uniform
+            const int k1 = r + kWave + lane < total ? r + kWave + lane : total - 1;
+            const Grad<S> r0 = item(r + lane), r1 = item(k1);
             L.res[lane] = r0;
             L.res[kWave + lane] = r1;
-        } else if (b + lane < total) {
-            L.res[lane] = item(b + lane);
+        } else if (r + lane < total) {
+            L.res[lane] = item(r + lane);
         }
         wave_lds_sync();
-        const int lo = first > b ? first : b, hi = last < b + 2 * kWave ? last : b + 2 * kWave;
-        for (int j = lo; j < hi; ++j) {  // this lane's items of the round, in slot order
-            const Grad<S> r = L.res[j - b];
-            acc.g += r.g;
-            acc.dx += r.dx;
-            acc.dy += r.dy;
-            acc.dz += r.dz;
+        const int lo = first > r ? first : r, hi = last < r + 2 * kWave ? last : r + 2 * kWave;
+        for (int k = lo; k < hi; ++k) {  // this lane's items of the round, in slot order
+            const Grad<S> q = L.res[k - r];
+            acc.g += q.g;
+            acc.dx += q.dx;
+            acc.dy += q.dy;
+            acc.dz += q.dz;
         }
         wave_lds_sync();
     }
-    store_grad(in, adj_sdf, adj_deform, px, py, pz, acc, adj.flags);
+    return acc;
 }
 
-// The touched segments of a block (bits of `act`, segment lo + bit) dealt round-robin over its
-// waves, each wave's next segment loaded while it gathers the current one. (Taking them from a
-// shared counter, as the emission kernels do, measured slower here: the gathers' costs vary
-// less.)
-template <typename S, bool DEF, bool RECOMP>
-__device__ __forceinline__ void bwd_run(const In<S> &in, const SegCtx &sc, int64_t lo, const SegPos &lp, uint64_t act,
-                                        const AdjIn<S> &adj, S *__restrict__ adj_sdf, S *__restrict__ adj_deform,
-                                        BwdLds<S> &L, int wave, int lane) {
-    uint64_t mine = 0;
-    for (int k = 0; act; ++k, act &= act - 1)
-        if ((k & (kWavesPerBlock - 1)) == wave) mine |= act & (0ull - act);
-    if (!mine) return;
-    int i = __builtin_ctzll(mine);
-    BwdSegIn nxt = bwd_load<RECOMP>(in.geo, sc, lo + i, pos_of_lane(lp, i), lane);
-    while (mine) {
-        const BwdSegIn cur = nxt;
-        mine &= mine - 1;
-        if (mine) {
-            i = __builtin_ctzll(mine);
-            nxt = bwd_load<RECOMP>(in.geo, sc, lo + i, pos_of_lane(lp, i), lane);
-        }
-        bwd_segment<S, DEF, RECOMP>(in, sc, cur, adj, adj_sdf, adj_deform, L, lane);
-    }
-}
-
-template <typename S, bool DEF, bool RECOMP>
-__global__ __launch_bounds__(kBlock) void bwd_mc_kernel(In<S> in, const SegBase *__restrict__ seg, AdjIn<S> adj,
-                                                        S *__restrict__ adj_sdf, S *__restrict__ adj_deform,
-                                                        int run, int64_t nblocks) {
-    __shared__ BwdLds<S> s_lds[kWavesPerBlock];
-    const int tid = threadIdx.x, wave = wave_id(), lane = tid % kWave;
+// What a lane knows of its segment in the backward: its place, its stored positions and the index of
+// the sample at its position 0.
+struct BwdSeg {
+    SegPos sp;
+    uint64_t have;
+    int64_t at;
+    uint32_t rows;
+};
+template <typename S>
+__device__ __forceinline__ BwdSeg bwd_seg(const In<S> &in, int64_t s, bool valid) {
     const Geo &g = in.geo;
-    const SegCtx sc = seg_ctx(seg, planes_of(seg, g.nseg));
-    const int64_t lo = xcd_block(blockIdx.x, nblocks) * run, hi = lo + run < g.nseg ? lo + run : g.nseg;
-    const int64_t t = lo + lane;
-    const SegPos lp = seg_pos(g, t);
-    const bool touched = t < hi && seg_touched(seg, g, t, lp);
-    uint64_t act = __ballot(touched);
-    // untouched segments get zero gradients (unless accumulating), dealt round-robin as well
-    uint64_t idle = (adj.flags & DISO_FLAG_ACCUMULATE) ? 0ull : __ballot(t < hi && !touched);
-    for (int k = 0; idle; ++k, idle &= idle - 1)
-        if ((k & (kWavesPerBlock - 1)) == wave) {
-            const SegPos sp = pos_of_lane(lp, __builtin_ctzll(idle));
-            store_grad(in, adj_sdf, adj_deform, sp.px, sp.py, sp.chunk * kWave + lane, Grad<S>{S(0), S(0), S(0), S(0)},
-                       adj.flags);
+    BwdSeg r;
+    r.sp = seg_pos(g, s);
+    const int x = r.sp.px - g.off, y = r.sp.py - g.off, z = r.sp.chunk * kWave - g.off;
+    const bool row = (unsigned)x < (unsigned)g.n0 && (unsigned)y < (unsigned)g.n1;
+    r.have = row && valid ? diso_bits::low_bits(g.n2 - z) & ~diso_bits::low_bits(-z) : 0ull;
+    r.at = ((int64_t)x * g.n1 + y) * g.n2 + z;
+    r.rows = (x + 1 < g.n0 ? 1u : 0u) | (y + 1 < g.n1 ? 2u : 0u) | (x > 0 ? 8u : 0u) | (y > 0 ? 16u : 0u);
+    return r;
+}
+
+// Crossing planes of lane i's segment s, as BwdLds::pl.
+__device__ __forceinline__ BwdPlanes stored_planes(const SegCtx &sc, const Geo &g, int64_t s, const SegPos &sp) {
+    BwdPlanes r;
+    const bool rx = sp.px > 0, ry = sp.py > 0;
+    const int64_t sm0 = rx ? s - xstride(g) : s, s0m = ry ? s - g.nchunk : s;
+    const Plane2 a = sc.xy[s], b = sc.xy[sm0], c = sc.xy[s0m];
+    const uint64_t az = sc.za[s].a, bz = sc.za[sm0].a, cz = sc.za[s0m].a;
+    r.w[0] = a.a, r.w[1] = a.b, r.w[2] = az;
+    r.w[3] = rx ? b.a : 0, r.w[4] = rx ? b.b : 0, r.w[5] = rx ? bz : 0;
+    r.w[6] = ry ? c.a : 0, r.w[7] = ry ? c.b : 0, r.w[8] = ry ? cz : 0;
+    r.w[9] = sp.chunk > 0 ? sc.za[s - 1].a : 0ull;
+    return r;
+}
+// Positions with an incident crossing edge.
+__device__ __forceinline__ uint64_t touched_bits(const uint64_t *w) {
+    return w[0] | w[1] | w[2] | w[3] | w[7] | diso_bits::down1(w[2], w[9]);
+}
+
+// Zero gradients of those of kBwdGroup segments from lo on that the gathering waves leave out (the samples of
+// consecutive segments are contiguous, so runs of them are zeroed together).
+template <typename S, bool DEF, bool RECOMP>
+__device__ __forceinline__ void bwd_zero(const In<S> &in, const SegCtx &sc, int64_t lo, S *__restrict__ adj_sdf,
+                                         S *__restrict__ adj_deform, int lane) {
+    const Geo &g = in.geo;
+    const int64_t all = (int64_t)g.n0 * g.n1 * g.n2, s = lo + lane;
+    const int n = g.nseg - lo < kBwdGroup ? (int)(g.nseg - lo) : kBwdGroup;
+    const BwdSeg q = bwd_seg(in, lane < n ? s : lo, lane < n);
+    bool touched = false;
+    if (lane < n)
+        touched = RECOMP ? q.have && seg_touched(sc.seg, g, s, q.sp)
+                         : (touched_bits(stored_planes(sc, g, s, q.sp).w) & q.have) != 0;
+    const int64_t start = lane < n ? sample_start(g, q.sp) : all;
+    const int64_t end = lo + n < g.nseg ? sample_start(g, seg_pos(g, lo + n)) : all;
+    for (uint64_t idle = ~__ballot(touched) & diso_bits::low_bits(n); idle;) {  // wave-uniform
+        const int a = (int)__builtin_ctzll(idle);
+        const uint64_t rest = ~(idle >> a);
+        const int len = rest ? (int)__builtin_ctzll(rest) : kWave;
+        const int64_t i0 = readlane64(start, a), i1 = a + len < n ? readlane64(start, a + len) : end;
+        fill_zero(adj_sdf, i0, i1, lane);
+        if (DEF) fill_zero(adj_deform, 3 * i0, 3 * i1, lane);
+        idle &= ~(diso_bits::low_bits(len) << a);
+    }
+}
+
+// Gather of the segments [lo, lo + n) of a grid (n <= kBwdTile) by one wave: 64 of their touched
+// vertices at a time, each segment's gradients then written as a row, zeros included.
+template <typename S, bool DEF, bool RECOMP>
+__device__ __forceinline__ void bwd_tile(const In<S> &in, const SegCtx &sc, int64_t lo, int n, const AdjIn<S> &adj,
+                                         S *__restrict__ adj_sdf, S *__restrict__ adj_deform, BwdLds<S> &L, int part, int lane) {
+    const Geo &g = in.geo;
+    const bool acc = (adj.flags & DISO_FLAG_ACCUMULATE) != 0;
+    const int64_t s = lo + (lane < n ? lane : 0);  // lane i: segment lo + i
+    const BwdSeg q = bwd_seg(in, s, lane < n);
+    const int64_t sm0 = q.sp.px > 0 ? s - xstride(g) : s, s0m = q.sp.py > 0 ? s - g.nchunk : s;
+    const int64_t v00 = sc.seg[s].v, vm0 = sc.seg[sm0].v, v0m = sc.seg[s0m].v;  // (issued with the planes)
+    uint64_t cand, T = 0;
+    if constexpr (RECOMP) {
+        // the planes from the samples, for the segments that can have a touched vertex (by the bases)
+        cand = __ballot(q.have && seg_touched(sc.seg, g, s, q.sp));
+        for (uint64_t c = cand; c; c &= c - 1) {  // wave-uniform
+            const int j = (int)__builtin_ctzll(c);
+            const BwdPlanes p = recompute_planes(in, pos_of_lane(q.sp, j), lane);
+            if (lane == 0)
+                for (int k = 0; k < 10; ++k) L.pl[j][k] = p.w[k];
         }
-    bwd_run<S, DEF, RECOMP>(in, sc, lo, lp, act, adj, adj_sdf, adj_deform, s_lds[wave], wave, lane);
+        wave_lds_sync();
+        if ((cand >> lane) & 1) T = touched_bits(L.pl[lane]) & q.have;
+    } else {
+        const BwdPlanes p = stored_planes(sc, g, s, q.sp);
+        T = touched_bits(p.w) & q.have;
+        cand = __ballot(T != 0);
+        if (lane < n)
+            for (int k = 0; k < 10; ++k) L.pl[lane][k] = p.w[k];
+    }
+    if (!cand) return;
+    const int64_t v0 = readlane64(v00, 0);
+    if (lane < n) {
+        L.at[lane] = q.at;
+        L.px[lane] = q.sp.px;
+        L.py[lane] = q.sp.py;
+        L.z0[lane] = q.sp.chunk * kWave;
+        L.rows[lane] = q.rows;
+        L.base[lane][0] = (int32_t)(v00 - v0);
+        L.base[lane][1] = (int32_t)(vm0 - v0);
+        L.base[lane][2] = (int32_t)(v0m - v0);
+    }
+    const uint32_t cT = (uint32_t)__popcll(T), iT = wave_incl_dpp(cT);
+    const int pre = (int)(iT - cT), total = __builtin_amdgcn_readlane((int)iT, kWave - 1);
+    for (int c0 = part * kWave; c0 < total || (RECOMP && c0 == 0); c0 += kBwdParts<RECOMP> * kWave) {  // wave-uniform
+        const int nv = total - c0 < kWave ? total - c0 : kWave;
+        const uint64_t segs = __ballot(T != 0 && pre < c0 + nv && (int)iT > c0);
+        for (uint64_t a = segs; a; a &= a - 1) {
+            const int j = (int)__builtin_ctzll(a);
+            const uint64_t t = (uint64_t)readlane64((int64_t)T, j);
+            const int k = __builtin_amdgcn_readlane(pre, j) - c0 + lanes_below(t);
+            if (__builtin_amdgcn_inverse_ballot_w64(t) && k >= 0 && k < kWave) L.list[k] = (uint16_t)(j << 6 | lane);
+        }
+        wave_lds_sync();
+        Grad<S> r = {S(0), S(0), S(0), S(0)};
+        if (nv > 0) r = bwd_chunk<S, DEF>(in, adj, v0 - sc.v0, nv, L, lane);
+        // rows of the segments with a vertex in the chunk (and, with the first chunk, of those that
+        // turned out to have none)
+        for (uint64_t a = segs | (RECOMP && c0 == 0 && !acc ? cand & ~__ballot(T != 0) : 0ull); a; a &= a - 1) {
+            const int j = (int)__builtin_ctzll(a);
+            const uint64_t t = (uint64_t)readlane64((int64_t)T, j), h = (uint64_t)readlane64((int64_t)q.have, j);
+            const int at = __builtin_amdgcn_readlane(pre, j) - c0, k = at + lanes_below(t);
+            const int from = (k & (kWave - 1)) << 2;
+            Grad<S> w;
+            w.g = from_lane(r.g, from);
+            if (DEF) {
+                w.dx = from_lane(r.dx, from);
+                w.dy = from_lane(r.dy, from);
+                w.dz = from_lane(r.dz, from);
+            }
+            const bool mine = __builtin_amdgcn_inverse_ballot_w64(t) && k >= 0 && k < nv;
+            const bool zero = at >= 0 && __builtin_amdgcn_inverse_ballot_w64(h & ~t);  // with the segment's first vertex
+            const int64_t i = readlane64(q.at, j) + lane;
+            if (acc) {
+                if (mine) {
+                    adj_sdf[i] += w.g;
+                    if (DEF) {
+                        adj_deform[3 * i + 0] += w.dx;
+                        adj_deform[3 * i + 1] += w.dy;
+                        adj_deform[3 * i + 2] += w.dz;
+                    }
+                }
+            } else if (mine || zero) {
+                put(adj_sdf + i, mine ? w.g : S(0));
+                if (DEF) {
+                    put(adj_deform + 3 * i + 0, mine ? w.dx : S(0));
+                    put(adj_deform + 3 * i + 1, mine ? w.dy : S(0));
+                    put(adj_deform + 3 * i + 2, mine ? w.dz : S(0));
+                }
+            }
+        }
+        wave_lds_sync();
+    }
+}
+
+// Block k of the blocks of one grid (bwd_blocks of them).
+template <typename S, bool DEF, bool RECOMP>
+__device__ __forceinline__ void bwd_wave(const In<S> &in, const SegCtx &sc, int64_t k, int tile, const AdjIn<S> &adj,
+                                         S *__restrict__ adj_sdf, S *__restrict__ adj_deform) {
+    __shared__ BwdLds<S> s_lds;
+    const int lane = threadIdx.x, parts = kBwdParts<RECOMP>, per = kBwdGroup / tile * parts + 1;
+    const int64_t group = k / per;
+    const int i = (int)(k - group * per);
+    if (i == 0) {
+        if (!(adj.flags & DISO_FLAG_ACCUMULATE)) bwd_zero<S, DEF, RECOMP>(in, sc, group * kBwdGroup, adj_sdf, adj_deform, lane);
+        return;
+    }
+    const int64_t lo = group * kBwdGroup + (i - 1) / parts * tile, left = in.geo.nseg - lo;
+    if (left > 0) bwd_tile<S, DEF, RECOMP>(in, sc, lo, (int)(left < tile ? left : tile), adj, adj_sdf, adj_deform, s_lds, (i - 1) % parts, lane);
+}
+
+template <typename S, bool DEF, bool RECOMP>
+__global__ __launch_bounds__(kWave) void bwd_mc_kernel(In<S> in, const SegBase *__restrict__ seg, AdjIn<S> adj,
+                                                       S *__restrict__ adj_sdf, S *__restrict__ adj_deform,
+                                                       int tile, int64_t nblocks) {
+    const SegCtx sc = seg_ctx(seg, planes_of(seg, in.geo.nseg));
+    const int64_t b = xcd_stripe(blockIdx.x, nblocks);
+    if (b < nblocks) bwd_wave<S, DEF, RECOMP>(in, sc, b, tile, adj, adj_sdf, adj_deform);
 }
 
 // Per-edge upstream gradient of a DMC forward: ge[q] = sum over the quad's corners v of
@@ -2209,36 +2282,22 @@ __global__ __launch_bounds__(kBlock) void dmc_edge_grad_batch_kernel(const Batch
 }
 
 template <typename S, bool DEF, bool RECOMP>
-__global__ __launch_bounds__(kBlock) void bwd_batch_kernel(const BatchGrid<S> *__restrict__ grids,
+__global__ __launch_bounds__(kWave) void bwd_batch_kernel(const BatchGrid<S> *__restrict__ grids,
                                                            const int32_t *__restrict__ gl,
                                                            const int64_t *__restrict__ rf, int m,
                                                            const SegBase *__restrict__ seg,
                                                            Planes planes,
                                                            const S *__restrict__ ge, int64_t nblocks) {
-    __shared__ BwdLds<S> s_lds[kWavesPerBlock];
-    const int tid = threadIdx.x, wave = wave_id(), lane = tid % kWave;
-    const int64_t b = xcd_block(blockIdx.x, nblocks);
+    const int64_t b = xcd_stripe(blockIdx.x, nblocks);
+    if (b >= nblocks) return;
     const int j = find_group(rf, m, b);
     const BatchGrid<S> &G = grids[gl[j]];
     const In<S> in = G.in;
-    const Geo &g = in.geo;
     const SegCtx sc = batch_ctx(G, seg, planes);
     // DMC grids gather the per-edge gradients (already divided by the normalisation)
     const AdjIn<S> adj = G.algo == DISO_DMC ? AdjIn<S>{ge + 3 * G.q_first, G.nf, G.flags & ~DISO_FLAG_NORMALIZE, G.nm}
                                             : AdjIn<S>{G.adj, G.nv, G.flags, G.nm};
-    const int64_t lo = (b - rf[j]) * G.run, hi = lo + G.run < g.nseg ? lo + G.run : g.nseg;
-    const int64_t t = lo + lane;
-    const SegPos lp = seg_pos(g, t);
-    const bool touched = t < hi && seg_touched(sc.seg, g, t, lp);
-    uint64_t act = __ballot(touched);
-    uint64_t idle = (adj.flags & DISO_FLAG_ACCUMULATE) ? 0ull : __ballot(t < hi && !touched);
-    for (int k = 0; idle; ++k, idle &= idle - 1)
-        if ((k & (kWavesPerBlock - 1)) == wave) {
-            const SegPos sp = pos_of_lane(lp, __builtin_ctzll(idle));
-            store_grad(in, G.adj_sdf, G.adj_deform, sp.px, sp.py, sp.chunk * kWave + lane,
-                       Grad<S>{S(0), S(0), S(0), S(0)}, adj.flags);
-        }
-    bwd_run<S, DEF, RECOMP>(in, sc, lo, lp, act, adj, G.adj_sdf, G.adj_deform, s_lds[wave], wave, lane);
+    bwd_wave<S, DEF, RECOMP>(in, sc, b - rf[j], G.tile, adj, G.adj_sdf, G.adj_deform);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2564,7 +2623,17 @@ int launch_count(int algo, const void *sdf, double iso, const Geo &g, void *seg,
     return check_hip(hipGetLastError(), "count kernel launch");
 }
 
-int64_t row_blocks(const Geo &g) { return (g.nseg + run_for(g.nseg) - 1) / run_for(g.nseg); }
+// The run length is what four gathering waves take: a wave's tile is a quarter of it, down to a power
+// of two (tiles divide the kBwdGroup segments that share a zeroing wave).
+int bwd_tile_of(int64_t nseg) {
+    int t = 1;
+    while (2 * t <= run_for(nseg) / kWavesPerBlock && 2 * t <= kBwdTile) t *= 2;
+    return t;
+}
+int64_t bwd_blocks(int64_t nseg, bool recompute) {
+    const int parts = recompute ? kBwdParts<true> : kBwdParts<false>;
+    return (nseg + kBwdGroup - 1) / kBwdGroup * (kBwdGroup / bwd_tile_of(nseg) * parts + 1);
+}
 
 template <typename S>
 Norm<S> norm_of(const Geo &g) {
@@ -2624,8 +2693,8 @@ int launch_backward(int algo, const void *sdf, const void *deform, double iso, i
     a.n = nverts;
     a.flags = flags;
     a.nm = norm_of<S>(g);
-    const int run = run_for(g.nseg);
-    const int64_t nb = row_blocks(g);
+    const int tile = bwd_tile_of(g.nseg);
+    const int64_t nb = bwd_blocks(g.nseg, (flags & DISO_FLAG_RECOMPUTE) != 0);
     const SegBase *sb = (const SegBase *)seg;
     S *gs = (S *)adj_sdf, *gd = (S *)(deform ? adj_deform : nullptr);
     if (algo == DISO_DMC) {
@@ -2641,16 +2710,16 @@ int launch_backward(int algo, const void *sdf, const void *deform, double iso, i
         a.n = nfaces;
         a.flags = flags & ~DISO_FLAG_NORMALIZE;  // applied by the edge gradient kernel
     }
-    const dim3 grid((unsigned)nb), block(kBlock);
+    const dim3 grid((unsigned)stripe_blocks(nb)), block(kWave);
     const bool rec = (flags & DISO_FLAG_RECOMPUTE) != 0;
     if (deform && rec)
-        hipLaunchKernelGGL((bwd_mc_kernel<S, true, true>), grid, block, 0, st, in, sb, a, gs, gd, run, nb);
+        hipLaunchKernelGGL((bwd_mc_kernel<S, true, true>), grid, block, 0, st, in, sb, a, gs, gd, tile, nb);
     else if (deform)
-        hipLaunchKernelGGL((bwd_mc_kernel<S, true, false>), grid, block, 0, st, in, sb, a, gs, gd, run, nb);
+        hipLaunchKernelGGL((bwd_mc_kernel<S, true, false>), grid, block, 0, st, in, sb, a, gs, gd, tile, nb);
     else if (rec)
-        hipLaunchKernelGGL((bwd_mc_kernel<S, false, true>), grid, block, 0, st, in, sb, a, gs, gd, run, nb);
+        hipLaunchKernelGGL((bwd_mc_kernel<S, false, true>), grid, block, 0, st, in, sb, a, gs, gd, tile, nb);
     else
-        hipLaunchKernelGGL((bwd_mc_kernel<S, false, false>), grid, block, 0, st, in, sb, a, gs, gd, run, nb);
+        hipLaunchKernelGGL((bwd_mc_kernel<S, false, false>), grid, block, 0, st, in, sb, a, gs, gd, tile, nb);
     return check_hip(hipGetLastError(), "backward kernel launch");
 }
 
@@ -2836,7 +2905,7 @@ std::vector<BatchGrid<S>> batch_desc(const diso_grid_t *grids, const BatchLayout
         D.adj_sdf = (S *)G.adj_sdf;
         D.adj_deform = (S *)G.adj_deform;
         D.q_first = q;
-        D.run = run_for(L.geo[i].nseg);
+        D.tile = bwd_tile_of(L.geo[i].nseg);
         if (G.algo == DISO_DMC) q += G.totals.n_faces;
     }
     return d;
@@ -2975,8 +3044,6 @@ int batch_count(diso_grid_t *grids, const BatchLayout &L, void *ws, void *ctl, h
     return DISO_OK;
 }
 
-int64_t runs_of(const Geo &g, int run) { return (g.nseg + run - 1) / run; }
-
 template <typename S>
 int batch_emit(const diso_grid_t *grids, const BatchLayout &L, void *ws, hipStream_t st) {
     Group gr[4];  // MC, MC + deform, DMC, DMC + deform
@@ -3032,7 +3099,8 @@ int batch_backward(const diso_grid_t *grids, const BatchLayout &L, void *ws, voi
             if (!G.faces || !G.vinfo) return fail(DISO_E_INVALID, "grid %d: DMC backward needs quads and vinfo", i);
             gr[4].add(i, (G.totals.n_faces + kBlock - 1) / kBlock);
         }
-        gr[2 * (G.deform != nullptr) + ((G.flags & DISO_FLAG_RECOMPUTE) != 0)].add(i, runs_of(L.geo[i], run_for(L.geo[i].nseg)));
+        gr[2 * (G.deform != nullptr) + ((G.flags & DISO_FLAG_RECOMPUTE) != 0)].add(
+            i, bwd_blocks(L.geo[i].nseg, (G.flags & DISO_FLAG_RECOMPUTE) != 0));
     }
     int rc = upload_batch<S>(ws, L, batch_desc<S>(grids, L), gr, 5, st);
     if (rc) return rc;
@@ -3048,15 +3116,15 @@ int batch_backward(const diso_grid_t *grids, const BatchLayout &L, void *ws, voi
     for (int k = 0; k < 4; ++k) {
         const int64_t nb = gr[k].blocks();
         if (!nb) continue;
-        const dim3 grid((unsigned)nb), block(kBlock);
+        const dim3 grid((unsigned)stripe_blocks(nb));
         const int32_t *gl = P.gl(L, k, w);
         const int64_t *rf = P.rf(L, k, w);
         const int m = gr[k].m();
         switch (k) {
-            case 0: hipLaunchKernelGGL((bwd_batch_kernel<S, false, false>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
-            case 1: hipLaunchKernelGGL((bwd_batch_kernel<S, false, true>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
-            case 2: hipLaunchKernelGGL((bwd_batch_kernel<S, true, false>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
-            default: hipLaunchKernelGGL((bwd_batch_kernel<S, true, true>), grid, block, 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
+            case 0: hipLaunchKernelGGL((bwd_batch_kernel<S, false, false>), grid, dim3(kWave), 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
+            case 1: hipLaunchKernelGGL((bwd_batch_kernel<S, false, true>), grid, dim3(kWave), 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
+            case 2: hipLaunchKernelGGL((bwd_batch_kernel<S, true, false>), grid, dim3(kWave), 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
+            default: hipLaunchKernelGGL((bwd_batch_kernel<S, true, true>), grid, dim3(kWave), 0, st, P.desc, gl, rf, m, P.seg, P.planes, ge, nb); break;
         }
         rc = check_hip(hipGetLastError(), "batch backward kernel launch");
         if (rc) return rc;
