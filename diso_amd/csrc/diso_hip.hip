@@ -1789,36 +1789,69 @@ __device__ __forceinline__ int64_t sample_start(const Geo &g, const SegPos &sp) 
     return x * plane + (int64_t)y * g.n2 + (z < 0 ? 0 : (z < g.n2 ? z : g.n2));
 }
 
-// Inside and below bits of a segment's row of samples (wave-uniform row).
+// Inside and below bits of a row's 64 samples from conceptual z0 on, for the wave-uniform row (px,
+// py): the load (at a valid address, whatever the row) and the compares. Positions outside the stored
+// grid take the pad's bits.
 struct SideBits {
     uint64_t in, below;
 };
 template <typename S>
-__device__ __forceinline__ SideBits row_bits(const In<S> &in, int px, int py, int z0, int lane) {
-    const S v = sample(in, px, py, z0 + lane);
-    return SideBits{__ballot(v >= in.iso), __ballot(v < in.iso)};
+__device__ __forceinline__ S row_sample(const In<S> &in, int px, int py, int zv) {
+    const Geo &g = in.geo;
+    const int x = px - g.off, y = py - g.off;
+    const bool row = (unsigned)x < (unsigned)g.n0 && (unsigned)y < (unsigned)g.n1;  // uniform
+    return in.sdf[(row ? ((int64_t)x * g.n1 + y) * g.n2 : 0) + zv];
+}
+template <typename S>
+__device__ __forceinline__ SideBits row_bits(const In<S> &in, int px, int py, uint64_t zs, S v) {
+    const Geo &g = in.geo;
+    const bool row = (unsigned)(px - g.off) < (unsigned)g.n0 && (unsigned)(py - g.off) < (unsigned)g.n1;
+    const uint64_t st = row ? zs : 0ull, pi = in.pad >= in.iso ? ~0ull : 0ull, pb = in.pad < in.iso ? ~0ull : 0ull;
+    return SideBits{(__ballot(v >= in.iso) & st) | (pi & ~st), (__ballot(v < in.iso) & st) | (pb & ~st)};
 }
 __device__ __forceinline__ uint64_t cross_bits(SideBits a, SideBits b) { return (a.below & b.in) | (b.below & a.in); }
 __device__ __forceinline__ SideBits side_up(SideBits a, SideBits next, int bit) {
     return SideBits{diso_bits::up1(a.in, next.in >> bit), diso_bits::up1(a.below, next.below >> bit)};
 }
 
-// The crossing planes of BwdLds::pl from the samples (the recomputing backward): returns them in
-// scalar registers, the same in every lane.
+// The crossing planes of BwdLds::pl from the samples (the recomputing backward), in two steps, so that
+// the loads of one segment are in flight while another's are used: the samples of the segment's row
+// and of the six around it that own or end its edges, and per lane one of the four positions past
+// the segment's ends that count; then the planes, in scalar registers.
 struct BwdPlanes {
     uint64_t w[10];
 };
 template <typename S>
-__device__ __forceinline__ BwdPlanes recompute_planes(const In<S> &in, const SegPos &sp, int lane) {
+struct BwdRows {
+    S c, xp, yp, xm, ym, xmyp, xpym, e;
+};
+template <typename S>
+__device__ __forceinline__ BwdRows<S> recompute_load(const In<S> &in, const SegPos &sp, int lane) {
+    const Geo &g = in.geo;
+    const int px = sp.px, py = sp.py, z0 = sp.chunk * kWave, z = z0 - g.off + lane;
+    const int zv = z < 0 ? 0 : (z < g.n2 ? z : g.n2 - 1);
+    BwdRows<S> r;
+    r.c = row_sample(in, px, py, zv);
+    r.xp = row_sample(in, px + 1, py, zv);
+    r.yp = row_sample(in, px, py + 1, zv);
+    r.xm = row_sample(in, px - 1, py, zv);
+    r.ym = row_sample(in, px, py - 1, zv);
+    r.xmyp = row_sample(in, px - 1, py + 1, zv);
+    r.xpym = row_sample(in, px + 1, py - 1, zv);
+    // lanes 0-2: position z0 + 64 of rows (0,0), (-1,0), (0,-1); the others: position z0 - 1 of row (0,0)
+    r.e = sample(in, px - (lane == 1), py - (lane == 2), lane < 3 ? z0 + kWave : z0 - 1);
+    return r;
+}
+template <typename S>
+__device__ __forceinline__ BwdPlanes recompute_planes(const In<S> &in, const SegPos &sp, const BwdRows<S> &v) {
     const Geo &g = in.geo;
     const int px = sp.px, py = sp.py, z0 = sp.chunk * kWave;
-    const SideBits c = row_bits(in, px, py, z0, lane), xp = row_bits(in, px + 1, py, z0, lane),
-                   yp = row_bits(in, px, py + 1, z0, lane), xm = row_bits(in, px - 1, py, z0, lane),
-                   ym = row_bits(in, px, py - 1, z0, lane), xmyp = row_bits(in, px - 1, py + 1, z0, lane),
-                   xpym = row_bits(in, px + 1, py - 1, z0, lane);
-    // lanes 0-2: position z0 + 64 of rows (0,0), (-1,0), (0,-1); lane 3: position z0 - 1 of row (0,0)
-    const S e = sample(in, px - (lane == 1), py - (lane == 2), lane == 3 ? z0 - 1 : z0 + kWave);
-    const SideBits eb{__ballot(e >= in.iso), __ballot(e < in.iso)};
+    const uint64_t zs = diso_bits::low_bits(g.n2 + g.off - z0) & ~diso_bits::low_bits(g.off - z0);
+    const SideBits c = row_bits(in, px, py, zs, v.c), xp = row_bits(in, px + 1, py, zs, v.xp),
+                   yp = row_bits(in, px, py + 1, zs, v.yp), xm = row_bits(in, px - 1, py, zs, v.xm),
+                   ym = row_bits(in, px, py - 1, zs, v.ym), xmyp = row_bits(in, px - 1, py + 1, zs, v.xmyp),
+                   xpym = row_bits(in, px + 1, py - 1, zs, v.xpym);
+    const SideBits eb{__ballot(v.e >= in.iso), __ballot(v.e < in.iso)};
     const uint64_t am = diso_bits::low_bits(g.g2 - 1 - z0);  // positions that anchor a cell
     const bool ax = px < g.g0 - 1, ay = py < g.g1 - 1;
     const uint64_t m00 = ax && ay ? am : 0ull, mx = px > 0 && ay ? am : 0ull, my = py > 0 && ax ? am : 0ull;
@@ -2000,11 +2033,21 @@ __device__ __forceinline__ void bwd_tile(const In<S> &in, const SegCtx &sc, int6
     if constexpr (RECOMP) {
         // the planes from the samples, for the segments that can have a touched vertex (by the bases)
         cand = __ballot(q.have && seg_touched(sc.seg, g, s, q.sp));
-        for (uint64_t c = cand; c; c &= c - 1) {  // wave-uniform
-            const int j = (int)__builtin_ctzll(c);
-            const BwdPlanes p = recompute_planes(in, pos_of_lane(q.sp, j), lane);
-            if (lane == 0)
-                for (int k = 0; k < 10; ++k) L.pl[j][k] = p.w[k];
+        if (cand) {
+            int j = (int)__builtin_ctzll(cand);
+            BwdRows<S> rows = recompute_load(in, pos_of_lane(q.sp, j), lane);
+            for (uint64_t c = cand & (cand - 1);; c &= c - 1) {  // wave-uniform
+                const BwdRows<S> cur = rows;
+                const int at = j;
+                if (c) {
+                    j = (int)__builtin_ctzll(c);
+                    rows = recompute_load(in, pos_of_lane(q.sp, j), lane);
+                }
+                const BwdPlanes p = recompute_planes(in, pos_of_lane(q.sp, at), cur);
+                if (lane == 0)
+                    for (int k = 0; k < 10; ++k) L.pl[at][k] = p.w[k];
+                if (!c) break;
+            }
         }
         wave_lds_sync();
         if ((cand >> lane) & 1) T = touched_bits(L.pl[lane]) & q.have;
