@@ -1022,10 +1022,10 @@ __device__ __forceinline__ void store_vertex(S *__restrict__ verts, int64_t i, i
 
 // Active cells in units of 64, one lane per cell, whatever segments they lie in (so that lanes are
 // full on sparse surfaces too). A unit's cells are found from the segments between its first one and
-// the next unit's first one: lane i loads segment U0 + i and each segment with cells writes them to
-// `list` at its place. Where more than 64 segments lie in between (a sparse stretch), each lane
-// searches its cell's segment instead. Returns the number of cells; lane k < n gets cell k's segment
-// (of the launch) and position in it, the other lanes a copy of one of them.
+// the next unit's first one: lane i loads segment U0 + i (unit_load, a unit ahead) and each segment
+// with cells writes them to `list` at its place. Where more than 64 segments lie in between (a sparse
+// stretch), each lane searches its cell's segment instead. unit_cells returns the number of cells;
+// lane k < n gets cell k's segment (of the launch) and position in it, the other lanes a copy of one.
 struct UnitGrid {
     const SegBase *__restrict__ seg;  // launch-level arrays
     Planes P;
@@ -1049,15 +1049,32 @@ __device__ __forceinline__ int select64(uint64_t m, int r) {
     return p;
 }
 
-__device__ __forceinline__ int unit_cells(const UnitGrid &G, uint32_t u, uint32_t nunits, uint16_t *list, int lane,
-                                          uint32_t *s_out, int *l_out) {
+struct UnitLoad {
+    uint32_t u;
+    int64_t U0, U1;  // first and last segment that can hold its cells
+    uint64_t A;      // lane i: segment U0 + i
+    uint16_t abase;
+};
+__device__ __forceinline__ UnitLoad unit_load(const UnitGrid &G, uint32_t u, uint32_t nunits, int lane) {
+    UnitLoad r;
+    r.u = u;
     const int64_t a = G.P.unit[u], b = u + 1 < nunits ? (int64_t)G.P.unit[u + 1] : G.last;
-    const int64_t U0 = a > G.first ? a : G.first, U1 = b < G.last ? b : G.last;
-    const uint16_t c0 = (uint16_t)(u * (uint32_t)kWave);  // number of the unit's first cell
+    r.U0 = a > G.first ? a : G.first;
+    r.U1 = b < G.last ? b : G.last;
+    const int64_t s = r.U0 + lane <= r.U1 ? r.U0 + lane : r.U1;
+    r.A = G.P.za[s].b;
+    r.abase = G.P.abase[s];
+    return r;
+}
+
+__device__ __forceinline__ int unit_cells(const UnitGrid &G, const UnitLoad &U, uint16_t *list, int lane,
+                                          uint32_t *s_out, int *l_out) {
+    const int64_t U0 = U.U0, U1 = U.U1;
+    const uint16_t c0 = (uint16_t)(U.u * (uint32_t)kWave);  // number of the unit's first cell
     if (U1 - U0 < kWave) {  // wave-uniform
         const bool in = lane <= (int)(U1 - U0);
-        const uint64_t A = in ? G.P.za[U0 + lane].b : 0ull;
-        const int st = in ? (int)(int16_t)(uint16_t)(G.P.abase[U0 + lane] - c0) : 0;
+        const uint64_t A = in ? U.A : 0ull;
+        const int st = in ? (int)(int16_t)(uint16_t)(U.abase - c0) : 0;
         const int s0 = __builtin_amdgcn_readfirstlane(st);
         const int k0 = s0 > 0 ? s0 : 0;  // cells of the unit that belong to the grid before (a batch)
         int n = 0;
@@ -1099,14 +1116,32 @@ __device__ __forceinline__ int unit_cells(const UnitGrid &G, uint32_t u, uint32_
     return n;
 }
 
-// The units of a launch as a wave goes through them: XCD x takes the x-th eighth, its waves in turn,
-// so that at any time an XCD's waves work on neighbouring cells (whose rows share its L2). Calls
-// f(unit) for each of this wave's units. The grid has a multiple of eight blocks.
+// A wave's units first, first + step, ... below hi: work(load, next) for each, which returns next(), the
+// load of the unit after (called where those loads should be issued: before the work's own stores,
+// which the in-order memory counter would otherwise put between them and their use).
 template <typename F>
-__device__ __forceinline__ void for_units(uint32_t lo, uint32_t hi, int64_t block, int64_t nblocks, int wave, F f) {
-    const uint32_t n = hi - lo, xcd = (uint32_t)(block % 8), per = (uint32_t)(nblocks / 8) * kWavesPerBlock;
-    const uint32_t u0 = lo + (uint32_t)((uint64_t)n * xcd / 8), u1 = lo + (uint32_t)((uint64_t)n * (xcd + 1) / 8);
-    for (uint32_t u = u0 + (uint32_t)(block / 8) * kWavesPerBlock + (uint32_t)wave; u < u1; u += per) f(u);
+__device__ __forceinline__ void unit_loop(const UnitGrid &G, uint32_t first, uint32_t hi, uint32_t step, uint32_t nunits,
+                                          int lane, F work) {
+    if (first >= hi) return;  // wave-uniform
+    UnitLoad cur = unit_load(G, first, nunits, lane);
+    for (uint32_t u = first;;) {
+        const bool more = step < hi - u;
+        const uint32_t un = more ? u + step : u;
+        cur = work(cur, [&]() { return unit_load(G, un, nunits, lane); });
+        if (!more) break;
+        u = un;
+    }
+}
+
+// The units of a launch as a wave goes through them: XCD x takes the x-th eighth, its waves in turn,
+// so that at any time an XCD's waves work on neighbouring cells (whose rows share its L2). The grid
+// has a multiple of eight blocks.
+template <typename F>
+__device__ __forceinline__ void for_units(const UnitGrid &G, uint32_t nunits, int64_t block, int64_t nblocks, int wave,
+                                          int lane, F work) {
+    const uint32_t xcd = (uint32_t)(block % 8), per = (uint32_t)(nblocks / 8) * kWavesPerBlock;
+    const uint32_t u0 = (uint32_t)((uint64_t)nunits * xcd / 8), u1 = (uint32_t)((uint64_t)nunits * (xcd + 1) / 8);
+    unit_loop(G, u0 + (uint32_t)(block / 8) * kWavesPerBlock + (uint32_t)wave, u1, per, nunits, lane, work);
 }
 
 __device__ __forceinline__ int bit_at(uint64_t w, int l) {
@@ -1134,15 +1169,15 @@ struct RowEdges {
     }
 };
 
-template <typename S, bool DEF>
-__device__ __forceinline__ void emit_mc_unit(const In<S> &in, const UnitGrid &G, uint32_t u, uint32_t nunits,
+template <typename S, bool DEF, typename Next>
+__device__ __forceinline__ UnitLoad emit_mc_unit(const In<S> &in, const UnitGrid &G, const UnitLoad &U, Next next,
                                              S *__restrict__ verts, void *__restrict__ faces, const OutCfg &out,
                                              const Norm<S> &nm, const uint64_t *s_case, McEmitLds &L, int lane) {
     wave_lds_sync();  // the previous unit's LDS reads are done
     uint32_t s;
     int l;
-    const int n = unit_cells(G, u, nunits, L.tri, lane, &s, &l);
-    if (n == 0) return;  // wave-uniform
+    const int n = unit_cells(G, U, L.tri, lane, &s, &l);
+    if (n == 0) return next();  // wave-uniform
     const Geo &g = in.geo;
     const SegPos sp = seg_pos(g, (int64_t)s - G.first);
     const bool on = lane < n;
@@ -1217,6 +1252,7 @@ __device__ __forceinline__ void emit_mc_unit(const In<S> &in, const UnitGrid &G,
     for (int t = 0; t < 5; ++t) L.tri[t < ntri ? pt + t : 5 * kWave] = (uint16_t)((lane << 3) | t);
     wave_lds_sync();
 
+    const UnitLoad after = next();
     for (int k = lane; k < tv; k += kWave) {
         const int it = L.vert[k], src = it >> 2, a = it & 3;
         const V3<S> p = edge_vertex<S, DEF>(in, L.cx[src], L.cy[src], L.cz[src], a);
@@ -1233,6 +1269,7 @@ __device__ __forceinline__ void emit_mc_unit(const In<S> &in, const UnitGrid &G,
         store_tri(faces, f, vbase + cand[DISO_MC_EDGE(w, 3 * t)], vbase + cand[DISO_MC_EDGE(w, 3 * t + 1)],
                   vbase + cand[DISO_MC_EDGE(w, 3 * t + 2)], out.flags);
     }
+    return after;
 }
 
 __device__ __forceinline__ void load_mc_cases(uint64_t *s_case) {
@@ -1252,8 +1289,8 @@ __global__ __launch_bounds__(kBlock, 6) void emit_mc_kernel(In<S> in, const SegB
     __syncthreads();
     const uint32_t nunits = *planes.nunits;
     const UnitGrid G{seg, planes, 0, in.geo.nseg - 1, 0, 0};
-    for_units(0, nunits, blockIdx.x, gridDim.x, wave, [&](uint32_t u) {
-        emit_mc_unit<S, DEF>(in, G, u, nunits, verts, faces, out, nm, s_case, s_lds[wave], lane);
+    for_units(G, nunits, blockIdx.x, gridDim.x, wave, lane, [&](const UnitLoad &U, auto next) {
+        return emit_mc_unit<S, DEF>(in, G, U, next, verts, faces, out, nm, s_case, s_lds[wave], lane);
     });
 }
 
@@ -1406,16 +1443,16 @@ __device__ __forceinline__ V3<S> patch_edge_vertex(const In<S> &in, int x, int y
 
 // One unit of 64 active cells: its patch vertices and the quads of the edges its cells own. Both are
 // contiguous rows of the output, in the cells' order.
-template <typename S, bool DEF>
-__device__ __forceinline__ void emit_dmc_unit(const In<S> &in, const UnitGrid &G, uint32_t u, uint32_t nunits,
+template <typename S, bool DEF, typename Next>
+__device__ __forceinline__ UnitLoad emit_dmc_unit(const In<S> &in, const UnitGrid &G, const UnitLoad &U, Next next,
                                               S *__restrict__ verts, void *__restrict__ faces,
                                               uint8_t *__restrict__ vinfo, const OutCfg &out, const Norm<S> &nm,
                                               const uint64_t *s_case, DmcEmitLds<S> &L, int lane) {
     wave_lds_sync();  // the previous unit's LDS reads are done
     uint32_t s;
     int l;
-    const int n = unit_cells(G, u, nunits, L.eitem, lane, &s, &l);
-    if (n == 0) return;  // wave-uniform
+    const int n = unit_cells(G, U, L.eitem, lane, &s, &l);
+    if (n == 0) return next();  // wave-uniform
     const Geo &g = in.geo;
     const SegPos sp = seg_pos(g, (int64_t)s - G.first);
     const int px = sp.px, py = sp.py, z = sp.chunk * kWave + l;
@@ -1510,6 +1547,7 @@ __device__ __forceinline__ void emit_dmc_unit(const In<S> &in, const UnitGrid &G
     L.nd[lane] = (uint8_t)(rx && ry ? cxy : 0u);
     wave_lds_sync();
 
+    const UnitLoad after = next();
     // quads: corner 0 is the own cell's vertex; corners B, C, D those of the other three cells around
     // the edge (X: -y, -y below, below; Y: below, -x below, -x; Z: -x, -x-y, -y), in that order or,
     // where the edge leaves the inside, in reverse. A cell below a row's cell at z has its patches
@@ -1604,6 +1642,7 @@ __device__ __forceinline__ void emit_dmc_unit(const In<S> &in, const UnitGrid &G
         store_vertex(verts, pbase + k, out.vcap, epilogue(V3<S>{sx2 * r, sy2 * r, sz2 * r}, out.flags, nm));
         if (pbase + k < out.vcap) put(vinfo + pbase + k, (uint8_t)(num | (pk << 3)));
     }
+    return after;
 }
 
 // The DMC case words with each code's own_kinds in the free top byte, in LDS.
@@ -1624,8 +1663,8 @@ __global__ __launch_bounds__(kBlock, 5) void emit_dmc_kernel(In<S> in, const Seg
     __syncthreads();
     const uint32_t nunits = *planes.nunits;
     const UnitGrid G{seg, planes, 0, in.geo.nseg - 1, 0, 0};
-    for_units(0, nunits, blockIdx.x, gridDim.x, wave, [&](uint32_t u) {
-        emit_dmc_unit<S, DEF>(in, G, u, nunits, verts, faces, vinfo, out, nm, s_case, s_lds[wave], lane);
+    for_units(G, nunits, blockIdx.x, gridDim.x, wave, lane, [&](const UnitLoad &U, auto next) {
+        return emit_dmc_unit<S, DEF>(in, G, U, next, verts, faces, vinfo, out, nm, s_case, s_lds[wave], lane);
     });
 }
 
@@ -2257,7 +2296,7 @@ template <typename S, typename F>
 __device__ __forceinline__ void batch_units(const BatchGrid<S> *__restrict__ grids, const int32_t *__restrict__ gl,
                                             const int64_t *__restrict__ rf, int m, const SegBase *__restrict__ seg,
                                             const Planes &planes, const uint32_t *__restrict__ range, int64_t nblocks,
-                                            int wave, F f) {
+                                            int wave, int lane, F f) {
     const int64_t b = xcd_block(blockIdx.x, nblocks);
     const int j = find_group(rf, m, b);
     const int gi = gl[j];
@@ -2268,8 +2307,8 @@ __device__ __forceinline__ void batch_units(const BatchGrid<S> *__restrict__ gri
     const UnitGrid G{seg, planes, first, first + in.geo.nseg - 1, seg[first].v, seg[first].f};
     const OutCfg out{B.flags, B.vcap, B.fcap};
     const uint32_t nunits = *planes.nunits, hi = range[2 * gi + 1], step = (uint32_t)(rf[j + 1] - rf[j]) * kWavesPerBlock;
-    for (uint32_t u = range[2 * gi] + (uint32_t)(b - rf[j]) * kWavesPerBlock + (uint32_t)wave; u < hi; u += step)
-        f(in, G, B, out, u, nunits);
+    unit_loop(G, range[2 * gi] + (uint32_t)(b - rf[j]) * kWavesPerBlock + (uint32_t)wave, hi, step, nunits, lane,
+              [&](const UnitLoad &U, auto next) { return f(in, G, B, out, U, next); });
 }
 
 template <typename S, bool DEF>
@@ -2283,9 +2322,9 @@ __global__ __launch_bounds__(kBlock, 6) void emit_mc_batch_kernel(const BatchGri
     const int wave = wave_id(), lane = threadIdx.x % kWave;
     load_mc_cases(s_case);
     __syncthreads();
-    batch_units(grids, gl, rf, m, seg, planes, range, nblocks, wave,
-                [&](const In<S> &in, const UnitGrid &G, const BatchGrid<S> &B, const OutCfg &out, uint32_t u, uint32_t nunits) {
-                    emit_mc_unit<S, DEF>(in, G, u, nunits, B.verts, B.faces, out, B.nm, s_case, s_lds[wave], lane);
+    batch_units(grids, gl, rf, m, seg, planes, range, nblocks, wave, lane,
+                [&](const In<S> &in, const UnitGrid &G, const BatchGrid<S> &B, const OutCfg &out, const UnitLoad &U, auto next) {
+                    return emit_mc_unit<S, DEF>(in, G, U, next, B.verts, B.faces, out, B.nm, s_case, s_lds[wave], lane);
                 });
 }
 
@@ -2300,9 +2339,9 @@ __global__ __launch_bounds__(kBlock, 5) void emit_dmc_batch_kernel(const BatchGr
     const int wave = wave_id(), lane = threadIdx.x % kWave;
     load_dmc_cases(s_case);
     __syncthreads();
-    batch_units(grids, gl, rf, m, seg, planes, range, nblocks, wave,
-                [&](const In<S> &in, const UnitGrid &G, const BatchGrid<S> &B, const OutCfg &out, uint32_t u, uint32_t nunits) {
-                    emit_dmc_unit<S, DEF>(in, G, u, nunits, (S *)B.verts, B.faces, B.vinfo, out, B.nm, s_case, s_lds[wave], lane);
+    batch_units(grids, gl, rf, m, seg, planes, range, nblocks, wave, lane,
+                [&](const In<S> &in, const UnitGrid &G, const BatchGrid<S> &B, const OutCfg &out, const UnitLoad &U, auto next) {
+                    return emit_dmc_unit<S, DEF>(in, G, U, next, (S *)B.verts, B.faces, B.vinfo, out, B.nm, s_case, s_lds[wave], lane);
                 });
 }
 
