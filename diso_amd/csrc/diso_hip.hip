@@ -2550,7 +2550,7 @@ __global__ __launch_bounds__(kSplitBlock) void split_emit_kernel(const void *__r
         // rows run.. of the first half, or of the second half at the rank among the others
         Index2 *t1 = reinterpret_cast<Index2 *>(tris + 6 * run);
         Index2 *t2 = reinterpret_cast<Index2 *>(tris + 6 * (n1 + (base - run) - nf));
-        for (int i = lane; i < 3 * n; i += kWave) put((i < 3 * nf ? t1 : t2) + i, row[i]);
+        for (int i = lane; i < 3 * n; i += kWave) __builtin_nontemporal_store(row[i], (i < 3 * nf ? t1 : t2) + i);  // (8-byte aligned)
         wave_lds_sync();
         run += nf;
     }
