@@ -113,20 +113,6 @@ __device__ __forceinline__ S sample(const In<S> &in, int x, int y, int z) {
     return ok ? v : in.pad;
 }
 
-template <typename S, bool DEF>
-__device__ __forceinline__ V3<S> deform_at(const In<S> &in, int x, int y, int z) {
-    V3<S> r = {S(0), S(0), S(0)};
-    if (DEF) {
-        const bool ok = in_data(in, x, y, z);
-        const S *d = in.deform + 3 * (ok ? data_index(in, x, y, z) : 0);
-        const S dx = d[0], dy = d[1], dz = d[2];
-        r.x = ok ? dx : S(0);
-        r.y = ok ? dy : S(0);
-        r.z = ok ? dz : S(0);
-    }
-    return r;
-}
-
 // clamp(x, a, b) = min(max(a, x), b) as in src/cumc.cu:80-91.
 template <typename S>
 __device__ __forceinline__ S clamp01(S v) {
@@ -350,8 +336,8 @@ __device__ __forceinline__ V3<S> lerp_vertex(int x, int y, int z, int axis, S d0
     return r;
 }
 
-// Samples and deforms of both endpoints of the edge from (x,y,z) along `axis`, as sample() and
-// deform_at() read them: the second endpoint's index is the first's plus the axis stride (one
+// Samples and deforms of both endpoints of the edge from (x,y,z) along `axis`, the pad value and a
+// zero deform where an endpoint is not stored: the second endpoint's index is the first's plus the axis stride (one
 // index product per edge instead of two).
 template <typename S, bool DEF>
 struct EdgeEnds {
@@ -1333,7 +1319,7 @@ static_assert(tables_agree(), "edge / quad tables");
 // Edges of a dual cell that start at its own z (the other four, on its top face, are the next
 // position's): kinds 0..7 in ascending edge number, with the edge's offsets and axis as bit masks
 // over the kinds. Top edges 2, 6, 10, 11 are kinds 0, 3, 7, 6 of the next position.
-__device__ constexpr int kind_edge(int k) { return k + (k >= 2) + (k >= 5); }  // 0 1 3 4 5 7 8 9
+__host__ __device__ constexpr int kind_edge(int k) { return k + (k >= 2) + (k >= 5); }  // 0 1 3 4 5 7 8 9
 constexpr int kTopEdges[4] = {2, 6, 10, 11}, kTopKinds[4] = {0, 3, 7, 6};
 constexpr int kKindX = 0x92, kKindY = 0x38, kKindAxisZ = 0x36, kKindAxisY = 0xC0;
 __device__ constexpr bool kinds_ok() {
@@ -1350,6 +1336,19 @@ __device__ constexpr bool kinds_ok() {
     return true;
 }
 static_assert(kinds_ok(), "edge kinds");
+// An edge of the cell as a bit: its kind at the cell's own position, or 8 + its kind at the next.
+__host__ __device__ constexpr int edge_bit(int e) {
+    for (int k = 0; k < 8; ++k)
+        if (kind_edge(k) == e) return k;
+    for (int t = 0; t < 4; ++t)
+        if (kTopEdges[t] == e) return 8 + kTopKinds[t];
+    return 16;
+}
+__host__ __device__ constexpr uint64_t edge_bits() {  // all twelve, four bits each
+    uint64_t w = 0;
+    for (int e = 0; e < 12; ++e) w |= (uint64_t)edge_bit(e) << (4 * e);
+    return w;
+}
 // The kinds that cross in a cell of code c (Morton corner order); a cell of the inverted code has
 // the same. And the top edges that cross, as kinds of the next position.
 __host__ __device__ constexpr uint32_t own_kinds(uint32_t c) {
@@ -1371,7 +1370,9 @@ struct DmcEmitLds {
     // kinds that cross (bits 16-23), its code (bits 24-31); entry 0: the code of the cell below cell
     // 0; entry n + 1: the slots and kinds of the position above the last cell
     uint32_t cw[kWave + 2];
-    int32_t cx[kWave + 1], cy[kWave + 1], cz[kWave + 1];  // the cells' positions (and that one's)
+    int64_t idx[kWave + 1];                         // the cells (and that position): index of the sample
+    S cx[kWave + 1], cy[kWave + 1], cz[kWave + 1];  // there (as if it were stored), position, and which
+    uint8_t stored[kWave + 1];                      // of the corners are stored (bit dx | dy << 1 | dz << 2)
     uint16_t pp[kWave];            // patches of the unit before the cell's
     uint8_t patch[kWave * 4 + 1];  // patch items: cell * 4 + patch
     uint8_t quad[kWave * 3 + 1];   // quad items: cell * 4 + axis
@@ -1387,8 +1388,8 @@ struct DmcEmitLds {
     };
 };
 
-// Edge masks of the patches of every DMC case, 16 bits per patch (patch k in bits 16k..16k+11),
-// derived at compile time from the case table.
+// Edges of the patches of every DMC case as edge_bit()s, 16 bits per patch, derived at compile time
+// from the case table.
 struct PatchEdgeTable {
     uint64_t m[256];
 };
@@ -1399,7 +1400,7 @@ constexpr PatchEdgeTable make_patch_edges() {
         uint64_t w = 0;
         for (int e = 0; e < 12; ++e) {
             const int k = DISO_DMC_PATCH_OF(cases[c], e);
-            if (k < 4) w |= 1ull << (16 * k + e);
+            if (k < 4) w |= 1ull << (16 * k + edge_bit(e));
         }
         t.m[c] = w;
     }
@@ -1407,47 +1408,97 @@ constexpr PatchEdgeTable make_patch_edges() {
 }
 __constant__ PatchEdgeTable kDmcPatchEdges = make_patch_edges();
 
-// 1/n for the possible patch sizes (n = 1..7), correctly rounded at compile time.
+// An edge kind: its ends' sample indices relative to the position's and their bits in the stored
+// corners, its start's offset and its direction.
 template <typename S>
-struct RcpTable {
-    S r[8];
+struct alignas(16) KindEnds {
+    int64_t d0, d1;
+    S ox, oy, ax, ay, az;
+    uint16_t c0, c1;
 };
+
+// The tables of the DMC emission, in LDS: the case words with each code's own_kinds in the free top
+// byte, the patches' edges, the edge kinds in the grid's strides, and 1/n for the possible patch sizes
+// (n = 1..7; correctly rounded).
 template <typename S>
-constexpr RcpTable<S> make_rcp() {
-    RcpTable<S> t{};
-    for (int n = 1; n < 8; ++n) t.r[n] = S(1) / S(n);
-    return t;
-}
-__constant__ RcpTable<float> kRcpF = make_rcp<float>();
-__constant__ RcpTable<double> kRcpD = make_rcp<double>();
-template <typename S>
-__device__ __forceinline__ S rcp_small(int n);
-template <>
-__device__ __forceinline__ float rcp_small<float>(int n) { return kRcpF.r[n]; }
-template <>
-__device__ __forceinline__ double rcp_small<double>(int n) { return kRcpD.r[n]; }
+struct DmcTables {
+    uint64_t cases[256], edges[256];
+    KindEnds<S> kind[8];
+    S rcp[8];
+    __device__ __forceinline__ void load(const Geo &g) {
+        const int t = threadIdx.x;
+        for (int i = t; i < 256; i += kBlock) {
+            cases[i] = kDmcCase[i] | (uint64_t)own_kinds((uint32_t)i) << 56;
+            edges[i] = kDmcPatchEdges.m[i];
+        }
+        if (t < 8) {
+            const int dx = (kKindX >> t) & 1, dy = (kKindY >> t) & 1;
+            const int a = (kKindAxisZ >> t) & 1 ? 2 : (kKindAxisY >> t) & 1;
+            const int64_t sy = g.n2, sx = (int64_t)g.n1 * g.n2, d0 = (dx ? sx : 0) + (dy ? sy : 0);
+            const int c0 = dx | dy << 1;
+            kind[t] = KindEnds<S>{d0, d0 + (a == 0 ? sx : (a == 1 ? sy : 1)), S(dx), S(dy),
+                                  S(a == 0), S(a == 1), S(a == 2), (uint16_t)c0, (uint16_t)(c0 + (1 << a))};
+            rcp[t] = t ? S(1) / S(t) : S(0);
+        }
+    }
+};
 
 // Patches before position l of a segment (b = bits below l).
 __device__ __forceinline__ int patches_below(uint64_t A, Plane2 m, uint64_t b) {
     return (int)__popcll(A & b) + (int)__popcll(m.a & b) + 2 * (int)__popcll(m.b & b);
 }
-// MC vertex of an edge as a patch sums it: zero where the edge does not cross (on NaN samples only,
-// for an edge whose ends' inside bits differ).
+// Which corners of the cell at a position are stored samples (bit dx | dy << 1 | dz << 2).
+__device__ __forceinline__ uint32_t stored_corners(const Geo &g, int x, int y, int z) {
+    const int a = x - g.off, b = y - g.off, c = z - g.off;
+    const uint32_t mx = ((unsigned)a < (unsigned)g.n0 ? 0x55u : 0u) | ((unsigned)(a + 1) < (unsigned)g.n0 ? 0xaau : 0u);
+    const uint32_t my = ((unsigned)b < (unsigned)g.n1 ? 0x33u : 0u) | ((unsigned)(b + 1) < (unsigned)g.n1 ? 0xccu : 0u);
+    const uint32_t mz = ((unsigned)c < (unsigned)g.n2 ? 0x0fu : 0u) | ((unsigned)(c + 1) < (unsigned)g.n2 ? 0xf0u : 0u);
+    return mx & my & mz;
+}
+
+// MC vertex of the edge of kind K at a position (c: its coordinates; stored, idx: as in DmcEmitLds) as
+// a patch sums it, lerp_vertex()'s expression: zero where the edge does not cross (on NaN samples only,
+// for an edge whose ends' inside bits differ). An end that is not stored reads as the pad value with a
+// zero deform (it loads element 0, so no lane needs its own execution mask around the loads).
 template <typename S, bool DEF>
-__device__ __forceinline__ V3<S> patch_edge_vertex(const In<S> &in, int x, int y, int z, int axis) {
-    const EdgeEnds<S, DEF> e = edge_ends<S, DEF>(in, x, y, z, axis);
-    const V3<S> p = lerp_vertex<S, DEF>(x, y, z, axis, e.d0, e.d1, e.f0, e.f1, in.iso);
-    const bool nan = e.d0 != e.d0 || e.d1 != e.d1;
-    return V3<S>{nan ? S(0) : p.x, nan ? S(0) : p.y, nan ? S(0) : p.z};
+__device__ __forceinline__ V3<S> patch_edge_vertex(const In<S> &in, const KindEnds<S> &K, int64_t idx, uint32_t stored,
+                                                   V3<S> c) {
+    const bool ok0 = (stored >> K.c0) & 1, ok1 = (stored >> K.c1) & 1;
+    const int64_t j0 = ok0 ? idx + K.d0 : 0, j1 = ok1 ? idx + K.d1 : 0;
+    S d0 = in.sdf[j0], d1 = in.sdf[j1];
+    V3<S> f0{}, f1{};
+    if (DEF) {
+        f0 = V3<S>{in.deform[3 * j0], in.deform[3 * j0 + 1], in.deform[3 * j0 + 2]};
+        f1 = V3<S>{in.deform[3 * j1], in.deform[3 * j1 + 1], in.deform[3 * j1 + 2]};
+    }
+    if (__any(!ok0 || !ok1)) {  // wave-uniform
+        d0 = ok0 ? d0 : in.pad;
+        d1 = ok1 ? d1 : in.pad;
+        f0 = V3<S>{ok0 ? f0.x : S(0), ok0 ? f0.y : S(0), ok0 ? f0.z : S(0)};
+        f1 = V3<S>{ok1 ? f1.x : S(0), ok1 ? f1.y : S(0), ok1 ? f1.z : S(0)};
+    }
+    const S t = interp_t(d0, d1, in.iso);
+    // (positions are whole numbers below 2^21: their sums are exact)
+    V3<S> p0 = {c.x + K.ox, c.y + K.oy, c.z}, p1 = {p0.x + K.ax, p0.y + K.ay, p0.z + K.az};
+    if (DEF) {
+        p0 = add3(p0, f0);
+        p1 = add3(p1, f1);
+    }
+    const bool nan = __builtin_isunordered(d0, d1);
+    return V3<S>{nan ? S(0) : p0.x + (p1.x - p0.x) * t, nan ? S(0) : p0.y + (p1.y - p0.y) * t,
+                 nan ? S(0) : p0.z + (p1.z - p0.z) * t};
 }
 
 // One unit of 64 active cells: its patch vertices and the quads of the edges its cells own. Both are
-// contiguous rows of the output, in the cells' order.
+// contiguous rows of the output, in the cells' order. Bound by vector instructions (four fifths of the
+// issue slots on white noise), so what a cell's edges share is worked out once per cell, and the rest
+// comes from small tables. Per edge position, index and bounds, and per patch the slots bit by bit:
+// 128x120x136 white noise 104 us, 256^3 noisy 173, 512^3 430; so 96, 163, 396.
 template <typename S, bool DEF, typename Next>
 __device__ __forceinline__ UnitLoad emit_dmc_unit(const In<S> &in, const UnitGrid &G, const UnitLoad &U, Next next,
                                               S *__restrict__ verts, void *__restrict__ faces,
                                               uint8_t *__restrict__ vinfo, const OutCfg &out, const Norm<S> &nm,
-                                              const uint64_t *s_case, DmcEmitLds<S> &L, int lane) {
+                                              const DmcTables<S> &T, DmcEmitLds<S> &L, int lane) {
     wave_lds_sync();  // the previous unit's LDS reads are done
     uint32_t s;
     int l;
@@ -1490,7 +1541,7 @@ __device__ __forceinline__ UnitLoad emit_dmc_unit(const In<S> &in, const UnitGri
     // (top edges) the next position, an edge counts as not crossing
     const bool gx = px + 1 < g.g0 - 1, gy = py + 1 < g.g1 - 1, gz = z + 1 < g.g2 - 1;
     const uint32_t keep = (gx ? 0xffu : 0x7du) & (gy ? 0xffu : 0xd7u) & (gx && gy ? 0xffu : 0xefu);
-    const uint64_t cwd = s_case[code];
+    const uint64_t cwd = T.cases[code];
     const uint32_t kb = on ? (uint32_t)(cwd >> 56) & keep : 0u;
     const int np = on ? DISO_DMC_NPATCH(cwd) : 0;
     const int ex = on ? bit_at(qxy.a, l) : 0, ey = on ? bit_at(qxy.b, l) : 0, ez = on ? bit_at(qza.a, l) : 0;
@@ -1507,18 +1558,24 @@ __device__ __forceinline__ UnitLoad emit_dmc_unit(const In<S> &in, const UnitGri
     const int nslot = te + __popc(hk);
     const bool slots = nslot <= kEdgeSlots;  // wave-uniform
 
+    const uint32_t stored = stored_corners(g, px, py, z);
+    const int64_t idx = data_index(in, px, py, z);
     if (on) {
         // bit 11: the top edges are the next cell's (they cross only where its position has a cell)
         L.cw[lane + 1] = (uint32_t)(pe + 1) | (uint32_t)bit_at(inside, l) << 10 | (gz ? 1u << 11 : 0u) | kb << 16 | code << 24;
-        L.cx[lane] = px;
-        L.cy[lane] = py;
-        L.cz[lane] = z;
+        L.idx[lane] = idx;
+        L.cx[lane] = S(px);
+        L.cy[lane] = S(py);
+        L.cz[lane] = S(z);
+        L.stored[lane] = (uint8_t)stored;
         L.pp[lane] = (uint16_t)pp;
     }
     if (lane == n - 1) {
-        L.cx[n] = px;
-        L.cy[n] = py;
-        L.cz[n] = z + 1;
+        L.idx[n] = idx + 1;
+        L.cx[n] = S(px);
+        L.cy[n] = S(py);
+        L.cz[n] = S(z + 1);
+        L.stored[n] = (uint8_t)(stored >> 4);  // (no edge of it that counts runs along z)
         L.cw[n + 1] = (uint32_t)(te + 1) | hk << 16;
     }
     if (lane == 0) L.cw[0] = (rz ? cz1 : 0u) << 24;
@@ -1560,11 +1617,11 @@ __device__ __forceinline__ UnitLoad emit_dmc_unit(const In<S> &in, const UnitGri
         const uint32_t w = L.cw[src + 1], wb = L.cw[src] >> 24, nc = L.nc[src], nd = L.nd[src];
         const int32_t f0 = L.pp[src], fx0 = L.nf[0][src], fy0 = L.nf[1][src], fw0 = L.nf[2][src];
         const bool isx = axis == 0, isy = axis == 1;
-        const uint32_t czb = L.cz[src] > 0 ? wb : 0u;
-        const uint64_t wa = s_case[w >> 24];
-        const uint64_t wB = s_case[isx ? (nc >> 16) & 0xff : (isy ? czb : nc & 0xff)];
-        const uint64_t wC = s_case[isx ? nc >> 24 : (isy ? (nc >> 8) & 0xff : nd)];
-        const uint64_t wD = s_case[isx ? czb : (isy ? nc & 0xff : (nc >> 16) & 0xff)];
+        const uint32_t czb = L.cz[src] > S(0) ? wb : 0u;
+        const uint64_t wa = T.cases[w >> 24];
+        const uint64_t wB = T.cases[isx ? (nc >> 16) & 0xff : (isy ? czb : nc & 0xff)];
+        const uint64_t wC = T.cases[isx ? nc >> 24 : (isy ? (nc >> 8) & 0xff : nd)];
+        const uint64_t wD = T.cases[isx ? czb : (isy ? nc & 0xff : (nc >> 16) & 0xff)];
         const int pa = (int)(wa >> (isx ? 0 : (isy ? 24 : 9))) & 7;         // edges 0, 8, 3
         const int pB = (int)(wB >> (isx ? 12 : (isy ? 33 : 3))) & 7;        // edges 4, 11, 1
         const int pC = (int)(wC >> (isx ? 18 : (isy ? 30 : 15))) & 7;       // edges 6, 10, 5
@@ -1584,8 +1641,8 @@ __device__ __forceinline__ UnitLoad emit_dmc_unit(const In<S> &in, const UnitGri
         // MC vertex of every crossing edge of the cells, once
         for (int i = lane; i < nslot; i += kWave) {
             const int it = L.eitem[i + 1], src = it >> 3, k = it & 7;
-            const int dx = (kKindX >> k) & 1, dy = (kKindY >> k) & 1, a = (kKindAxisZ >> k) & 1 ? 2 : (kKindAxisY >> k) & 1;
-            const V3<S> p = patch_edge_vertex<S, DEF>(in, L.cx[src] + dx, L.cy[src] + dy, L.cz[src], a);
+            const V3<S> p = patch_edge_vertex<S, DEF>(in, T.kind[k], L.idx[src], L.stored[src],
+                                                      V3<S>{L.cx[src], L.cy[src], L.cz[src]});
             L.ev[0][i + 1] = p.x;
             L.ev[1][i + 1] = p.y;
             L.ev[2][i + 1] = p.z;
@@ -1596,75 +1653,74 @@ __device__ __forceinline__ UnitLoad emit_dmc_unit(const In<S> &in, const UnitGri
     for (int k = lane; k < tp; k += kWave) {
         const int it = L.patch[k], src = it >> 2, pk = it & 3;
         const uint32_t w0 = L.cw[src + 1];
-        unsigned em = (unsigned)(kDmcPatchEdges.m[w0 >> 24] >> (16 * pk)) & 0xfffu;
+        const uint32_t em = (uint32_t)(T.edges[w0 >> 24] >> (16 * pk)) & 0xffffu;
         const int num = __popc(em);
         S sx2 = S(0), sy2 = S(0), sz2 = S(0);
         if (slots) {
-            // the slots of all twelve edges first, then all twelve vertices added in ascending edge
-            // order, edges outside the patch (or not counted as crossing) reading the zero entry: the
-            // running sum starts at +0 and so is never -0, and adding +0 leaves it unchanged
+            // the slots of all twelve edges first (as byte offsets), then all twelve vertices added in
+            // ascending edge order, edges outside the patch (or not counted as crossing) reading the
+            // zero entry: the running sum starts at +0 and so is never -0, and adding +0 leaves it
+            // unchanged
             const uint32_t w1 = L.cw[src + 2];
             const uint32_t k0 = (w0 >> 16) & 0xff, k1 = (w0 >> 11) & 1 ? (w1 >> 16) & 0xff : 0u;
-            int r0 = (int)(w0 & 0x3ff);
+            const int e0 = (int)(em & k0), e1 = (int)((em >> 8) & k1);
+            int r0 = (int)(w0 & 0x3ff) * (int)sizeof(S);
             const int r1 = (int)(w1 & 0x3ff);
             int sl[12];
 #pragma unroll
             for (int k2 = 0; k2 < 8; ++k2) {
-                const int e = kind_edge(k2), x = (int)(k0 >> k2) & 1;
-                sl[e] = (x & (int)(em >> e)) ? r0 : 0;
-                r0 += x;
+                sl[kind_edge(k2)] = r0 & __builtin_amdgcn_sbfe(e0, k2, 1);
+                r0 += (int)__builtin_amdgcn_ubfe(k0, k2, 1) * (int)sizeof(S);
             }
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const int e = kTopEdges[t], kd = kTopKinds[t];
-                sl[e] = ((k1 >> kd) & (em >> e) & 1) ? r1 + __popc(k1 & ((1u << kd) - 1)) : 0;
+                const int kd = kTopKinds[t];
+                sl[kTopEdges[t]] =
+                    (r1 + __popc(k1 & ((1u << kd) - 1))) * (int)sizeof(S) & __builtin_amdgcn_sbfe(e1, kd, 1);
             }
 #pragma unroll
             for (int e = 0; e < 12; ++e) {
-                sx2 += L.ev[0][sl[e]];
-                sy2 += L.ev[1][sl[e]];
-                sz2 += L.ev[2][sl[e]];
+                const char *at = reinterpret_cast<const char *>(L.ev[0]) + sl[e];
+                sx2 += reinterpret_cast<const S *>(at)[0];
+                sy2 += reinterpret_cast<const S *>(at)[kEdgeSlots + 1];
+                sz2 += reinterpret_cast<const S *>(at)[2 * (kEdgeSlots + 1)];
             }
         } else {
-            const int x0 = L.cx[src], y0 = L.cy[src], z0 = L.cz[src];
-            const bool okx = x0 + 1 < g.g0 - 1, oky = y0 + 1 < g.g1 - 1, okz = z0 + 1 < g.g2 - 1;
-            while (em) {  // ascending edge order
-                const int e = __ffs(em) - 1;
-                em &= em - 1;
-                if ((eox(e) && !okx) || (eoy(e) && !oky) || (eoz(e) && !okz)) continue;
-                const V3<S> p = patch_edge_vertex<S, DEF>(in, x0 + eox(e), y0 + eoy(e), z0 + eoz(e), eax(e));
+            const V3<S> c = {L.cx[src], L.cy[src], L.cz[src]};
+            const bool okx = (int)c.x + 1 < g.g0 - 1, oky = (int)c.y + 1 < g.g1 - 1, okz = (int)c.z + 1 < g.g2 - 1;
+            constexpr uint64_t kEdgeBits = edge_bits();
+            for (int e = 0; e < 12; ++e) {  // ascending edge order
+                const int bit = (int)(kEdgeBits >> (4 * e)) & 15, up = bit >> 3;
+                if (!((em >> bit) & 1) || (eox(e) && !okx) || (eoy(e) && !oky) || (eoz(e) && !okz)) continue;
+                const V3<S> p = patch_edge_vertex<S, DEF>(in, T.kind[bit & 7], L.idx[src] + up, L.stored[src] >> (4 * up),
+                                                          V3<S>{c.x, c.y, c.z + S(up)});
                 sx2 += p.x;
                 sy2 += p.y;
                 sz2 += p.z;
             }
         }
-        const S r = rcp_small<S>(num);
+        const S r = T.rcp[num];
         store_vertex(verts, pbase + k, out.vcap, epilogue(V3<S>{sx2 * r, sy2 * r, sz2 * r}, out.flags, nm));
         if (pbase + k < out.vcap) put(vinfo + pbase + k, (uint8_t)(num | (pk << 3)));
     }
     return after;
 }
 
-// The DMC case words with each code's own_kinds in the free top byte, in LDS.
-__device__ __forceinline__ void load_dmc_cases(uint64_t *s_case) {
-    for (int i = threadIdx.x; i < 256; i += kBlock) s_case[i] = kDmcCase[i] | (uint64_t)own_kinds((uint32_t)i) << 56;
-}
-
 template <typename S, bool DEF>
 __global__ __launch_bounds__(kBlock, 5) void emit_dmc_kernel(In<S> in, const SegBase *__restrict__ seg, Planes planes,
                                                           S *__restrict__ verts, void *__restrict__ faces,
                                                           uint8_t *__restrict__ vinfo, OutCfg out, Norm<S> nm) {
-    __shared__ uint64_t s_case[256];
+    __shared__ DmcTables<S> s_tab;
     __shared__ DmcEmitLds<S> s_lds[kWavesPerBlock];
     const int wave = wave_id(), lane = threadIdx.x % kWave;
     const SegBase *tot = seg + in.geo.nseg;
     if (tot[0].v > out.fcap || tot[0].f > out.vcap) return;
-    load_dmc_cases(s_case);
+    s_tab.load(in.geo);
     __syncthreads();
     const uint32_t nunits = *planes.nunits;
     const UnitGrid G{seg, planes, 0, in.geo.nseg - 1, 0, 0};
     for_units(G, nunits, blockIdx.x, gridDim.x, wave, lane, [&](const UnitLoad &U, auto next) {
-        return emit_dmc_unit<S, DEF>(in, G, U, next, verts, faces, vinfo, out, nm, s_case, s_lds[wave], lane);
+        return emit_dmc_unit<S, DEF>(in, G, U, next, verts, faces, vinfo, out, nm, s_tab, s_lds[wave], lane);
     });
 }
 
@@ -2291,18 +2347,21 @@ __global__ void batch_totals_kernel(const BatchGrid<S> *__restrict__ grids, int 
 }
 
 // Batched emission: a grid's blocks go through its units in turn. Units are of the whole batch, so a
-// grid's first and last may hold cells of its neighbours too (unit_cells leaves them out).
-template <typename S, typename F>
+// grid's first and last may hold cells of its neighbours too (unit_cells leaves them out). tables(geo)
+// fills the block's tables.
+template <typename S, typename T, typename F>
 __device__ __forceinline__ void batch_units(const BatchGrid<S> *__restrict__ grids, const int32_t *__restrict__ gl,
                                             const int64_t *__restrict__ rf, int m, const SegBase *__restrict__ seg,
                                             const Planes &planes, const uint32_t *__restrict__ range, int64_t nblocks,
-                                            int wave, int lane, F f) {
+                                            int wave, int lane, T tables, F f) {
     const int64_t b = xcd_block(blockIdx.x, nblocks);
     const int j = find_group(rf, m, b);
     const int gi = gl[j];
     const BatchGrid<S> &B = grids[gi];
     if (B.nv > B.vcap || B.nf > B.fcap) return;
     const In<S> in = B.in;
+    tables(in.geo);
+    __syncthreads();
     const int64_t first = B.seg_first;
     const UnitGrid G{seg, planes, first, first + in.geo.nseg - 1, seg[first].v, seg[first].f};
     const OutCfg out{B.flags, B.vcap, B.fcap};
@@ -2320,9 +2379,7 @@ __global__ __launch_bounds__(kBlock, 6) void emit_mc_batch_kernel(const BatchGri
     __shared__ uint64_t s_case[256];
     __shared__ McEmitLds s_lds[kWavesPerBlock];
     const int wave = wave_id(), lane = threadIdx.x % kWave;
-    load_mc_cases(s_case);
-    __syncthreads();
-    batch_units(grids, gl, rf, m, seg, planes, range, nblocks, wave, lane,
+    batch_units(grids, gl, rf, m, seg, planes, range, nblocks, wave, lane, [&](const Geo &) { load_mc_cases(s_case); },
                 [&](const In<S> &in, const UnitGrid &G, const BatchGrid<S> &B, const OutCfg &out, const UnitLoad &U, auto next) {
                     return emit_mc_unit<S, DEF>(in, G, U, next, B.verts, B.faces, out, B.nm, s_case, s_lds[wave], lane);
                 });
@@ -2334,14 +2391,12 @@ __global__ __launch_bounds__(kBlock, 5) void emit_dmc_batch_kernel(const BatchGr
                                                                 const int64_t *__restrict__ rf, int m,
                                                                 const SegBase *__restrict__ seg, Planes planes,
                                                                 const uint32_t *__restrict__ range, int64_t nblocks) {
-    __shared__ uint64_t s_case[256];
+    __shared__ DmcTables<S> s_tab;
     __shared__ DmcEmitLds<S> s_lds[kWavesPerBlock];
     const int wave = wave_id(), lane = threadIdx.x % kWave;
-    load_dmc_cases(s_case);
-    __syncthreads();
-    batch_units(grids, gl, rf, m, seg, planes, range, nblocks, wave, lane,
+    batch_units(grids, gl, rf, m, seg, planes, range, nblocks, wave, lane, [&](const Geo &g) { s_tab.load(g); },
                 [&](const In<S> &in, const UnitGrid &G, const BatchGrid<S> &B, const OutCfg &out, const UnitLoad &U, auto next) {
-                    return emit_dmc_unit<S, DEF>(in, G, U, next, (S *)B.verts, B.faces, B.vinfo, out, B.nm, s_case, s_lds[wave], lane);
+                    return emit_dmc_unit<S, DEF>(in, G, U, next, (S *)B.verts, B.faces, B.vinfo, out, B.nm, s_tab, s_lds[wave], lane);
                 });
 }
 
