@@ -2,27 +2,28 @@
 //
 // Work decomposition
 //   The (virtually padded) grid G = [g0,g1,g2] is cut into "segments": one z-row (px,py) of the
-//   grid, split into chunks of 64 consecutive z positions. One wave64 owns one segment, lane l
-//   the position pz = 64*chunk + l. Segment order (px, py, chunk) is the grid's linear order
+//   grid, split into chunks of 64 consecutive z positions, bit l of a 64-bit plane standing for
+//   position pz = 64*chunk + l. Segment order (px, py, chunk) is the grid's linear order
 //   (x-major, z fastest), which is the order in which the reference emits its vertices and faces
 //   (used cells in increasing linear cell id, src/cumc.cu:299-311,370-410,564-610). So the output
 //   position of any cell's first vertex / face is
-//       base(segment) + exclusive prefix, within the wave, of the per-cell counts,
-//   and only the per-segment bases are stored (16 bytes per 64 cells). The count pass also stores
-//   one 16-bit classification word per position (code, owned crossings, inside bit, face count),
-//   which the later passes read instead of re-classifying (the recompute-classification backward
-//   re-derives the crossings from the samples instead). In-wave prefixes come from bit-plane
-//   ballots and v_mbcnt.
+//       base(segment) + bits of the segment's planes below its position,
+//   and only the per-segment bases are stored (16 bytes per 64 cells). The count pass also stores the
+//   classification as bit planes and codes (struct Planes), which the later passes read instead of
+//   re-classifying (the recompute-classification backward re-derives the crossings from the samples
+//   instead), and deals the active cells into units of 64, the emission's work items: a surface
+//   fills few positions of a segment, and a wave that took segments would run half empty.
 //
 // Kernels
-//   count_kernel          classify + count + single-pass decoupled look-back scan of segment
-//                         counts (also over the segments of a batch of grids).
+//   mask_kernel           the samples' inside and below bits as planes, and their flags.
+//   count_kernel          classify + count, a lane per segment, + single-pass decoupled look-back
+//                         scan of segment counts (also over the segments of a batch of grids).
 //   emit_mc_kernel        MC vertices and triangles (+ shift / normalise / int64 epilogue).
 //   emit_dmc_kernel       DMC vertices (patch means) and quads.
 //   dmc_edge_grad_kernel  DMC backward, first step: per crossing edge, the sum of its <= 4 quad
 //                         corners' vertex gradients / patch sizes.
-//   bwd_mc_kernel         MC gather backward (DMC: on those edge gradients): one lane per grid
-//                         vertex sums its <= 6 incident edges, deterministic, no atomics.
+//   bwd_mc_kernel         MC gather backward (DMC: on those edge gradients): one lane per touched
+//                         grid vertex sums its <= 6 incident edges, deterministic, no atomics.
 //   split_*_kernel        DiffDMC's quad -> triangle split.
 //   *_batch_kernel        the same passes over many grids in one launch.
 //
@@ -917,16 +918,15 @@ __global__ __launch_bounds__(kCountBlock, kCountWaves / 2) void count_kernel(Cou
 // ------------------------------------------------------------------------------------------
 // Pass 2: emission
 //
-// Work compaction: each lane publishes its work items (MC vertices and triangle corners; DMC
-// patch vertices and quads) into a dense per-wave list in LDS at its in-wave prefix, and the wave
-// then processes the list 64 items at a time. Every item is computed exactly once (a lane-per-
-// cell loop would make the whole wave execute the union of all lanes' branches), and item k is
-// the segment's k-th output row, so consecutive lanes write consecutive rows (coalesced stores).
+// Work compaction, twice. A wave takes units of 64 active cells, wherever they lie: 256^3 noisy, MC /
+// DMC 156 / 289 us with a wave per segment, 124 / 163 so; 384^3 smooth 217 and 63. And each lane
+// publishes its cell's items (MC vertices and triangles; DMC edge vertices, patch vertices and
+// quads) into a dense per-wave list in LDS at its in-wave prefix, which the wave then processes 64
+// items at a time. Every item is computed exactly once, and item k is the unit's k-th output row, so
+// consecutive lanes write consecutive rows (coalesced stores). MC is bound by the latency between a
+// unit's dependent loads (vector instructions take two fifths of the issue slots).
 
-// Emission and backward blocks each take a run of `run` (<= 64) consecutive segments (so per-block
-// setup, such as the case tables in LDS, is paid once per run) and share its segments with work
-// among their waves (emission: from a shared counter, run_segments; backward: round-robin); the
-// rest cost one lane-parallel load of the run's bases. The run length is a launch parameter
+// Largest run length: the segments that four gathering waves take (bwd_tile_of), a launch parameter
 // (diso_set_param).
 constexpr int kMaxRun = kWave;
 
@@ -1286,7 +1286,7 @@ __global__ __launch_bounds__(kBlock, 6) void emit_mc_kernel(In<S> in, const SegB
 // Quad item = (lane, axis, leaving) of an owned crossing edge (src/cudualmc.cu:1027-1056): its
 // corners are the vertices of the patches holding the edge in the four cells around it, which
 // lie in rows R00, Rm0 (-x), R0m (-y), Rmm (-x-y) at this z and z-1. Cell codes come from the
-// count pass's classification words, so no sample is read to classify.
+// count pass, so no sample is read to classify.
 
 // Quad stencil (src/cudualmc.cu:504-513) as cell index ci and edge id: entry k of type ty.
 // Types 3..5 (edges leaving the inside) list the cells of types 0..2 in the order 0,3,2,1.
@@ -2302,10 +2302,9 @@ __global__ __launch_bounds__(kBlock) void dmc_edge_grad_kernel(const void *__res
 // The count pass runs once over the concatenation of all grids' segments (a grid's segments are
 // consecutive, grids in batch order), so one single-pass scan yields every grid's bases; a grid's
 // own output rows are its bases minus those of its first segment. Emission and backward launch
-// one block per run of segments of one grid: a launch covers the runs of every grid of one
-// kind (algorithm x deform x recompute), listed in `gl` with the prefix of their run counts in
-// `rf`; a block finds its grid by binary search over `rf`.
-
+// blocks of one grid: a launch covers the blocks of every grid of one kind (algorithm x deform x
+// recompute), listed in `gl` with the prefix of their block counts in `rf`; a block finds its grid
+// by binary search over `rf`.
 
 template <typename S>
 __device__ __forceinline__ SegCtx batch_ctx(const BatchGrid<S> &G, const SegBase *seg, const Planes &q) {
@@ -2988,7 +2987,7 @@ int64_t align256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 constexpr int kBatchGroups = 9;  // emit: MC/DMC x deform; backward: deform x recompute; DMC edges
 
 // Where everything of a batch lives in its workspace: the device descriptors, the launch-group
-// tables, the per-grid totals, then the segment bases and classification words of all grids.
+// tables, the per-grid totals, then the segment bases and classification planes of all grids.
 struct BatchLayout {
     int n = 0;
     int64_t nseg = 0;

@@ -203,7 +203,7 @@ class Extractor:
             counted.quads, counted.vinfo = faces, vinfo
         if flags & _lib.FLAG_RECOMPUTE:
             # The backward will re-derive the classification from the samples: keep only the
-            # segment bases and release the classification words.
+            # segment bases and release the stored classification.
             counted.seg = counted.seg[:self._sizes(counted.dims, flags)[1]].clone()
         return verts, faces
 

@@ -49,7 +49,7 @@ class Request:
         return (self.isovalue, self.normalize, self.return_quads)
 
     def workspace(self):
-        """Device bytes of the counting pass's workspace: a 16-bit word per padded position and a
+        """Device bytes of the counting pass's workspace: two bytes per padded position and a
         16-byte base per 64 positions."""
         X, Y, Z = (int(d) for d in self.sdf.shape)
         pos = (X + 2) * (Y + 2) * (Z + 2)

@@ -43,7 +43,7 @@ enum {
     DISO_FLAG_ACCUMULATE = 1 << 5,  /* backward adds into the gradient buffers instead of
                                        overwriting them                                        */
     DISO_FLAG_RECOMPUTE = 1 << 6    /* backward re-derives the crossing masks from the samples
-                                       instead of reading the classification words, so only
+                                       instead of reading the stored classification, so only
                                        the bases prefix of seg (diso_seg_bytes with this flag)
                                        must be kept from the forward                           */
 };
@@ -78,7 +78,7 @@ typedef struct {
 } diso_totals_t;
 
 /* Size in bytes of the per-call segment workspace ("seg") for a grid of dims (X,Y,Z): the
- * per-segment vertex/face bases and a 16-bit classification word per grid position, written by
+ * per-segment vertex/face bases and the classification (two bytes per grid position), written by
  * diso_count and read by diso_emit / diso_backward. It needs no initialisation. Keep it (with the
  * same inputs) to run diso_backward later; that is the state the reference keeps inside CuMC
  * between forward and backward (src/cumc.h:73-99). With DISO_FLAG_RECOMPUTE in `flags` the size
