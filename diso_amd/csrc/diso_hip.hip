@@ -1749,20 +1749,20 @@ struct AdjIn {
     Norm<S> nm;  // upstream scaling by 1/(dims-1) when the forward normalised
 };
 
+// Row i < n of the upstream gradient.
 template <typename S>
-__device__ __forceinline__ V3<S> load_adj(const AdjIn<S> &a, int64_t i) {
-    V3<S> r = {S(0), S(0), S(0)};
-    if (i >= 0 && i < a.n) {
-        r.x = a.adj[3 * i + 0];
-        r.y = a.adj[3 * i + 1];
-        r.z = a.adj[3 * i + 2];
-        if (a.flags & DISO_FLAG_NORMALIZE) {  // grad of verts / (dims - 1): g / (dims - 1)
-            r.x = div_by(r.x, a.nm.c[0], a.nm.r[0]);
-            r.y = div_by(r.y, a.nm.c[1], a.nm.r[1]);
-            r.z = div_by(r.z, a.nm.c[2], a.nm.r[2]);
-        }
+__device__ __forceinline__ V3<S> load_adj_at(const AdjIn<S> &a, int64_t i) {
+    V3<S> r = {a.adj[3 * i + 0], a.adj[3 * i + 1], a.adj[3 * i + 2]};
+    if (a.flags & DISO_FLAG_NORMALIZE) {  // grad of verts / (dims - 1): g / (dims - 1)
+        r.x = div_by(r.x, a.nm.c[0], a.nm.r[0]);
+        r.y = div_by(r.y, a.nm.c[1], a.nm.r[1]);
+        r.z = div_by(r.z, a.nm.c[2], a.nm.r[2]);
     }
     return r;
+}
+template <typename S>
+__device__ __forceinline__ V3<S> load_adj(const AdjIn<S> &a, int64_t i) {
+    return i >= 0 && i < a.n ? load_adj_at(a, i) : V3<S>{S(0), S(0), S(0)};
 }
 
 template <typename S>
@@ -2243,38 +2243,81 @@ __global__ __launch_bounds__(kWave) void bwd_mc_kernel(In<S> in, const SegBase *
     if (b < nblocks) bwd_wave<S, DEF, RECOMP>(in, sc, b, tile, adj, adj_sdf, adj_deform);
 }
 
+// A quad's four indices in 16-byte loads (any address an index may have).
+typedef int64_t Index2 __attribute__((ext_vector_type(2), aligned(8)));
+typedef int32_t Index4 __attribute__((ext_vector_type(4), aligned(4)));
+struct QuadIds {
+    Index2 a, b;
+};
+__device__ __forceinline__ QuadIds load_quad(const void *__restrict__ quads, int64_t q, int flags) {
+    if (flags & DISO_FLAG_INDEX64) {
+        const Index2 *p = reinterpret_cast<const Index2 *>(static_cast<const int64_t *>(quads) + 4 * q);
+        return QuadIds{p[0], p[1]};
+    }
+    const Index4 v = *reinterpret_cast<const Index4 *>(static_cast<const int32_t *>(quads) + 4 * q);
+    return QuadIds{Index2{v.x, v.y}, Index2{v.z, v.w}};
+}
+
 // Per-edge upstream gradient of a DMC forward: ge[q] = sum over the quad's corners v of
-// (dL/dv) / (edges in v's patch), corners in the quad's order.
+// (dL/dv) / (edges in v's patch), corners in the quad's order, for a wave's 64 quads from q0 on. Bound
+// by the latency of the gather: a corner out of range adds nothing, but loads row 0, so that all four
+// corners' loads are in flight together (a branch around each: 256^3 noisy 63 us, 512^3 123; so 59,
+// 118). The quads are read once, by non-temporal loads, so that they do not displace what the gather
+// after this re-reads (with ordinary loads it takes 136 us, so 120); 64-bit ones pass through LDS, each
+// load covering whole lines (without that, 63 us, and a batch's 381 instead of 321).
 template <typename S>
-__device__ __forceinline__ void edge_grad_one(const void *__restrict__ quads, int64_t q,
-                                              const uint8_t *__restrict__ vinfo, const AdjIn<S> &adj, const S *s_rcp,
-                                              S *__restrict__ ge) {
+__device__ __forceinline__ void edge_grad_wave(const void *__restrict__ quads, int64_t q0, int64_t n,
+                                               const uint8_t *__restrict__ vinfo, const AdjIn<S> &adj, const S *s_rcp,
+                                               Index2 *s_quad, S *__restrict__ ge) {
     const bool compat = (adj.flags & DISO_FLAG_REFERENCE_COMPAT) != 0;
-    V3<S> sum = {S(0), S(0), S(0)};
-    // the quad's four indices: one 16-byte non-temporal load when they are 32-bit and aligned (a
-    // stream read once, kept out of the caches the following gather re-reads samples from)
-    int64_t qv[4];
-    if (!(adj.flags & DISO_FLAG_INDEX64) && ((uintptr_t)quads & 15) == 0) {  // uniform
-        const i32x4 r = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(quads) + q);
-        qv[0] = r.x;
-        qv[1] = r.y;
-        qv[2] = r.z;
-        qv[3] = r.w;
+    const int lane = threadIdx.x % kWave;
+    const int64_t q = q0 + lane, left = n - q0;
+    if (left <= 0) return;  // wave-uniform
+    QuadIds w;
+    if (adj.flags & DISO_FLAG_INDEX64) {
+        const Index2 *p = reinterpret_cast<const Index2 *>(static_cast<const int64_t *>(quads) + 4 * q0);
+        const int last = left < kWave ? 2 * (int)left - 1 : 2 * kWave - 1;
+        s_quad[lane] = __builtin_nontemporal_load(p + (lane < last ? lane : last));
+        s_quad[lane + kWave] = __builtin_nontemporal_load(p + (lane + kWave < last ? lane + kWave : last));
+        wave_lds_sync();
+        w = QuadIds{s_quad[2 * lane], s_quad[2 * lane + 1]};
     } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) qv[k] = load_index(quads, 4 * q + k, adj.flags);
+        const Index4 *p = reinterpret_cast<const Index4 *>(static_cast<const int32_t *>(quads) + 4 * q0);
+        const Index4 v = __builtin_nontemporal_load(p + (lane < left ? lane : 0));
+        w = QuadIds{Index2{v.x, v.y}, Index2{v.z, v.w}};
     }
+    const int64_t qv[4] = {w.a.x, w.a.y, w.b.x, w.b.y};
+    V3<S> sum = {S(0), S(0), S(0)};
+    if (adj.n > 0) {  // uniform
+        int64_t at[4];
+        bool ok[4];
+        int info[4];
+        V3<S> a[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int64_t v = qv[k];
-        if (v < 0 || v >= adj.n) continue;
-        const int info = vinfo[v];
-        const V3<S> a = load_adj(adj, compat ? v - (info >> 3) : v);
-        const S r = s_rcp[info & 7];
-        sum.x += a.x * r;
-        sum.y += a.y * r;
-        sum.z += a.z * r;
+        for (int k = 0; k < 4; ++k) {
+            ok[k] = (qv[k] >= 0) & (qv[k] < adj.n);
+            at[k] = ok[k] ? qv[k] : 0;
+            info[k] = vinfo[at[k]];
+        }
+        if (compat) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int64_t first = at[k] - (info[k] >> 3);
+                ok[k] &= first >= 0;
+                at[k] = first >= 0 ? first : 0;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a[k] = load_adj_at(adj, at[k]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const S r = s_rcp[info[k] & 7];
+            sum.x += ok[k] ? a[k].x * r : S(0);
+            sum.y += ok[k] ? a[k].y * r : S(0);
+            sum.z += ok[k] ? a[k].z * r : S(0);
+        }
     }
+    if (lane >= left) return;
     ge[3 * q + 0] = sum.x;
     ge[3 * q + 1] = sum.y;
     ge[3 * q + 2] = sum.z;
@@ -2286,14 +2329,15 @@ __global__ __launch_bounds__(kBlock) void dmc_edge_grad_kernel(const void *__res
                                                                const uint8_t *__restrict__ vinfo, AdjIn<S> adj,
                                                                S *__restrict__ ge) {
     __shared__ S s_rcp[8];
+    __shared__ Index2 s_quad[kWavesPerBlock][2 * kWave];
     if (threadIdx.x < 8) s_rcp[threadIdx.x] = threadIdx.x ? S(1) / S(threadIdx.x) : S(0);
     __syncthreads();
     // nq may be a capacity: the quads are the first tot->v rows (the count pass's total)
     const int64_t n = tot->v < nq ? tot->v : nq;
     // each XCD takes a contiguous eighth of the quads, so the vertex rows a quad shares with the
     // quads of the previous plane are still in that XCD's L2
-    const int64_t q = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (q < n) edge_grad_one(quads, q, vinfo, adj, s_rcp, ge);
+    const int64_t q0 = xcd_block(blockIdx.x, gridDim.x) * kBlock + wave_id() * kWave;
+    edge_grad_wave(quads, q0, n, vinfo, adj, s_rcp, s_quad[wave_id()], ge);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2406,15 +2450,15 @@ __global__ __launch_bounds__(kBlock) void dmc_edge_grad_batch_kernel(const Batch
                                                                      const int64_t *__restrict__ rf, int m,
                                                                      S *__restrict__ ge) {
     __shared__ S s_rcp[8];
+    __shared__ Index2 s_quad[kWavesPerBlock][2 * kWave];
     if (threadIdx.x < 8) s_rcp[threadIdx.x] = threadIdx.x ? S(1) / S(threadIdx.x) : S(0);
     __syncthreads();
     const int64_t b = xcd_block(blockIdx.x, gridDim.x);  // as dmc_edge_grad_kernel
     const int j = find_group(rf, m, b);
     const BatchGrid<S> &G = grids[gl[j]];
-    const int64_t q = (b - rf[j]) * kBlock + threadIdx.x;
-    if (q >= G.nf) return;
+    const int64_t q0 = (b - rf[j]) * kBlock + wave_id() * kWave;
     const AdjIn<S> a{G.adj, G.nv, G.flags, G.nm};
-    edge_grad_one(G.faces, q, G.vinfo, a, s_rcp, ge + 3 * G.q_first);
+    edge_grad_wave(G.faces, q0, G.nf, G.vinfo, a, s_rcp, s_quad[wave_id()], ge + 3 * G.q_first);
 }
 
 template <typename S, bool DEF, bool RECOMP>
@@ -2496,21 +2540,7 @@ __device__ __forceinline__ V3<S> load_vert(const S *__restrict__ v, int64_t i) {
     return {v[3 * i + 0], v[3 * i + 1], v[3 * i + 2]};
 }
 
-// A quad's four indices in 16-byte loads (any address an index may have).
-typedef int64_t Index2 __attribute__((ext_vector_type(2), aligned(8)));
-typedef int32_t Index4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t Count4 __attribute__((ext_vector_type(kSplitWaves), aligned(4)));  // a block's counts
-struct QuadIds {
-    Index2 a, b;
-};
-__device__ __forceinline__ QuadIds load_quad(const void *__restrict__ quads, int64_t q, int flags) {
-    if (flags & DISO_FLAG_INDEX64) {
-        const Index2 *p = reinterpret_cast<const Index2 *>(static_cast<const int64_t *>(quads) + 4 * q);
-        return QuadIds{p[0], p[1]};
-    }
-    const Index4 v = *reinterpret_cast<const Index4 *>(static_cast<const int32_t *>(quads) + 4 * q);
-    return QuadIds{Index2{v.x, v.y}, Index2{v.z, v.w}};
-}
 
 template <typename S>
 __global__ __launch_bounds__(kSplitBlock) void split_score_kernel(const S *__restrict__ verts, int64_t nv,
