@@ -1,7 +1,7 @@
 """Thin host-side driver of libdiso_hip.so for torch tensors.
 
 `Extractor` is the counterpart of the reference's engine objects (CuMC, src/cumc.h:70-139;
-CUDualMC, src/cudualmc.h:70-150): it owns the scan control workspace of each device it has run
+CUDualMC, src/cudualmc.h:70-150): it owns the scan control workspace of each stream it has run
 on (zero-filled once, grown on demand) and runs the count / emit / backward passes on the
 current torch stream. Per-call state (the segment bases the backward needs) is returned to the
 caller instead of being kept inside the object, so one extractor can serve many grids whose
@@ -73,6 +73,10 @@ def _stream(device):
     return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
 
+def _capturing():
+    return torch.cuda.is_current_stream_capturing()
+
+
 class Extractor:
     def __init__(self, algo, dtype):
         if dtype not in _DTYPES:
@@ -80,7 +84,8 @@ class Extractor:
         self.algo = algo
         self.dtype = dtype
         self.code = _DTYPES[dtype]
-        self._ctl = {}
+        self._ctl = {}  # (device, stream) -> control block (ctl_for)
+        self._first = {}  # device -> the first of them, for captures
         self._guess = {}  # (device, dims, flags) -> (vertices, faces) of the last call
         self._need = {}  # (dims, flags) -> workspace bytes (_sizes)
         _lib.lib()  # fail loudly now if the HIP library is not there
@@ -109,14 +114,32 @@ class Extractor:
             self._need[key] = got
         return got
 
-    def ctl_for(self, device, dims, flags):
+    def ctl_for(self, device, dims, flags, capturing=False):
+        """The control block of the current stream. One per stream, because consecutive calls may use
+        it only in stream order: a forward returns as soon as its totals are known, while blocks of
+        its count may still be reading and clearing the block's words. A capture takes the device's
+        first block, which is kept as long as this object (or, without one, a block that each replay
+        clears)."""
         need = self._sizes(dims, flags)[2]
-        key = device.index
-        ctl = self._ctl.get(key)
-        if ctl is None or ctl.numel() < need:
-            # Grown buffers start zero-filled; the scan keeps them consistent from then on (its
-            # words carry their call's epoch, so not even a timed-out call needs a reset).
-            ctl = torch.zeros(max(need, 1 << 16) * 5 // 4, dtype=torch.uint8, device=device)
+        key = (device.index, _stream(device).value)
+        if not capturing:
+            ctl = self._ctl.get(key)
+            if ctl is not None and ctl.numel() >= need:
+                return ctl
+            capturing = _capturing()
+        first = self._first.get(device.index)
+        if first is not None and first.numel() < need:
+            first = None
+        if capturing and first is not None:
+            return first
+        # New blocks start zero-filled; the scan keeps them consistent from then on (its words carry
+        # their call's epoch, so not even a timed-out call needs a reset).
+        ctl = torch.zeros(max(need, 1 << 16) * 5 // 4, dtype=torch.uint8, device=device)
+        if not capturing:
+            if first is None:
+                self._first[device.index] = ctl
+            if len(self._ctl) >= 64:
+                self._ctl.clear()  # many streams: start over (freed memory goes back to its own stream)
             self._ctl[key] = ctl
         return ctl
 

@@ -25,7 +25,7 @@ import ctypes
 import torch
 
 from . import _lib
-from .engine import _DTYPES, Extractor, _ptr, _stream
+from .engine import _DTYPES, Extractor, _capturing, _ptr, _stream
 
 __all__ = ["FixedExtractor"]
 
@@ -45,7 +45,7 @@ class _FixedExtract(torch.autograd.Function):
         if nseg < 0 or off < 0:
             _lib.check(min(nseg, off), "workspace sizing")
         seg = torch.empty(nseg, dtype=torch.uint8, device=dev)
-        ctl = ex.ctl_for(dev, dims, flags)
+        ctl = ex.ctl_for(dev, dims, flags, _capturing())
         st = _stream(dev)
         rc = L.diso_count(ex.algo, ex.code, _ptr(grid), *dims, iso, flags, _ptr(seg), nseg, _ptr(ctl), ctl.numel(),
                           None, st)

@@ -1,0 +1,78 @@
+"""One module on several streams, and extractions from several host threads (needs a GPU). A forward
+returns before its count kernel has ended, so what calls share must be ordered by more than the host."""
+import threading
+
+import pytest
+import torch
+
+import diso_amd
+from diso_amd import _lib
+from tests.helpers import check_against_oracle, inputs
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _grids(n, dims, seed):
+    return [torch.tensor(inputs(dims, "noise" if i % 2 else "noisy_box", seed + i, "float32", False)[0], device=DEV)
+            for i in range(n)]
+
+
+@pytest.mark.parametrize("spins", [0, None])
+@pytest.mark.parametrize("algo", ["mc", "dmc"])
+def test_one_module_on_alternating_streams(algo, spins):
+    """Sequential calls from one thread, each on the other stream, none synchronised: each as alone.
+    (With recount spins 0 a block that finds a predecessor's word missing counts that range itself.)"""
+    print(f"case streams {algo} spins={spins}", flush=True)
+    L = _lib.lib()
+    before = L.diso_get_param(_lib.PARAM_RECOUNT_SPINS)
+    make = diso_amd.DiffMC if algo == "mc" else diso_amd.DiffDMC
+    kw = {} if algo == "mc" else {"return_quads": True}
+    grids = _grids(4, (70, 61, 130), 40)
+    want = [make()(g, **kw) for g in grids]
+    for g, (v, f) in zip(grids[:2], want):
+        check_against_oracle(algo, g.cpu().numpy(), None, v, f)
+    mod, streams = make(), [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    got = []
+    try:
+        if spins is not None:
+            _lib.check(L.diso_set_param(_lib.PARAM_RECOUNT_SPINS, spins), "spins")
+        for k in range(60):
+            with torch.cuda.stream(streams[k % 2]):
+                got.append(mod(grids[k % 4], **kw))
+        torch.cuda.synchronize()
+    finally:
+        L.diso_set_param(_lib.PARAM_RECOUNT_SPINS, before)
+    for k, (v, f) in enumerate(got):
+        assert torch.equal(v, want[k % 4][0]) and torch.equal(f, want[k % 4][1]), k
+
+
+def test_extractions_from_several_threads():
+    """Threads with a module of their own on one stream, and on one of their own each."""
+    print("case threads", flush=True)
+    grids = _grids(6, (40, 51, 70), 60)
+    want = [diso_amd.DiffMC()(g) for g in grids]
+    for own_stream in (False, True):
+        torch.cuda.synchronize()
+        got, errors = [None] * len(grids), []
+
+        def work(i):
+            try:
+                mod = diso_amd.DiffMC()
+                st = torch.cuda.Stream() if own_stream else torch.cuda.default_stream()
+                with torch.cuda.stream(st):
+                    for _ in range(20):
+                        got[i] = mod(grids[i])
+                    st.synchronize()
+            except Exception as e:  # reported below
+                errors.append(e)
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(len(grids))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not errors, errors
+        for (v, f), (w, x) in zip(got, want):
+            assert torch.equal(v, w) and torch.equal(f, x)
