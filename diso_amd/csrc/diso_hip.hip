@@ -563,6 +563,15 @@ __device__ __forceinline__ void mask_tile(const In<S> &in, int64_t first, int64_
     const uint64_t own = lane >= 1 && lane <= n ? have : 0ull;
     uint32_t fl = ((~I & ~E & own) ? DISO_TOTAL_HAS_BELOW : 0u) | ((I & ~E & own) ? DISO_TOTAL_HAS_ABOVE : 0u) |
                   ((~I & E & own) ? DISO_TOTAL_HAS_NAN : 0u);
+    if (in.iso != in.iso) {  // every compare fails: no sample is below or above, and E says nothing of NaN
+        fl = 0u;
+        const int end = own ? g.n2 - z0 : 0;
+#pragma unroll 1
+        for (int l = 0; l < kWave && l < end; ++l) {
+            const S v = in.sdf[ro + l];
+            fl |= v != v ? DISO_TOTAL_HAS_NAN : 0u;
+        }
+    }
     fl = wave_or(fl);
     if ((fl & DISO_TOTAL_HAS_NAN) && lane == 0) __hip_atomic_store(nan, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // the previous lane's top bit (its chunk precedes this one, unless this is the row's first)
