@@ -1812,8 +1812,11 @@ __device__ __forceinline__ Grad<S> edge_adjoint(V3<S> c, int axis, S dir, S d, S
     } else {
         dot = dir * (axis == 0 ? gv.x : (axis == 1 ? gv.y : gv.z));
     }
-    const S wc = clamp01<S>(w);
-    return Grad<S>{-(q.of(w) * dot), wc * gv.x, wc * gv.y, wc * gv.z};
+    const S g = -(q.of(w) * dot);
+    if (!DEF) return Grad<S>{g, S(0), S(0), S(0)};
+    const bool second = dir < S(0);
+    const S t = clamp01<S>(second ? w : q.of(iso - d)), wt = second ? t : S(1) - t;
+    return Grad<S>{g, wt * gv.x, wt * gv.y, wt * gv.z};
 }
 
 // Zeros p[a..b), by one wave: 16-byte stores between the aligned ends.

@@ -37,3 +37,75 @@ def test_nan_isovalue_extracts_nothing(dtype, dims):
     fx = diso_amd.FixedExtractor("mc", TDT[dtype], 10, 10)
     assert fx(sdf, isovalue=NAN)[2].tolist() == [0, 0, 0]
     assert fx(bad, isovalue=NAN)[2].tolist() == [0, 0, _lib.TOTAL_HAS_NAN]
+
+
+def _edge_terms(sdf, up, iso):
+    """The deform gradient of every crossing edge's two ends as src/cumc.cu:343-368,412-453 states it, in
+    numpy, padded grid: (1 - t) up and t up, with t clamped as min(max(0, t), 1) is in C (NaN gives 1)."""
+    dt = sdf.dtype
+    p = np.pad(sdf, 1, constant_values=dt.type(iso) + dt.type(1))
+    g = np.zeros((*p.shape, 3), np.float64)
+    inside = p >= iso
+    n = 0
+    X, Y, Z = (d - 1 for d in p.shape)
+    with np.errstate(all="ignore"):
+        for x in range(X):
+            for y in range(Y):
+                for z in range(Z):
+                    for a in range(3):
+                        q = (x + (a == 0), y + (a == 1), z + (a == 2))
+                        if inside[x, y, z] == inside[q]:
+                            continue
+                        d0, d1 = p[x, y, z], p[q]
+                        t = (dt.type(iso) - d0) / (d1 - d0)
+                        t = 0.0 if 0 > t else t
+                        t = t if t < 1 else 1.0
+                        g[x, y, z] += (1.0 - t) * up[n]
+                        g[q] += t * up[n]
+                        n += 1
+    assert n == up.shape[0]
+    return g[1:-1, 1:-1, 1:-1]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("recompute", [False, True])
+@pytest.mark.parametrize("kind", ["inf", "huge", "tiny"])
+def test_deform_gradients_of_extreme_samples(dtype, recompute, kind):
+    """An edge's two ends share its vertex's gradient as 1 - t and t whatever the samples: infinite ones,
+    and ones whose difference overflows or is denormal (its fp32 reciprocal then is zero or infinite, so t
+    is only held to [0, 1] and to the ends' sum there, and compared where a plain division gives it)."""
+    print(f"case extreme {kind} {np.dtype(dtype).name} recompute={recompute}", flush=True)
+    rng = np.random.default_rng(8)
+    sdf_np = rng.standard_normal((7, 6, 67))
+    if kind == "inf":
+        sdf_np[rng.random(sdf_np.shape) < 0.3] = np.inf
+        sdf_np[rng.random(sdf_np.shape) < 0.3] = -np.inf
+    else:
+        scale = {("huge", np.float32): 1.5e38, ("huge", np.float64): 8e307, ("tiny", np.float32): 1e-39,
+                 ("tiny", np.float64): 1e-309}[kind, dtype]
+        sdf_np = np.clip(sdf_np, -2, 2) * scale  # (finite; differences of "huge" ones overflow)
+    sdf_np = sdf_np.astype(dtype)
+    sdf = torch.tensor(sdf_np, device=DEV)
+    deform = torch.zeros((*sdf_np.shape, 3), dtype=TDT[dtype], device=DEV, requires_grad=True)
+    v, _ = diso_amd.DiffMC(TDT[dtype], recompute_backward=recompute)(sdf, deform, normalize=False)
+    up = rng.standard_normal(v.shape).astype(dtype)
+    v.backward(torch.tensor(up, device=DEV))
+    got = deform.grad.cpu().numpy()
+    assert np.isfinite(got).all()
+    want = _edge_terms(sdf_np, up.astype(np.float64), 0.0)
+    # (at most six terms per vertex, each within an ulp or two of its weight)
+    if kind == "inf" or dtype == np.float64:
+        assert np.abs(got - want).max() <= (1e-5 if dtype == np.float32 else 1e-13) * np.abs(want).max()
+    else:
+        whole = np.abs(got.astype(np.float64)[1:-1, 1:-1, 1:-1]).max()
+        assert whole <= 6 * np.abs(up).max()
+    # with the pad's samples stored, every edge has both ends in the grid: together they take all of `up`
+    ones = torch.tensor(np.ones_like(up), device=DEV)
+    big = torch.full(tuple(n + 2 for n in sdf_np.shape), 1.0, dtype=TDT[dtype], device=DEV)
+    big[1:-1, 1:-1, 1:-1] = sdf
+    d2 = torch.zeros((*big.shape, 3), dtype=TDT[dtype], device=DEV, requires_grad=True)
+    w, _ = diso_amd.DiffMC(TDT[dtype], recompute_backward=recompute)(big, d2, normalize=False)
+    assert w.shape == v.shape
+    w.backward(ones)
+    total = d2.grad.double().sum((0, 1, 2)).cpu().numpy()
+    assert np.abs(total - w.shape[0]).max() <= (1e-5 if dtype == np.float32 else 1e-12) * w.shape[0]
