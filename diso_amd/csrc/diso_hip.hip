@@ -44,6 +44,7 @@
 
 #include "diso_hip.h"
 #include "diso_bits.h"
+#include "diso_launch.h"
 #include "diso_scan_word.h"
 #include "diso_tables.h"
 
@@ -165,27 +166,12 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
     return v;
 }
 
-// Block index remap: the dispatcher deals consecutive workgroups round-robin to the 8 XCDs;
-// this gives each XCD a contiguous run of logical blocks so that neighbouring rows (which a
-// block re-reads as halo) share one XCD's L2.
-__device__ __forceinline__ int64_t xcd_block(int64_t bid, int64_t nb) {
-    int64_t q = nb / 8, r = nb % 8;
-    int64_t xcd = bid % 8, k = bid / 8;
-    return xcd * q + (xcd < r ? xcd : r) + k;
-}
+using diso_launch::stripe_blocks;
+using diso_launch::xcd_block;
+using diso_launch::xcd_stripe;
 
-// The same in kStripes turns: an XCD takes one of every eight stripes of consecutive blocks, so that
-// work that is uneven over the grid (a surface's faces) is spread over the XCDs while neighbouring
-// rows still mostly share one. The grid is padded to `stripe_blocks` blocks; returns a block >= nb for
-// the padding. The 256^3 noisy gather, in one turn (an eighth of the grid per XCD: the planes of a
-// box's face fall to one) 176 us, in 2, 4, 8, 16, 32 turns 170, 141, 135, 131, 132 us.
-constexpr int64_t kStripes = 16;
-__host__ __device__ __forceinline__ int64_t stripe_len(int64_t nb) { return (nb + 8 * kStripes - 1) / (8 * kStripes); }
-__host__ __device__ __forceinline__ int64_t stripe_blocks(int64_t nb) { return stripe_len(nb) * 8 * kStripes; }
-__device__ __forceinline__ int64_t xcd_stripe(int64_t bid, int64_t nb) {
-    const int64_t c = stripe_len(nb), k = bid / 8, turn = k / c;
-    return (turn * 8 + bid % 8) * c + (k - turn * c);
-}
+// The block's number in a launch of diso_launch::shape_of.
+__device__ __forceinline__ int64_t block_number() { return (int64_t)blockIdx.y * gridDim.x + blockIdx.x; }
 
 struct SegBase {
     int64_t v;  // first vertex (MC) / first quad (DMC) of the segment
@@ -593,7 +579,7 @@ template <typename S, bool BATCH>
 __global__ __launch_bounds__(kBlock) void mask_kernel(CountSrc<S> src, const BatchGrid<S> *__restrict__ grids,
                                                       Planes out, uint8_t *ctl) {
     const int lane = threadIdx.x % kWave;
-    const int64_t lo = ((int64_t)blockIdx.x * kWavesPerBlock + wave_id()) * kMaskTile;
+    const int64_t lo = (block_number() * kWavesPerBlock + wave_id()) * kMaskTile;
     const int64_t hi = lo + kMaskTile < src.nseg ? lo + kMaskTile : src.nseg;
     uint32_t *nan = &reinterpret_cast<CtlHeader *>(ctl)->nan;
     if (lo >= hi) return;
@@ -2251,7 +2237,7 @@ __global__ __launch_bounds__(kWave) void bwd_mc_kernel(In<S> in, const SegBase *
                                                        S *__restrict__ adj_sdf, S *__restrict__ adj_deform,
                                                        int tile, int64_t nblocks) {
     const SegCtx sc = seg_ctx(seg, planes_of(seg, in.geo.nseg));
-    const int64_t b = xcd_stripe(blockIdx.x, nblocks);
+    const int64_t b = xcd_stripe(block_number(), nblocks);
     if (b < nblocks) bwd_wave<S, DEF, RECOMP>(in, sc, b, tile, adj, adj_sdf, adj_deform);
 }
 
@@ -2409,7 +2395,8 @@ __device__ __forceinline__ void batch_units(const BatchGrid<S> *__restrict__ gri
                                             const int64_t *__restrict__ rf, int m, const SegBase *__restrict__ seg,
                                             const Planes &planes, const uint32_t *__restrict__ range, int64_t nblocks,
                                             int wave, int lane, T tables, F f) {
-    const int64_t b = xcd_block(blockIdx.x, nblocks);
+    if (block_number() >= nblocks) return;
+    const int64_t b = xcd_block(block_number(), nblocks);
     const int j = find_group(rf, m, b);
     const int gi = gl[j];
     const BatchGrid<S> &B = grids[gi];
@@ -2480,7 +2467,7 @@ __global__ __launch_bounds__(kWave) void bwd_batch_kernel(const BatchGrid<S> *__
                                                            const SegBase *__restrict__ seg,
                                                            Planes planes,
                                                            const S *__restrict__ ge, int64_t nblocks) {
-    const int64_t b = xcd_stripe(blockIdx.x, nblocks);
+    const int64_t b = xcd_stripe(block_number(), nblocks);
     if (b >= nblocks) return;
     const int j = find_group(rf, m, b);
     const BatchGrid<S> &G = grids[gl[j]];
@@ -2779,8 +2766,14 @@ int64_t count_blocks(int64_t nseg, int resident_per_cu) {
     return nb < 1 ? 1 : nb;
 }
 
-int64_t mask_blocks(int64_t nseg) {
-    return (nseg + kMaskTile * kWavesPerBlock - 1) / (kMaskTile * kWavesPerBlock);
+// The launch shape of at least `blocks` blocks whose kernel takes them by block_number().
+dim3 shape_of(int64_t blocks, int threads) {
+    const diso_launch::Shape s = diso_launch::shape_of(blocks, threads);
+    return dim3(s.x, s.y);
+}
+
+dim3 mask_shape(int64_t nseg) {
+    return shape_of((nseg + kMaskTile * kWavesPerBlock - 1) / (kMaskTile * kWavesPerBlock), kBlock);
 }
 
 template <typename S>
@@ -2804,7 +2797,7 @@ int launch_count(int algo, const void *sdf, double iso, const Geo &g, void *seg,
     (void)ctl_bytes;
     SegBase *sb = (SegBase *)seg;
     const Planes P = planes_of(sb, g.nseg);
-    hipLaunchKernelGGL((mask_kernel<S, false>), dim3((unsigned)mask_blocks(g.nseg)), dim3(kBlock), 0, st, src,
+    hipLaunchKernelGGL((mask_kernel<S, false>), mask_shape(g.nseg), dim3(kBlock), 0, st, src,
                        (const BatchGrid<S> *)nullptr, P, (uint8_t *)ctl);
     int rc = check_hip(hipGetLastError(), "mask kernel launch");
     if (rc) return rc;
@@ -2907,7 +2900,7 @@ int launch_backward(int algo, const void *sdf, const void *deform, double iso, i
         a.n = nfaces;
         a.flags = flags & ~DISO_FLAG_NORMALIZE;  // applied by the edge gradient kernel
     }
-    const dim3 grid((unsigned)stripe_blocks(nb)), block(kWave);
+    const dim3 grid = shape_of(stripe_blocks(nb), kWave), block(kWave);
     const bool rec = (flags & DISO_FLAG_RECOMPUTE) != 0;
     if (deform && rec)
         hipLaunchKernelGGL((bwd_mc_kernel<S, true, true>), grid, block, 0, st, in, sb, a, gs, gd, tile, nb);
@@ -3213,7 +3206,7 @@ int batch_count(diso_grid_t *grids, const BatchLayout &L, void *ws, void *ctl, h
     src.ngrids = L.n;
     src.nseg = L.nseg;
     src.recount_spins = (uint32_t)g_params.recount_spins;
-    hipLaunchKernelGGL((mask_kernel<S, true>), dim3((unsigned)mask_blocks(L.nseg)), dim3(kBlock), 0, st, src,
+    hipLaunchKernelGGL((mask_kernel<S, true>), mask_shape(L.nseg), dim3(kBlock), 0, st, src,
                        (const BatchGrid<S> *)P.desc, P.planes, (uint8_t *)ctl);
     if ((rc = check_hip(hipGetLastError(), "batch mask kernel launch"))) return rc;
     const int64_t nb = count_blocks(L.nseg, count_resident_per_cu<count_kernel<S, DISO_MC, true>>());
@@ -3261,7 +3254,7 @@ int batch_emit(const diso_grid_t *grids, const BatchLayout &L, void *ws, hipStre
     for (int k = 0; k < 4; ++k) {
         const int64_t nb = gr[k].blocks();
         if (!nb) continue;
-        const dim3 grid((unsigned)nb), block(kBlock);
+        const dim3 grid = shape_of(nb, kBlock), block(kBlock);
         const int32_t *gl = P.gl(L, k, w);
         const int64_t *rf = P.rf(L, k, w);
         const int m = gr[k].m();
@@ -3313,7 +3306,7 @@ int batch_backward(const diso_grid_t *grids, const BatchLayout &L, void *ws, voi
     for (int k = 0; k < 4; ++k) {
         const int64_t nb = gr[k].blocks();
         if (!nb) continue;
-        const dim3 grid((unsigned)stripe_blocks(nb));
+        const dim3 grid = shape_of(stripe_blocks(nb), kWave);
         const int32_t *gl = P.gl(L, k, w);
         const int64_t *rf = P.rf(L, k, w);
         const int m = gr[k].m();
