@@ -16,7 +16,7 @@ LIB_PATH = os.environ.get("DISO_AMD_LIB") or os.path.join(HERE, "libdiso_hip.so"
 SOURCES = [os.path.join(HERE, "csrc", "diso_hip.hip")]
 HEADERS = [os.path.join(ROOT, "include", "diso_hip.h"), os.path.join(HERE, "csrc", "diso_tables.h"),
            os.path.join(HERE, "csrc", "diso_scan_word.h"), os.path.join(HERE, "csrc", "diso_bits.h"),
-           os.path.join(HERE, "csrc", "diso_launch.h")]
+           os.path.join(HERE, "csrc", "diso_launch.h"), os.path.join(HERE, "csrc", "diso_host.h")]
 
 # Flags: gfx950 only; no FP contraction and correctly rounded division so results match an IEEE
 # evaluation of the reference's expressions; packed-fp32 instructions disabled.

@@ -33,7 +33,6 @@
 // backward uses one hardware reciprocal per edge (gradients are compared within a tolerance).
 #include <hip/hip_runtime.h>
 
-#include <sched.h>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -44,6 +43,7 @@
 
 #include "diso_hip.h"
 #include "diso_bits.h"
+#include "diso_host.h"
 #include "diso_launch.h"
 #include "diso_scan_word.h"
 #include "diso_tables.h"
@@ -2999,20 +2999,15 @@ Landing &landing() {
     return l;
 }
 
-// Waits until the count has written number `seq`. The stream's state is looked at only now and then
-// (it tells of a failed launch, or of work ahead in the stream that makes the wait long).
+// Waits until the count has written number `seq`; the stream's state tells of a failed launch.
 int wait_totals(const HostTotals *h, uint64_t seq, hipStream_t st) {
-    for (uint32_t spins = 1;; ++spins) {
-        if (__atomic_load_n(&h->seq, __ATOMIC_ACQUIRE) == seq) return DISO_OK;
-        if (spins % 4096 == 0) {
-            const hipError_t e = hipStreamQuery(st);
-            if (e != hipSuccess && e != hipErrorNotReady) return check_hip(e, "count pass");
-            if (e == hipSuccess && __atomic_load_n(&h->seq, __ATOMIC_ACQUIRE) != seq)
-                return fail(DISO_E_HIP, "count pass ended without totals");
-            if (spins > (1u << 16)) sched_yield();
-        }
-        __builtin_ia32_pause();
-    }
+    auto written = [&]() { return __atomic_load_n(&h->seq, __ATOMIC_ACQUIRE) == seq; };
+    return diso_host::wait_until(written, [&]() {
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady) return (int)DISO_OK;
+        if (e != hipSuccess) return check_hip(e, "count pass");
+        return written() ? (int)DISO_OK : fail(DISO_E_HIP, "count pass ended without totals");
+    });
 }
 
 // ---- batches

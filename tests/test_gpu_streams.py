@@ -1,6 +1,7 @@
 """One module on several streams, and extractions from several host threads (needs a GPU). A forward
 returns before its count kernel has ended, so what calls share must be ordered by more than the host."""
 import threading
+import time
 
 import pytest
 import torch
@@ -76,3 +77,28 @@ def test_extractions_from_several_threads():
         assert not errors, errors
         for (v, f), (w, x) in zip(got, want):
             assert torch.equal(v, w) and torch.equal(f, x)
+
+
+def test_a_long_wait_does_not_hold_a_core():
+    """With some 300 ms of work ahead in the stream, the waiting thread's own time stays a fraction."""
+    print("case long wait", flush=True)
+    sdf = _grids(1, (30, 31, 32), 80)[0]
+    mod = diso_amd.DiffMC()
+    want = mod(sdf)  # (the next call has a size estimate)
+    big = torch.ones(1 << 29, device=DEV)
+    torch.cuda.synchronize()
+    big.mul_(1.0)
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    for _ in range(10):
+        big.mul_(1.0)
+    torch.cuda.synchronize()
+    n = int(3.0 / (time.perf_counter() - t0)) + 1  # some 0.3 s of them
+    for _ in range(n):
+        big.mul_(1.0)
+    w0, c0 = time.perf_counter(), time.thread_time()
+    got = mod(sdf)
+    wall, own = time.perf_counter() - w0, time.thread_time() - c0
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert wall > 0.1, "the work ahead was too short for this test"
+    assert own < 0.3 * wall, (own, wall)

@@ -1,0 +1,82 @@
+"""The forward's host wait (diso_amd/csrc/diso_host.h), compiled with g++: a long wait sleeps instead of
+holding a core, a short one sees its word at once, and an error ends the wait."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = r"""
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+#include <atomic>
+#include <thread>
+#include "diso_host.h"
+using namespace diso_host;
+
+#define CHECK(c) do { if (!(c)) { printf("FAIL line %d: %s\n", __LINE__, #c); return 1; } } while (0)
+
+static int64_t cpu_ns() {
+    timespec t;
+    clock_gettime(CLOCK_THREAD_CPUTIME_ID, &t);
+    return (int64_t)t.tv_sec * 1000000000 + t.tv_nsec;
+}
+static void sleep_ns(int64_t ns) {
+    const timespec t{(time_t)(ns / 1000000000), (long)(ns % 1000000000)};
+    nanosleep(&t, nullptr);
+}
+
+// A wait for a word that another thread sets after `ns`: the wait's CPU time, and how late it saw it.
+static void timed(int64_t ns, int64_t *cpu, int64_t *late, int *troubles) {
+    std::atomic<int64_t> set{0};
+    std::thread t([&] { sleep_ns(ns); set.store(now_ns(), std::memory_order_release); });
+    const int64_t c0 = cpu_ns();
+    *troubles = 0;
+    wait_until([&] { return set.load(std::memory_order_acquire) != 0; }, [&] { ++*troubles; return 0; });
+    *late = now_ns() - set.load();
+    *cpu = cpu_ns() - c0;
+    t.join();
+}
+
+int main(int argc, char **argv) {
+    int64_t cpu, late;
+    int troubles;
+    if (!strcmp(argv[1], "long")) {
+        timed(400000000, &cpu, &late, &troubles);
+        printf("cpu %lld us, late %lld us, looks at the stream %d\n", (long long)cpu / 1000, (long long)late / 1000, troubles);
+        CHECK(cpu < 100000000 && troubles > 10);
+    } else if (!strcmp(argv[1], "short")) {
+        int64_t best = 1 << 30;  // (the machine may be busy: the best of some)
+        for (int i = 0; i < 20; ++i) {
+            timed(200000, &cpu, &late, &troubles);
+            best = late < best ? late : best;
+        }
+        printf("late %lld ns\n", (long long)best);
+        CHECK(best < 50000);
+        CHECK(wait_until([] { return true; }, [] { return 7; }) == 0);
+    } else {
+        int n = 0;
+        CHECK(wait_until([] { return false; }, [&] { return ++n == 3 ? 7 : 0; }) == 7 && n == 3);
+    }
+    printf("ok\n");
+    return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    d = tmp_path_factory.mktemp("wait")
+    src, exe = d / "wait.cpp", d / "wait"
+    src.write_text(PROGRAM)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-I" + os.path.join(ROOT, "diso_amd", "csrc"), "-o", str(exe),
+                    str(src)], check=True)
+    return str(exe)
+
+
+@pytest.mark.parametrize("what", ["long", "short", "error"])
+def test_host_wait(program, what):
+    r = subprocess.run([program, what], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and "ok" in r.stdout, r.stdout[-500:] + r.stderr[-500:]
