@@ -2981,17 +2981,19 @@ int read_totals(const Geo &g, const void *seg, diso_totals_t *t, hipStream_t st,
     return DISO_OK;
 }
 
-// This thread's landing place for totals written by the count kernel, kept for the life of the
-// process, and the number of its next call (a kernel of an abandoned call writes an old number).
+// This thread's landing place for totals written by the count kernel (handed to a later thread when
+// this one ends), and the number of its next call (a kernel of an abandoned call writes an old number).
 struct Landing {
     HostTotals *host = nullptr;
     uint64_t seq = 0;
 };
+Landing *make_landing() { return new Landing; }
 Landing &landing() {
-    thread_local Landing l;
+    Landing &l = *diso_host::thread_object<Landing, make_landing>();
     if (!l.host) {
         void *q = nullptr;
-        if (hipHostMalloc(&q, sizeof(HostTotals), hipHostMallocCoherent | hipHostMallocMapped) == hipSuccess) {
+        if (hipHostMalloc(&q, sizeof(HostTotals), hipHostMallocCoherent | hipHostMallocMapped | hipHostMallocPortable) ==
+            hipSuccess) {
             l.host = (HostTotals *)q;
             l.host->seq = 0;
         }

@@ -1,10 +1,14 @@
-// diso_host.h - how a host thread waits for a word that a kernel writes.
+// diso_host.h - host-side helpers of the waiting forward: how a thread waits for a word that a kernel
+// writes, and objects that host threads take turns to own.
 //
-// Plain C++, so it is testable on the CPU.
+// Plain C++, so both are testable on the CPU.
 #pragma once
 
 #include <stdint.h>
 #include <time.h>
+
+#include <mutex>
+#include <vector>
 
 namespace diso_host {
 
@@ -40,6 +44,37 @@ inline int wait_until(Done done, Trouble trouble) {
             looks = 1023;  // one look, then here again
         }
     }
+}
+
+// An object per host thread, taken over by a later thread when its owner ends: as many are made as
+// threads have held one at a time.
+template <class T, T *(*Make)()>
+T *thread_object() {
+    struct Pool {
+        std::mutex mu;
+        std::vector<T *> free;
+    };
+    static Pool *const pool = new Pool;  // (outlives every thread)
+    struct Holder {
+        T *obj = nullptr;
+        ~Holder() {
+            if (!obj) return;
+            std::lock_guard<std::mutex> lock(pool->mu);
+            pool->free.push_back(obj);
+        }
+    };
+    static thread_local Holder mine;
+    if (!mine.obj) {
+        {
+            std::lock_guard<std::mutex> lock(pool->mu);
+            if (!pool->free.empty()) {
+                mine.obj = pool->free.back();
+                pool->free.pop_back();
+            }
+        }
+        if (!mine.obj) mine.obj = Make();
+    }
+    return mine.obj;
 }
 
 }  // namespace diso_host

@@ -1,5 +1,6 @@
-"""The forward's host wait (diso_amd/csrc/diso_host.h), compiled with g++: a long wait sleeps instead of
-holding a core, a short one sees its word at once, and an error ends the wait."""
+"""The forward's host wait and its per-thread landing places (diso_amd/csrc/diso_host.h), compiled with
+g++: a long wait sleeps instead of holding a core, a short one sees its word at once, an error ends the
+wait, and threads that come and go do not each leave an object behind."""
 import os
 import subprocess
 
@@ -40,6 +41,13 @@ static void timed(int64_t ns, int64_t *cpu, int64_t *late, int *troubles) {
     t.join();
 }
 
+static std::atomic<int> made{0};
+struct Obj {
+    int n;
+};
+static Obj *make() { return new Obj{++made}; }
+static Obj *get() { return thread_object<Obj, make>(); }
+
 int main(int argc, char **argv) {
     int64_t cpu, late;
     int troubles;
@@ -56,9 +64,21 @@ int main(int argc, char **argv) {
         printf("late %lld ns\n", (long long)best);
         CHECK(best < 50000);
         CHECK(wait_until([] { return true; }, [] { return 7; }) == 0);
-    } else {
+    } else if (!strcmp(argv[1], "error")) {
         int n = 0;
         CHECK(wait_until([] { return false; }, [&] { return ++n == 3 ? 7 : 0; }) == 7 && n == 3);
+    } else {
+        Obj *const main_obj = get();
+        CHECK(main_obj == get() && made == 1);
+        for (int i = 0; i < 100; ++i)
+            std::thread([&] { Obj *o = get(); if (o == main_obj || o != get()) abort(); }).join();
+        CHECK(made == 2);  // the main thread's, and one that a hundred threads took in turn
+        std::atomic<int> in{0};
+        std::vector<std::thread> ts;
+        for (int i = 0; i < 8; ++i)
+            ts.emplace_back([&] { Obj *o = get(); ++in; while (in < 8) std::this_thread::yield(); if (o != get()) abort(); });
+        for (auto &t : ts) t.join();
+        CHECK(made == 9);  // eight at a time, besides the main thread's
     }
     printf("ok\n");
     return 0;
@@ -76,7 +96,7 @@ def program(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize("what", ["long", "short", "error"])
-def test_host_wait(program, what):
+@pytest.mark.parametrize("what", ["long", "short", "error", "threads"])
+def test_wait_and_thread_objects(program, what):
     r = subprocess.run([program, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and "ok" in r.stdout, r.stdout[-500:] + r.stderr[-500:]
