@@ -3508,8 +3508,9 @@ int diso_extract(int algo, int dtype, const void *sdf, const void *deform, int64
     rc = f32 ? launch_count<float>(algo, sdf, iso, g, seg, ctl, ctl_bytes, st, land.host, seq)
              : launch_count<double>(algo, sdf, iso, g, seg, ctl, ctl_bytes, st, land.host, seq);
     if (rc) return rc;
-    rc = f32 ? launch_emit<float>(algo, sdf, deform, iso, flags, g, seg, verts, vert_capacity, faces, face_capacity, vinfo, st)
-             : launch_emit<double>(algo, sdf, deform, iso, flags, g, seg, verts, vert_capacity, faces, face_capacity, vinfo, st);
+    if (vert_capacity || face_capacity)  // (else nothing could be written)
+        rc = f32 ? launch_emit<float>(algo, sdf, deform, iso, flags, g, seg, verts, vert_capacity, faces, face_capacity, vinfo, st)
+                 : launch_emit<double>(algo, sdf, deform, iso, flags, g, seg, verts, vert_capacity, faces, face_capacity, vinfo, st);
     const int rw = wait_totals(land.host, seq, st);
     if (rc || rw) return rc ? rc : rw;
     const HostTotals h = *land.host;

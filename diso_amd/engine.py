@@ -105,7 +105,8 @@ class Extractor:
         got = self._need.get(key)
         if got is None:
             L = _lib.lib()
-            got = (L.diso_seg_bytes(*dims, flags & ~_lib.FLAG_RECOMPUTE), L.diso_seg_bytes(*dims, flags),
+            seg = L.diso_seg_bytes(*dims, flags & ~_lib.FLAG_RECOMPUTE)
+            got = (seg, L.diso_seg_bytes(*dims, flags) if flags & _lib.FLAG_RECOMPUTE else seg,
                    L.diso_ctl_bytes(*dims, flags))
             if min(got) < 0:
                 _lib.check(min(got), "workspace sizing")
@@ -114,14 +115,14 @@ class Extractor:
             self._need[key] = got
         return got
 
-    def ctl_for(self, device, dims, flags, capturing=False):
+    def ctl_for(self, device, dims, flags, capturing=False, stream=None):
         """The control block of the current stream. One per stream, because consecutive calls may use
         it only in stream order: a forward returns as soon as its totals are known, while blocks of
         its count may still be reading and clearing the block's words. A capture takes the device's
         first block, which is kept as long as this object (or, without one, a block that each replay
         clears)."""
         need = self._sizes(dims, flags)[2]
-        key = (device.index, _stream(device).value)
+        key = (device.index, (_stream(device) if stream is None else stream).value)
         if not capturing:
             ctl = self._ctl.get(key)
             if ctl is not None and ctl.numel() >= need:
@@ -167,27 +168,28 @@ class Extractor:
         dev = grid.device
         key = (dev.index, dims, flags)
         guess = self._guess.get(key)
-        if guess is None:
-            counted = self.count(grid, iso, flags)
-            self._remember(key, counted.n_verts, counted.n_faces)
-            return counted
         nseg = self._sizes(dims, flags)[0]
         seg = torch.empty(nseg, dtype=torch.uint8, device=dev)
-        ctl = self.ctl_for(dev, dims, flags)
+        stream = _stream(dev)
+        ctl = self.ctl_for(dev, dims, flags, stream=stream)
         dmc = self.algo == _lib.DMC
-        vcap, fcap = guess[0] + guess[0] // 4 + 1024, guess[1] + guess[1] // 4 + 1024
-        verts = torch.empty((vcap, 3), dtype=self.dtype, device=dev)
-        faces = torch.empty((fcap, 4 if dmc else 3), dtype=torch.int64 if flags & _lib.FLAG_INDEX64 else torch.int32,
-                            device=dev)
-        vinfo = torch.empty(vcap, dtype=torch.uint8, device=dev) if dmc else None
+        vcap = fcap = 0
+        verts = faces = vinfo = None
+        if guess is not None:
+            vcap, fcap = guess[0] + guess[0] // 4 + 1024, guess[1] + guess[1] // 4 + 1024
+            verts = torch.empty((vcap, 3), dtype=self.dtype, device=dev)
+            faces = torch.empty((fcap, 4 if dmc else 3),
+                                dtype=torch.int64 if flags & _lib.FLAG_INDEX64 else torch.int32, device=dev)
+            vinfo = torch.empty(vcap, dtype=torch.uint8, device=dev) if dmc else None
         tot = _lib.Totals()
         rc = _lib.lib().diso_extract(self.algo, self.code, grid.data_ptr(), 0 if deform is None else deform.data_ptr(),
                                      *dims, iso, flags, seg.data_ptr(), nseg, ctl.data_ptr(), ctl.numel(),
-                                     verts.data_ptr(), vcap, faces.data_ptr(), fcap,
-                                     vinfo.data_ptr() if dmc else 0, tot, _stream(dev))
+                                     0 if verts is None else verts.data_ptr(), vcap,
+                                     0 if faces is None else faces.data_ptr(), fcap,
+                                     0 if vinfo is None else vinfo.data_ptr(), tot, stream)
         _lib.check(rc, "extraction")
         counted = Counted(seg, tot, dims, iso, flags)
-        if tot.n_verts <= vcap and tot.n_faces <= fcap:
+        if verts is not None and tot.n_verts <= vcap and tot.n_faces <= fcap:
             counted.spec = (verts, faces, vinfo)
         self._remember(key, tot.n_verts, tot.n_faces)
         return counted

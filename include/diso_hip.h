@@ -143,7 +143,7 @@ int diso_emit(int algo, int dtype, const void *sdf, const void *deform, int64_t 
  * suffice (an estimate from an earlier grid): enqueues diso_count and diso_emit and returns as soon
  * as the totals are known, which the counting pass writes to host memory itself, while the emission
  * may still run. If the totals exceed the capacities nothing has been written: call diso_emit with
- * larger buffers. The reference reads its counts back with three blocking copies (src/cumc.cu:651-723).
+ * larger buffers. With both capacities zero (no estimate yet) only the totals are taken. The reference reads its counts back with three blocking copies (src/cumc.cu:651-723).
  * Waits for the host, so it cannot be captured in a graph. On return the counting pass may still be
  * using `ctl` (and the emission `seg`): their next use must be ordered after it, on the same stream
  * or by an event. */

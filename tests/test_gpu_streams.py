@@ -102,3 +102,21 @@ def test_a_long_wait_does_not_hold_a_core():
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     assert wall > 0.1, "the work ahead was too short for this test"
     assert own < 0.3 * wall, (own, wall)
+
+
+def test_first_forward_takes_written_totals(monkeypatch):
+    """A module's first forward on a size has no estimate to emit with, but waits for its totals as later
+    ones do: no copy, no stream synchronisation (which made first calls slower than later ones)."""
+    print("case first forward", flush=True)
+    sdf = _grids(1, (12, 13, 14), 90)[0]
+    monkeypatch.setattr(diso_amd.engine.Extractor, "count", None)  # the pass that copies and synchronises
+    for algo, make, kw in (("mc", diso_amd.DiffMC, {}), ("dmc", diso_amd.DiffDMC, {"return_quads": True})):
+        for recompute in (False, True):
+            mod = make(recompute_backward=recompute)
+            for _ in range(2):
+                v, f = mod(sdf, **kw)
+                check_against_oracle(algo, sdf.cpu().numpy(), None, v, f)
+        empty = make()
+        for _ in range(2):
+            assert empty(torch.ones_like(sdf), **kw)[0].shape == (0, 3)
+            assert empty(torch.ones((1, 1, 1), device=DEV), **kw)[0].shape == (0, 3)
