@@ -459,16 +459,6 @@ __device__ __forceinline__ void st_relaxed(uint64_t *p, uint64_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__device__ __forceinline__ int64_t wave_incl64(int64_t v) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-        int64_t u = __shfl_up(v, o, kWave);
-        if (lane >= o) v += u;
-    }
-    return v;
-}
-
 // What a count launch classifies: one grid (`in`, algorithm ALGO), or (BATCH) the concatenated
 // segments of several grids, each with its own descriptor; then per-grid sample flags are
 // or-ed into gflags[grid] (zero on entry) and the scan runs over all segments in order.
@@ -985,11 +975,6 @@ __device__ __forceinline__ void store_quad(void *__restrict__ faces, int64_t q, 
             for (int j = 0; j < 4; ++j) put(f + j, (int32_t)(base + rel[j]));
         }
     }
-}
-
-__device__ __forceinline__ int64_t load_index(const void *__restrict__ faces, int64_t i, int flags) {
-    return (flags & DISO_FLAG_INDEX64) ? reinterpret_cast<const int64_t *>(faces)[i]
-                                       : (int64_t) reinterpret_cast<const int32_t *>(faces)[i];
 }
 
 template <typename S>
@@ -2788,13 +2773,12 @@ In<S> make_in(const void *sdf, const void *deform, double iso, const Geo &g) {
 }
 
 template <typename S>
-int launch_count(int algo, const void *sdf, double iso, const Geo &g, void *seg, void *ctl,
-                 int64_t ctl_bytes, hipStream_t st, HostTotals *host = nullptr, uint64_t seq = 0) {
+int launch_count(int algo, const void *sdf, double iso, const Geo &g, void *seg, void *ctl, hipStream_t st,
+                 HostTotals *host = nullptr, uint64_t seq = 0) {
     CountSrc<S> src{};
     src.in = make_in<S>(sdf, nullptr, iso, g);
     src.nseg = g.nseg;
     src.recount_spins = (uint32_t)g_params.recount_spins;
-    (void)ctl_bytes;
     SegBase *sb = (SegBase *)seg;
     const Planes P = planes_of(sb, g.nseg);
     hipLaunchKernelGGL((mask_kernel<S, false>), mask_shape(g.nseg), dim3(kBlock), 0, st, src,
@@ -3409,8 +3393,8 @@ int diso_count(int algo, int dtype, const void *sdf, int64_t X, int64_t Y, int64
         return fail(DISO_E_CAPACITY, "ctl workspace too small: %lld < %lld bytes", (long long)ctl_bytes,
                     (long long)ctl_bytes_for(g));
     hipStream_t st = (hipStream_t)stream;
-    rc = dtype == DISO_F32 ? launch_count<float>(algo, sdf, iso, g, seg, ctl, ctl_bytes, st)
-                           : launch_count<double>(algo, sdf, iso, g, seg, ctl, ctl_bytes, st);
+    rc = dtype == DISO_F32 ? launch_count<float>(algo, sdf, iso, g, seg, ctl, st)
+                           : launch_count<double>(algo, sdf, iso, g, seg, ctl, st);
     if (rc) return rc;
     if (totals_host) {
         rc = read_totals(g, seg, totals_host, st);
@@ -3438,8 +3422,8 @@ int diso_count_noalloc(int algo, int dtype, const void *sdf, int64_t X, int64_t 
     void *ctl = nullptr;
     rc = noalloc_ctl(st, &ctl);
     if (rc) return rc;
-    rc = dtype == DISO_F32 ? launch_count<float>(algo, sdf, iso, g, seg, ctl, kNoallocCtlBytes, st)
-                           : launch_count<double>(algo, sdf, iso, g, seg, ctl, kNoallocCtlBytes, st);
+    rc = dtype == DISO_F32 ? launch_count<float>(algo, sdf, iso, g, seg, ctl, st)
+                           : launch_count<double>(algo, sdf, iso, g, seg, ctl, st);
     if (rc) return rc;
     if (totals_host) {
         rc = read_totals(g, seg, totals_host, st, false);
@@ -3505,8 +3489,8 @@ int diso_extract(int algo, int dtype, const void *sdf, const void *deform, int64
     if (!land.host) return fail(DISO_E_HIP, "pinned allocation failed");
     const uint64_t seq = ++land.seq;
     const bool f32 = dtype == DISO_F32;
-    rc = f32 ? launch_count<float>(algo, sdf, iso, g, seg, ctl, ctl_bytes, st, land.host, seq)
-             : launch_count<double>(algo, sdf, iso, g, seg, ctl, ctl_bytes, st, land.host, seq);
+    rc = f32 ? launch_count<float>(algo, sdf, iso, g, seg, ctl, st, land.host, seq)
+             : launch_count<double>(algo, sdf, iso, g, seg, ctl, st, land.host, seq);
     if (rc) return rc;
     if (vert_capacity || face_capacity)  // (else nothing could be written)
         rc = f32 ? launch_emit<float>(algo, sdf, deform, iso, flags, g, seg, verts, vert_capacity, faces, face_capacity, vinfo, st)

@@ -109,3 +109,66 @@ def test_deform_gradients_of_extreme_samples(dtype, recompute, kind):
     w.backward(ones)
     total = d2.grad.double().sum((0, 1, 2)).cpu().numpy()
     assert np.abs(total - w.shape[0]).max() <= (1e-5 if dtype == np.float32 else 1e-12) * w.shape[0]
+
+
+def _crossing_vertices(sdf, iso):
+    """Marching Cubes vertices of a padded grid in linear order, x, y, z edges of each position in turn: an
+    edge crosses where one end is >= iso and the other < iso, which no NaN is."""
+    dt = sdf.dtype
+    p = np.pad(sdf, 1, constant_values=dt.type(iso) + dt.type(1))
+    out = []
+    for x, y, z in np.ndindex(*(d - 1 for d in p.shape)):
+        for a in range(3):
+            d0, d1 = p[x, y, z], p[x + (a == 0), y + (a == 1), z + (a == 2)]
+            if (d0 >= iso and d1 < iso) or (d0 < iso and d1 >= iso):
+                v = np.array([x, y, z], dt)
+                v[a] += ((v[a] + dt.type(1)) - v[a]) * ((dt.type(iso) - d0) / (d1 - d0))
+                out.append(v - dt.type(1))
+    return np.array(out, dt).reshape(-1, 3)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("share", [0.0, 0.03, 0.6])  # (0: one sample)
+def test_nan_samples_where_nothing_raises(dtype, share):
+    """FixedExtractor leaves the NaN flag to its caller. NaN samples are outside, edges that end in one do
+    not cross; stored and recomputed classification agree, and a clean grid after it is extracted clean."""
+    from oracle import oracle as O
+    from tests.torch_counts import expected_counts
+
+    print(f"case nan samples {np.dtype(dtype).name} {share}", flush=True)
+    rng = np.random.default_rng(12)
+    dims = (9, 8, 70)
+    clean = rng.standard_normal(dims).astype(dtype)
+    bad = clean.copy()
+    bad[rng.random(dims) < share] = NAN
+    bad[4, 4, 63] = NAN
+    counts = expected_counts(torch.tensor(bad), {k: torch.tensor(t, dtype=torch.int64) for k, t in O.expand_tables().items()})
+    want = _crossing_vertices(bad, 0.0)
+    n = 4 * clean.size
+    for algo in ("mc", "dmc"):
+        outs = []
+        for recompute in (False, True):
+            fx = diso_amd.FixedExtractor(algo, TDT[dtype], 2 * n, 3 * n, recompute_backward=recompute)
+            for k in range(3):  # bad, clean, bad: through one control block
+                s = torch.tensor(clean if k == 1 else bad, device=DEV, requires_grad=True)
+                v, f, c = fx(s, normalize=False)
+                nv, nf, flags = c.tolist()
+                v.backward(torch.ones_like(v))
+                if k == 1:
+                    assert not flags & _lib.TOTAL_HAS_NAN
+                    mod = diso_amd.DiffMC(TDT[dtype]) if algo == "mc" else diso_amd.DiffDMC(TDT[dtype])
+                    s2 = torch.tensor(clean, device=DEV, requires_grad=True)
+                    w, g = mod(s2, normalize=False, **({} if algo == "mc" else {"return_quads": True}))
+                    w.backward(torch.ones_like(w))
+                    assert torch.equal(v[:nv], w) and torch.equal(f[:nf], g) and torch.equal(s.grad, s2.grad)
+                    continue
+                assert flags & _lib.TOTAL_HAS_NAN
+                if algo == "mc":
+                    assert nv == want.shape[0] and nf == counts[1]
+                    assert np.array_equal(v[:nv].detach().cpu().numpy(), want)
+                else:
+                    assert nv == counts[2] and nf == want.shape[0] and torch.isfinite(v[:nv]).all()
+                outs.append((v[:nv].detach(), f[:nf], s.grad))
+        for o in outs[1:]:
+            assert all(torch.equal(x, y) for x, y in zip(o, outs[0]))
+            assert torch.isfinite(o[2]).all()
