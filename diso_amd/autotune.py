@@ -8,8 +8,8 @@ together; batched backward: each grid's own run length). Results never depend on
 the parameters; speed does, by device and grid size.
 
 `tune()` times, per bucket, the count launches of DiffMC + DiffDMC for every count-blocks choice
-and their emission + backward launches for every run length (the two parameters act on different
-kernels, so they are searched independently), on a rounded box with noise and a deformation at
+and their emission + backward launches for every run length with a gather tile of its own (the two
+parameters act on different kernels, so they are searched independently), on a rounded box with noise and a deformation at
 the bucket's size. It applies the fastest and can save them to tuning.json under the device name;
 `load()` (called when the library is first loaded) applies the saved choice.
 
@@ -25,7 +25,7 @@ from . import _lib
 
 TUNING_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuning.json")
 BUCKET_SIZES = (32, 64, 128, 256, 512)  # representative cubic grid per bucket (bucket b: index b)
-RUNS = (1, 2, 4, 8, 16, 32, 64)
+RUNS = (4, 8, 16, 32)  # the run lengths with tiles of their own (1, 2, 4, 8 segments a wave)
 COUNT_BLOCKS_PER_CU = (1, 2, 3, 4)
 _applied = {"source": "library defaults"}
 
@@ -171,6 +171,13 @@ def _bucket_launches(n, dev):
     return count, emit_backward
 
 
+def _choose(times):
+    """The smallest value whose time is within 1 % of the fastest's (runs of one value differ by that
+    much; of two equal ones the smaller is the better one for the smaller grids of the bucket)."""
+    limit = 1.01 * min(times.values())
+    return min(k for k, t in times.items() if t <= limit)
+
+
 def tune(sizes=BUCKET_SIZES, reps=10, save=False, path=TUNING_FILE, verbose=True):
     """Per bucket, the count-blocks choice with the fastest MC + DMC count launches and the run
     length with the fastest MC + DMC emission + backward launches (GPU time of graph replays,
@@ -192,7 +199,7 @@ def tune(sizes=BUCKET_SIZES, reps=10, save=False, path=TUNING_FILE, verbose=True
         for r in RUNS:
             _set(_lib.PARAM_RUN, b, r, "set run length")
             t_run[r] = _gpu_ms(emit_backward, reps, inner)
-        best_c, best_r = min(t_cpc, key=t_cpc.get), min(t_run, key=t_run.get)
+        best_c, best_r = _choose(t_cpc), _choose(t_run)
         _set(_lib.PARAM_COUNT_BLOCKS_PER_CU, b, best_c, "set count blocks per CU")
         _set(_lib.PARAM_RUN, b, best_r, "set run length")
         table[key] = {"run": best_r, "count_blocks_per_cu": best_c}

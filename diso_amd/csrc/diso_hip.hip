@@ -1811,7 +1811,10 @@ __device__ __forceinline__ void fill_zero(S *__restrict__ p, int64_t a, int64_t 
 // touched vertices at a time in turn (a tile of a surface that runs along z holds up to 512). On
 // 256^3 noisy / 203x256x181 smooth: tiles of 8 in one part 131 / 64 us, in two 127 / 60, in four 148 /
 // 64; tiles of 4 in one part 129 / 60, of 16 149 / 83; groups of 64, 32, 16 segments 127 / 60,
-// 128 / 55, 132 / 57. (A recomputing wave does not share a tile: each would recompute the planes.)
+// 128 / 55, 132 / 57. (A recomputing wave does not share a tile: each would recompute the planes. A tile
+// of one segment has no second 64 vertices.) Small grids want smaller tiles (the tuned run lengths): one
+// wave's chain of chunks is the kernel's time there. 32^3 noisy, tiles of 1, 2, 4, 8: 5.2, 6.3, 7.0, 10.1
+// us; 64^3 19.9, 19.9, 11.4, 11.4.
 constexpr int kBwdTile = 8;
 constexpr int kBwdGroup = 32;
 template <bool RECOMP>
@@ -2206,7 +2209,7 @@ template <typename S, bool DEF, bool RECOMP>
 __device__ __forceinline__ void bwd_wave(const In<S> &in, const SegCtx &sc, int64_t k, int tile, const AdjIn<S> &adj,
                                          S *__restrict__ adj_sdf, S *__restrict__ adj_deform) {
     __shared__ BwdLds<S> s_lds;
-    const int lane = threadIdx.x, parts = kBwdParts<RECOMP>, per = kBwdGroup / tile * parts + 1;
+    const int lane = threadIdx.x, parts = tile > 1 ? kBwdParts<RECOMP> : 1, per = kBwdGroup / tile * parts + 1;
     const int64_t group = k / per;
     const int i = (int)(k - group * per);
     if (i == 0) {
@@ -2643,8 +2646,8 @@ int check_hip(hipError_t e, const char *what) {
     return fail(DISO_E_HIP, "%s: %s", what, hipGetErrorString(e));
 }
 
-// Launch parameters (diso_set_param, diso_set_bucket_param): emission / backward run length and
-// count blocks per CU, each per size bucket, and the recount spins. A launch takes the bucket of
+// Launch parameters (diso_set_param, diso_set_bucket_param): the segments that four waves of the
+// backward take and count blocks per CU, each per size bucket, and the recount spins. A launch takes the bucket of
 // its segment count (a batched launch: the segments of all its grids); the bucket limits lie
 // between the segment counts of cubic grids of 32, 64, 128, 256 and 512 samples per side with
 // the virtual pad (1,156 / 8,712 / 50,700 / 332,820 / 2,377,764 segments).
@@ -2805,8 +2808,9 @@ int bwd_tile_of(int64_t nseg) {
     return t;
 }
 int64_t bwd_blocks(int64_t nseg, bool recompute) {
-    const int parts = recompute ? kBwdParts<true> : kBwdParts<false>;
-    return (nseg + kBwdGroup - 1) / kBwdGroup * (kBwdGroup / bwd_tile_of(nseg) * parts + 1);
+    const int tile = bwd_tile_of(nseg);
+    const int parts = tile == 1 ? 1 : (recompute ? kBwdParts<true> : kBwdParts<false>);
+    return (nseg + kBwdGroup - 1) / kBwdGroup * (kBwdGroup / tile * parts + 1);
 }
 
 template <typename S>

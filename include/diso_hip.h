@@ -225,15 +225,16 @@ int diso_batch_backward(int dtype, const diso_grid_t *grids, int n, void *seg, i
  * diso_amd/autotune.py picks them per machine and grid size). Results do not depend on them.
  * No counterpart in the reference, whose block size is a compile-time constant
  * (src/cumc.cu:93, BLOCK_SIZE 512).
- *  DISO_PARAM_RUN: segments per emission / backward block, 1..64 (default 32).
+ *  DISO_PARAM_RUN: segments that four waves of the backward take, 1..64 (default 32). A wave's
+ *    tile is a quarter of it, rounded down to a power of two, at least 1 and at most 8.
  *  DISO_PARAM_COUNT_BLOCKS_PER_CU: resident blocks per CU of the count pass, 1..4 (default 4).
  *  DISO_PARAM_RECOUNT_SPINS: reads of a predecessor's unpublished aggregate before a count block
  *    counts that range itself, 0..2^20 (default 8192; 0 counts every predecessor not already
  *    published, which tests use to exercise that path).
  * The first two have one value per size bucket. A launch takes the bucket of its segment count
- * (a batched count: of all its grids together; a batched emission or backward: each grid its own
- * run length); buckets 0..4 hold grids of about 32^3, 64^3,
- * 128^3, 256^3 and 512^3 samples (limits 3,200 / 21,000 / 130,000 / 900,000 segments).
+ * (a batched count: of all its grids together; a batched backward: each grid its own run length);
+ * buckets 0..4 hold grids of about 32^3, 64^3, 128^3, 256^3 and 512^3 samples (limits 3,200 /
+ * 21,000 / 130,000 / 900,000 segments).
  * diso_set_param sets every bucket; diso_get_param returns bucket 3's value. */
 enum {
     DISO_PARAM_RUN = 0,
