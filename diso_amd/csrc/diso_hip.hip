@@ -990,8 +990,8 @@ __device__ __forceinline__ void store_vertex(S *__restrict__ verts, int64_t i, i
 // full on sparse surfaces too). A unit's cells are found from the segments between its first one and
 // the next unit's first one: lane i loads segment U0 + i (unit_load, a unit ahead) and each segment
 // with cells writes them to `list` at its place. Where more than 64 segments lie in between (a sparse
-// stretch), each lane searches its cell's segment instead. unit_cells returns the number of cells;
-// lane k < n gets cell k's segment (of the launch) and position in it, the other lanes a copy of one.
+// stretch), each lane searches its cell's segment instead. unit_cells returns the number of cells
+// (of the part of the unit that the load stands for); lane k < n gets cell k's segment (of the launch) and position in it, the other lanes a copy of one.
 struct UnitGrid {
     const SegBase *__restrict__ seg;  // launch-level arrays
     Planes P;
@@ -1017,13 +1017,17 @@ __device__ __forceinline__ int select64(uint64_t m, int r) {
 
 struct UnitLoad {
     uint32_t u;
+    int from, to;    // which of its cells
     int64_t U0, U1;  // first and last segment that can hold its cells
     uint64_t A;      // lane i: segment U0 + i
     uint16_t abase;
 };
-__device__ __forceinline__ UnitLoad unit_load(const UnitGrid &G, uint32_t u, uint32_t nunits, int lane) {
+__device__ __forceinline__ UnitLoad unit_load(const UnitGrid &G, uint32_t part, int split, uint32_t nunits, int lane) {
     UnitLoad r;
+    const uint32_t u = part >> split;
     r.u = u;
+    r.from = (int)(part & ((1u << split) - 1)) * (kWave >> split);
+    r.to = r.from + (kWave >> split);
     const int64_t a = G.P.unit[u], b = u + 1 < nunits ? (int64_t)G.P.unit[u + 1] : G.last;
     r.U0 = a > G.first ? a : G.first;
     r.U1 = b < G.last ? b : G.last;
@@ -1042,26 +1046,28 @@ __device__ __forceinline__ int unit_cells(const UnitGrid &G, const UnitLoad &U, 
         const uint64_t A = in ? U.A : 0ull;
         const int st = in ? (int)(int16_t)(uint16_t)(U.abase - c0) : 0;
         const int s0 = __builtin_amdgcn_readfirstlane(st);
-        const int k0 = s0 > 0 ? s0 : 0;  // cells of the unit that belong to the grid before (a batch)
+        const int k0 = s0 > U.from ? s0 : U.from;  // (in a batch, the first s0 cells belong to the grid before)
+        const int len = U.to - k0;
         int n = 0;
         for (uint64_t act = __ballot(A != 0); act; act &= act - 1) {
             const int j = (int)__builtin_ctzll(act);
             const uint64_t m = (uint64_t)readlane64((int64_t)A, j);
             const int at = __builtin_amdgcn_readlane(st, j) - k0;
-            if (at >= kWave - k0) break;
+            if (at >= len) break;
             const int k = at + lanes_below(m);
-            if (__builtin_amdgcn_inverse_ballot_w64(m) && k >= 0 && k < kWave - k0) list[k] = (uint16_t)(j << 6 | lane);
+            if (__builtin_amdgcn_inverse_ballot_w64(m) && k >= 0 && k < len) list[k] = (uint16_t)(j << 6 | lane);
             n = at + (int)__popcll(m);
         }
-        n = n < kWave - k0 ? n : kWave - k0;
+        n = n < len ? n : len;
+        if (n <= 0) return 0;
         wave_lds_sync();
-        const int w = n > 0 ? list[lane < n ? lane : n - 1] : 0;
+        const int w = list[lane < n ? lane : n - 1];
         *s_out = (uint32_t)(U0 + (w >> 6));
         *l_out = w & 63;
         wave_lds_sync();
         return n;
     }
-    const int s0 = (int)(int16_t)(uint16_t)(G.P.abase[U0] - c0), k0 = s0 > 0 ? s0 : 0;
+    const int s0 = (int)(int16_t)(uint16_t)(G.P.abase[U0] - c0), k0 = s0 > U.from ? s0 : U.from;
     const int c = k0 + lane;  // this lane's cell of the unit
     int64_t lo = U0, hi = U1;
     while (lo < hi) {  // the last segment whose cells start at or before c
@@ -1073,7 +1079,7 @@ __device__ __forceinline__ int unit_cells(const UnitGrid &G, const UnitLoad &U, 
     }
     const uint64_t A = G.P.za[lo].b;
     const int r = c - (int)(int16_t)(uint16_t)(G.P.abase[lo] - c0);
-    const uint64_t ok = __ballot(c < kWave && r < (int)__popcll(A));
+    const uint64_t ok = __ballot(c < U.to && r < (int)__popcll(A));
     const int n = (int)__popcll(ok);  // the valid lanes are the first ones
     const int l = (ok >> lane) & 1 ? select64(A, r) : 0;
     const int from = lane < n ? lane : 0;
@@ -1086,14 +1092,14 @@ __device__ __forceinline__ int unit_cells(const UnitGrid &G, const UnitLoad &U, 
 // load of the unit after (called where those loads should be issued: before the work's own stores,
 // which the in-order memory counter would otherwise put between them and their use).
 template <typename F>
-__device__ __forceinline__ void unit_loop(const UnitGrid &G, uint32_t first, uint32_t hi, uint32_t step, uint32_t nunits,
-                                          int lane, F work) {
+__device__ __forceinline__ void unit_loop(const UnitGrid &G, uint32_t first, uint32_t hi, uint32_t step, int split,
+                                          uint32_t nunits, int lane, F work) {
     if (first >= hi) return;  // wave-uniform
-    UnitLoad cur = unit_load(G, first, nunits, lane);
+    UnitLoad cur = unit_load(G, first, split, nunits, lane);
     for (uint32_t u = first;;) {
         const bool more = step < hi - u;
         const uint32_t un = more ? u + step : u;
-        cur = work(cur, [&]() { return unit_load(G, un, nunits, lane); });
+        cur = work(cur, [&]() { return unit_load(G, un, split, nunits, lane); });
         if (!more) break;
         u = un;
     }
@@ -1101,13 +1107,19 @@ __device__ __forceinline__ void unit_loop(const UnitGrid &G, uint32_t first, uin
 
 // The units of a launch as a wave goes through them: XCD x takes the x-th eighth, its waves in turn,
 // so that at any time an XCD's waves work on neighbouring cells (whose rows share its L2). The grid
-// has a multiple of eight blocks.
+// has a multiple of eight blocks. Where there are few units, the time is one wave's chain through one:
+// a unit is then cut in two or four, up to kFewParts parts in all (two waves per SIMD). 32^3 noisy, MC /
+// DMC 6.6 / 10.4 us whole and 5.7 / 7.8 so, 64^3 6.7 / 10.6 and 6.4 / 9.3; with up to 4096 parts 64^3 takes
+// 8.4 / 11.4.
+constexpr uint32_t kFewParts = 2048;
 template <typename F>
 __device__ __forceinline__ void for_units(const UnitGrid &G, uint32_t nunits, int64_t block, int64_t nblocks, int wave,
                                           int lane, F work) {
     const uint32_t xcd = (uint32_t)(block % 8), per = (uint32_t)(nblocks / 8) * kWavesPerBlock;
-    const uint32_t u0 = (uint32_t)((uint64_t)nunits * xcd / 8), u1 = (uint32_t)((uint64_t)nunits * (xcd + 1) / 8);
-    unit_loop(G, u0 + (uint32_t)(block / 8) * kWavesPerBlock + (uint32_t)wave, u1, per, nunits, lane, work);
+    const int split = nunits <= kFewParts / 4 ? 2 : (nunits <= kFewParts / 2 ? 1 : 0);
+    const uint64_t parts = (uint64_t)nunits << split;
+    const uint32_t u0 = (uint32_t)(parts * xcd / 8), u1 = (uint32_t)(parts * (xcd + 1) / 8);
+    unit_loop(G, u0 + (uint32_t)(block / 8) * kWavesPerBlock + (uint32_t)wave, u1, per, split, nunits, lane, work);
 }
 
 __device__ __forceinline__ int bit_at(uint64_t w, int l) {
@@ -2396,7 +2408,7 @@ __device__ __forceinline__ void batch_units(const BatchGrid<S> *__restrict__ gri
     const UnitGrid G{seg, planes, first, first + in.geo.nseg - 1, seg[first].v, seg[first].f};
     const OutCfg out{B.flags, B.vcap, B.fcap};
     const uint32_t nunits = *planes.nunits, hi = range[2 * gi + 1], step = (uint32_t)(rf[j + 1] - rf[j]) * kWavesPerBlock;
-    unit_loop(G, range[2 * gi] + (uint32_t)(b - rf[j]) * kWavesPerBlock + (uint32_t)wave, hi, step, nunits, lane,
+    unit_loop(G, range[2 * gi] + (uint32_t)(b - rf[j]) * kWavesPerBlock + (uint32_t)wave, hi, step, 0, nunits, lane,
               [&](const UnitLoad &U, auto next) { return f(in, G, B, out, U, next); });
 }
 
@@ -2825,11 +2837,14 @@ Norm<S> norm_of(const Geo &g) {
 }
 
 // Blocks of a unit emission whose cells number at most `cells` (a cell has at least one triangle /
-// patch, so a face / vertex capacity bounds them): a wave per unit, at most kUnitBlocksPerCU blocks
-// per CU (then each wave goes through several units), a multiple of the eight XCDs.
+// patch, so a face / vertex capacity bounds them): a wave per unit or part of one, at most
+// kUnitBlocksPerCU blocks per CU (then each wave goes through several units), a multiple of the eight
+// XCDs.
 constexpr int kUnitBlocksPerCU = 10;
 int64_t unit_blocks(int64_t cells) {
     int64_t nb = cells / (kWave * kWavesPerBlock) + 1;
+    constexpr int64_t few = kFewParts / kWavesPerBlock;  // (for_units may cut units in four)
+    if (nb < few) nb = 4 * nb < few ? 4 * nb : few;
     const int64_t most = (int64_t)cu_count() * kUnitBlocksPerCU;
     if (nb > most) nb = most;
     return (nb + 7) / 8 * 8;

@@ -91,3 +91,24 @@ def test_split_at_unit_edges(nq, idx):
     want, _, _ = O.split_quads(verts, quads)
     got = diso_amd.split_quads(torch.tensor(verts, device=DEV), torch.tensor(quads, dtype=idx, device=DEV))
     assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("algo", [O.MC, O.DMC])
+@pytest.mark.parametrize("n,units", [(20, (1, 512)), (36, (513, 1024)), (45, (1025, 4000))])
+def test_units_cut_in_parts(algo, n, units):
+    """White noise of which nearly every cell is active, at sizes whose units are cut in four, in two and
+    not at all."""
+    print(f"case parts algo={algo} n={n}", flush=True)
+    rng = np.random.default_rng(13)
+    sdf_np, def_np = rng.standard_normal((n, n, n)).astype(np.float32), (rng.random((n, n, n, 3)) * 0.6 - 0.3).astype(np.float32)
+    ins = np.pad(sdf_np, 1, constant_values=1) >= 0
+    cubes = [ins[i:n + 1 + i, j:n + 1 + j, k:n + 1 + k] for i in (0, 1) for j in (0, 1) for k in (0, 1)]
+    active = int((np.any(cubes, 0) & ~np.all(cubes, 0)).sum())
+    assert units[0] <= (active + 63) // 64 <= units[1]
+    ref = O.Extractor(algo, np.float32)
+    rv, rf = ref.forward(sdf_np, def_np, 0.0, True, return_quads=True)
+    mod = (diso_amd.DiffMC if algo == O.MC else diso_amd.DiffDMC)()
+    kw = {"return_quads": True} if algo == O.DMC else {}
+    for _ in range(2):  # without and with a size estimate: exact and larger capacities
+        v, f = mod(torch.tensor(sdf_np, device=DEV), torch.tensor(def_np, device=DEV), 0.0, **kw)
+        assert np.array_equal(f.cpu().numpy(), rf) and np.array_equal(v.cpu().numpy(), rv)
