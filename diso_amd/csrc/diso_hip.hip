@@ -591,12 +591,13 @@ __global__ __launch_bounds__(kBlock) void mask_kernel(CountSrc<S> src, const Bat
 }
 
 // An edge with a NaN end does not cross: takes such edges out of a segment's crossings (from the
-// samples; only called when the launch holds a NaN).
+// samples; only called when the launch holds a NaN). Each lane goes through its own segment's positions
+// with a crossing; through all 64 in turn, a NaN cost a 256^3 count 230 us more on any surface.
 template <typename S>
 __device__ __forceinline__ void drop_nan_edges(const In<S> &in, const SegPos &sp, uint64_t &X, uint64_t &Y, uint64_t &Z) {
 #pragma unroll 1
-    for (int l = 0; l < kWave; ++l) {
-        const int z = sp.chunk * kWave + l;
+    for (uint64_t todo = X | Y | Z; todo; todo &= todo - 1) {
+        const int l = (int)__builtin_ctzll(todo), z = sp.chunk * kWave + l;
         const S a = sample(in, sp.px, sp.py, z), x = sample(in, sp.px + 1, sp.py, z), y = sample(in, sp.px, sp.py + 1, z),
                 u = sample(in, sp.px, sp.py, z + 1);
         X &= ~((uint64_t)(a != a || x != x) << l);
