@@ -144,54 +144,53 @@ class Extractor:
             self._ctl[key] = ctl
         return ctl
 
-    def count(self, grid, iso, flags):
-        dims = tuple(int(d) for d in grid.shape)
-        L = _lib.lib()
-        nseg = self._sizes(dims, flags)[0]
-        seg = torch.empty(nseg, dtype=torch.uint8, device=grid.device)
-        ctl = self.ctl_for(grid.device, dims, flags)
-        tot = _lib.Totals()
-        rc = L.diso_count(self.algo, self.code, _ptr(grid), *dims, float(iso), flags, _ptr(seg), nseg,
-                          _ptr(ctl), ctl.numel(), ctypes.byref(tot), _stream(grid.device))
-        _lib.check(rc, "count pass")
-        return Counted(seg, tot, dims, float(iso), flags)
-
-    def count_speculative(self, grid, deform, iso, flags):
-        """The counting pass, and, when an earlier call on a grid of these dims gives a size
-        estimate, the emission queued right behind it into buffers of that size plus a margin
-        (diso_extract): the host then waits only for the counts, which the counting kernel writes
-        to host memory, so its work until the next launch overlaps the emission instead of leaving
-        the device idle. If the counts fit, `counted.spec` holds the emitted buffers (emit() returns
-        views of them); otherwise emit() runs the emission again at the exact size (the queued one
-        writes nothing when the counts exceed its capacities)."""
+    def _extract(self, grid, deform, iso, flags, verts=None, faces=None, vinfo=None):
+        """diso_extract: the counting pass, and behind it the emission into the given buffers (none: no
+        emission). Waits only for the counts, which the counting kernel writes to host memory."""
         dims = tuple(grid.shape)
         dev = grid.device
-        key = (dev.index, dims, flags)
-        guess = self._guess.get(key)
         nseg = self._sizes(dims, flags)[0]
         seg = torch.empty(nseg, dtype=torch.uint8, device=dev)
         stream = _stream(dev)
         ctl = self.ctl_for(dev, dims, flags, stream=stream)
-        dmc = self.algo == _lib.DMC
-        vcap = fcap = 0
-        verts = faces = vinfo = None
-        if guess is not None:
+        tot = _lib.Totals()
+        vp, vcap, fp, fcap, ip = 0, 0, 0, 0, 0
+        if verts is not None:
+            vp, vcap, fp, fcap = verts.data_ptr(), verts.shape[0], faces.data_ptr(), faces.shape[0]
+            ip = 0 if vinfo is None else vinfo.data_ptr()
+        rc = _lib.lib().diso_extract(self.algo, self.code, grid.data_ptr(), 0 if deform is None else deform.data_ptr(),
+                                     *dims, iso, flags, seg.data_ptr(), nseg, ctl.data_ptr(), ctl.numel(), vp, vcap, fp,
+                                     fcap, ip, tot, stream)
+        _lib.check(rc, "extraction")
+        return Counted(seg, tot, dims, iso, flags)
+
+    def count(self, grid, iso, flags):
+        """The counting pass alone."""
+        return self._extract(grid, None, float(iso), flags)
+
+    def count_speculative(self, grid, deform, iso, flags):
+        """The counting pass, and, when an earlier call on a grid of these dims gives a size
+        estimate, the emission queued right behind it into buffers of that size plus a margin: the
+        host then waits only for the counts, so its work until the next launch overlaps the emission
+        instead of leaving the device idle. If the counts fit, `counted.spec` holds the emitted
+        buffers (emit() returns views of them); otherwise emit() runs the emission again at the exact
+        size (the queued one writes nothing when the counts exceed its capacities)."""
+        dev = grid.device
+        key = (dev.index, tuple(grid.shape), flags)
+        guess = self._guess.get(key)
+        if guess is None:
+            counted = self.count(grid, iso, flags)
+        else:
+            dmc = self.algo == _lib.DMC
             vcap, fcap = guess[0] + guess[0] // 4 + 1024, guess[1] + guess[1] // 4 + 1024
             verts = torch.empty((vcap, 3), dtype=self.dtype, device=dev)
             faces = torch.empty((fcap, 4 if dmc else 3),
                                 dtype=torch.int64 if flags & _lib.FLAG_INDEX64 else torch.int32, device=dev)
             vinfo = torch.empty(vcap, dtype=torch.uint8, device=dev) if dmc else None
-        tot = _lib.Totals()
-        rc = _lib.lib().diso_extract(self.algo, self.code, grid.data_ptr(), 0 if deform is None else deform.data_ptr(),
-                                     *dims, iso, flags, seg.data_ptr(), nseg, ctl.data_ptr(), ctl.numel(),
-                                     0 if verts is None else verts.data_ptr(), vcap,
-                                     0 if faces is None else faces.data_ptr(), fcap,
-                                     0 if vinfo is None else vinfo.data_ptr(), tot, stream)
-        _lib.check(rc, "extraction")
-        counted = Counted(seg, tot, dims, iso, flags)
-        if verts is not None and tot.n_verts <= vcap and tot.n_faces <= fcap:
-            counted.spec = (verts, faces, vinfo)
-        self._remember(key, tot.n_verts, tot.n_faces)
+            counted = self._extract(grid, deform, iso, flags, verts, faces, vinfo)
+            if counted.n_verts <= vcap and counted.n_faces <= fcap:
+                counted.spec = (verts, faces, vinfo)
+        self._remember(key, counted.n_verts, counted.n_faces)
         return counted
 
     def _remember(self, key, n_verts, n_faces):

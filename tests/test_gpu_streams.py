@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import diso_amd
+import diso_amd._C  # noqa: F401
 from diso_amd import _lib
 from tests.helpers import check_against_oracle, inputs
 
@@ -104,12 +105,17 @@ def test_a_long_wait_does_not_hold_a_core():
     assert own < 0.3 * wall, (own, wall)
 
 
-def test_first_forward_takes_written_totals(monkeypatch):
-    """A module's first forward on a size has no estimate to emit with, but waits for its totals as later
-    ones do: no copy, no stream synchronisation (which made first calls slower than later ones)."""
+def test_forwards_take_written_totals(monkeypatch):
+    """A module's first forward on a size has no estimate to emit with, and the binding classes never
+    have one, but all wait for their totals as later forwards do: no copy, no stream synchronisation
+    (which made them slower than before the count became two launches)."""
     print("case first forward", flush=True)
     sdf = _grids(1, (12, 13, 14), 90)[0]
-    monkeypatch.setattr(diso_amd.engine.Extractor, "count", None)  # the pass that copies and synchronises
+
+    def refuse(*args):  # the pass that copies and synchronises
+        raise AssertionError("diso_count called")
+
+    monkeypatch.setattr(_lib.lib(), "diso_count", refuse)
     for algo, make, kw in (("mc", diso_amd.DiffMC, {}), ("dmc", diso_amd.DiffDMC, {"return_quads": True})):
         for recompute in (False, True):
             mod = make(recompute_backward=recompute)
@@ -120,3 +126,9 @@ def test_first_forward_takes_written_totals(monkeypatch):
         for _ in range(2):
             assert empty(torch.ones_like(sdf), **kw)[0].shape == (0, 3)
             assert empty(torch.ones((1, 1, 1), device=DEV), **kw)[0].shape == (0, 3)
+    padded = torch.nn.functional.pad(sdf, (1,) * 6, value=1.0)
+    for algo, cls in (("mc", diso_amd._C.CUMCFloat), ("dmc", diso_amd._C.CUDMCFloat)):
+        v, f = cls().forward(padded, 0.0)
+        w, g = (diso_amd.DiffMC()(sdf, normalize=False) if algo == "mc" else
+                diso_amd.DiffDMC()(sdf, normalize=False, return_quads=True))
+        assert torch.equal(v - 1, w) and torch.equal(f.long(), g)
