@@ -88,6 +88,7 @@ class Extractor:
         self._first = {}  # device -> the first of them, for captures
         self._guess = {}  # (device, dims, flags) -> (vertices, faces) of the last call
         self._need = {}  # (dims, flags) -> workspace bytes (_sizes)
+        self._at = {}  # (dims, flags) -> offset of the totals (_totals_at)
         _lib.lib()  # fail loudly now if the HIP library is not there
 
     def check_grid(self, grid, name="grid"):
@@ -113,6 +114,18 @@ class Extractor:
             if len(self._need) >= 256:
                 self._need.clear()
             self._need[key] = got
+        return got
+
+    def _totals_at(self, dims, flags):
+        """Offset of the totals in the segment workspace (asked once per dims and flags)."""
+        got = self._at.get((dims, flags))
+        if got is None:
+            got = _lib.lib().diso_totals_offset(*dims, flags)
+            if got < 0:
+                _lib.check(got, "workspace sizing")
+            if len(self._at) >= 256:
+                self._at.clear()
+            self._at[(dims, flags)] = got
         return got
 
     def ctl_for(self, device, dims, flags, capturing=False, stream=None):

@@ -38,15 +38,13 @@ class _FixedExtract(torch.autograd.Function):
         L = _lib.lib()
         ex = fx.ex
         dev = grid.device
-        dims = tuple(int(d) for d in grid.shape)
+        dims = tuple(grid.shape)
         dmc = ex.algo == _lib.DMC
-        nseg = L.diso_seg_bytes(*dims, flags & ~_lib.FLAG_RECOMPUTE)
-        off = L.diso_totals_offset(*dims, flags)
-        if nseg < 0 or off < 0:
-            _lib.check(min(nseg, off), "workspace sizing")
+        nseg, kept, _ = ex._sizes(dims, flags)
+        off = ex._totals_at(dims, flags)
         seg = torch.empty(nseg, dtype=torch.uint8, device=dev)
-        ctl = ex.ctl_for(dev, dims, flags, _capturing())
         st = _stream(dev)
+        ctl = ex.ctl_for(dev, dims, flags, _capturing(), st)
         rc = L.diso_count(ex.algo, ex.code, _ptr(grid), *dims, iso, flags, _ptr(seg), nseg, _ptr(ctl), ctl.numel(),
                           None, st)
         _lib.check(rc, "count pass")
@@ -60,7 +58,7 @@ class _FixedExtract(torch.autograd.Function):
         tot = seg[off:off + 32].view(torch.int64)  # (crossing edges, MC triangles | DMC vertices, flags, algo)
         counts = torch.stack([tot[1], tot[0], tot[2]]) if dmc else tot[:3].clone()
         if flags & _lib.FLAG_RECOMPUTE:
-            seg = seg[:L.diso_seg_bytes(*dims, flags)].clone()  # the bases (and totals) only
+            seg = seg[:kept].clone()  # the bases (and totals) only
         ctx.fx, ctx.iso, ctx.flags, ctx.dims, ctx.seg = fx, iso, flags, dims, seg
         ctx.save_for_backward(grid, deform, faces if dmc else None, vinfo if dmc else None)
         ctx.mark_non_differentiable(faces, counts)
