@@ -116,7 +116,8 @@ DISO_BITS_HD int popc64(uint64_t v) {
 DISO_BITS_HD uint64_t low_bits(int n) { return n >= 64 ? ~0ull : (n <= 0 ? 0ull : ((1ull << n) - 1)); }
 
 // 8 bytes b[i] (i = plane) of eight positions each, to 8 codes (byte j = position j, bit i = plane
-// i): an 8 x 8 bit transpose in two 32-bit halves (planes 0-3, planes 4-7).
+// i): an 8 x 8 bit transpose in two 32-bit halves (planes 0-3, planes 4-7), by exchanging blocks of
+// 1, 2 and 4 bits (H. S. Warren, Hacker's Delight, "Transposing a bit matrix").
 DISO_BITS_HD void transpose8(uint32_t &lo, uint32_t &hi) {
     uint32_t t;
     t = (lo ^ (lo >> 7)) & 0x00AA00AAu;

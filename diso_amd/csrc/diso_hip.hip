@@ -417,11 +417,11 @@ __device__ __forceinline__ int find_group(const int64_t *__restrict__ rf, int m,
 // segment counts in the same launch.
 //
 // The scan (single pass). The segments are split into G contiguous ranges, one per block. A block
-// counts its segments (writing each segment's planes, and its counts into `seg`), publishes its
-// aggregate as one self-contained 64-bit word, reads the aggregates of all its predecessors in
-// parallel (a look-back over the whole window at once: no chain of inclusive prefixes, so the wait
-// is one memory latency rather than one per predecessor), and finally scans its own segment counts
-// into segment bases. Aggregate words are accessed with agent-scope
+// counts its segments (writing each segment's planes, and keeping its counts), publishes its
+// aggregate as two 64-bit words, each with the call's tag, so that a reader takes them only when both
+// are this call's, reads the aggregates of all its predecessors in parallel (a look-back over the whole
+// window at once: no chain of inclusive prefixes, so the wait is one memory latency rather than one per
+// predecessor), and finally scans its own segment counts into segment bases. Aggregate words are accessed with agent-scope
 // atomics only, so they are coherent across the XCDs' L2s without fences. Two word buffers
 // alternate between calls; each call clears the one the next call uses (up to the extent that
 // was written), and the last block advances the epoch once every block has published (and so has

@@ -1,8 +1,8 @@
 // diso_scan_word.h - aggregate words of the single-pass scan's control block.
 //
-// The control block holds a header (an epoch counter) and two buffers of 64-bit words, one word
+// The control block holds a header (an epoch counter) and two buffers of 64-bit words, two words
 // per count block. Call number `epoch` uses buffer (epoch & 1): every block publishes its
-// aggregate there, tagged with tag(epoch) = 1 + epoch % 3, and reads its predecessors' words from
+// aggregate there, both words tagged with tag(epoch) = 1 + epoch % 3, and reads its predecessors' words from
 // it; it clears its share of the other buffer for the next call; the call's last block advances
 // the epoch. A word counts as published for a call only when its tag is that call's tag, so a
 // word written late by a block of an earlier call (one whose last block gave up waiting for it)

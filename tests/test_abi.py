@@ -35,7 +35,7 @@ def test_workspace_sizes():
     n = 256
     seg = L.diso_seg_bytes(n, n, n, _lib.FLAG_VIRTUAL_PAD)
     # one 16-byte base per (row, 64-wide z chunk) of the padded grid, plus two totals entries, then
-    # one 16-bit classification word per lane of every segment
+    # two bytes of classification per position of every segment
     nseg = (n + 2) * (n + 2) * ((n + 2 + 63) // 64)
     assert seg == (nseg + 2) * 16 + nseg * 64 * 2
     # a recompute-classification backward keeps only the bases
