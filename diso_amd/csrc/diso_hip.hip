@@ -3512,6 +3512,13 @@ int diso_extract(int algo, int dtype, const void *sdf, const void *deform, int64
     if ((vert_capacity && !verts) || (face_capacity && !faces)) return fail(DISO_E_INVALID, "null output buffer");
     if (algo == DISO_DMC && vert_capacity && !vinfo) return fail(DISO_E_INVALID, "DMC needs a vinfo buffer");
     hipStream_t st = (hipStream_t)stream;
+    if (st) {  // (the null stream cannot be captured) a captured count would never write what is waited for
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        rc = check_hip(hipStreamIsCapturing(st, &cap), "capture status");
+        if (rc) return rc;
+        if (cap != hipStreamCaptureStatusNone)
+            return fail(DISO_E_INVALID, "the stream is being captured: the totals cannot be waited for");
+    }
     Landing &land = landing();
     if (!land.host) return fail(DISO_E_HIP, "pinned allocation failed");
     const uint64_t seq = ++land.seq;

@@ -132,3 +132,30 @@ def test_forwards_take_written_totals(monkeypatch):
         w, g = (diso_amd.DiffMC()(sdf, normalize=False) if algo == "mc" else
                 diso_amd.DiffDMC()(sdf, normalize=False, return_quads=True))
         assert torch.equal(v - 1, w) and torch.equal(f.long(), g)
+
+
+@pytest.mark.parametrize("known", [False, True])
+def test_a_capture_refuses_to_wait(known):
+    """A module's forward waits for its totals, so it is refused while its stream is captured, at once and
+    before anything is recorded; the module works on afterwards."""
+    print(f"case capture known={known}", flush=True)
+    sdf = _grids(1, (20, 21, 22), 95)[0]
+    want = diso_amd.DiffDMC()(sdf, return_quads=True)
+    mod = diso_amd.DiffDMC()
+    if known:
+        mod(sdf, return_quads=True)
+    torch.cuda.synchronize()
+    x = torch.ones(8, device=DEV)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x.add_(1)
+        with pytest.raises(RuntimeError, match="captured"):
+            mod(sdf, return_quads=True)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert (x == 2).all()
+    for stream in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(stream):
+            v, f = mod(sdf, return_quads=True)
+            stream.synchronize()
+        assert torch.equal(v, want[0]) and torch.equal(f, want[1])
