@@ -143,10 +143,11 @@ int diso_emit(int algo, int dtype, const void *sdf, const void *deform, int64_t 
  * suffice (an estimate from an earlier grid): enqueues diso_count and diso_emit and returns as soon
  * as the totals are known, which the counting pass writes to host memory itself, while the emission
  * may still run. If the totals exceed the capacities nothing has been written: call diso_emit with
- * larger buffers. With both capacities zero (no estimate yet) only the totals are taken. The reference reads its counts back with three blocking copies (src/cumc.cu:651-723).
- * The host waits, so a stream that is being captured is refused (DISO_E_INVALID). On return the counting pass may still be
- * using `ctl` (and the emission `seg`): their next use must be ordered after it, on the same stream
- * or by an event. */
+ * larger buffers. With both capacities zero (no estimate yet) only the totals are taken. The
+ * reference reads its counts back with three blocking copies (src/cumc.cu:651-723).
+ * The host waits, so a stream that is being captured is refused (DISO_E_INVALID). On return the
+ * counting pass may still be using `ctl` (and the emission `seg`): their next use must be ordered
+ * after it, on the same stream or by an event. */
 int diso_extract(int algo, int dtype, const void *sdf, const void *deform, int64_t X, int64_t Y,
                  int64_t Z, double iso, int flags, void *seg, int64_t seg_bytes, void *ctl,
                  int64_t ctl_bytes, void *verts, int64_t vert_capacity, void *faces,
