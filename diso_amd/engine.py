@@ -162,10 +162,12 @@ class Extractor:
         emission). Waits only for the counts, which the counting kernel writes to host memory."""
         dims = tuple(grid.shape)
         dev = grid.device
-        nseg = self._sizes(dims, flags)[0]
+        nseg, _, need = self._sizes(dims, flags)
         seg = torch.empty(nseg, dtype=torch.uint8, device=dev)
         stream = _stream(dev)
-        ctl = self.ctl_for(dev, dims, flags, stream=stream)
+        ctl = self._ctl.get((dev.index, stream.value))
+        if ctl is None or ctl.numel() < need:
+            ctl = self.ctl_for(dev, dims, flags, stream=stream)
         tot = _lib.Totals()
         vp, vcap, fp, fcap, ip = 0, 0, 0, 0, 0
         if verts is not None:
